@@ -324,6 +324,8 @@ int mdattn_fwd_fp8_bias(void* stream, const void* q8, const void* k8, const void
  *   lse          f32 [B,H,Sq] as written by the forward
  *   workspace    f32 device buffer of at least mdattn_bwd_workspace_floats(B,H,Sq) elements, 16-byte aligned;
  *                scratch of the call (per padded q row: -lse in log2 units and -rowsum(dout*out)), nothing to keep
+ *                A larger workspace lets a pass with few rows of its own be split over the other sequence (partial
+ *                gradients in f32, summed in a fixed order; same result up to f32 summation order)
  * Two passes, no atomics: dq; then dk and dv together.  When scale * log2(e) == 1 (the caller's q carries the softmax
  * scale, as for the forward) the logits need no multiply; dq is then the gradient for the q that was passed.
  * Requires D == 128 or D == 64 (LTX-2's audio stream); sequence strides below 2^23 elements and

@@ -59,6 +59,11 @@ SIGNATURES = {
     "mdattn_finalize": ([_P, _P, _P, _L], _I),
 }
 
+# what csrc/mdattn_host.h declares: entry points for this package's own host side
+HOST_SIGNATURES = {
+    "mdattn_bwd_split_workspace_floats": ([_I, _I, _I, _I, _I], _L),
+}
+
 _lib = None
 
 
@@ -71,7 +76,7 @@ def load() -> ctypes.CDLL:
           f"{LIB_PATH} is missing: build it with `python -m maxdiffusion_amd.build` "
           "(there is no non-HIP fallback for this path)")
     lib = ctypes.CDLL(LIB_PATH)
-    for name, (argtypes, restype) in SIGNATURES.items():
+    for name, (argtypes, restype) in {**SIGNATURES, **HOST_SIGNATURES}.items():
       fn = getattr(lib, name)
       fn.argtypes = argtypes
       fn.restype = restype

@@ -26,6 +26,7 @@
 #include <mutex>
 
 #include "mdattn_common.h"
+#include "mdattn_host.h"
 
 namespace mdattn {
 namespace {
@@ -91,6 +92,11 @@ struct BwdArgs {
   float c, scale;
   const float* bias;   // BIAS: additive per-key bias [B, bias_sb] in natural-log units (mdattn_fwd_bf16_bias)
   int64_t bias_sb;
+  // stream split: the tiles of the stream are dealt to nsplit workgroups per entity tile, tps tiles each; with nsplit > 1
+  // a workgroup leaves f32 partial sums [split][B*H][Se][HD] (part: out's, part2: out2's) for bwd_reduce_kernel
+  int nsplit, tps;
+  float* part;
+  float* part2;
 };
 
 // MODE 0: dq (entity = q rows, stream = keys); 3: dk and dv in one pass (entity = key rows, stream = q rows).
@@ -133,10 +139,15 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   const int wg = blockIdx.x;
   const int w = (wg & 7) * a.chunk + (wg >> 3);
   if (w >= a.total) return;
-  const int bh = w / a.net, et = w - bh * a.net;
+  // entity tiles fastest: neighbouring workgroups walk the same piece of the stream
+  const int bhs = w / a.net, et = w - bhs * a.net;
+  const int bh = bhs / a.nsplit, sp = bhs - bh * a.nsplit;
   const int b = bh / a.H, h = bh - b * a.H;
   const int r0 = et * (NW * 32) + wave * 32;
-  const int nt = (a.Ss + kBT - 1) / kBT;
+  // this workgroup's stream: rows ss0 .. ss0 + Ss - 1 of the sequence (never empty); everything below counts from ss0
+  const int ss0 = sp * a.tps * kBT;
+  const int Ss = a.Ss - ss0 < a.tps * kBT ? a.Ss - ss0 : a.tps * kBT;
+  const int nt = (Ss + kBT - 1) / kBT;
   const float c = a.c;
 
   // ---- entity fragments
@@ -153,23 +164,23 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       for (int s = 0; s < NJ; ++s) ef2[s] = *reinterpret_cast<const bf16x8*>(p2 + s * 16);
     }
   }
-  const float* lrow = a.lse2 + ((int64_t)b * a.H + h) * a.Sp;
-  const float* drow = a.delta + ((int64_t)b * a.H + h) * a.Sp;
+  const float* lrow = a.lse2 + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
+  const float* drow = a.delta + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
   float nlse_e = 0.f, ndelta_e = 0.f;  // the workspace holds both negated
   if constexpr (MODE == 0) {
     nlse_e = lrow[erow];
     ndelta_e = drow[erow];
   }
   // key bias in log2 units: a per-lane scalar when the keys are the entity rows, sixteen values per tile otherwise
-  [[maybe_unused]] const float* bias_row = BIAS ? a.bias + b * a.bias_sb : nullptr;
+  [[maybe_unused]] const float* bias_row = BIAS ? a.bias + b * a.bias_sb + (MODE == 0 ? ss0 : 0) : nullptr;
   [[maybe_unused]] float bias_e = 0.f;
   if constexpr (BIAS && MODE != 0) bias_e = bias_row[erow] * kLog2e;
 
   // ---- direct global -> LDS loads of one stream tile (layouts and lane maps of the forward kernel)
-  const __bf16* s1p = a.s1 + b * a.s1_sb + h * a.s1_sh;
-  const __bf16* s2p = HAS2 ? a.s2 + b * a.s2_sb + h * a.s2_sh : nullptr;
-  const __bf16* s3p = a.s3 + b * a.s3_sb + h * a.s3_sh;
-  [[maybe_unused]] const __bf16* s4p = BOTH ? a.s4 + b * a.s4_sb + h * a.s4_sh : nullptr;
+  const __bf16* s1p = a.s1 + b * a.s1_sb + h * a.s1_sh + ss0 * a.s1_ss;
+  const __bf16* s2p = HAS2 ? a.s2 + b * a.s2_sb + h * a.s2_sh + ss0 * a.s2_ss : nullptr;
+  const __bf16* s3p = a.s3 + b * a.s3_sb + h * a.s3_sh + ss0 * a.s3_ss;
+  [[maybe_unused]] const __bf16* s4p = BOTH ? a.s4 + b * a.s4_sb + h * a.s4_sh + ss0 * a.s4_ss : nullptr;
   constexpr int RPI = L::RPI;
   const int grow = HD == 128 ? lane >> 4 : lane >> 3;
   // lane -> logical 16-byte chunk stored at this lane's position (a wave fills the row groups wave, wave + NW, ...)
@@ -210,7 +221,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         lds_dma4((MODE != 0 ? lrow : bias_row) + t * kBT, oa, A1 + kBAux * 2u);
       }
     }
-    if (t * kBT + kBT <= a.Ss) {  // a full tile: uniform row-group bases, one per-lane offset per stream
+    if (t * kBT + kBT <= Ss) {  // a full tile: uniform row-group bases, one per-lane offset per stream
       unsigned o1 = ofs1, o2 = ofs2, o3 = ofs3, o4 = ofs4;
       if constexpr (REFORM) {
         int ln = lane;
@@ -234,7 +245,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       for (int i = 0; i < (kBT / RPI) / NW; ++i) {
         const int g = wave + NW * i;
         int rr = t * kBT + RPI * g + grow;
-        rr = rr < a.Ss ? rr : a.Ss - 1;
+        rr = rr < Ss ? rr : Ss - 1;
         lds_dma16(s1p + (int64_t)rr * a.s1_ss + acol, A1 + (unsigned)(g * kBGK) * 2u);
         if constexpr (HAS2) lds_dma16(s2p + (int64_t)rr * a.s2_ss + acol, A2 + (unsigned)(g * kBGK) * 2u);
         lds_dma16(s3p + (int64_t)rr * a.s3_ss + bcol, Bt + (unsigned)(g * kBGV) * 2u);
@@ -350,7 +361,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         const int sbase = t * kBT + 4 * hh;
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          if (sbase + 8 * (i >> 2) + (i & 3) >= a.Ss) S[i] = -INFINITY;
+          if (sbase + 8 * (i >> 2) + (i & 3) >= Ss) S[i] = -INFINITY;
       }
     }
     bf16x8 W[2];
@@ -369,7 +380,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
               const f32x4 bv = *reinterpret_cast<const f32x4*>(aux + 8 * (2 * hb + g) + 4 * hh);
 #pragma unroll
               for (int e = 0; e < 4; ++e)
-                nl[4 * g + e] = col + e < a.Ss ? __builtin_fmaf(bv[e], kLog2e, nlse_e) : -INFINITY;  // whatever the padding holds
+                nl[4 * g + e] = col + e < Ss ? __builtin_fmaf(bv[e], kLog2e, nlse_e) : -INFINITY;  // whatever the padding holds
             }
           }
         } else {
@@ -432,6 +443,23 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 
   const int row = r0 + l32;
   const float osc = HAS2 ? a.scale : 1.0f;  // dq = scale * dS k, dk = scale * dS^T q
+  if (a.nsplit > 1) {  // partial sums over this workgroup's share of the stream, in f32
+    if (row < a.Se) {
+      const int64_t nbh = a.total / (a.net * a.nsplit);
+      const int64_t o = (((int64_t)sp * nbh + bh) * a.Se + row) * HD + 4 * hh;
+#pragma unroll
+      for (int db = 0; db < ND; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          *reinterpret_cast<f32x4*>(a.part + o + db * 32 + 8 * g) =
+              f32x4{acc[db][4 * g] * osc, acc[db][4 * g + 1] * osc, acc[db][4 * g + 2] * osc, acc[db][4 * g + 3] * osc};
+          if constexpr (BOTH)
+            *reinterpret_cast<f32x4*>(a.part2 + o + db * 32 + 8 * g) =
+                f32x4{acc2[db][4 * g], acc2[db][4 * g + 1], acc2[db][4 * g + 2], acc2[db][4 * g + 3]};
+        }
+    }
+    return;
+  }
   if (row < a.Se) {
     __bf16* orow = a.out + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_ss + 4 * hh;
 #pragma unroll
@@ -502,12 +530,70 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const __bf16* out, const 
   }
 }
 
+// Sums the partial gradients of a split pass in the order of the splits and rounds them to bf16: one 16-byte store per
+// lane, blockIdx.y = tensor.  Bound by the partials' bytes: 12.8 us for 63 MB (4.9 TB/s).
+struct BwdReduceArgs {
+  const float* part[2];
+  __bf16* out[2];
+  int64_t sb[2], ss[2], sh[2];
+  int H, S, nsplit;
+  int64_t chunks;  // B*H*S*HD/8
+};
+template <int HD>
+__global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.chunks) return;
+  const int t = blockIdx.y;
+  constexpr int CPR = HD / 8;
+  const int c = (int)(i % CPR);
+  const int64_t row = i / CPR;
+  const int s = (int)(row % a.S);
+  const int64_t bh = row / a.S;
+  const int64_t b = bh / a.H, h = bh - b * a.H;
+  const float4* p = reinterpret_cast<const float4*>(a.part[t]) + 2 * i;
+  float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < a.nsplit; ++k, p += 2 * a.chunks) {
+    const float4 u = ld_nt(p), v = ld_nt(p + 1);
+    f[0] += u.x; f[1] += u.y; f[2] += u.z; f[3] += u.w; f[4] += v.x; f[5] += v.y; f[6] += v.z; f[7] += v.w;
+  }
+  *reinterpret_cast<uint4*>(a.out[t] + b * a.sb[t] + (int64_t)s * a.ss[t] + h * a.sh[t] + c * 8) = pack8(f);
+}
+
+// Into how many pieces a pass cuts its stream.  A pass has one workgroup per (batch, head, entity tile); cross-attention's
+// dk / dv pass (512 keys: two tiles per head) would leave most of the chip idle while each workgroup walks every query
+// row.  The cost of n pieces, in tiles: rounds of workgroups times (tiles per workgroup + 2 for a workgroup's start), the
+// write and read-back of n f32 partials, and the launch that sums them.  12 heads x 32,760 queries x 512 keys: the dk / dv
+// pass takes 1312 us in one piece (24 workgroups) and 201 us in ten, + 13 us of bwd_reduce_kernel.  Pieces under 16
+// tiles (512 rows) spend as long starting and writing partials as walking.
+constexpr int kMinSplitTiles = 16, kMaxSplit = 32;
+struct BwdSplit {
+  int nsplit, tps;
+  int64_t floats;  // of one tensor's partials
+};
+// entity rows Se, stream rows Ss; tensors: gradients the pass produces (2 in the dk / dv pass)
+inline BwdSplit bwd_split(int64_t BH, int Se, int Ss, int D, int tensors) {
+  const int rows = D == 128 ? bwd_waves<128>() * 32 : bwd_waves<64>() * 32;
+  const int slots = D == 128 ? 256 : 3 * 256;              // workgroups the chip holds at once
+  const double tile_us = tensors == 2 ? 1.7 : 1.2;         // a workgroup's time per stream tile
+  const int64_t entities = BH * ((Se + rows - 1) / rows), floats = BH * Se * D;
+  const double partial = 2.0 * tensors * (double)floats * 4 / 5e6 / tile_us;  // written and read at 5 TB/s
+  const int nt = (Ss + kBT - 1) / kBT;
+  BwdSplit best{1, nt, 0};
+  double best_cost = (double)((entities + slots - 1) / slots) * (nt + 2);
+  for (int n = 2; n <= kMaxSplit && nt / n >= kMinSplitTiles; ++n) {
+    const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
+    const double cost = (double)((entities * ns + slots - 1) / slots) * (tps + 2) + partial * ns + 5.0 / tile_us;
+    if (cost < best_cost * 0.95) { best_cost = cost; best = {ns, tps, ns * floats}; }
+  }
+  return best;
+}
+
 template <int MODE, int HD, bool BIAS, bool PRE>
 int launch_bwd_as(hipStream_t st, BwdArgs a, int B) {
   constexpr int lds_bytes = 2 * bwd_slot_elems<MODE, HD, BIAS>() * 2;
   constexpr int NW = bwd_waves<HD>();
   a.net = (a.Se + NW * 32 - 1) / (NW * 32);
-  const int64_t total = (int64_t)B * a.H * a.net;
+  const int64_t total = (int64_t)B * a.H * a.net * a.nsplit;
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
@@ -538,6 +624,20 @@ int launch_bwd_any(hipStream_t st, const BwdArgs& a, int B, int D) {
   return a.bias ? launch_bwd<MODE, 64, true>(st, a, B) : launch_bwd<MODE, 64, false>(st, a, B);
 }
 
+int launch_bwd_reduce(hipStream_t st, const BwdArgs& a, int B, int D) {
+  BwdReduceArgs r;
+  r.part[0] = a.part; r.part[1] = a.part2;
+  r.out[0] = a.out; r.out[1] = a.part2 ? a.out2 : nullptr;
+  r.sb[0] = a.o_sb; r.ss[0] = a.o_ss; r.sh[0] = a.o_sh;
+  r.sb[1] = a.o2_sb; r.ss[1] = a.o2_ss; r.sh[1] = a.o2_sh;
+  r.H = a.H; r.S = a.Se; r.nsplit = a.nsplit;
+  r.chunks = (int64_t)B * a.H * a.Se * (D / 8);
+  const dim3 grid((unsigned)((r.chunks + 255) / 256), a.part2 ? 2 : 1);
+  if (D == 128) MDATTN_LAUNCH(bwd_reduce_kernel<128>, grid, dim3(256), 0, st, r);
+  else MDATTN_LAUNCH(bwd_reduce_kernel<64>, grid, dim3(256), 0, st, r);
+  return launch_status();
+}
+
 }  // namespace
 }  // namespace mdattn
 
@@ -546,6 +646,12 @@ using namespace mdattn;
 extern "C" int64_t mdattn_bwd_workspace_floats(int B, int H, int Sq) {
   if (B <= 0 || H <= 0 || Sq <= 0) return 0;
   return 2 * (int64_t)B * H * (((int64_t)Sq + 31) / 32 * 32);
+}
+
+extern "C" int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || (D != 128 && D != 64)) return 0;
+  const int64_t BH = (int64_t)B * H;
+  return mdattn_bwd_workspace_floats(B, H, Sq) + bwd_split(BH, Sq, Skv, D, 1).floats + 2 * bwd_split(BH, Skv, Sq, D, 2).floats;
 }
 
 // Shared body of mdattn_bwd_bf16 and mdattn_bwd_bf16_static: validation, the preparation kernel and the two passes.
@@ -584,6 +690,13 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
                      (const __bf16*)dout, lse, lse2, delta, H, Sq, Sp, D, rows, o_strides->batch, o_strides->seq, o_strides->head);
   if (launch_status() != MDATTN_OK) return MDATTN_E_LAUNCH;
 
+  // stream splits, when the caller's workspace holds their partials (it always holds lse2 and delta)
+  const int64_t BH = (int64_t)B * H;
+  BwdSplit sq = bwd_split(BH, Sq, Skv, D, 1), skv = bwd_split(BH, Skv, Sq, D, 2);
+  if (workspace_floats < 2 * rows + sq.floats + 2 * skv.floats) {
+    sq = {1, (Skv + kBT - 1) / kBT, 0};
+    skv = {1, (Sq + kBT - 1) / kBT, 0};
+  }
   BwdArgs a;
   a.lse2 = lse2; a.delta = delta; a.H = H; a.Sp = Sp; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;
@@ -594,8 +707,10 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.e1_sb, a.e1_ss, a.e1_sh, q_strides); set(a.e2_sb, a.e2_ss, a.e2_sh, o_strides);
   set(a.s1_sb, a.s1_ss, a.s1_sh, k_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, v_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, k_strides);
   set(a.o_sb, a.o_ss, a.o_sh, q_strides);
+  a.nsplit = sq.nsplit; a.tps = sq.tps; a.part = workspace + 2 * rows; a.part2 = nullptr;
   int rc = launch_bwd_any<0>(st, a, B, D);
   if (rc != MDATTN_OK) return rc;
+  if (sq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B, D)) != MDATTN_OK) return rc;
   // dk and dv in one pass: entity k / v, stream q (scores, and accumulate for dk), dout (dP, and accumulate for dv)
   a.e1 = (const __bf16*)k; a.e2 = (const __bf16*)v; a.s1 = (const __bf16*)q; a.s2 = (const __bf16*)dout; a.s3 = (const __bf16*)q;
   a.s4 = (const __bf16*)dout;
@@ -604,7 +719,10 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.s1_sb, a.s1_ss, a.s1_sh, q_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, o_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, q_strides);
   set(a.s4_sb, a.s4_ss, a.s4_sh, o_strides);
   set(a.o_sb, a.o_ss, a.o_sh, k_strides); set(a.o2_sb, a.o2_ss, a.o2_sh, v_strides);
-  return launch_bwd_any<3>(st, a, B, D);
+  a.nsplit = skv.nsplit; a.tps = skv.tps; a.part = workspace + 2 * rows + sq.floats; a.part2 = a.part + skv.floats;
+  rc = launch_bwd_any<3>(st, a, B, D);
+  if (rc == MDATTN_OK && skv.nsplit > 1) rc = launch_bwd_reduce(st, a, B, D);
+  return rc;
 }
 
 
@@ -680,6 +798,6 @@ extern "C" int mdattn_bwd_bf16_static(void* stream, const void* q, const void* k
   if (need > (int64_t)MDATTN_BWD_STATIC_MAX_FLOATS) return MDATTN_E_TOOBIG;
   float* ws = scratch_on_current_device();
   if (!ws) return MDATTN_E_LAUNCH;
-  return bwd_run((hipStream_t)stream, q, k, v, out, dout, lse, dq, dk, dv, ws, need, B, H, Sq, Skv, D,
+  return bwd_run((hipStream_t)stream, q, k, v, out, dout, lse, dq, dk, dv, ws, MDATTN_BWD_STATIC_MAX_FLOATS, B, H, Sq, Skv, D,
                  q_strides, k_strides, v_strides, o_strides, scale, nullptr, 0);
 }

@@ -394,7 +394,7 @@ def flash_attention_backward(q, k, v, out, dout, lse, scale: float | None = None
   if dq.stride() != q.stride() or dk.stride() != k.stride() or dv.stride() != v.stride():
     raise ValueError("q, k, v must be dense tensors (their gradients take the same strides)")
   lib = _lib.load()
-  nws = lib.mdattn_bwd_workspace_floats(b, h, sq)
+  nws = lib.mdattn_bwd_split_workspace_floats(b, h, sq, skv, d) or lib.mdattn_bwd_workspace_floats(b, h, sq)
   ws = torch.empty(nws, dtype=torch.float32, device=q.device)
   sq_, sk_, sv_, so_ = _strides(q), _strides(k), _strides(v), _strides(out)
   args = (_stream(), _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws), nws,

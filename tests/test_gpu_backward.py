@@ -298,3 +298,27 @@ def test_backward_over_kv_chunks_with_the_merged_lse(dev, D):
     rl = rel_l2(to_np(got.to(torch.bfloat16)), to_np(want))
     print(f"D={D} {name}: chunked vs unsplit rel-l2 {rl:.3e}", flush=True)
     assert rl <= 1e-2, name  # bf16 roundings of the merged out and of the partial dq
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("sq,skv,masked", [(2100, 63, False), (1025, 257, True), (33, 1999, False), (5, 1030, True)])
+def test_backward_split_over_the_other_sequence(dev, lib, D, sq, skv, masked):
+  """Few rows on one side, many on the other: the pass that owns the few is split over the many (uneven pieces, a ragged
+  last tile).  Bars of the unsplit passes: the partials are f32 and summed in a fixed order."""
+  B, H = 1, 2
+  assert lib.mdattn_bwd_split_workspace_floats(B, H, sq, skv, D) > lib.mdattn_bwd_workspace_floats(B, H, sq)
+  q, do = O.normal_bf16((B, sq, H, D), 0), O.normal_bf16((B, sq, H, D), 3)
+  k, v = O.normal_bf16((B, skv, H, D), 1), O.normal_bf16((B, skv, H, D), 2)
+  keep = np.ones((B, skv), bool)
+  keep[:, ::5] = not masked
+  qd, kd, vd, dod = (to_dev_bf16(x, dev) for x in (q, k, v, do))
+  bias = ops.key_mask_bias(torch.from_numpy(keep).to(dev)) if masked else None
+  out, lse = ops.flash_attention(qd, kd, vd, return_lse=True, key_bias=bias)
+  got = ops.flash_attention_backward(qd, kd, vd, out, dod, lse, key_bias=bias)
+  again = ops.flash_attention_backward(qd, kd, vd, out, dod, lse, key_bias=bias)
+  assert all(torch.equal(a, b) for a, b in zip(got, again))
+  rq, rk, rv = O.attention_bwd(hsd(q), hsd(k[:, keep[0]]), hsd(v[:, keep[0]]), hsd(do), D**-0.5)
+  dk, dv = to_np(got[1]), to_np(got[2])
+  assert not dk[:, ~keep[0]].any() and not dv[:, ~keep[0]].any()
+  for g, r, name in ((to_np(got[0]), rq, "dq"), (dk[:, keep[0]], rk, "dk"), (dv[:, keep[0]], rv, "dv")):
+    _check(hsd(g), r, f"{name} Sq={sq} Skv={skv} D={D} masked={masked}")
