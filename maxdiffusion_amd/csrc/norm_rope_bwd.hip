@@ -243,32 +243,47 @@ __global__ __launch_bounds__(512) void norm_rope_fullrow_bwd_kernel(NormRopeBwdF
   }
 }
 
-// Second stage: out[col] = sum over the nb partial rows, in a fixed order.  A workgroup covers 64 columns (16 lanes x
-// float4) with 16 row slices; the slices are combined through LDS.  Column col goes to outs[col / seglen][col % seglen].
+// Second stage: out[col] = sum over the nb partial rows, in a fixed order.  A workgroup covers 32 columns (8 lanes x
+// float4, one 128-byte line per row) with 128 row slices: with few columns (512 per-head, 1,536 at 12 heads) the launch is
+// a handful of workgroups and its time is the length of a lane's chain of loads, so the rows are spread over as many lanes
+// as a workgroup holds and eight loads are in flight per lane.  Against 64 columns x 16 slices of 256 lanes: 512 columns
+// 21.8 -> 4.7 us, 1,536 columns 17 -> 4.9 us, 10,240 columns 10.0 -> 5.4 us.  Slices are combined inside the wave, then
+// through LDS.  Column col goes to outs[col / seglen][col % seglen].
 struct ColsumArgs {
   const float* part;
   float* outs[4];
   int nb, ncols, seglen;
 };
 
-__global__ __launch_bounds__(256) void colsum_kernel(ColsumArgs a) {
-  const int tid = threadIdx.x, lane16 = tid & 15, slice = tid >> 4;
-  const int col = blockIdx.x * 64 + lane16 * 4;
-  __shared__ float4 sm[16][16];
+__global__ __launch_bounds__(1024) void colsum_kernel(ColsumArgs a) {
+  const int tid = threadIdx.x, lane8 = tid & 7, slice = tid >> 3;
+  const int col = blockIdx.x * 32 + lane8 * 4;
+  __shared__ float4 sm[16][8];
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [&](const float4& v) { acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w; };
   if (col < a.ncols) {
-    for (int r = slice; r < a.nb; r += 16) {
-      const float4 v = *reinterpret_cast<const float4*>(a.part + (int64_t)r * a.ncols + col);
-      acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+    const float* p = a.part + col;
+    int r = slice;
+    for (; r + 7 * 128 < a.nb; r += 8 * 128) {
+      float4 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float4*>(p + (int64_t)(r + j * 128) * a.ncols);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) add(v[j]);
     }
+#pragma unroll 4
+    for (; r < a.nb; r += 128) add(*reinterpret_cast<const float4*>(p + (int64_t)r * a.ncols));
   }
-  sm[slice][lane16] = acc;
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1)
+    add(make_float4(__shfl_xor(acc.x, o), __shfl_xor(acc.y, o), __shfl_xor(acc.z, o), __shfl_xor(acc.w, o)));
+  if ((tid & 63) < 8) sm[tid >> 6][lane8] = acc;
   __syncthreads();
-  if (slice == 0 && col < a.ncols) {
-    float4 tot = sm[0][lane16];
+  if (tid < 8 && col < a.ncols) {
+    float4 tot = sm[0][lane8];
 #pragma unroll
     for (int s = 1; s < 16; ++s) {
-      const float4 v = sm[s][lane16];
+      const float4 v = sm[s][lane8];
       tot.x += v.x; tot.y += v.y; tot.z += v.z; tot.w += v.w;
     }
     const int seg = col / a.seglen, i = col - seg * a.seglen;  // seglen % 4 == 0: a float4 never straddles segments
@@ -589,7 +604,7 @@ static int launch_colsum(hipStream_t st, const float* part, int nb, int ncols, i
   ColsumArgs c;
   c.part = part; c.nb = nb; c.ncols = ncols; c.seglen = seglen;
   c.outs[0] = o0; c.outs[1] = o1; c.outs[2] = o2; c.outs[3] = o3;
-  MDATTN_LAUNCH(colsum_kernel, dim3((ncols + 63) / 64), dim3(256), 0, st, c);
+  MDATTN_LAUNCH(colsum_kernel, dim3((ncols + 31) / 32), dim3(1024), 0, st, c);
   return launch_status();
 }
 
