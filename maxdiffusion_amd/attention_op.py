@@ -212,19 +212,19 @@ class _HipNormRopeFullrow(torch.autograd.Function):
   recomputed); the reference differentiates through these lines by JAX autodiff (attention_flax.py:2655-2677)."""
 
   @staticmethod
-  def forward(ctx, q, k, wq, wk, cos, sin, heads, eps, out_layout, q_mul):
-    q_out, k_out = ops.norm_rope_fullrow(q, k, wq, wk, cos, sin, heads, eps, out_layout, q_mul)
-    ctx.save_for_backward(q, k, wq, wk, cos, sin)
-    ctx.cfg = (heads, eps, q_mul)
+  def forward(ctx, q, k, wq, wk, table, heads, eps, out_layout, q_mul):
+    q_out, k_out = ops.norm_rope_fullrow(q, k, wq, wk, table, None, heads, eps, out_layout, q_mul)
+    ctx.save_for_backward(q, k, wq, wk, *_saved_table(table)[:2])
+    ctx.cfg = (heads, eps, q_mul, _saved_table(table)[2])
     return q_out, k_out
 
   @staticmethod
   def backward(ctx, gq, gk):
     q, k, wq, wk, cos, sin = ctx.saved_tensors
-    heads, eps, q_mul = ctx.cfg
-    dq, dk, dwq, dwk = ops.norm_rope_fullrow_backward(q, k, wq, wk, cos, sin, heads, gq.to(torch.bfloat16),
+    heads, eps, q_mul, kind = ctx.cfg
+    dq, dk, dwq, dwk = ops.norm_rope_fullrow_backward(q, k, wq, wk, ops.RopeTable(cos, sin, kind), None, heads, gq.to(torch.bfloat16),
                                                       gk.to(torch.bfloat16) if k is not None else None, eps, q_mul)
-    return dq, dk, dwq.to(wq.dtype), (dwk.to(wk.dtype) if k is not None else None), None, None, None, None, None, None
+    return dq, dk, dwq.to(wq.dtype), (dwk.to(wk.dtype) if k is not None else None), None, None, None, None, None
 
 
 class _HipNormRopeQkv(torch.autograd.Function):
@@ -233,47 +233,47 @@ class _HipNormRopeQkv(torch.autograd.Function):
   gradient (v only gains a bias, whose gradient is the token sum)."""
 
   @staticmethod
-  def forward(ctx, qkv, bias, wq, wk, cos, sin, heads, eps, out_layout, q_mul):
-    q_out, k_out, v_out = ops.norm_rope_qkv(qkv, wq, wk, cos, sin, heads, bias, eps, out_layout, q_mul)
-    ctx.save_for_backward(qkv, bias, wq, wk, cos, sin)
-    ctx.cfg = (heads, eps, q_mul)
+  def forward(ctx, qkv, bias, wq, wk, table, heads, eps, out_layout, q_mul):
+    q_out, k_out, v_out = ops.norm_rope_qkv(qkv, wq, wk, table, None, heads, bias, eps, out_layout, q_mul)
+    ctx.save_for_backward(qkv, bias, wq, wk, *_saved_table(table)[:2])
+    ctx.cfg = (heads, eps, q_mul, _saved_table(table)[2])
     return q_out, k_out, v_out
 
   @staticmethod
   def backward(ctx, gq, gk, gv):
     qkv, bias, wq, wk, cos, sin = ctx.saved_tensors
-    heads, eps, q_mul = ctx.cfg
+    heads, eps, q_mul, kind = ctx.cfg
     b, s, n3 = qkv.shape
     n = n3 // 3
     dqkv = torch.empty((b, s, n3), dtype=torch.bfloat16, device=qkv.device)
-    res = ops.norm_rope_fullrow_backward(qkv[:, :, :n], qkv[:, :, n:2 * n], wq, wk, cos, sin, heads, gq.to(torch.bfloat16),
+    res = ops.norm_rope_fullrow_backward(qkv[:, :, :n], qkv[:, :, n:2 * n], wq, wk, ops.RopeTable(cos, sin, kind), None, heads, gq.to(torch.bfloat16),
                                          gk.to(torch.bfloat16), eps, q_mul, bias=None if bias is None else bias[:2 * n].contiguous(),
                                          dq=dqkv[:, :, :n], dk=dqkv[:, :, n:2 * n])
     dqkv[:, :, 2 * n:].unflatten(2, (heads, n // heads)).copy_(gv)
     dbias = None
     if bias is not None:
       dbias = torch.cat([res[4], gv.float().sum(dim=(0, 1)).reshape(n)]).to(bias.dtype)
-    return dqkv, dbias, res[2].to(wq.dtype), res[3].to(wk.dtype), None, None, None, None, None, None
+    return dqkv, dbias, res[2].to(wq.dtype), res[3].to(wk.dtype), None, None, None, None, None
 
 
 class _HipNormRopePerhead(torch.autograd.Function):
   """The Flux prologue with its HIP backward (attention_flax.py:2989-3020)."""
 
   @staticmethod
-  def forward(ctx, q, k, wq, wk, wq_txt, wk_txt, cos, sin, eps, n_txt, out_layout, q_mul):
-    q_out, k_out = ops.norm_rope_perhead(q, k, wq, wk, cos, sin, eps, wq_txt, wk_txt, n_txt, out_layout, q_mul)
-    ctx.save_for_backward(q, k, wq, wk, wq_txt, wk_txt, cos, sin)
-    ctx.cfg = (eps, n_txt, q_mul)
+  def forward(ctx, q, k, wq, wk, wq_txt, wk_txt, table, eps, n_txt, out_layout, q_mul):
+    q_out, k_out = ops.norm_rope_perhead(q, k, wq, wk, table, None, eps, wq_txt, wk_txt, n_txt, out_layout, q_mul)
+    ctx.save_for_backward(q, k, wq, wk, wq_txt, wk_txt, *_saved_table(table)[:2])
+    ctx.cfg = (eps, n_txt, q_mul, _saved_table(table)[2])
     return q_out, k_out
 
   @staticmethod
   def backward(ctx, gq, gk):
     q, k, wq, wk, wq_txt, wk_txt, cos, sin = ctx.saved_tensors
-    eps, n_txt, q_mul = ctx.cfg
+    eps, n_txt, q_mul, kind = ctx.cfg
     dq, dk, dwq, dwk, dwq_t, dwk_t = ops.norm_rope_perhead_backward(
-        q, k, wq, wk, cos, sin, gq.to(torch.bfloat16), gk.to(torch.bfloat16) if k is not None else None, eps, wq_txt, wk_txt, n_txt, q_mul)
+        q, k, wq, wk, ops.RopeTable(cos, sin, kind), None, gq.to(torch.bfloat16), gk.to(torch.bfloat16) if k is not None else None, eps, wq_txt, wk_txt, n_txt, q_mul)
     cast = lambda g, w: None if g is None else g.to(w.dtype)
-    return dq, dk, cast(dwq, wq), cast(dwk, wk), cast(dwq_t, wq_txt), cast(dwk_t, wk_txt), None, None, None, None, None, None
+    return dq, dk, cast(dwq, wq), cast(dwk, wk), cast(dwq_t, wq_txt), cast(dwk_t, wk_txt), None, None, None, None, None
 
 
 class _HipNormRopeRows(torch.autograd.Function):
@@ -308,12 +308,12 @@ def hip_norm_rope_qkv(qkv, wq, wk, freqs_cis, heads: int, bias=None, eps: float 
   without them.  Differentiable with respect to qkv, bias and the norm weights; `inplace=True` (the fused buffer
   itself becomes the three operands) is for inference only, since the backward needs the projection output."""
   b, s, n3 = qkv.shape
-  cos, sin = _split_table(freqs_cis, s, n3 // 3 // heads)
+  table = _rope_table(freqs_cis, s, n3 // 3 // heads)
   if _wants_grad(qkv, wq, wk, bias):
     if inplace:
       raise ValueError("inplace=True overwrites the projection output that the backward pass needs")
-    return _HipNormRopeQkv.apply(qkv, bias, wq, wk, cos, sin, heads, eps, out_layout, q_mul)
-  return ops.norm_rope_qkv(qkv, wq, wk, cos, sin, heads, bias, eps, out_layout, q_mul, inplace)
+    return _HipNormRopeQkv.apply(qkv, bias, wq, wk, table, heads, eps, out_layout, q_mul)
+  return ops.norm_rope_qkv(qkv, wq, wk, table, None, heads, bias, eps, out_layout, q_mul, inplace)
 
 
 def hip_norm_rope_ltx2(query, key, norm_q_scale, norm_k_scale, heads: int, rotary_emb=None, k_rotary_emb=None,
@@ -520,6 +520,27 @@ def _split_table(freqs_cis, seq: int, d: int):
   return cos.to(torch.float32).contiguous(), sin.to(torch.float32).contiguous()
 
 
+def _rope_table(freqs_cis, seq: int, d: int, per_head: bool = False):
+  """A rotary table as the prologue kernels take it (ops.RopeTable, or None): a dense complex64 table -- for the per-head
+  form also the f32 tuple repeated pairwise and the matrix form -- is read in place; any other goes through
+  `_split_table`."""
+  if freqs_cis is None:
+    return None
+  in_place = lambda t, dtype, shape: t.dtype == dtype and t.is_contiguous() and t.numel() == math.prod(shape) and t.data_ptr() % 16 == 0
+  if isinstance(freqs_cis, (tuple, list)):
+    if per_head and all(in_place(t, torch.float32, (seq, d)) for t in freqs_cis):
+      return ops.RopeTable(*freqs_cis, 2)
+  elif in_place(freqs_cis, torch.complex64, (seq, d // 2)) and not freqs_cis.is_conj():
+    return ops.RopeTable(freqs_cis, None, 1)
+  elif per_head and in_place(freqs_cis, torch.float32, (seq, d // 2, 4)):
+    return ops.RopeTable(freqs_cis, None, 3)
+  return ops.RopeTable(*_split_table(freqs_cis, seq, d), 0)
+
+
+def _saved_table(table):
+  return (None, None, 0) if table is None else (table.cos, table.sin, table.kind)
+
+
 def hip_norm_rope(q, k, wq, wk, freqs_cis, heads: int, eps: float = 1e-6, per_head: bool = False,
                   wq_txt=None, wk_txt=None, n_txt: int = 0, out_layout: str = "bshd", q_mul: float = 1.0):
   """The fused prologue the attention modules call in place of their inline norm + rope.
@@ -535,12 +556,12 @@ def hip_norm_rope(q, k, wq, wk, freqs_cis, heads: int, eps: float = 1e-6, per_he
   """
   if per_head:
     b, s, h, d = q.shape
-    cos, sin = _split_table(freqs_cis, s, d)
+    table = _rope_table(freqs_cis, s, d, per_head=True)
     if _wants_grad(q, k, wq, wk, wq_txt, wk_txt):
-      return _HipNormRopePerhead.apply(q, k, wq, wk, wq_txt, wk_txt, cos, sin, eps, n_txt, out_layout, q_mul)
-    return ops.norm_rope_perhead(q, k, wq, wk, cos, sin, eps, wq_txt, wk_txt, n_txt, out_layout, q_mul)
+      return _HipNormRopePerhead.apply(q, k, wq, wk, wq_txt, wk_txt, table, eps, n_txt, out_layout, q_mul)
+    return ops.norm_rope_perhead(q, k, wq, wk, table, None, eps, wq_txt, wk_txt, n_txt, out_layout, q_mul)
   b, s, n = q.shape
-  cos, sin = _split_table(freqs_cis, s, n // heads)
+  table = _rope_table(freqs_cis, s, n // heads)
   if _wants_grad(q, k, wq, wk):
-    return _HipNormRopeFullrow.apply(q, k, wq, wk, cos, sin, heads, eps, out_layout, q_mul)
-  return ops.norm_rope_fullrow(q, k, wq, wk, cos, sin, heads, eps, out_layout, q_mul)
+    return _HipNormRopeFullrow.apply(q, k, wq, wk, table, heads, eps, out_layout, q_mul)
+  return ops.norm_rope_fullrow(q, k, wq, wk, table, None, heads, eps, out_layout, q_mul)

@@ -79,6 +79,33 @@ __device__ __forceinline__ void st_nt(uint4* p, const uint4& u) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
 
+// Four consecutive rotation angles' cos and sin, group i (of four) of a rotary table in one of the layouts of
+// mdattn_host.h's MDATTN_TABLE_*: the table is read as the model made it (splitting a complex table into planes first was
+// two strided copies, 10 us and two launches of a 160 us call at 4,680 tokens).
+template <int TABLE>
+__device__ __forceinline__ void load_rope4(const float4* cos, const float4* sin, int64_t i, float* cc, float* sv) {
+  if constexpr (TABLE == 0) {  // planes [S, D/2]
+    const float4 c = cos[i], s = sin[i];
+    cc[0] = c.x; cc[1] = c.y; cc[2] = c.z; cc[3] = c.w;
+    sv[0] = s.x; sv[1] = s.y; sv[2] = s.z; sv[3] = s.w;
+  } else if constexpr (TABLE == 1) {  // complex [S, D/2]
+    const float4 a = cos[2 * i], b = cos[2 * i + 1];
+    cc[0] = a.x; cc[1] = a.z; cc[2] = b.x; cc[3] = b.z;
+    sv[0] = a.y; sv[1] = a.w; sv[2] = b.y; sv[3] = b.w;
+  } else if constexpr (TABLE == 2) {  // planes [S, D], each angle for both of its pair
+    const float4 a = cos[2 * i], b = cos[2 * i + 1], c = sin[2 * i], d = sin[2 * i + 1];
+    cc[0] = a.x; cc[1] = a.z; cc[2] = b.x; cc[3] = b.z;
+    sv[0] = c.x; sv[1] = c.z; sv[2] = d.x; sv[3] = d.z;
+  } else {  // matrices [S, D/2, 2, 2] = [[cos, -sin], [sin, cos]]
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 m = cos[4 * i + j];
+      cc[j] = m.x;
+      sv[j] = m.z;
+    }
+  }
+}
+
 // Direct global -> LDS load of 16 bytes per lane: lane i's bytes land at lds_addr + 16*i (the LDS base
 // travels in M0).  Written as inline assembly so that the loads stay asynchronous: the compiler cannot
 // tell which LDS bytes such a load writes and would otherwise wait for it before the next LDS read.
@@ -121,6 +148,12 @@ struct AttnArgs {
 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// a rotary table of layout `table` (0: planes, cos and sin; 1: complex; 2: repeated planes; 3: matrices): both pointers or none
+// for the planes, cos alone for the others
+inline bool table_ok(const float* cos, const float* sin, int table) {
+  if (table < 0 || table > 3) return false;
+  return table == 0 || table == 2 ? (cos == nullptr) == (sin == nullptr) : sin == nullptr;
+}
 inline bool strides_ok(const mdattn_strides* s, int64_t mult) {
   return s && s->batch % mult == 0 && s->seq % mult == 0 && s->head % mult == 0 && s->seq > 0 && s->head > 0 && s->batch >= 0;
 }

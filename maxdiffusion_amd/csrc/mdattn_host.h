@@ -3,6 +3,8 @@
 #pragma once
 #include <stdint.h>
 
+#include "mdattn.h"
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -11,6 +13,38 @@ extern "C" {
  * (cross-attention: dk / dv of a few hundred keys) is split over the other sequence: mdattn_bwd_workspace_floats plus the
  * f32 partial gradients.  With less, the call runs unsplit. */
 int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D);
+
+/* The prologue and its backward with the rotary table in the layout the model made it in:
+ *   PLANES    cos, sin f32 [S, D/2] (the layout of mdattn.h's entry points)
+ *   COMPLEX   cos = complex64 [S, D/2], sin null
+ *   REPEATED  cos, sin f32 [S, D], each angle for both members of its pair      (per-head forms only)
+ *   MATRIX    cos = f32 [S, D/2, 2, 2] = [[cos, -sin], [sin, cos]], sin null     (per-head forms only)
+ * No table: cos null, sin null, PLANES. */
+#define MDATTN_TABLE_PLANES 0
+#define MDATTN_TABLE_COMPLEX 1
+#define MDATTN_TABLE_REPEATED 2
+#define MDATTN_TABLE_MATRIX 3
+int mdattn_host_norm_rope_fullrow(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out, const void* wq,
+                                  const void* wk, const float* cos, const float* sin, int table, int B, int S, int H, int D,
+                                  float eps, float q_mul, int64_t in_stride_batch, int64_t in_stride_seq, const mdattn_strides* out_strides);
+int mdattn_host_norm_rope_qkv(void* stream, const void* qkv, const void* bias, void* q_out, void* k_out, void* v_out, const void* wq,
+                              const void* wk, const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps,
+                              float q_mul, int64_t qkv_stride_batch, int64_t qkv_stride_seq, const mdattn_strides* out_strides);
+int mdattn_host_norm_rope_perhead(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out, const void* wq,
+                                  const void* wk, const void* wq_txt, const void* wk_txt, int n_txt, const float* cos, const float* sin,
+                                  int table, int B, int S, int H, int D, float eps, float q_mul, const mdattn_strides* in_strides,
+                                  const mdattn_strides* out_strides);
+int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in, const void* k_in, const void* bias, const void* gq, const void* gk,
+                                      void* dq_in, void* dk_in, const void* wq, const void* wk, float* dwq, float* dwk, float* dbias,
+                                      const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps, float q_mul,
+                                      int64_t in_stride_batch, int64_t in_stride_seq, int64_t dx_stride_batch, int64_t dx_stride_seq,
+                                      const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats);
+int mdattn_host_norm_rope_perhead_bwd(void* stream, const void* q_in, const void* k_in, const void* gq, const void* gk, void* dq_in,
+                                      void* dk_in, const void* wq, const void* wk, const void* wq_txt, const void* wk_txt, int n_txt,
+                                      float* dwq, float* dwk, float* dwq_txt, float* dwk_txt, const float* cos, const float* sin,
+                                      int table, int B, int S, int H, int D, float eps, float q_mul, const mdattn_strides* in_strides,
+                                      const mdattn_strides* dx_strides, const mdattn_strides* g_strides, float* workspace,
+                                      int64_t workspace_floats);
 
 #ifdef __cplusplus
 }

@@ -1,7 +1,10 @@
 // Fused q/k RMSNorm + interleaved-pair RoPE for gfx950.  HBM-bound: every q and k element is
 // read once (16-byte loads) and written once (16-byte stores); statistics, scale and rotation
 // are f32 in registers with a single rounding to bf16.
+#include <type_traits>
+
 #include "mdattn_common.h"
+#include "mdattn_host.h"
 
 namespace mdattn {
 
@@ -11,6 +14,7 @@ struct NormRopeFullArgs {
   const uint4* w[2];
   const float4* cos;
   const float4* sin;
+  int table;              // MDATTN_TABLE_PLANES or MDATTN_TABLE_COMPLEX
   int S, H, D, N;         // N = H*D
   float eps, inv_n;
   float q_mul;            // constant folded into the q output before its rounding
@@ -25,7 +29,9 @@ struct NormRopeFullArgs {
 // One workgroup (256 lanes) per token row; lane t owns 16-byte chunks t, t+256, ... (<= MAXC).
 // FUSED: the row is the output of a fused q|k|v projection; the projection biases are added in f32 before the
 // statistics, and the value block is passed through (bias added, laid out like q and k) in the same launch.
-template <int MAXC, bool FUSED = false>
+// TAB1: every chunk of a lane sits at the same offset inside its head (256 a multiple of D/8), so one slice of the table
+// row serves them all, and it is requested with the row instead of behind the statistics' barrier.
+template <int MAXC, bool FUSED, bool TAB1>
 __global__ __launch_bounds__(256) void norm_rope_fullrow_kernel(NormRopeFullArgs a) {
   const int tid = threadIdx.x;
   const int s = blockIdx.x, b = blockIdx.y;
@@ -57,6 +63,18 @@ __global__ __launch_bounds__(256) void norm_rope_fullrow_kernel(NormRopeFullArgs
       }
     }
   }
+  const bool rope = a.cos != nullptr, cplx = a.table == MDATTN_TABLE_COMPLEX;
+  const int halfd4 = a.D >> 3;  // groups of four angles per table row
+  // two float4 per group either way: cos and sin of four angles, or the two halves of four complex numbers
+  float4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
+  auto load_table = [&](int d) __attribute__((always_inline)) {
+    const int64_t i = (int64_t)s * halfd4 + (d >> 3);
+    const float4* p0 = cplx ? a.cos + 2 * i : a.cos + i;
+    const float4* p1 = cplx ? p0 + 1 : a.sin + i;
+    cs = *p0;
+    sn = *p1;
+  };
+  if (TAB1 && rope) load_table((tid << 3) % a.D);
   // value of chunk c of tensor t as the statistics and the output see it: the projection plus its bias
   auto chunk_f32 = [&](int t, int i, int c, float* f) __attribute__((always_inline)) {
     unpack8(raw[t][i], f);
@@ -102,20 +120,15 @@ __global__ __launch_bounds__(256) void norm_rope_fullrow_kernel(NormRopeFullArgs
     }
   }
 
-  const bool rope = a.cos != nullptr;
-  const int halfd4 = a.D >> 3;  // float4 chunks per table row
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
     const int c = tid + i * 256;
     if (c < nchunks) {
       const int e = c << 3;
       const int h = e / a.D, d = e - h * a.D;
-      float4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
-      if (rope) {
-        cs = a.cos[(int64_t)s * halfd4 + (d >> 3)];
-        sn = a.sin[(int64_t)s * halfd4 + (d >> 3)];
-      }
-      const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
+      if (!TAB1 && rope) load_table(d);
+      const float cc[4] = {cs.x, cplx ? cs.z : cs.y, cplx ? sn.x : cs.z, cplx ? sn.z : cs.w};
+      const float sv[4] = {cplx ? cs.y : sn.x, cplx ? cs.w : sn.y, cplx ? sn.y : sn.z, sn.w};
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         if (t < ntens) {
@@ -166,8 +179,11 @@ struct NormRopeHeadArgs {
 };
 
 // LPR = D/8 lanes per (token, head) row; each lane owns one 16-byte chunk; RPT rows per lane group
-// in flight so that enough bytes are outstanding per CU.
-template <int LPR, int RPT>
+// in flight so that enough bytes are outstanding per CU.  TABLE: layout of the rotary table (MDATTN_TABLE_*), at compile
+// time so that its loads move up to the rows'.  A slice is read once per token and lane, not per head: 24 heads x 4,608
+// tokens on the repeated table take 26.1 us (39.9 us with a read per head); 24.8 us on planes, which took two copies of
+// 5.3 us to make.
+template <int LPR, int RPT, int TABLE>
 __global__ __launch_bounds__(256) void norm_rope_perhead_kernel(NormRopeHeadArgs a) {
   constexpr int D = LPR * 8;
   constexpr int GROUPS = 256 / LPR;
@@ -195,14 +211,12 @@ __global__ __launch_bounds__(256) void norm_rope_perhead_kernel(NormRopeHeadArgs
     for (int t = 0; t < 2; ++t)
       if (t < ntens) raw[t][r] = ld_nt(a.x_in[t] + (iofs >> 3) + lane);
   }
+  float cc[4] = {1.f, 1.f, 1.f, 1.f}, sv[4] = {0.f, 0.f, 0.f, 0.f};
+  if (rope) load_rope4<TABLE>(a.cos, a.sin, (int64_t)tok[0] * LPR + lane, cc, sv);
 #pragma unroll
   for (int r = 0; r < RPT; ++r) {
-    float4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
-    if (rope) {
-      cs = a.cos[(int64_t)tok[r] * LPR + lane];
-      sn = a.sin[(int64_t)tok[r] * LPR + lane];
-    }
-    const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
+    // a lane's rows are neighbouring heads, nearly always of one token
+    if (r > 0 && rope && tok[r] != tok[r - 1]) load_rope4<TABLE>(a.cos, a.sin, (int64_t)tok[r] * LPR + lane, cc, sv);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       if (t < ntens) {
@@ -354,14 +368,15 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(NormRopeRowsArgs a)
 
 using namespace mdattn;
 
-extern "C" int mdattn_norm_rope_fullrow(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out,
-                                        const void* wq, const void* wk, const float* cos, const float* sin,
+extern "C" int mdattn_host_norm_rope_fullrow(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out,
+                                        const void* wq, const void* wk, const float* cos, const float* sin, int table,
                                         int B, int S, int H, int D, float eps, float q_mul,
                                         int64_t in_stride_batch, int64_t in_stride_seq,
                                         const mdattn_strides* out_strides) {
   if (!q_in || !q_out || !wq || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !out_strides) return MDATTN_E_BADARG;
   if ((k_in == nullptr) != (k_out == nullptr) || (k_in && !wk)) return MDATTN_E_BADARG;
-  if ((cos == nullptr) != (sin == nullptr)) return MDATTN_E_BADARG;
+  if (!table_ok(cos, sin, table)) return MDATTN_E_BADARG;
+  if (table != MDATTN_TABLE_PLANES && table != MDATTN_TABLE_COMPLEX) return MDATTN_E_UNSUPPORTED;
   if (!(eps >= 0.f) || !(q_mul > 0.f) || !(q_mul < 1e30f)) return MDATTN_E_BADARG;
   const int64_t N = (int64_t)H * D;
   if (D % 8 != 0 || N > 8192) return MDATTN_E_UNSUPPORTED;
@@ -376,7 +391,7 @@ extern "C" int mdattn_norm_rope_fullrow(void* stream, const void* q_in, const vo
   a.x_in[0] = (const uint4*)q_in; a.x_in[1] = (const uint4*)k_in;
   a.x_out[0] = (uint4*)q_out; a.x_out[1] = (uint4*)k_out;
   a.w[0] = (const uint4*)wq; a.w[1] = (const uint4*)wk;
-  a.cos = (const float4*)cos; a.sin = (const float4*)sin;
+  a.cos = (const float4*)cos; a.sin = (const float4*)sin; a.table = table;
   a.S = S; a.H = H; a.D = D; a.N = (int)N; a.eps = eps; a.inv_n = 1.0f / (float)N; a.q_mul = q_mul;
   a.in_sb = in_stride_batch; a.in_ss = in_stride_seq;
   a.out_sb = out_strides->batch; a.out_ss = out_strides->seq; a.out_sh = out_strides->head;
@@ -384,19 +399,23 @@ extern "C" int mdattn_norm_rope_fullrow(void* stream, const void* q_in, const vo
   dim3 grid(S, B), block(256);
   hipStream_t st = (hipStream_t)stream;
   const int nchunks = (int)(N / 8);
-  if (nchunks <= 256) MDATTN_LAUNCH(norm_rope_fullrow_kernel<1>, grid, block, 0, st, a);
-  else if (nchunks <= 512) MDATTN_LAUNCH(norm_rope_fullrow_kernel<2>, grid, block, 0, st, a);
-  else if (nchunks <= 768) MDATTN_LAUNCH(norm_rope_fullrow_kernel<3>, grid, block, 0, st, a);
-  else MDATTN_LAUNCH(norm_rope_fullrow_kernel<4>, grid, block, 0, st, a);
+  void (*kern)(NormRopeFullArgs);
+  const bool tab1 = 256 % (D / 8) == 0;
+  if (nchunks <= 256) kern = tab1 ? norm_rope_fullrow_kernel<1, false, true> : norm_rope_fullrow_kernel<1, false, false>;
+  else if (nchunks <= 512) kern = tab1 ? norm_rope_fullrow_kernel<2, false, true> : norm_rope_fullrow_kernel<2, false, false>;
+  else if (nchunks <= 768) kern = tab1 ? norm_rope_fullrow_kernel<3, false, true> : norm_rope_fullrow_kernel<3, false, false>;
+  else kern = tab1 ? norm_rope_fullrow_kernel<4, false, true> : norm_rope_fullrow_kernel<4, false, false>;
+  MDATTN_LAUNCH(kern, grid, block, 0, st, a);
   return launch_status();
 }
 
-extern "C" int mdattn_norm_rope_qkv(void* stream, const void* qkv, const void* bias, void* q_out, void* k_out, void* v_out,
-                                    const void* wq, const void* wk, const float* cos, const float* sin,
+extern "C" int mdattn_host_norm_rope_qkv(void* stream, const void* qkv, const void* bias, void* q_out, void* k_out, void* v_out,
+                                    const void* wq, const void* wk, const float* cos, const float* sin, int table,
                                     int B, int S, int H, int D, float eps, float q_mul,
                                     int64_t qkv_stride_batch, int64_t qkv_stride_seq, const mdattn_strides* out_strides) {
   if (!qkv || !q_out || !k_out || !wq || !wk || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !out_strides) return MDATTN_E_BADARG;
-  if ((cos == nullptr) != (sin == nullptr)) return MDATTN_E_BADARG;
+  if (!table_ok(cos, sin, table)) return MDATTN_E_BADARG;
+  if (table != MDATTN_TABLE_PLANES && table != MDATTN_TABLE_COMPLEX) return MDATTN_E_UNSUPPORTED;
   if (bias && !v_out) return MDATTN_E_BADARG;  // the value block needs its bias too: it cannot stay where it is
   if (!(eps >= 0.f) || !(q_mul > 0.f) || !(q_mul < 1e30f)) return MDATTN_E_BADARG;
   const int64_t N = (int64_t)H * D;
@@ -415,28 +434,31 @@ extern "C" int mdattn_norm_rope_qkv(void* stream, const void* qkv, const void* b
   a.w[0] = (const uint4*)wq; a.w[1] = (const uint4*)wk;
   const uint4* bb = (const uint4*)bias;
   a.bias[0] = bb; a.bias[1] = bb ? bb + N / 8 : nullptr; a.bias[2] = bb ? bb + 2 * N / 8 : nullptr;
-  a.cos = (const float4*)cos; a.sin = (const float4*)sin;
+  a.cos = (const float4*)cos; a.sin = (const float4*)sin; a.table = table;
   a.S = S; a.H = H; a.D = D; a.N = (int)N; a.eps = eps; a.inv_n = 1.0f / (float)N; a.q_mul = q_mul;
   a.in_sb = qkv_stride_batch; a.in_ss = qkv_stride_seq;
   a.out_sb = out_strides->batch; a.out_ss = out_strides->seq; a.out_sh = out_strides->head;
   dim3 grid(S, B), block(256);
   hipStream_t st = (hipStream_t)stream;
   const int nchunks = (int)(N / 8);
-  if (nchunks <= 256) MDATTN_LAUNCH((norm_rope_fullrow_kernel<1, true>), grid, block, 0, st, a);
-  else if (nchunks <= 512) MDATTN_LAUNCH((norm_rope_fullrow_kernel<2, true>), grid, block, 0, st, a);
-  else if (nchunks <= 768) MDATTN_LAUNCH((norm_rope_fullrow_kernel<3, true>), grid, block, 0, st, a);
-  else MDATTN_LAUNCH((norm_rope_fullrow_kernel<4, true>), grid, block, 0, st, a);
+  void (*kern)(NormRopeFullArgs);
+  const bool tab1 = 256 % (D / 8) == 0;
+  if (nchunks <= 256) kern = tab1 ? norm_rope_fullrow_kernel<1, true, true> : norm_rope_fullrow_kernel<1, true, false>;
+  else if (nchunks <= 512) kern = tab1 ? norm_rope_fullrow_kernel<2, true, true> : norm_rope_fullrow_kernel<2, true, false>;
+  else if (nchunks <= 768) kern = tab1 ? norm_rope_fullrow_kernel<3, true, true> : norm_rope_fullrow_kernel<3, true, false>;
+  else kern = tab1 ? norm_rope_fullrow_kernel<4, true, true> : norm_rope_fullrow_kernel<4, true, false>;
+  MDATTN_LAUNCH(kern, grid, block, 0, st, a);
   return launch_status();
 }
 
-extern "C" int mdattn_norm_rope_perhead(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out,
+extern "C" int mdattn_host_norm_rope_perhead(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out,
                                         const void* wq, const void* wk, const void* wq_txt, const void* wk_txt,
-                                        int n_txt, const float* cos, const float* sin, int B, int S, int H, int D,
+                                        int n_txt, const float* cos, const float* sin, int table, int B, int S, int H, int D,
                                         float eps, float q_mul, const mdattn_strides* in_strides,
                                         const mdattn_strides* out_strides) {
   if (!q_in || !q_out || !wq || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !in_strides || !out_strides) return MDATTN_E_BADARG;
   if ((k_in == nullptr) != (k_out == nullptr) || (k_in && !wk)) return MDATTN_E_BADARG;
-  if ((cos == nullptr) != (sin == nullptr)) return MDATTN_E_BADARG;
+  if (!table_ok(cos, sin, table)) return MDATTN_E_BADARG;
   if (n_txt < 0 || n_txt > S || !(eps >= 0.f) || !(q_mul > 0.f) || !(q_mul < 1e30f)) return MDATTN_E_BADARG;
   if (D != 64 && D != 128 && D != 256) return MDATTN_E_UNSUPPORTED;
   if (!aligned16(q_in) || !aligned16(q_out) || !aligned16(wq) || !aligned16(k_in) || !aligned16(k_out) ||
@@ -460,10 +482,41 @@ extern "C" int mdattn_norm_rope_perhead(void* stream, const void* q_in, const vo
   if (nblocks > 0x7FFFFFFF) return MDATTN_E_UNSUPPORTED;
   dim3 grid((unsigned)nblocks), block(256);
   hipStream_t st = (hipStream_t)stream;
-  if (lpr == 8) MDATTN_LAUNCH((norm_rope_perhead_kernel<8, RPT>), grid, block, 0, st, a);
-  else if (lpr == 16) MDATTN_LAUNCH((norm_rope_perhead_kernel<16, RPT>), grid, block, 0, st, a);
-  else MDATTN_LAUNCH((norm_rope_perhead_kernel<32, RPT>), grid, block, 0, st, a);
+  auto pick = [&](auto t) {
+    constexpr int T = decltype(t)::value;
+    return lpr == 8 ? norm_rope_perhead_kernel<8, RPT, T> : lpr == 16 ? norm_rope_perhead_kernel<16, RPT, T> : norm_rope_perhead_kernel<32, RPT, T>;
+  };
+  void (*kern)(NormRopeHeadArgs) = table == 0 ? pick(std::integral_constant<int, 0>{}) : table == 1 ? pick(std::integral_constant<int, 1>{})
+                                 : table == 2 ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 3>{});
+  MDATTN_LAUNCH(kern, grid, block, 0, st, a);
   return launch_status();
+}
+
+// The C ABI's forms take the table as two planes [S, D/2].
+extern "C" int mdattn_norm_rope_fullrow(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out,
+                                        const void* wq, const void* wk, const float* cos, const float* sin,
+                                        int B, int S, int H, int D, float eps, float q_mul,
+                                        int64_t in_stride_batch, int64_t in_stride_seq,
+                                        const mdattn_strides* out_strides) {
+  return mdattn_host_norm_rope_fullrow(stream, q_in, k_in, q_out, k_out, wq, wk, cos, sin, MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul,
+                                       in_stride_batch, in_stride_seq, out_strides);
+}
+
+extern "C" int mdattn_norm_rope_qkv(void* stream, const void* qkv, const void* bias, void* q_out, void* k_out, void* v_out,
+                                    const void* wq, const void* wk, const float* cos, const float* sin,
+                                    int B, int S, int H, int D, float eps, float q_mul,
+                                    int64_t qkv_stride_batch, int64_t qkv_stride_seq, const mdattn_strides* out_strides) {
+  return mdattn_host_norm_rope_qkv(stream, qkv, bias, q_out, k_out, v_out, wq, wk, cos, sin, MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul,
+                                   qkv_stride_batch, qkv_stride_seq, out_strides);
+}
+
+extern "C" int mdattn_norm_rope_perhead(void* stream, const void* q_in, const void* k_in, void* q_out, void* k_out,
+                                        const void* wq, const void* wk, const void* wq_txt, const void* wk_txt,
+                                        int n_txt, const float* cos, const float* sin, int B, int S, int H, int D,
+                                        float eps, float q_mul, const mdattn_strides* in_strides,
+                                        const mdattn_strides* out_strides) {
+  return mdattn_host_norm_rope_perhead(stream, q_in, k_in, q_out, k_out, wq, wk, wq_txt, wk_txt, n_txt, cos, sin, MDATTN_TABLE_PLANES, B, S,
+                                       H, D, eps, q_mul, in_strides, out_strides);
 }
 
 extern "C" int mdattn_norm_rope_rows(void* stream, const void* x_in, int x_is_f32, void* x_out, const float* w,

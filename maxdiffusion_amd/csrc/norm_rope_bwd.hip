@@ -10,7 +10,10 @@
 // gradients are reduced without atomics in two stages: every workgroup accumulates its tokens' contributions to
 // its lanes' columns in registers and writes one partial row to the workspace; a second kernel sums the partial rows
 // in a fixed order, so results are bit-reproducible.
+#include <type_traits>
+
 #include "mdattn_common.h"
+#include "mdattn_host.h"
 
 namespace mdattn {
 
@@ -30,6 +33,7 @@ struct NormRopeBwdFullArgs {
   const uint4* bias[2];   // BIAS: the projection biases the forward added (null: none)
   const float4* cos;
   const float4* sin;
+  int table;              // MDATTN_TABLE_PLANES or MDATTN_TABLE_COMPLEX
   float* part;            // [nb][ncols] partial weight (and bias) gradients
   int S, H, D, N, ntok, nb, ncols;
   float eps, inv_n, q_mul;
@@ -85,7 +89,7 @@ __global__ __launch_bounds__(512) void norm_rope_fullrow_bwd_kernel(NormRopeBwdF
     al[2 * (i * NT + tid) + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
     coff[i] = cc;
     goff[i] = (int)(h * a.g_sh) + d;
-    if (i < TC) tofs[i] = d >> 3;
+    if (i < TC) tofs[i] = (d >> 3) * (a.table == MDATTN_TABLE_COMPLEX ? 2 : 1);
 #pragma unroll
     for (int j = 0; j < 8; ++j) { if constexpr (BIAS) { accb[i][j] = 0.f; bf[i][j] = 0.f; } }
     if constexpr (BIAS) {
@@ -96,9 +100,11 @@ __global__ __launch_bounds__(512) void norm_rope_fullrow_bwd_kernel(NormRopeBwdF
     const float4 v0 = base[2 * (i * NT + tid)], v1 = base[2 * (i * NT + tid) + 1];
     f[0] = v0.x; f[1] = v0.y; f[2] = v0.z; f[3] = v0.w; f[4] = v1.x; f[5] = v1.y; f[6] = v1.z; f[7] = v1.w;
   };
+  // two float4 per chunk either way: cos and sin of four angles, or the two halves of four complex numbers
+  const bool cplx = a.table == MDATTN_TABLE_COMPLEX;
   const float4* cosp = rope ? a.cos : reinterpret_cast<const float4*>(a.w[t]);  // norm only: any readable address, unused
-  const float4* sinp = rope ? a.sin : reinterpret_cast<const float4*>(a.w[t]);
-  const int64_t tstride = rope ? halfd4 : 0;
+  const float4* sinp = rope ? (cplx ? a.cos + 1 : a.sin) : cosp;
+  const int64_t tstride = rope ? (cplx ? 2 * halfd4 : halfd4) : 0;
 
   struct RowBuf {
     uint4 x[MAXC], g[MAXC];
@@ -148,7 +154,8 @@ __global__ __launch_bounds__(512) void norm_rope_fullrow_bwd_kernel(NormRopeBwdF
       }
       if (rope) {
         const float4 cs = r.cs[TAB1 ? 0 : i], sn = r.sn[TAB1 ? 0 : i];
-        const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
+        const float cc[4] = {cs.x, cplx ? cs.z : cs.y, cplx ? sn.x : cs.z, cplx ? sn.z : cs.w};
+        const float sv[4] = {cplx ? cs.y : sn.x, cplx ? cs.w : sn.y, cplx ? sn.y : sn.z, sn.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           dy[i][2 * j] = __builtin_fmaf(gf[2 * j], cc[j], gf[2 * j + 1] * sv[j]);
@@ -301,7 +308,7 @@ struct NormRopeBwdHeadArgs {
   const float4* cos;
   const float4* sin;
   float* part;  // [nb][4*D]: [tensor][image | text][D]
-  int S, H, n_txt, nb;
+  int S, H, n_txt, nb, run;
   int64_t rows;  // B*S*H
   float eps, q_mul;
   int64_t in_sb, in_ss, in_sh, dx_sb, dx_ss, dx_sh, g_sb, g_ss, g_sh;
@@ -309,7 +316,7 @@ struct NormRopeBwdHeadArgs {
 
 // LPR = D/8 lanes per (token, head) row, one 16-byte chunk per lane; a workgroup's 256/LPR lane groups walk the rows
 // in strides.  Both row sums stay inside the lane group (no LDS, no barrier in the loop).
-template <int LPR>
+template <int LPR, int TABLE>
 __global__ __launch_bounds__(256) void norm_rope_perhead_bwd_kernel(NormRopeBwdHeadArgs a) {
   constexpr int D = LPR * 8;
   constexpr int GROUPS = 256 / LPR;
@@ -336,7 +343,13 @@ __global__ __launch_bounds__(256) void norm_rope_perhead_bwd_kernel(NormRopeBwdH
     return v;
   };
 
-  for (int64_t row = (int64_t)blockIdx.x * GROUPS + grp; row < a.rows; row += (int64_t)a.nb * GROUPS) {
+  // a lane group takes `run` consecutive rows (neighbouring heads, nearly always of one token) per turn, so that a slice of
+  // the table is read once per token rather than once per head
+  int64_t tab_s = -1;
+  float cc[4] = {1.f, 1.f, 1.f, 1.f}, sv[4] = {0.f, 0.f, 0.f, 0.f};
+  int left = a.run;
+  const int64_t hop = (int64_t)(a.nb * GROUPS - 1) * a.run + 1;  // from the last row of a turn to the first of the next
+  for (int64_t row = ((int64_t)blockIdx.x * GROUPS + grp) * a.run; row < a.rows;) {
     const int h = (int)(row % a.H);
     const int64_t bs = row / a.H;
     const int s = (int)(bs % a.S);
@@ -351,12 +364,10 @@ __global__ __launch_bounds__(256) void norm_rope_perhead_bwd_kernel(NormRopeBwdH
         xr[t] = ld_nt(a.x_in[t] + (iofs >> 3) + lane);
         gr[t] = ld_nt(a.g[t] + (gofs >> 3) + lane);
       }
-    float4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
-    if (rope) {
-      cs = a.cos[(int64_t)s * LPR + lane];
-      sn = a.sin[(int64_t)s * LPR + lane];
+    if (rope && s != tab_s) {
+      load_rope4<TABLE>(a.cos, a.sin, (int64_t)s * LPR + lane, cc, sv);
+      tab_s = s;
     }
-    const float cc[4] = {cs.x, cs.y, cs.z, cs.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       if (t < ntens) {
@@ -391,6 +402,9 @@ __global__ __launch_bounds__(256) void norm_rope_perhead_bwd_kernel(NormRopeBwdH
         st_nt(a.dx[t] + (dofs >> 3) + lane, pack8(du));
       }
     }
+    left -= 1;
+    row += left ? 1 : hop;
+    if (!left) left = a.run;
   }
 
   // the workgroup's lane groups -> one partial row
@@ -625,17 +639,18 @@ static int partial_rows(int64_t units, int64_t ncols, int64_t floats, int reside
   return (int)nb;
 }
 
-extern "C" int mdattn_norm_rope_fullrow_bwd(void* stream, const void* q_in, const void* k_in, const void* bias,
+extern "C" int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in, const void* k_in, const void* bias,
                                             const void* gq, const void* gk, void* dq_in, void* dk_in,
                                             const void* wq, const void* wk, float* dwq, float* dwk, float* dbias,
-                                            const float* cos, const float* sin, int B, int S, int H, int D, float eps, float q_mul,
+                                            const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps, float q_mul,
                                             int64_t in_stride_batch, int64_t in_stride_seq,
                                             int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides,
                                             float* workspace, int64_t workspace_floats) {
   if (!q_in || !gq || !dq_in || !wq || !dwq || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !g_strides || !workspace) return MDATTN_E_BADARG;
   const bool has_k = k_in != nullptr;
   if (has_k != (gk != nullptr) || has_k != (dk_in != nullptr) || has_k != (dwk != nullptr) || (has_k && !wk)) return MDATTN_E_BADARG;
-  if ((cos == nullptr) != (sin == nullptr)) return MDATTN_E_BADARG;
+  if (!table_ok(cos, sin, table)) return MDATTN_E_BADARG;
+  if (table != MDATTN_TABLE_PLANES && table != MDATTN_TABLE_COMPLEX) return MDATTN_E_UNSUPPORTED;
   if ((bias == nullptr) != (dbias == nullptr) || (bias && !has_k)) return MDATTN_E_BADARG;  // the fused q|k|v form carries both
   if (!(eps >= 0.f) || !(q_mul > 0.f) || !(q_mul < 1e30f)) return MDATTN_E_BADARG;
   const int64_t N = (int64_t)H * D;
@@ -674,7 +689,7 @@ extern "C" int mdattn_norm_rope_fullrow_bwd(void* stream, const void* q_in, cons
   a.w[0] = (const uint4*)wq; a.w[1] = (const uint4*)wk;
   const uint4* bb = (const uint4*)bias;
   a.bias[0] = bb; a.bias[1] = bb ? bb + N / 8 : nullptr;
-  a.cos = (const float4*)cos; a.sin = (const float4*)sin;
+  a.cos = (const float4*)cos; a.sin = (const float4*)sin; a.table = table;
   a.part = workspace;
   a.S = S; a.H = H; a.D = D; a.N = (int)N; a.ntok = (int)ntok; a.nb = nb; a.ncols = (int)ncols;
   a.eps = eps; a.inv_n = 1.0f / (float)N; a.q_mul = q_mul;
@@ -689,17 +704,17 @@ extern "C" int mdattn_norm_rope_fullrow_bwd(void* stream, const void* q_in, cons
   return launch_colsum(st, workspace, nb, (int)ncols, (int)N, dwq, dwk, nullptr, nullptr);
 }
 
-extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, const void* k_in, const void* gq, const void* gk,
+extern "C" int mdattn_host_norm_rope_perhead_bwd(void* stream, const void* q_in, const void* k_in, const void* gq, const void* gk,
                                             void* dq_in, void* dk_in, const void* wq, const void* wk, const void* wq_txt,
                                             const void* wk_txt, int n_txt, float* dwq, float* dwk, float* dwq_txt, float* dwk_txt,
-                                            const float* cos, const float* sin, int B, int S, int H, int D, float eps, float q_mul,
+                                            const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps, float q_mul,
                                             const mdattn_strides* in_strides, const mdattn_strides* dx_strides,
                                             const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats) {
   if (!q_in || !gq || !dq_in || !wq || !dwq || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !in_strides || !dx_strides || !g_strides || !workspace)
     return MDATTN_E_BADARG;
   const bool has_k = k_in != nullptr;
   if (has_k != (gk != nullptr) || has_k != (dk_in != nullptr) || has_k != (dwk != nullptr) || (has_k && !wk)) return MDATTN_E_BADARG;
-  if ((cos == nullptr) != (sin == nullptr)) return MDATTN_E_BADARG;
+  if (!table_ok(cos, sin, table)) return MDATTN_E_BADARG;
   if ((wq_txt == nullptr) != (dwq_txt == nullptr) || (wk_txt == nullptr) != (dwk_txt == nullptr)) return MDATTN_E_BADARG;
   if (n_txt < 0 || n_txt > S || !(eps >= 0.f) || !(q_mul > 0.f) || !(q_mul < 1e30f)) return MDATTN_E_BADARG;
   if (D != 64 && D != 128 && D != 256) return MDATTN_E_UNSUPPORTED;
@@ -712,10 +727,15 @@ extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, cons
   const int64_t rows = (int64_t)B * S * H;
   const int64_t ncols = 4 * (int64_t)D;
   const int lds = groups * 4 * D * (int)sizeof(float);  // 32 KB for every supported D
-  void (*kern)(NormRopeBwdHeadArgs) = lpr == 8 ? norm_rope_perhead_bwd_kernel<8> : lpr == 16 ? norm_rope_perhead_bwd_kernel<16> : norm_rope_perhead_bwd_kernel<32>;
-  static ResidentCache resident[3];
+  auto pick = [&](auto t) {
+    constexpr int T = decltype(t)::value;
+    return lpr == 8 ? norm_rope_perhead_bwd_kernel<8, T> : lpr == 16 ? norm_rope_perhead_bwd_kernel<16, T> : norm_rope_perhead_bwd_kernel<32, T>;
+  };
+  void (*kern)(NormRopeBwdHeadArgs) = table == 0 ? pick(std::integral_constant<int, 0>{}) : table == 1 ? pick(std::integral_constant<int, 1>{})
+                                    : table == 2 ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 3>{});
+  static ResidentCache resident[3][4];
   const int nb = partial_rows((rows + groups - 1) / groups, ncols, workspace_floats,
-                              resident_blocks(resident[lpr == 8 ? 0 : lpr == 16 ? 1 : 2], reinterpret_cast<const void*>(kern), 256, lds));
+                              resident_blocks(resident[lpr == 8 ? 0 : lpr == 16 ? 1 : 2][table], reinterpret_cast<const void*>(kern), 256, lds));
   if (nb < 1) return MDATTN_E_BADARG;
 
   NormRopeBwdHeadArgs a;
@@ -726,7 +746,9 @@ extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, cons
   a.w_txt[0] = (const uint4*)wq_txt; a.w_txt[1] = has_k ? (const uint4*)wk_txt : nullptr;
   a.cos = (const float4*)cos; a.sin = (const float4*)sin;
   a.part = workspace;
-  a.S = S; a.H = H; a.n_txt = n_txt; a.nb = nb; a.rows = rows; a.eps = eps; a.q_mul = q_mul;
+  a.S = S; a.H = H; a.n_txt = n_txt; a.nb = nb; a.rows = rows;
+  a.run = rows >= 4 * (int64_t)nb * groups ? 4 : 1;  // short inputs: every lane group its own row
+  a.eps = eps; a.q_mul = q_mul;
   a.in_sb = in_strides->batch; a.in_ss = in_strides->seq; a.in_sh = in_strides->head;
   a.dx_sb = dx_strides->batch; a.dx_ss = dx_strides->seq; a.dx_sh = dx_strides->head;
   a.g_sb = g_strides->batch; a.g_ss = g_strides->seq; a.g_sh = g_strides->head;
@@ -736,6 +758,30 @@ extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, cons
   if (rc != MDATTN_OK) return rc;
   // columns: [q image][q text][k image][k text], each D wide; outputs that do not exist are skipped
   return launch_colsum(st, workspace, nb, (int)ncols, D, dwq, dwq_txt, dwk, has_k ? dwk_txt : nullptr);
+}
+
+// The C ABI's forms take the table as two planes [S, D/2].
+extern "C" int mdattn_norm_rope_fullrow_bwd(void* stream, const void* q_in, const void* k_in, const void* bias,
+                                            const void* gq, const void* gk, void* dq_in, void* dk_in,
+                                            const void* wq, const void* wk, float* dwq, float* dwk, float* dbias,
+                                            const float* cos, const float* sin, int B, int S, int H, int D, float eps, float q_mul,
+                                            int64_t in_stride_batch, int64_t in_stride_seq,
+                                            int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides,
+                                            float* workspace, int64_t workspace_floats) {
+  return mdattn_host_norm_rope_fullrow_bwd(stream, q_in, k_in, bias, gq, gk, dq_in, dk_in, wq, wk, dwq, dwk, dbias, cos, sin,
+                                           MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul, in_stride_batch, in_stride_seq, dx_stride_batch,
+                                           dx_stride_seq, g_strides, workspace, workspace_floats);
+}
+
+extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, const void* k_in, const void* gq, const void* gk,
+                                            void* dq_in, void* dk_in, const void* wq, const void* wk, const void* wq_txt,
+                                            const void* wk_txt, int n_txt, float* dwq, float* dwk, float* dwq_txt, float* dwk_txt,
+                                            const float* cos, const float* sin, int B, int S, int H, int D, float eps, float q_mul,
+                                            const mdattn_strides* in_strides, const mdattn_strides* dx_strides,
+                                            const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats) {
+  return mdattn_host_norm_rope_perhead_bwd(stream, q_in, k_in, gq, gk, dq_in, dk_in, wq, wk, wq_txt, wk_txt, n_txt, dwq, dwk, dwq_txt,
+                                           dwk_txt, cos, sin, MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul, in_strides, dx_strides,
+                                           g_strides, workspace, workspace_floats);
 }
 
 extern "C" int mdattn_norm_rope_rows_bwd(void* stream, const void* x_in, int x_is_f32, const void* g, void* dx, const float* w,

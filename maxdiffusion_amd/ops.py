@@ -49,7 +49,8 @@ def _ptr(t):
 
 
 def _stream():
-  return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+  # the raw handle of the current stream of the current device (building a torch.cuda.Stream object around it costs 10 us)
+  return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _check_dev(*ts):
@@ -81,13 +82,34 @@ def _table(t, s, d, name):
   return t
 
 
+class RopeTable:
+  """A rotary table as a model made it, for the hooks of `attention_op`: the kernels read it in place.  `kind` is
+  mdattn_host.h's MDATTN_TABLE_*: 0 cos, sin f32 [S, D/2]; 1 cos complex64 [S, D/2]; 2 cos, sin f32 [S, D] (repeated
+  pairwise); 3 cos f32 [S, D/2, 2, 2].  Passed in place of `cos`, with `sin` None."""
+  __slots__ = ("cos", "sin", "kind")
+
+  def __init__(self, cos, sin, kind):
+    self.cos, self.sin, self.kind = cos, sin, kind
+
+
+def _table_args(cos, sin, s, d):
+  """(cos pointer, sin pointer, kind) of the table arguments of a prologue call."""
+  if isinstance(cos, RopeTable):
+    if cos.kind:
+      _check_dev(cos.cos, cos.sin)
+      return _ptr(cos.cos), _ptr(cos.sin), cos.kind
+    cos, sin = cos.cos, cos.sin
+  _check_dev(cos, sin)
+  return _ptr(_table(cos, s, d, "cos")), _ptr(_table(sin, s, d, "sin")), 0
+
+
 def norm_rope_fullrow(q, k, wq, wk, cos, sin, heads: int, eps: float = 1e-6, out_layout: str = "bshd", q_mul: float = 1.0):
   """q, k: bf16 [B, S, H*D] (k may be None) -> (q_out, k_out) logical [B,S,H,D] views in `out_layout`.
 
   RMSNorm over H*D, then rotation of interleaved pairs by the [S, D/2] table (cos/sin None: norm only).
   `q_mul` is multiplied into q_out before its single rounding (see FOLDED_Q_MUL / FOLDED_SCALE).
   """
-  _check_dev(q, k, wq, wk, cos, sin)
+  _check_dev(q, k, wq, wk)
   if q.dim() != 3 or q.dtype != torch.bfloat16 or q.stride(2) != 1:
     raise ValueError("q must be bf16 [B, S, H*D] with a contiguous last axis")
   b, s, n = q.shape
@@ -96,12 +118,12 @@ def norm_rope_fullrow(q, k, wq, wk, cos, sin, heads: int, eps: float = 1e-6, out
   d = n // heads
   if k is not None and (k.shape != q.shape or k.dtype != q.dtype or k.stride() != q.stride()):
     raise ValueError("k must match q in shape, dtype and strides")
-  cos, sin = _table(cos, s, d, "cos"), _table(sin, s, d, "sin")
+  pcos, psin, kind = _table_args(cos, sin, s, d)
   q_out = _alloc_like_layout(b, s, heads, d, out_layout, torch.bfloat16, q.device)
   k_out = _alloc_like_layout(b, s, heads, d, out_layout, torch.bfloat16, q.device) if k is not None else None
   st = _strides(q_out)
-  rc = _lib.load().mdattn_norm_rope_fullrow(
-      _stream(), _ptr(q), _ptr(k), _ptr(q_out), _ptr(k_out), _ptr(wq), _ptr(wk), _ptr(cos), _ptr(sin),
+  rc = _lib.load().mdattn_host_norm_rope_fullrow(
+      _stream(), _ptr(q), _ptr(k), _ptr(q_out), _ptr(k_out), _ptr(wq), _ptr(wk), pcos, psin, kind,
       b, s, heads, d, eps, q_mul, q.stride(0), q.stride(1), ctypes.byref(st))
   _lib.check(rc, "mdattn_norm_rope_fullrow")
   return q_out, k_out
@@ -114,13 +136,13 @@ def norm_rope_qkv(qkv, wq, wk, cos, sin, heads: int, bias=None, eps: float = 1e-
   bias bf16 [3*H*D] or None: the projections' biases, added in f32 before the statistics.  Returns (q, k, v) logical
   [B,S,H,D] views.  Without bias v is a view of the fused buffer itself (never copied).  inplace=True writes q, k
   (and the biased v) back into the fused buffer, which then holds the three attention operands."""
-  _check_dev(qkv, wq, wk, cos, sin, bias)
+  _check_dev(qkv, wq, wk, bias)
   if qkv.dim() != 3 or qkv.dtype != torch.bfloat16 or qkv.stride(2) != 1 or qkv.shape[2] % (3 * heads):
     raise ValueError("qkv must be bf16 [B, S, 3*H*D] with a contiguous last axis")
   b, s, n3 = qkv.shape
   n = n3 // 3
   d = n // heads
-  cos, sin = _table(cos, s, d, "cos"), _table(sin, s, d, "sin")
+  pcos, psin, kind = _table_args(cos, sin, s, d)
   if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != n3 or not bias.is_contiguous()):
     raise ValueError("bias must be a contiguous bf16 [3*H*D] tensor")
   blocks = [qkv[:, :, i * n:(i + 1) * n].unflatten(2, (heads, d)) for i in range(3)]  # views of the fused buffer
@@ -132,8 +154,8 @@ def norm_rope_qkv(qkv, wq, wk, cos, sin, heads: int, bias=None, eps: float = 1e-
     k_out = _alloc_like_layout(b, s, heads, d, out_layout, torch.bfloat16, qkv.device)
     v_out = _alloc_like_layout(b, s, heads, d, out_layout, torch.bfloat16, qkv.device) if bias is not None else None
   st = _strides(q_out)
-  rc = _lib.load().mdattn_norm_rope_qkv(
-      _stream(), _ptr(qkv), _ptr(bias), _ptr(q_out), _ptr(k_out), _ptr(v_out), _ptr(wq), _ptr(wk), _ptr(cos), _ptr(sin),
+  rc = _lib.load().mdattn_host_norm_rope_qkv(
+      _stream(), _ptr(qkv), _ptr(bias), _ptr(q_out), _ptr(k_out), _ptr(v_out), _ptr(wq), _ptr(wk), pcos, psin, kind,
       b, s, heads, d, eps, q_mul, qkv.stride(0), qkv.stride(1), ctypes.byref(st))
   _lib.check(rc, "mdattn_norm_rope_qkv")
   return q_out, k_out, (v_out if v_out is not None else blocks[2])
@@ -172,19 +194,19 @@ def norm_rope_perhead(q, k, wq, wk, cos, sin, eps: float = 1e-6, wq_txt=None, wk
                       out_layout: str = "bshd", q_mul: float = 1.0):
   """q, k: bf16 logical [B, S, H, D] views (k may be None); RMSNorm over D per head, then RoPE.
   `q_mul` is multiplied into q_out before its single rounding."""
-  _check_dev(q, k, wq, wk, wq_txt, wk_txt, cos, sin)
+  _check_dev(q, k, wq, wk, wq_txt, wk_txt)
   if q.dtype != torch.bfloat16:
     raise ValueError("q must be bf16")
   b, s, h, d = q.shape
   if k is not None and (k.shape != q.shape or k.stride() != q.stride() or k.dtype != q.dtype):
     raise ValueError("k must match q in shape, dtype and strides")
-  cos, sin = _table(cos, s, d, "cos"), _table(sin, s, d, "sin")
+  pcos, psin, kind = _table_args(cos, sin, s, d)
   q_out = _alloc_like_layout(b, s, h, d, out_layout, torch.bfloat16, q.device)
   k_out = _alloc_like_layout(b, s, h, d, out_layout, torch.bfloat16, q.device) if k is not None else None
   si, so = _strides(q), _strides(q_out)
-  rc = _lib.load().mdattn_norm_rope_perhead(
+  rc = _lib.load().mdattn_host_norm_rope_perhead(
       _stream(), _ptr(q), _ptr(k), _ptr(q_out), _ptr(k_out), _ptr(wq), _ptr(wk), _ptr(wq_txt), _ptr(wk_txt), n_txt,
-      _ptr(cos), _ptr(sin), b, s, h, d, eps, q_mul, ctypes.byref(si), ctypes.byref(so))
+      pcos, psin, kind, b, s, h, d, eps, q_mul, ctypes.byref(si), ctypes.byref(so))
   _lib.check(rc, "mdattn_norm_rope_perhead")
   return q_out, k_out
 
@@ -210,7 +232,7 @@ def norm_rope_fullrow_backward(q, k, wq, wk, cos, sin, heads: int, gq, gk, eps: 
   the prologue's outputs.  Returns (dq, dk, dwq, dwk) -- dq, dk bf16 shaped and strided like q, k (or written into
   the given dq / dk, which may be the column blocks of a fused gradient buffer), dwq, dwk f32 [H*D] -- plus dbias
   f32 [2*H*D] when bias is given."""
-  _check_dev(q, k, wq, wk, cos, sin, gq, gk, bias, dq, dk)
+  _check_dev(q, k, wq, wk, gq, gk, bias, dq, dk)
   if q.dim() != 3 or q.dtype != torch.bfloat16 or q.stride(2) != 1:
     raise ValueError("q must be bf16 [B, S, H*D] with a contiguous last axis")
   b, s, n = q.shape
@@ -222,7 +244,7 @@ def norm_rope_fullrow_backward(q, k, wq, wk, cos, sin, heads: int, gq, gk, eps: 
     raise ValueError("k must match q in shape, dtype and strides")
   if has_k != (gk is not None):
     raise ValueError("gk must be given exactly when k is")
-  cos, sin = _table(cos, s, d, "cos"), _table(sin, s, d, "sin")
+  pcos, psin, kind = _table_args(cos, sin, s, d)
   gq = _grad_view(gq, (b, s, heads, d), "gq")
   if has_k:
     gk = _grad_view(gk, (b, s, heads, d), "gk")
@@ -242,9 +264,9 @@ def norm_rope_fullrow_backward(q, k, wq, wk, cos, sin, heads: int, gq, gk, eps: 
   dbias = torch.empty(2 * n, dtype=torch.float32, device=q.device) if bias is not None else None
   ws, nws = _bwd_workspace(b * s, (2 if has_k else 1) * (2 if bias is not None else 1) * n, q.device)
   st = _strides(gq)
-  rc = _lib.load().mdattn_norm_rope_fullrow_bwd(
+  rc = _lib.load().mdattn_host_norm_rope_fullrow_bwd(
       _stream(), _ptr(q), _ptr(k), _ptr(bias), _ptr(gq), _ptr(gk), _ptr(dq), _ptr(dk), _ptr(wq), _ptr(wk), _ptr(dwq), _ptr(dwk),
-      _ptr(dbias), _ptr(cos), _ptr(sin), b, s, heads, d, eps, q_mul, q.stride(0), q.stride(1), dq.stride(0), dq.stride(1),
+      _ptr(dbias), pcos, psin, kind, b, s, heads, d, eps, q_mul, q.stride(0), q.stride(1), dq.stride(0), dq.stride(1),
       ctypes.byref(st), _ptr(ws), nws)
   _lib.check(rc, "mdattn_norm_rope_fullrow_bwd")
   return (dq, dk, dwq, dwk) if bias is None else (dq, dk, dwq, dwk, dbias)
@@ -255,7 +277,7 @@ def norm_rope_perhead_backward(q, k, wq, wk, cos, sin, gq, gk, eps: float = 1e-6
   """Backward of `norm_rope_perhead`: q, k the saved bf16 logical [B,S,H,D] inputs (k may be None), gq, gk the
   gradients of its outputs.  Returns (dq, dk, dwq, dwk, dwq_txt, dwk_txt): dq, dk bf16 laid out like q; the weight
   gradients f32 [D] (the *_txt ones None when no text weights were given)."""
-  _check_dev(q, k, wq, wk, wq_txt, wk_txt, cos, sin, gq, gk)
+  _check_dev(q, k, wq, wk, wq_txt, wk_txt, gq, gk)
   if q.dtype != torch.bfloat16:
     raise ValueError("q must be bf16")
   b, s, h, d = q.shape
@@ -264,7 +286,7 @@ def norm_rope_perhead_backward(q, k, wq, wk, cos, sin, gq, gk, eps: float = 1e-6
     raise ValueError("k must match q in shape, dtype and strides")
   if has_k != (gk is not None):
     raise ValueError("gk must be given exactly when k is")
-  cos, sin = _table(cos, s, d, "cos"), _table(sin, s, d, "sin")
+  pcos, psin, kind = _table_args(cos, sin, s, d)
   gq = _grad_view(gq, q.shape, "gq")
   if has_k:
     gk = _grad_view(gk, q.shape, "gk")
@@ -278,9 +300,9 @@ def norm_rope_perhead_backward(q, k, wq, wk, cos, sin, gq, gk, eps: float = 1e-6
   dwk_t = f32() if (wk_txt is not None and has_k) else None
   ws, nws = _bwd_workspace(b * s * h, 4 * d, q.device)
   si, sd, sg = _strides(q), _strides(dq), _strides(gq)
-  rc = _lib.load().mdattn_norm_rope_perhead_bwd(
+  rc = _lib.load().mdattn_host_norm_rope_perhead_bwd(
       _stream(), _ptr(q), _ptr(k), _ptr(gq), _ptr(gk), _ptr(dq), _ptr(dk), _ptr(wq), _ptr(wk), _ptr(wq_txt),
-      _ptr(wk_txt if has_k else None), n_txt, _ptr(dwq), _ptr(dwk), _ptr(dwq_t), _ptr(dwk_t), _ptr(cos), _ptr(sin), b, s, h, d, eps, q_mul,
+      _ptr(wk_txt if has_k else None), n_txt, _ptr(dwq), _ptr(dwk), _ptr(dwq_t), _ptr(dwk_t), pcos, psin, kind, b, s, h, d, eps, q_mul,
       ctypes.byref(si), ctypes.byref(sd), ctypes.byref(sg), _ptr(ws), nws)
   _lib.check(rc, "mdattn_norm_rope_perhead_bwd")
   return dq, dk, dwq, dwk, dwq_t, dwk_t

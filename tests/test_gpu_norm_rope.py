@@ -226,3 +226,32 @@ def test_fused_qkv_rejects_a_bias_without_a_value_output(dev, lib):
   assert lib.mdattn_norm_rope_qkv(*args(fake, None, 1536)) == _lib.E_BADARG      # bias but nowhere to put v + bias
   assert lib.mdattn_norm_rope_qkv(*args(None, None, 1024)) == _lib.E_BADARG      # row stride below 3*H*D
   assert lib.mdattn_norm_rope_qkv(*args(P(0x1004), fake, 1536)) == _lib.E_ALIGN
+
+
+@pytest.mark.parametrize("form", ["complex", "repeated", "matrix"])
+@pytest.mark.parametrize("D,S", [(128, 37), (64, 130)])
+def test_rotary_tables_are_read_in_the_layout_the_model_made(dev, form, D, S):
+  """The hooks read a table in place; forward and backward equal, bit for bit, those on the planes split from it."""
+  from maxdiffusion_amd import attention_op as A
+  B, H = 2, 3
+  gen = torch.Generator(device=dev).manual_seed(D + S)
+  rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)
+  ang = torch.rand((S, D // 2), generator=gen, device=dev) * 6.28
+  cos, sin = torch.cos(ang), torch.sin(ang)
+  table = {"complex": torch.complex(cos, sin)[None, None],
+           "repeated": tuple(t.repeat_interleave(2, dim=1) for t in (cos, sin)),
+           "matrix": torch.stack([cos, -sin, sin, cos], dim=-1).reshape(S, D // 2, 2, 2)}[form]
+  for per_head in (False, True):
+    x = [rnd(B, S, H, D) if per_head else rnd(B, S, H * D) for _ in range(2)]
+    w = [(1 + 0.1 * rnd(D if per_head else H * D).float()).to(torch.bfloat16) for _ in range(2)]
+    g = [rnd(B, S, H, D) for _ in range(2)]
+    assert A._rope_table(table, S, D, per_head).kind == {"complex": 1, "repeated": 2, "matrix": 3}[form] or not (per_head or form == "complex")
+    leaves = [t.clone().requires_grad_(True) for t in (*x, *w)]
+    out = A.hip_norm_rope(*leaves, table, H, per_head=per_head)
+    got = torch.autograd.grad(out, leaves, g)
+    if per_head:
+      want, back = ops.norm_rope_perhead(*x, *w, cos, sin), ops.norm_rope_perhead_backward(*x, *w, cos, sin, *g)[:4]
+    else:
+      want, back = ops.norm_rope_fullrow(*x, *w, cos, sin, H), ops.norm_rope_fullrow_backward(*x, *w, cos, sin, H, *g)
+    assert all(torch.equal(a, b) for a, b in zip(out, want))
+    assert all(torch.equal(a, b.to(torch.bfloat16)) for a, b in zip(got, back))
