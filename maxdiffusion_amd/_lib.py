@@ -95,6 +95,29 @@ def load() -> ctypes.CDLL:
   return _lib
 
 
+_host = None
+
+
+def host():
+  """The C++ host path (csrc/host/torch_host.cc).  Loaded once, after libmdattn.so; raises if it has not been built."""
+  global _host
+  if _host is None:
+    lib = load()
+    from . import build
+
+    if not os.path.exists(build.HOST_EXT_PATH):
+      raise RuntimeError(f"{build.HOST_EXT_PATH} is missing: build it with `python -m maxdiffusion_amd.build`")
+    import importlib
+
+    import torch  # noqa: F401  (its libraries before ours)
+
+    ext = importlib.import_module("." + build.HOST_EXT_NAME, __package__)
+    if ext.build_id() != lib.mdattn_build_id().decode():
+      raise RuntimeError(f"{build.HOST_EXT_PATH} was built from other sources than libmdattn.so: rebuild with `python -m maxdiffusion_amd.build`")
+    _host = ext
+  return _host
+
+
 def strerror(code: int) -> str:
   return load().mdattn_strerror(code).decode()
 

@@ -19,7 +19,7 @@ import math
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 __all__ = [
     "KERNEL_REGISTRY", "register_kernel", "AttentionOp", "hip_flash_kernel", "hip_flash_fp8_kernel",
@@ -94,6 +94,10 @@ def _mask_bias(context, qv, kv):
 FOLD_SCALE_MIN_KEYS = 16384
 
 
+def _folds_scale(keys: int, d: int, scale: float) -> bool:
+  return keys * 128 >= FOLD_SCALE_MIN_KEYS * d and abs(scale * math.log2(math.e) - 1.0) > 1e-6
+
+
 def _pad_head_dim(qv, kv, vv):
   """Head dims below 128 other than 64 are zero-padded to the next size the kernels take (64 or 128), as the
   reference's flash wrappers pad them to 128 (attention_flax.py:223-259, `_pad_data_for_flash`): zero columns of q and
@@ -150,6 +154,18 @@ def hip_flash_kernel(q, k, v, context):
   """
   _reject_unsupported(context)
   heads = context["heads"]
+  scale = context["scale"]
+  mask = context.get("attention_mask")
+  if q.is_cuda:
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+      out = _lib.host().flash_autograd(q, k, v, heads, scale, mask)
+    else:
+      folds = mask is None and _folds_scale(k.shape[-2] if k.dim() == 4 else k.shape[1], q.shape[-1] if q.dim() == 4 else q.shape[-1] // heads, scale)
+      out = ops.flash_attention(q, k, v, scale=ops.FOLDED_SCALE if folds else scale, heads=heads, keep=mask,
+                                q_mul=scale * math.log2(math.e) if folds else 1.0)
+    if out is not None:
+      return out
+  # what the native path leaves: other dtypes, head dims to be padded, views to be copied, and every error
   qv, kv, vv = _as_bshd(q, heads), _as_bshd(k, heads), _as_bshd(v, heads)
   # LTX2 hands f32 q/k next to a v in the model dtype (norm dtype f32, attention_ltx2.py:415-432); the MFMA operands are
   # bf16.  Each such cast is one more pass over the tensor in HBM: `hip_norm_rope_ltx2` in front of this entry emits
@@ -160,18 +176,16 @@ def hip_flash_kernel(q, k, v, context):
   # segment ids (:390-438); rows without a kept key return 0 (:1552-1554)
   bias = _mask_bias(context, qv, kv)
   qv, kv, vv, d0 = _pad_head_dim(qv, kv, vv)
-  scale = context["scale"]
   if torch.is_grad_enabled() and (qv.requires_grad or kv.requires_grad or vv.requires_grad):
     out = hip_flash_attention_autograd(qv, kv, vv, scale, bias)
   else:
-    c = scale * math.log2(math.e)
-    if bias is None and kv.shape[1] * 128 >= FOLD_SCALE_MIN_KEYS * qv.shape[-1] and abs(c - 1.0) > 1e-6:
+    if bias is None and _folds_scale(kv.shape[1], qv.shape[-1], scale):
       # Long key sequences: q * (scale * log2 e), rounded to bf16 once, then scale = ln 2, on which the kernels drop the
       # multiply per logit (3.5 % of the launch at head dim 128, 7 % at 64) for one pass over q.  The reference's flash
       # wrappers round the same factors into their operands (k * scale and q * log2 e in bf16,
       # attention_flax.py:1783, :610).  Callers that apply the fused prologue with q_mul arrive here with scale = ln 2
       # already and skip this.
-      qv, scale = qv * c, ops.FOLDED_SCALE
+      qv, scale = qv * (scale * math.log2(math.e)), ops.FOLDED_SCALE
     out = ops.flash_attention(qv, kv, vv, scale=scale, key_bias=bias)
   b, s, h, d = out.shape
   out = out[..., :d0].reshape(b, s, h * d0)
@@ -294,7 +308,14 @@ class _HipNormRopeRows(torch.autograd.Function):
     return dx, dw, None, None, None, None, None
 
 
+_ROWS_MODES = {"none": 0, "interleaved": 1, "split": 2}
+
+
 def _norm_rope_rows(x, w, cos, sin, heads, mode, eps):
+  if x.is_cuda:
+    out = _lib.host().norm_rope_rows(x, w, cos, sin, heads, _ROWS_MODES[mode], eps)
+    if out is not None:
+      return out
   if _wants_grad(x, w):
     return _HipNormRopeRows.apply(x, w, cos, sin, heads, mode, eps)
   return ops.norm_rope_rows(x, w, cos, sin, heads=heads, mode=mode, eps=eps)
@@ -307,6 +328,10 @@ def hip_norm_rope_qkv(qkv, wq, wk, freqs_cis, heads: int, bias=None, eps: float 
   returns (q, k, v) logical [B,S,H,D] for `hip_flash`.  `bias`: the three Linear biases [3*H*D] when the GEMM ran
   without them.  Differentiable with respect to qkv, bias and the norm weights; `inplace=True` (the fused buffer
   itself becomes the three operands) is for inference only, since the backward needs the projection output."""
+  if qkv.is_cuda and bias is not None and not inplace and out_layout in _LAYOUTS:
+    out = _lib.host().norm_rope_qkv(qkv, bias, wq, wk, *_table_pair(freqs_cis), heads, eps, q_mul, out_layout == "bhsd")
+    if out is not None:
+      return tuple(out)
   b, s, n3 = qkv.shape
   table = _rope_table(freqs_cis, s, n3 // 3 // heads)
   if _wants_grad(qkv, wq, wk, bias):
@@ -537,6 +562,13 @@ def _rope_table(freqs_cis, seq: int, d: int, per_head: bool = False):
   return ops.RopeTable(*_split_table(freqs_cis, seq, d), 0)
 
 
+_LAYOUTS = ("bshd", "bhsd")
+
+
+def _table_pair(freqs_cis):
+  return freqs_cis if isinstance(freqs_cis, (tuple, list)) else (freqs_cis, None)
+
+
 def _saved_table(table):
   return (None, None, 0) if table is None else (table.cos, table.sin, table.kind)
 
@@ -554,6 +586,14 @@ def hip_norm_rope(q, k, wq, wk, freqs_cis, heads: int, eps: float = 1e-6, per_he
   context["scale"]=ops.FOLDED_SCALE the softmax scale is carried by the prologue, where the reference carries it by
   two bf16 multiplies of k and q (:1783, :610), and the attention kernel saves its multiply per logit.
   """
+  if q.is_cuda and out_layout in _LAYOUTS:
+    host, bhsd = _lib.host(), out_layout == "bhsd"
+    if per_head:
+      out = host.norm_rope_perhead(q, k, wq, wk, wq_txt, wk_txt, n_txt, *_table_pair(freqs_cis), eps, q_mul, bhsd)
+    else:
+      out = host.norm_rope(q, k, wq, wk, *_table_pair(freqs_cis), heads, eps, q_mul, bhsd)
+    if out is not None:
+      return (out[0], out[1] if k is not None else None)
   if per_head:
     b, s, h, d = q.shape
     table = _rope_table(freqs_cis, s, d, per_head=True)

@@ -15,6 +15,8 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libmdattn.so")
 FFI_LIB_PATH = os.path.join(PKG_DIR, "libmdattn_ffi.so")
+HOST_EXT_NAME = "_mdattn_torch"
+HOST_EXT_PATH = os.path.join(PKG_DIR, HOST_EXT_NAME + ".so")  # the torch-side host path in C++ (csrc/host/torch_host.cc)
 
 SOURCES = ["mdattn_api.hip", "norm_rope.hip", "norm_rope_bwd.hip", "attn_fwd_bf16.hip", "attn_fwd_fp8.hip", "attn_bwd_bf16.hip", "merge_quant.hip", "probes.hip",
            # the bodies of the XLA custom-call handlers on plain structs (no XLA header): part of the library
@@ -92,7 +94,7 @@ def source_id() -> str:
 
   h = hashlib.sha256(" ".join(HIPCC_FLAGS).encode())
   files = [os.path.join(CSRC, f) for f in sorted(os.listdir(CSRC)) if f.endswith((".hip", ".h"))]
-  for path in files + [os.path.join(CSRC, "ffi", "mdattn_marshal.cc"), os.path.join(INCLUDE, "mdattn.h"), os.path.join(INCLUDE, "mdattn_marshal.h")]:
+  for path in files + [os.path.join(CSRC, "ffi", "mdattn_marshal.cc"), os.path.join(CSRC, "host", "torch_host.cc"), os.path.join(INCLUDE, "mdattn.h"), os.path.join(INCLUDE, "mdattn_marshal.h")]:
     h.update(os.path.basename(path).encode())
     with open(path, "rb") as f:
       h.update(f.read())
@@ -116,8 +118,9 @@ def built_library_id(path: str | None = None) -> str | None:
 
 
 def library_is_current() -> bool:
-  """True when libmdattn.so exists and was built from the sources in this tree."""
-  return built_library_id() == source_id()
+  """True when libmdattn.so (and, where torch is installed, the host extension) exists and was built from the sources in
+  this tree."""
+  return built_library_id() == source_id() and (built_library_id(HOST_EXT_PATH) == source_id() or not _has_torch())
 
 
 def ensure_built(verbose: bool = True) -> str:
@@ -128,8 +131,65 @@ def ensure_built(verbose: bool = True) -> str:
   return LIB_PATH
 
 
+def _has_torch() -> bool:
+  import importlib.util
+
+  return importlib.util.find_spec("torch") is not None
+
+
+def _start_host_extension():
+  """Starts the compiler on csrc/host/torch_host.cc (host code only: g++); None where torch is absent."""
+  if not _has_torch():
+    return None
+  import sysconfig
+
+  from torch.utils.cpp_extension import include_paths
+
+  obj = HOST_EXT_PATH + f".{os.getpid()}.o"
+  cmd = [shutil.which("g++") or "g++", "-c", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+         f"-DTORCH_EXTENSION_NAME={HOST_EXT_NAME}", f'-DMDATTN_BUILD_ID="{source_id()}"', f"-I{INCLUDE}", f"-I{CSRC}", "-I/opt/rocm/include",
+         *[f"-isystem{p}" for p in include_paths()], f"-I{sysconfig.get_paths()['include']}",
+         os.path.join(CSRC, "host", "torch_host.cc"), "-o", obj]
+  return obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+
+
+def _finish_host_extension(job, verbose: bool) -> None:
+  from torch.utils.cpp_extension import library_paths
+
+  obj, proc = job
+  log, _ = proc.communicate()
+  try:
+    if proc.returncode != 0:
+      raise RuntimeError(f"g++ failed on csrc/host/torch_host.cc ({proc.returncode}):\n{log}")
+    tmp = HOST_EXT_PATH + f".{os.getpid()}.tmp"
+    link = [shutil.which("g++") or "g++", "-shared", obj, "-o", tmp, f"-L{PKG_DIR}", "-l:libmdattn.so", "-Wl,-rpath,$ORIGIN",
+            *[f"-L{p}" for p in library_paths()], "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(link, capture_output=True, text=True)
+    if r.returncode != 0:
+      raise RuntimeError(f"linking {HOST_EXT_PATH} failed ({r.returncode}):\n{r.stdout}{r.stderr}")
+    os.replace(tmp, HOST_EXT_PATH)
+    if verbose:
+      print(f"[maxdiffusion_amd.build] {HOST_EXT_PATH}", flush=True)
+  finally:
+    if os.path.exists(obj):
+      os.remove(obj)
+
+
 def build_library(verbose: bool = True) -> str:
-  """Compile every HIP source into maxdiffusion_amd/libmdattn.so.  Always recompiles."""
+  """Compile every HIP source into maxdiffusion_amd/libmdattn.so, and the host extension beside it.  Always recompiles."""
+  host = _start_host_extension()
+  try:
+    _build_hip(verbose)
+  except BaseException:
+    if host is not None:
+      host[1].kill()
+    raise
+  if host is not None:
+    _finish_host_extension(host, verbose)
+  return LIB_PATH
+
+
+def _build_hip(verbose: bool) -> str:
   # Linked under another name and moved into place: a process that has the previous library mapped keeps its own
   # file, and a later dlopen of the path finds the new one instead of the handle it already holds.
   tmp = LIB_PATH + f".{os.getpid()}.tmp"

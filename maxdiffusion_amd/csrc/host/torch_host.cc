@@ -1,0 +1,508 @@
+// The torch-side host path in C++: what ops.py and attention_op.py do around a C-ABI call (checks, strides, allocation,
+// the stream, the autograd node), for the inputs that need nothing unusual.  Every function returns None for any other
+// input -- another dtype, a CPU tensor, a shape the kernels refuse -- and the Python path beside the call takes over and
+// raises or converts as it always did; nothing is computed here that the kernels do not compute.
+//
+// Why native: a call of the smallest size is host time (4 heads x 126 tokens: 10 us of kernels).  The Python path took
+// 36.7 us for prologue + attention (ctypes' conversion of twenty arguments, four stride structs, the checks), this one
+// 16.5; a training step's backward runs in autograd's own thread without the interpreter: 255-465 us of host time per
+// step become 91-108.
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <pybind11/stl.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <array>
+#include <cmath>
+#include <optional>
+
+#include "mdattn.h"
+#include "mdattn_host.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+const void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+void* mut(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+float* f32(const Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
+
+Tensor value(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+// autograd's apply() takes an argument that may be missing as an optional, never as an undefined tensor
+OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; }
+bool bf16_on(const Tensor& t, const Tensor& ref) {
+  return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.get_device() == ref.get_device() && !t.is_neg();
+}
+bool wants_grad(std::initializer_list<const Tensor*> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : ts)
+    if (t->defined() && t->requires_grad()) return true;
+  return false;
+}
+// a backward call that the checks of its forward should have made impossible to fail
+void must(int rc, const char* where) { TORCH_CHECK(rc == MDATTN_OK, where, ": mdattn error ", rc, ": ", mdattn_strerror(rc)); }
+
+// [B,S,H,D] as the kernels walk it, over a rank-3 [B,S,H*D] or a rank-4 [B,H,S,D] tensor (attention_op._as_bshd)
+struct View {
+  int64_t b = 0, s = 0, h = 0, d = 0;
+  mdattn_strides st{0, 0, 0};
+};
+std::optional<View> as_view(const Tensor& t, int64_t heads) {
+  View v;
+  if (t.dim() == 3) {
+    const int64_t n = t.size(2);
+    if (t.stride(2) != 1 || heads <= 0 || n % heads) return std::nullopt;
+    v.b = t.size(0); v.s = t.size(1); v.h = heads; v.d = n / heads;
+    v.st = {t.stride(0), t.stride(1), v.d};
+  } else if (t.dim() == 4) {
+    if (t.stride(3) != 1) return std::nullopt;
+    v.b = t.size(0); v.h = t.size(1); v.s = t.size(2); v.d = t.size(3);
+    v.st = {t.stride(0), t.stride(2), t.stride(1)};
+  } else {
+    return std::nullopt;
+  }
+  return v;
+}
+// a logical [B,S,H,D] tensor
+mdattn_strides strides4(const Tensor& t) { return {t.stride(0), t.stride(1), t.stride(2)}; }
+
+Tensor alloc_bshd(const Tensor& like, int64_t b, int64_t s, int64_t h, int64_t d, bool bhsd) {
+  return bhsd ? at::empty({b, h, s, d}, like.options().dtype(at::kBFloat16)).permute({0, 2, 1, 3})
+              : at::empty({b, s, h, d}, like.options().dtype(at::kBFloat16));
+}
+// A gradient as the kernels read it: bf16, last axis contiguous, with the strides of `like` when given.
+Tensor grad_like(const Tensor& g, const Tensor& like) {
+  Tensor x = g.scalar_type() == at::kBFloat16 ? g : g.to(at::kBFloat16);
+  if (like.defined()) return x.strides() == like.strides() ? x : at::empty_strided(like.sizes(), like.strides(), x.options()).copy_(x);
+  return x.stride(-1) == 1 ? x : x.contiguous();
+}
+
+// ------------------------------------------------------------------------------------------------ attention
+int fwd(const Tensor& q, const Tensor& k, const Tensor& v, const View& vq, const View& vk, const View& vv, const Tensor& out, const Tensor& lse,
+        const Tensor& bias, double scale) {
+  const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
+  if (bias.defined())
+    return mdattn_fwd_bf16_bias(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st,
+                                &vk.st, &vv.st, &so, (float)scale, f32(bias), bias.stride(0));
+  return mdattn_fwd_bf16(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st, &vk.st,
+                         &vv.st, &so, (float)scale);
+}
+
+// q, k, v in the caller's own rank; out [B,Sq,H*D]
+struct FlashFn : torch::autograd::Function<FlashFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& bias_, int64_t heads, double scale) {
+    const Tensor bias = value(bias_);
+    const View vq = *as_view(q, heads), vk = *as_view(k, heads), vv = *as_view(v, heads);
+    Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
+    Tensor lse = at::empty({vq.b, vq.h, vq.s}, q.options().dtype(at::kFloat));
+    must(fwd(q, k, v, vq, vk, vv, out, lse, bias, scale), "mdattn_fwd_bf16");
+    ctx->save_for_backward({q, k, v, out, lse, bias});
+    ctx->saved_data["heads"] = heads;
+    ctx->saved_data["scale"] = scale;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &bias = saved[5];
+    const int64_t heads = ctx->saved_data["heads"].toInt();
+    const double scale = ctx->saved_data["scale"].toDouble();
+    const View vq = *as_view(q, heads), vk = *as_view(k, heads), vv = *as_view(v, heads);
+    const Tensor dout = grad_like(grads[0], out);
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    const int B = (int)vq.b, H = (int)vq.h, Sq = (int)vq.s, Skv = (int)vk.s, D = (int)vq.d;
+    const int64_t nws = mdattn_bwd_split_workspace_floats(B, H, Sq, Skv, D);
+    Tensor ws = at::empty({nws}, lse.options());
+    const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
+    const int rc = bias.defined()
+        ? mdattn_bwd_bf16_bias(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq, Skv,
+                               D, &vq.st, &vk.st, &vv.st, &so, (float)scale, f32(bias), bias.stride(0))
+        : mdattn_bwd_bf16(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq, Skv, D,
+                          &vq.st, &vk.st, &vv.st, &so, (float)scale);
+    must(rc, "mdattn_bwd_bf16");
+    return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
+  }
+};
+
+// [B,Skv] keep-mask (bool or uint8) -> additive bias f32 [B, ceil32(Skv)], or undefined when the mask needs the Python path
+Tensor mask_bias(const Tensor& keep, const View& vk, const Tensor& ref) {
+  if (!keep.is_cuda() || keep.get_device() != ref.get_device() || (keep.scalar_type() != at::kBool && keep.scalar_type() != at::kByte) ||
+      keep.dim() != 2 || keep.size(0) != vk.b || keep.size(1) != vk.s || !keep.is_contiguous())
+    return Tensor();
+  const int64_t cols = (vk.s + 31) / 32 * 32;
+  Tensor bias = at::empty({vk.b, cols}, keep.options().dtype(at::kFloat));
+  if (mdattn_key_mask_bias(stream(), ptr(keep), f32(bias), (int)vk.b, (int)vk.s, cols, -INFINITY) != MDATTN_OK) return Tensor();
+  return bias;
+}
+
+// The registry entry's operands, checked: false when the Python path has to take over
+bool flash_args(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep, View& vq, View& vk, View& vv,
+                Tensor& bias) {
+  if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q)) return false;
+  const auto a = as_view(q, heads), b = as_view(k, heads), c = as_view(v, heads);
+  if (!a || !b || !c || (a->d != 64 && a->d != 128) || a->b != b->b || a->b != c->b || a->h != b->h || a->h != c->h || a->d != b->d || a->d != c->d ||
+      b->s != c->s || !(scale > 0))
+    return false;
+  if (q.numel() == 0 || k.numel() == 0 || std::max(a->s, b->s) >= ((int64_t)1 << 31)) return false;
+  if (keep.has_value() && !(bias = mask_bias(*keep, *b, q)).defined()) return false;
+  vq = *a; vk = *b; vv = *c;
+  return true;
+}
+
+// The registry entry `hip_flash`: [B,S,H*D] or [B,H,S,D] operands -> [B,Sq,H*D]; q_mul is rounded into q first.
+OptTensor flash(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep, double q_mul) {
+  View vq, vk, vv;
+  Tensor bias;
+  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, bias)) return std::nullopt;
+  at::NoGradGuard guard;
+  Tensor qf = q;
+  if (q_mul != 1.0) {
+    qf = q.mul(q_mul);
+    const auto w = as_view(qf, heads);
+    if (!w) return std::nullopt;
+    vq = *w;
+  }
+  Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
+  if (fwd(qf, k, v, vq, vk, vv, out, Tensor(), bias, scale) != MDATTN_OK) return std::nullopt;
+  return out;
+}
+
+OptTensor flash_autograd(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep) {
+  View vq, vk, vv;
+  Tensor bias;
+  for (const Tensor* t : {&q, &k, &v})
+    if (!t->is_non_overlapping_and_dense()) return std::nullopt;  // their gradients take the same strides
+  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, bias)) return std::nullopt;
+  return FlashFn::apply(q, k, v, opt(bias), heads, scale);
+}
+
+// One ring step (ops.flash_attention_merge) on logical [B,S,H,D] views; false: the Python path takes it
+bool flash_merge(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o_run, const Tensor& lse_run, double scale) {
+  if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q) || q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || o_run.dim() != 4)
+    return false;
+  if (q.stride(3) != 1 || k.stride(3) != 1 || v.stride(3) != 1 || o_run.stride(3) != 1 || k.sizes() != v.sizes() || k.size(0) != q.size(0) ||
+      k.size(2) != q.size(2) || k.size(3) != q.size(3) || o_run.sizes() != q.sizes() || o_run.scalar_type() != at::kFloat || !o_run.is_cuda() ||
+      lse_run.scalar_type() != at::kFloat || !lse_run.is_cuda() || !lse_run.is_contiguous() || lse_run.dim() != 3 || lse_run.size(0) != q.size(0) ||
+      lse_run.size(1) != q.size(2) || lse_run.size(2) != q.size(1))
+    return false;
+  const mdattn_strides sq = strides4(q), sk = strides4(k), sv = strides4(v), so = strides4(o_run);
+  return mdattn_fwd_bf16_merge(stream(), ptr(q), ptr(k), ptr(v), f32(o_run), f32(lse_run), (int)q.size(0), (int)q.size(2), (int)q.size(1),
+                               (int)k.size(1), (int)q.size(3), &sq, &sk, &sv, &so, (float)scale) == MDATTN_OK;
+}
+
+// ------------------------------------------------------------------------------------------------ prologues
+// A rotary table in one of the layouts that the kernels read in place (attention_op._rope_table)
+struct Table {
+  Tensor cos, sin;
+  int64_t kind = MDATTN_TABLE_PLANES;
+};
+bool in_place(const Tensor& t, at::ScalarType dtype, int64_t numel, const Tensor& ref) {
+  return t.is_cuda() && t.get_device() == ref.get_device() && t.scalar_type() == dtype && t.is_contiguous() && t.numel() == numel &&
+         !t.is_conj() && !t.is_neg() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+}
+std::optional<Table> as_table(const OptTensor& a, const OptTensor& b, int64_t s, int64_t d, bool per_head, const Tensor& ref) {
+  Table t;
+  if (!a.has_value()) return t;
+  if (b.has_value()) {  // a (cos, sin) tuple
+    if (per_head && in_place(*a, at::kFloat, s * d, ref) && in_place(*b, at::kFloat, s * d, ref)) t.kind = MDATTN_TABLE_REPEATED;
+    else if (in_place(*a, at::kFloat, s * d / 2, ref) && in_place(*b, at::kFloat, s * d / 2, ref)) t.kind = MDATTN_TABLE_PLANES;
+    else return std::nullopt;
+    t.sin = *b;
+  } else if (in_place(*a, at::kComplexFloat, s * d / 2, ref)) {
+    t.kind = MDATTN_TABLE_COMPLEX;
+  } else if (per_head && in_place(*a, at::kFloat, s * d * 2, ref)) {
+    t.kind = MDATTN_TABLE_MATRIX;
+  } else {
+    return std::nullopt;
+  }
+  t.cos = *a;
+  return t;
+}
+const float* table_ptr(const Tensor& t) { return t.defined() ? static_cast<const float*>(t.data_ptr()) : nullptr; }
+bool weight_ok(const Tensor& w, int64_t n, const Tensor& ref) { return bf16_on(w, ref) && w.is_contiguous() && w.numel() == n; }
+
+struct Prologue {
+  int64_t heads, kind, n_txt = 0;
+  double eps, q_mul;
+  bool bhsd;
+  void save(AutogradContext* ctx) const {
+    ctx->saved_data["i"] = c10::List<int64_t>({heads, kind, n_txt});
+    ctx->saved_data["f"] = c10::List<double>({eps, q_mul});
+  }
+  static Prologue saved(AutogradContext* ctx) {
+    const auto i = ctx->saved_data["i"].toIntVector();
+    const auto f = ctx->saved_data["f"].toDoubleVector();
+    return {i[0], i[1], i[2], f[0], f[1], false};
+  }
+};
+
+// Wan: q, k [B,S,H*D] (k may be undefined) -> {q_out(, k_out)} or empty when a kernel refuses the request
+variable_list fullrow_run(const Tensor& q, const Tensor& k, const Tensor& wq, const Tensor& wk, const Tensor& cos, const Tensor& sin, const Prologue& p) {
+  const int64_t b = q.size(0), s = q.size(1), d = q.size(2) / p.heads;
+  Tensor qo = alloc_bshd(q, b, s, p.heads, d, p.bhsd), ko = k.defined() ? alloc_bshd(q, b, s, p.heads, d, p.bhsd) : Tensor();
+  const mdattn_strides so = strides4(qo);
+  const int rc = mdattn_host_norm_rope_fullrow(stream(), ptr(q), ptr(k), mut(qo), mut(ko), ptr(wq), ptr(wk), table_ptr(cos), table_ptr(sin), (int)p.kind,
+                                               (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps, (float)p.q_mul, q.stride(0), q.stride(1), &so);
+  if (rc != MDATTN_OK) return {};
+  return k.defined() ? variable_list{qo, ko} : variable_list{qo};
+}
+struct FullrowFn : torch::autograd::Function<FullrowFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const OptTensor& k_, const Tensor& wq, const OptTensor& wk_,
+                               const OptTensor& cos_, const OptTensor& sin_, const Prologue& p) {
+    const Tensor k = value(k_), wk = value(wk_), cos = value(cos_), sin = value(sin_);
+    variable_list out = fullrow_run(q, k, wq, wk, cos, sin, p);
+    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_fullrow refused the request");
+    ctx->save_for_backward({q, k, wq, wk, cos, sin});
+    p.save(ctx);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    const auto sv = ctx->get_saved_variables();
+    const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3];
+    const Prologue p = Prologue::saved(ctx);
+    const int64_t b = q.size(0), s = q.size(1), n = q.size(2), d = n / p.heads;
+    const bool has_k = k.defined();
+    const Tensor gq = grad_like(g[0], Tensor());
+    const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
+    Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = has_k ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
+    const auto fo = q.options().dtype(at::kFloat);
+    Tensor dwq = at::empty({n}, fo), dwk = has_k ? at::empty({n}, fo) : Tensor();
+    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, (has_k ? 2 : 1) * n);
+    Tensor ws = at::empty({nws}, fo);
+    const mdattn_strides sg = strides4(gq);
+    must(mdattn_host_norm_rope_fullrow_bwd(stream(), ptr(q), ptr(k), nullptr, ptr(gq), ptr(gk), mut(dq), mut(dk), ptr(wq), ptr(wk), f32(dwq), f32(dwk),
+                                           nullptr, table_ptr(sv[4]), table_ptr(sv[5]), (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps,
+                                           (float)p.q_mul, q.stride(0), q.stride(1), dq.stride(0), dq.stride(1), &sg, f32(ws), nws),
+         "mdattn_norm_rope_fullrow_bwd");
+    return {dq, dk, dwq.to(wq.scalar_type()), has_k ? dwk.to(wk.scalar_type()) : Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::optional<variable_list> norm_rope(const Tensor& q, const OptTensor& k_, const Tensor& wq, const OptTensor& wk_, const OptTensor& fa, const OptTensor& fb,
+                                       int64_t heads, double eps, double q_mul, bool bhsd) {
+  const Tensor k = value(k_), wk = value(wk_);
+  if (!q.is_cuda() || !bf16_on(q, q) || q.dim() != 3 || q.numel() == 0 || q.stride(2) != 1 || heads <= 0 || q.size(2) % heads) return std::nullopt;
+  const int64_t n = q.size(2);
+  if (!weight_ok(wq, n, q)) return std::nullopt;
+  if (k.defined() && (!bf16_on(k, q) || k.sizes() != q.sizes() || k.strides() != q.strides() || !wk.defined() || !weight_ok(wk, n, q))) return std::nullopt;
+  const auto t = as_table(fa, fb, q.size(1), n / heads, false, q);
+  if (!t) return std::nullopt;
+  const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
+  if (wants_grad({&q, &k, &wq, &wk})) {
+    if (!q.is_non_overlapping_and_dense()) return std::nullopt;
+    return FullrowFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(t->cos), opt(t->sin), p);
+  }
+  variable_list out = fullrow_run(q, k, wq, wk, t->cos, t->sin, p);
+  if (out.empty()) return std::nullopt;
+  return out;
+}
+
+// Flux: q, k logical [B,S,H,D]
+variable_list perhead_run(const Tensor& q, const Tensor& k, const Tensor& wq, const Tensor& wk, const Tensor& wqt, const Tensor& wkt, const Tensor& cos,
+                          const Tensor& sin, const Prologue& p) {
+  const int64_t b = q.size(0), s = q.size(1), h = q.size(2), d = q.size(3);
+  Tensor qo = alloc_bshd(q, b, s, h, d, p.bhsd), ko = k.defined() ? alloc_bshd(q, b, s, h, d, p.bhsd) : Tensor();
+  const mdattn_strides si = strides4(q), so = strides4(qo);
+  const int rc = mdattn_host_norm_rope_perhead(stream(), ptr(q), ptr(k), mut(qo), mut(ko), ptr(wq), ptr(wk), ptr(wqt), ptr(wkt), (int)p.n_txt,
+                                               table_ptr(cos), table_ptr(sin), (int)p.kind, (int)b, (int)s, (int)h, (int)d, (float)p.eps, (float)p.q_mul,
+                                               &si, &so);
+  if (rc != MDATTN_OK) return {};
+  return k.defined() ? variable_list{qo, ko} : variable_list{qo};
+}
+struct PerheadFn : torch::autograd::Function<PerheadFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const OptTensor& k_, const Tensor& wq, const OptTensor& wk_, const OptTensor& wqt_,
+                               const OptTensor& wkt_, const OptTensor& cos_, const OptTensor& sin_, const Prologue& p) {
+    const Tensor k = value(k_), wk = value(wk_), wqt = value(wqt_), wkt = value(wkt_), cos = value(cos_), sin = value(sin_);
+    variable_list out = perhead_run(q, k, wq, wk, wqt, wkt, cos, sin, p);
+    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_perhead refused the request");
+    ctx->save_for_backward({q, k, wq, wk, wqt, wkt, cos, sin});
+    p.save(ctx);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    const auto sv = ctx->get_saved_variables();
+    const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3], &wqt = sv[4], &wkt = sv[5];
+    const Prologue p = Prologue::saved(ctx);
+    const int64_t b = q.size(0), s = q.size(1), h = q.size(2), d = q.size(3);
+    const bool has_k = k.defined();
+    const Tensor gq = grad_like(g[0], Tensor());
+    const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
+    Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = has_k ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
+    const auto fo = q.options().dtype(at::kFloat);
+    auto dw = [&](bool want) { return want ? at::empty({d}, fo) : Tensor(); };
+    Tensor dwq = dw(true), dwk = dw(has_k), dwqt = dw(wqt.defined()), dwkt = dw(wkt.defined() && has_k);
+    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s * h, 4 * d);
+    Tensor ws = at::empty({nws}, fo);
+    const mdattn_strides si = strides4(q), sd = strides4(dq), sg = strides4(gq);
+    must(mdattn_host_norm_rope_perhead_bwd(stream(), ptr(q), ptr(k), ptr(gq), ptr(gk), mut(dq), mut(dk), ptr(wq), ptr(wk), ptr(wqt),
+                                           has_k ? ptr(wkt) : nullptr, (int)p.n_txt, f32(dwq), f32(dwk), f32(dwqt), f32(dwkt), table_ptr(sv[6]),
+                                           table_ptr(sv[7]), (int)p.kind, (int)b, (int)s, (int)h, (int)d, (float)p.eps, (float)p.q_mul, &si, &sd, &sg,
+                                           f32(ws), nws),
+         "mdattn_norm_rope_perhead_bwd");
+    auto cast = [](const Tensor& x, const Tensor& w) { return x.defined() ? x.to(w.scalar_type()) : Tensor(); };
+    return {dq, dk, cast(dwq, wq), cast(dwk, wk), cast(dwqt, wqt), cast(dwkt, wkt), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::optional<variable_list> norm_rope_perhead(const Tensor& q, const OptTensor& k_, const Tensor& wq, const OptTensor& wk_, const OptTensor& wqt_,
+                                               const OptTensor& wkt_, int64_t n_txt, const OptTensor& fa, const OptTensor& fb, double eps, double q_mul,
+                                               bool bhsd) {
+  const Tensor k = value(k_), wk = value(wk_), wqt = value(wqt_), wkt = value(wkt_);
+  if (!q.is_cuda() || !bf16_on(q, q) || q.dim() != 4 || q.numel() == 0 || q.stride(3) != 1) return std::nullopt;
+  const int64_t d = q.size(3);
+  if (!weight_ok(wq, d, q) || (wqt.defined() && !weight_ok(wqt, d, q)) || (wkt.defined() && !weight_ok(wkt, d, q))) return std::nullopt;
+  if (k.defined() ? (!bf16_on(k, q) || k.sizes() != q.sizes() || k.strides() != q.strides() || !wk.defined() || !weight_ok(wk, d, q)) : wkt.defined())
+    return std::nullopt;
+  const auto t = as_table(fa, fb, q.size(1), d, true, q);
+  if (!t) return std::nullopt;
+  const Prologue p{q.size(2), t->kind, n_txt, eps, q_mul, bhsd};
+  if (wants_grad({&q, &k, &wq, &wk, &wqt, &wkt})) {
+    if (!q.is_non_overlapping_and_dense()) return std::nullopt;
+    return PerheadFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(wqt), opt(wkt), opt(t->cos), opt(t->sin), p);
+  }
+  variable_list out = perhead_run(q, k, wq, wk, wqt, wkt, t->cos, t->sin, p);
+  if (out.empty()) return std::nullopt;
+  return out;
+}
+
+// Wan over one fused q|k|v projection output with its biases
+variable_list qkv_run(const Tensor& x, const Tensor& bias, const Tensor& wq, const Tensor& wk, const Tensor& cos, const Tensor& sin, const Prologue& p) {
+  const int64_t b = x.size(0), s = x.size(1), d = x.size(2) / 3 / p.heads;
+  Tensor o[3];
+  for (Tensor& t : o) t = alloc_bshd(x, b, s, p.heads, d, p.bhsd);
+  const mdattn_strides so = strides4(o[0]);
+  const int rc = mdattn_host_norm_rope_qkv(stream(), ptr(x), ptr(bias), mut(o[0]), mut(o[1]), mut(o[2]), ptr(wq), ptr(wk), table_ptr(cos), table_ptr(sin),
+                                           (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps, (float)p.q_mul, x.stride(0), x.stride(1), &so);
+  if (rc != MDATTN_OK) return {};
+  return {o[0], o[1], o[2]};
+}
+struct QkvFn : torch::autograd::Function<QkvFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& bias, const Tensor& wq, const Tensor& wk, const OptTensor& cos_,
+                               const OptTensor& sin_, const Prologue& p) {
+    const Tensor cos = value(cos_), sin = value(sin_);
+    variable_list out = qkv_run(x, bias, wq, wk, cos, sin, p);
+    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_qkv refused the request");
+    ctx->save_for_backward({x, bias, wq, wk, cos, sin});
+    p.save(ctx);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    const auto sv = ctx->get_saved_variables();
+    const Tensor &x = sv[0], &bias = sv[1], &wq = sv[2], &wk = sv[3];
+    const Prologue p = Prologue::saved(ctx);
+    const int64_t b = x.size(0), s = x.size(1), n = x.size(2) / 3, d = n / p.heads;
+    const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq);
+    Tensor dx = at::empty({b, s, 3 * n}, x.options());
+    const auto fo = x.options().dtype(at::kFloat);
+    Tensor dwq = at::empty({n}, fo), dwk = at::empty({n}, fo), db = at::empty({2 * n}, fo);
+    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, 4 * n);
+    Tensor ws = at::empty({nws}, fo);
+    const mdattn_strides sg = strides4(gq);
+    const char* xp = static_cast<const char*>(ptr(x));
+    char* dp = static_cast<char*>(mut(dx));
+    must(mdattn_host_norm_rope_fullrow_bwd(stream(), xp, xp + 2 * n, ptr(bias), ptr(gq), ptr(gk), dp, dp + 2 * n, ptr(wq), ptr(wk), f32(dwq), f32(dwk),
+                                           f32(db), table_ptr(sv[4]), table_ptr(sv[5]), (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps,
+                                           (float)p.q_mul, x.stride(0), x.stride(1), dx.stride(0), dx.stride(1), &sg, f32(ws), nws),
+         "mdattn_norm_rope_fullrow_bwd");
+    dx.narrow(2, 2 * n, n).unflatten(2, {p.heads, d}).copy_(g[2]);
+    Tensor dbias = at::cat({db, g[2].to(at::kFloat).sum(at::IntArrayRef{0, 1}).reshape({n})}).to(bias.scalar_type());
+    return {dx, dbias, dwq.to(wq.scalar_type()), dwk.to(wk.scalar_type()), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::optional<variable_list> norm_rope_qkv(const Tensor& x, const Tensor& bias, const Tensor& wq, const Tensor& wk, const OptTensor& fa, const OptTensor& fb,
+                                           int64_t heads, double eps, double q_mul, bool bhsd) {
+  if (!x.is_cuda() || !bf16_on(x, x) || x.dim() != 3 || x.numel() == 0 || x.stride(2) != 1 || heads <= 0 || x.size(2) % (3 * heads)) return std::nullopt;
+  const int64_t n = x.size(2) / 3;
+  if (!weight_ok(wq, n, x) || !weight_ok(wk, n, x) || !weight_ok(bias, 3 * n, x)) return std::nullopt;
+  const auto t = as_table(fa, fb, x.size(1), n / heads, false, x);
+  if (!t) return std::nullopt;
+  const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
+  if (wants_grad({&x, &bias, &wq, &wk})) return QkvFn::apply(x, bias, wq, wk, opt(t->cos), opt(t->sin), p);
+  variable_list out = qkv_run(x, bias, wq, wk, t->cos, t->sin, p);
+  if (out.empty()) return std::nullopt;
+  return out;
+}
+
+// LTX-2: one tensor, f32 weight, tables of its own size (mode 1) or [B,H,S,D/2] (mode 2)
+Tensor rows_run(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t heads, int64_t mode, double eps) {
+  const int64_t b = x.size(0), s = x.size(1), d = x.size(2) / heads;
+  Tensor out = at::empty({b, s, heads, d}, x.options().dtype(at::kBFloat16));
+  const mdattn_strides so = strides4(out);
+  const int rc = mdattn_norm_rope_rows(stream(), ptr(x), x.scalar_type() == at::kFloat, mut(out), f32(w), mode ? f32(cos) : nullptr,
+                                       mode ? f32(sin) : nullptr, (int)mode, (int)b, (int)s, (int)heads, (int)d, (float)eps, x.stride(0), x.stride(1), &so);
+  return rc == MDATTN_OK ? out : Tensor();
+}
+struct RowsFn : torch::autograd::Function<RowsFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& cos_, const OptTensor& sin_, int64_t heads,
+                        int64_t mode, double eps) {
+    const Tensor cos = value(cos_), sin = value(sin_);
+    Tensor out = rows_run(x, w, cos, sin, heads, mode, eps);
+    TORCH_CHECK(out.defined(), "mdattn_norm_rope_rows refused the request");
+    ctx->save_for_backward({x, w, cos, sin});
+    ctx->saved_data["i"] = c10::List<int64_t>({heads, mode});
+    ctx->saved_data["eps"] = eps;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto sv = ctx->get_saved_variables();
+    const Tensor &x = sv[0], &w = sv[1];
+    const auto iv = ctx->saved_data["i"].toIntVector();
+    const int64_t heads = iv[0], mode = iv[1], b = x.size(0), s = x.size(1), n = x.size(2);
+    const Tensor g = grad_like(grads[0], Tensor());
+    Tensor dx = at::empty_strided(x.sizes(), x.strides(), x.options());
+    Tensor dw = at::empty({n}, w.options());
+    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, n);
+    Tensor ws = at::empty({nws}, w.options());
+    const mdattn_strides sg = strides4(g);
+    must(mdattn_norm_rope_rows_bwd(stream(), ptr(x), x.scalar_type() == at::kFloat, ptr(g), mut(dx), f32(w), f32(dw), mode ? f32(sv[2]) : nullptr,
+                                   mode ? f32(sv[3]) : nullptr, (int)mode, (int)b, (int)s, (int)heads, (int)(n / heads),
+                                   (float)ctx->saved_data["eps"].toDouble(), x.stride(0), x.stride(1), dx.stride(0), dx.stride(1), &sg, f32(ws), nws),
+         "mdattn_norm_rope_rows_bwd");
+    return {dx, dw, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+OptTensor norm_rope_rows(const Tensor& x, const Tensor& w, const OptTensor& cos_, const OptTensor& sin_, int64_t heads, int64_t mode, double eps) {
+  const Tensor cos = value(cos_), sin = value(sin_);
+  if (!x.is_cuda() || (x.scalar_type() != at::kFloat && x.scalar_type() != at::kBFloat16) || x.is_neg() || x.dim() != 3 || x.numel() == 0 ||
+      x.stride(2) != 1 || heads <= 0 || x.size(2) % heads)
+    return std::nullopt;
+  const int64_t b = x.size(0), s = x.size(1), n = x.size(2);
+  if (!in_place(w, at::kFloat, n, x)) return std::nullopt;
+  if (mode) {
+    const std::array<int64_t, 3> full{b, s, n};
+    const std::array<int64_t, 4> half{b, heads, s, n / heads / 2};
+    const at::IntArrayRef want = mode == 1 ? at::IntArrayRef(full) : at::IntArrayRef(half);
+    for (const Tensor* t : {&cos, &sin})
+      if (!t->defined() || t->sizes() != want || !in_place(*t, at::kFloat, t->numel(), x)) return std::nullopt;
+  }
+  if (wants_grad({&x, &w})) {
+    if (!x.is_non_overlapping_and_dense()) return std::nullopt;
+    return RowsFn::apply(x, w, opt(cos), opt(sin), heads, mode, eps);
+  }
+  Tensor out = rows_run(x, w, cos, sin, heads, mode, eps);
+  if (!out.defined()) return std::nullopt;
+  return out;
+}
+
+// the id of the sources, behind the marker that build.py finds in the file (as in libmdattn.so)
+const char kBuildIdRecord[] = "mdattn-build-id:" MDATTN_BUILD_ID;
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("build_id", [] { return std::string(kBuildIdRecord + 16); });
+  m.def("flash", &flash);
+  m.def("flash_autograd", &flash_autograd);
+  m.def("flash_merge", &flash_merge);
+  m.def("norm_rope", &norm_rope);
+  m.def("norm_rope_perhead", &norm_rope_perhead);
+  m.def("norm_rope_qkv", &norm_rope_qkv);
+  m.def("norm_rope_rows", &norm_rope_rows);
+}

@@ -356,12 +356,18 @@ def key_mask_bias(keep: torch.Tensor, masked_value: float = -math.inf) -> torch.
 
 
 def flash_attention(q, k, v, scale: float | None = None, return_lse: bool = False, out_layout: str = "bshd", out=None,
-                    key_bias: torch.Tensor | None = None):
+                    key_bias: torch.Tensor | None = None, *, heads: int | None = None, keep: torch.Tensor | None = None, q_mul: float = 1.0):
   """softmax(scale * q k^T [+ key_bias]) v, non-causal.  q [B,Sq,H,D], k/v [B,Skv,H,D] logical views, bf16.
 
   `key_bias` f32 [B, >= Skv rounded up to 32] (see `key_mask_bias`) is added to the scaled logits of each key;
   -inf excludes a key.  Returns out (logical [B,Sq,H,D] in `out_layout`) and, if asked, lse f32 [B,H,Sq] (natural log).
+
+  The registry entries' form (`heads` given): q, k, v as the models hand them over, [B,S,H*D] or [B,H,S,D], with a
+  [B,Skv] keep-mask and a factor `q_mul` rounded into q; returns [B,Sq,H*D], or None when an operand needs a conversion
+  first (another dtype, a head dim to be padded, a mask to be copied).
   """
+  if heads is not None:
+    return _lib.host().flash(q, k, v, heads, scale, keep, q_mul)
   _check_dev(q, k, v)
   if not (q.dtype == k.dtype == v.dtype == torch.bfloat16):
     raise ValueError("flash_attention needs bf16 q, k, v")
@@ -536,6 +542,8 @@ def flash_attention_merge(q, k, v, o_run, lse_run, scale: float | None = None):
   """One ring step in one launch: attention of q [B,Sq,H,D] against the chunk k/v [B,Skv,H,D] (bf16 logical views),
   merged in place into (o_run f32 logical [B,Sq,H,D], lse_run f32 [B,H,Sq]) as `merge_partial` would merge the
   result of `flash_attention`; the chunk's own output is never stored."""
+  if q.is_cuda and _lib.host().flash_merge(q, k, v, o_run, lse_run, 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale):
+    return o_run, lse_run
   _check_dev(q, k, v, o_run, lse_run)
   if not (q.dtype == k.dtype == v.dtype == torch.bfloat16):
     raise ValueError("flash_attention_merge needs bf16 q, k, v")
