@@ -99,7 +99,7 @@ def _folds_scale(keys: int, d: int, scale: float) -> bool:
 
 
 def _pad_head_dim(qv, kv, vv):
-  """Head dims below 128 other than 64 are zero-padded to the next size the kernels take (64 or 128), as the
+  """Head dims below 128 that the kernels do not walk as they are (csrc/mdattn_common.h: native_head_dim) are zero-padded to the next size the kernels take (64 or 128), as the
   reference's flash wrappers pad them to 128 (attention_flax.py:223-259, `_pad_data_for_flash`): zero columns of q and
   k add nothing to a logit, zero columns of v give output columns that the caller of this helper slices off.  Returns
   the (possibly padded) views and the original head dim.  One more pass over each tensor; gradients flow through the
@@ -160,7 +160,8 @@ def hip_flash_kernel(q, k, v, context):
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
       out = _lib.host().flash_autograd(q, k, v, heads, scale, mask)
     else:
-      folds = mask is None and _folds_scale(k.shape[-2] if k.dim() == 4 else k.shape[1], q.shape[-1] if q.dim() == 4 else q.shape[-1] // heads, scale)
+      d = q.shape[-1] if q.dim() == 4 else q.shape[-1] // heads
+      folds = mask is None and _folds_scale(k.shape[-2] if k.dim() == 4 else k.shape[1], 64 if d <= 64 else 128, scale)
       out = ops.flash_attention(q, k, v, scale=ops.FOLDED_SCALE if folds else scale, heads=heads, keep=mask,
                                 q_mul=scale * math.log2(math.e) if folds else 1.0)
     if out is not None:

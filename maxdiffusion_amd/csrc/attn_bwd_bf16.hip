@@ -84,7 +84,7 @@ struct BwdArgs {
   int64_t s4_sb, s4_ss, s4_sh, o2_sb, o2_ss, o2_sh;
   const float* lse2;   // [B,H,Sp] -lse * log2(e), -inf on padded rows
   const float* delta;  // [B,H,Sp] -rowsum(dout * out)
-  int H, Se, Ss, Sp;
+  int H, Se, Ss, Sp, D;
   int net, total, chunk;
   int64_t e1_sb, e1_ss, e1_sh, e2_sb, e2_ss, e2_sh;
   int64_t s1_sb, s1_ss, s1_sh, s2_sb, s2_ss, s2_sh, s3_sb, s3_ss, s3_sh;
@@ -93,7 +93,7 @@ struct BwdArgs {
   const float* bias;   // BIAS: additive per-key bias [B, bias_sb] in natural-log units (mdattn_fwd_bf16_bias)
   int64_t bias_sb;
   // stream split: the tiles of the stream are dealt to nsplit workgroups per entity tile, tps tiles each; with nsplit > 1
-  // a workgroup leaves f32 partial sums [split][B*H][Se][HD] (part: out's, part2: out2's) for bwd_reduce_kernel
+  // a workgroup leaves f32 partial sums [split][B*H][Se][D] (part: out's, part2: out2's) for bwd_reduce_kernel
   int nsplit, tps;
   float* part;
   float* part2;
@@ -101,7 +101,10 @@ struct BwdArgs {
 
 // MODE 0: dq (entity = q rows, stream = keys); 3: dk and dv in one pass (entity = key rows, stream = q rows).
 // MODE 1 (dk alone) and 2 (dv alone) are the same body with one accumulator set; the library launches 0 and 3.
-template <int MODE, int HD, bool BIAS, bool PRE>
+// DC != 0: head dims other than HD (a.D, a multiple of 8 up to DC), as in the forward's flat schedule: the layout of HD, the
+// MFMAs that cover DC columns; chunks past a.D are zero in the entity fragments, any finite data in the stream tiles, and
+// not stored in the gradients.
+template <int MODE, int HD, bool BIAS, bool PRE, int DC>
 __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   static_assert(!(PRE && BIAS), "a biased logit is touched after the MFMAs anyway");
   extern __shared__ __attribute__((aligned(16))) char smem_raw_b[];
@@ -110,8 +113,9 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   constexpr bool HAS2 = MODE != 2;
   constexpr bool BOTH = MODE == 3;
   using L = BwdLayout<HD>;
-  constexpr int NJ = HD / 16;   // MFMAs per 32 x 32 block of a contraction over the head dim
-  constexpr int ND = HD / 32;   // 32-wide slabs of d = accumulators
+  constexpr bool PADDED = DC != 0;
+  constexpr int NJ = (PADDED ? DC : HD) / 16;         // MFMAs per 32 x 32 block of a contraction over the head dim
+  constexpr int ND = ((PADDED ? DC : HD) + 31) / 32;  // 32-wide slabs of d = accumulators
   constexpr int kBD = HD, kBGK = L::GA, kBGV = L::GB, kBTileA = L::TileA, kBTileB = L::TileB;
   constexpr int kBStage = bwd_slot_elems<MODE, HD, BIAS>();  // MODE 3: a second transposed-read tile (dout)
   constexpr bool AUX = MODE != 0 || BIAS;
@@ -154,14 +158,16 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   int erow = r0 + l32;
   erow = erow < a.Se ? erow : a.Se - 1;
   bf16x8 ef1[NJ], ef2[NJ];
+  const bf16x8 zero8 = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+  auto in_row = [&](int s) __attribute__((always_inline)) { return !PADDED || s * 16 + hh * 8 < a.D; };
   {
     const __bf16* p = a.e1 + b * a.e1_sb + h * a.e1_sh + (int64_t)erow * a.e1_ss + hh * 8;
 #pragma unroll
-    for (int s = 0; s < NJ; ++s) ef1[s] = *reinterpret_cast<const bf16x8*>(p + s * 16);
+    for (int s = 0; s < NJ; ++s) ef1[s] = in_row(s) ? *reinterpret_cast<const bf16x8*>(p + s * 16) : zero8;
     if constexpr (HAS2) {
       const __bf16* p2 = a.e2 + b * a.e2_sb + h * a.e2_sh + (int64_t)erow * a.e2_ss + hh * 8;
 #pragma unroll
-      for (int s = 0; s < NJ; ++s) ef2[s] = *reinterpret_cast<const bf16x8*>(p2 + s * 16);
+      for (int s = 0; s < NJ; ++s) ef2[s] = in_row(s) ? *reinterpret_cast<const bf16x8*>(p2 + s * 16) : zero8;
     }
   }
   const float* lrow = a.lse2 + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
@@ -184,8 +190,9 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   constexpr int RPI = L::RPI;
   const int grow = HD == 128 ? lane >> 4 : lane >> 3;
   // lane -> logical 16-byte chunk stored at this lane's position (a wave fills the row groups wave, wave + NW, ...)
-  const int acol = HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8;
-  const int bcol = HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8;
+  auto in_head = [&](int col) __attribute__((always_inline)) { return !PADDED || col < a.D ? col : 0; };
+  const int acol = in_head(HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8);
+  const int bcol = in_head(HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8);
   const unsigned smem_addr = lds_addr_of(smem);
   // byte offsets of this lane's chunk from the first row of its row group: the same for every full tile.  The merged
   // pass at head dim 128 has no registers to keep them in (spilled, every reload would wait for the load issued
@@ -193,8 +200,8 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   constexpr bool REFORM = BOTH && HD == 128;
   auto chunk_ofs = [&](int ln, int64_t ss, bool transposed) __attribute__((always_inline)) {
     const int gr = HD == 128 ? ln >> 4 : ln >> 3;
-    const int col = transposed ? (HD == 128 ? ((ln & 15) ^ (gr << 2)) * 8 : ((ln & 7) ^ (((gr >> 1) & 1) << 2)) * 8)
-                               : (HD == 128 ? ((ln & 15) ^ gr) * 8 : ((ln & 7) ^ ((4 * (wave & 1) + (gr >> 1)) & 7)) * 8);
+    const int col = in_head(transposed ? (HD == 128 ? ((ln & 15) ^ (gr << 2)) * 8 : ((ln & 7) ^ (((gr >> 1) & 1) << 2)) * 8)
+                                       : (HD == 128 ? ((ln & 15) ^ gr) * 8 : ((ln & 7) ^ ((4 * (wave & 1) + (gr >> 1)) & 7)) * 8));
     return (__umul24((unsigned)gr, (unsigned)ss) + (unsigned)col) * 2u;  // strides are below 2^23
   };
   [[maybe_unused]] const unsigned ofs1 = REFORM ? 0u : chunk_ofs(lane, a.s1_ss, false);
@@ -446,11 +453,12 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   if (a.nsplit > 1) {  // partial sums over this workgroup's share of the stream, in f32
     if (row < a.Se) {
       const int64_t nbh = a.total / (a.net * a.nsplit);
-      const int64_t o = (((int64_t)sp * nbh + bh) * a.Se + row) * HD + 4 * hh;
+      const int64_t o = (((int64_t)sp * nbh + bh) * a.Se + row) * (PADDED ? a.D : HD) + 4 * hh;
 #pragma unroll
       for (int db = 0; db < ND; ++db)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+          if (PADDED && db * 32 + 8 * g >= a.D) continue;
           *reinterpret_cast<f32x4*>(a.part + o + db * 32 + 8 * g) =
               f32x4{acc[db][4 * g] * osc, acc[db][4 * g + 1] * osc, acc[db][4 * g + 2] * osc, acc[db][4 * g + 3] * osc};
           if constexpr (BOTH)
@@ -466,6 +474,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     for (int db = 0; db < ND; ++db)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
+        if (PADDED && db * 32 + 8 * g >= a.D) continue;
         uint2 u;
         u.x = pack2(acc[db][4 * g] * osc, acc[db][4 * g + 1] * osc);
         u.y = pack2(acc[db][4 * g + 2] * osc, acc[db][4 * g + 3] * osc);
@@ -477,6 +486,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       for (int db = 0; db < ND; ++db)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+          if (PADDED && db * 32 + 8 * g >= a.D) continue;
           uint2 u;
           u.x = pack2(acc2[db][4 * g], acc2[db][4 * g + 1]);
           u.y = pack2(acc2[db][4 * g + 2], acc2[db][4 * g + 3]);
@@ -486,17 +496,17 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   }
 }
 
-template <int MODE, int HD, bool BIAS, bool PRE>
+template <int MODE, int HD, bool BIAS, bool PRE, int DC>
 __global__ __launch_bounds__((bwd_waves<HD>() * 64)) void attn_bwd_kernel(BwdArgs a) {
-  attn_bwd_body<MODE, HD, BIAS, PRE>(a);
+  attn_bwd_body<MODE, HD, BIAS, PRE, DC>(a);
 }
 // The dk / dv pass at head dim 128 wants a few registers more than half the register file (128 accumulators, 64 of
 // entity fragments, 32 of S and dP): held to two waves per SIMD, which the schedule needs to overlap one wave's
 // exponentials with the other's MFMAs; at one wave per SIMD it measured 28 % slower.  Head dim 64 fits three waves
 // per SIMD (3 % faster than two).
-template <int HD, bool BIAS, bool PRE>
+template <int HD, bool BIAS, bool PRE, int DC>
 __global__ __launch_bounds__((bwd_waves<HD>() * 64)) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 3 : 2, HD == 64 ? 3 : 2))) void attn_bwd_both_kernel(BwdArgs a) {
-  attn_bwd_body<3, HD, BIAS, PRE>(a);
+  attn_bwd_body<3, HD, BIAS, PRE, DC>(a);
 }
 
 // The workspace, both negated (they start the MFMA chains that they are subtracted from):
@@ -537,16 +547,15 @@ struct BwdReduceArgs {
   __bf16* out[2];
   int64_t sb[2], ss[2], sh[2];
   int H, S, nsplit;
-  int64_t chunks;  // B*H*S*HD/8
+  int cpr;         // 16-byte chunks per row, D/8
+  int64_t chunks;  // B*H*S*cpr
 };
-template <int HD>
 __global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= a.chunks) return;
   const int t = blockIdx.y;
-  constexpr int CPR = HD / 8;
-  const int c = (int)(i % CPR);
-  const int64_t row = i / CPR;
+  const int64_t row = i / a.cpr;
+  const int c = (int)(i - row * a.cpr);
   const int s = (int)(row % a.S);
   const int64_t bh = row / a.S;
   const int64_t b = bh / a.H, h = bh - b * a.H;
@@ -572,8 +581,8 @@ struct BwdSplit {
 };
 // entity rows Se, stream rows Ss; tensors: gradients the pass produces (2 in the dk / dv pass)
 inline BwdSplit bwd_split(int64_t BH, int Se, int Ss, int D, int tensors) {
-  const int rows = D == 128 ? bwd_waves<128>() * 32 : bwd_waves<64>() * 32;
-  const int slots = D == 128 ? 256 : 3 * 256;              // workgroups the chip holds at once
+  const int rows = D > 64 ? bwd_waves<128>() * 32 : bwd_waves<64>() * 32;
+  const int slots = D > 64 ? 256 : 3 * 256;                // workgroups the chip holds at once
   const double tile_us = tensors == 2 ? 1.7 : 1.2;         // a workgroup's time per stream tile
   const int64_t entities = BH * ((Se + rows - 1) / rows), floats = BH * Se * D;
   const double partial = 2.0 * tensors * (double)floats * 4 / 5e6 / tile_us;  // written and read at 5 TB/s
@@ -588,7 +597,7 @@ inline BwdSplit bwd_split(int64_t BH, int Se, int Ss, int D, int tensors) {
   return best;
 }
 
-template <int MODE, int HD, bool BIAS, bool PRE>
+template <int MODE, int HD, bool BIAS, bool PRE, int DC = 0>
 int launch_bwd_as(hipStream_t st, BwdArgs a, int B) {
   constexpr int lds_bytes = 2 * bwd_slot_elems<MODE, HD, BIAS>() * 2;
   constexpr int NW = bwd_waves<HD>();
@@ -598,8 +607,8 @@ int launch_bwd_as(hipStream_t st, BwdArgs a, int B) {
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
   void (*kern)(BwdArgs);
-  if constexpr (MODE == 3) kern = attn_bwd_both_kernel<HD, BIAS, PRE>;
-  else kern = attn_bwd_kernel<MODE, HD, BIAS, PRE>;
+  if constexpr (MODE == 3) kern = attn_bwd_both_kernel<HD, BIAS, PRE, DC>;
+  else kern = attn_bwd_kernel<MODE, HD, BIAS, PRE, DC>;
   static LdsOptIn opted;
   if (lds_opt_in(opted, reinterpret_cast<const void*>(kern), lds_bytes) != MDATTN_OK) return MDATTN_E_LAUNCH;
   MDATTN_LAUNCH(kern, dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
@@ -618,23 +627,30 @@ int launch_bwd(hipStream_t st, const BwdArgs& a, int B) {
   return launch_bwd_as<MODE, HD, BIAS, false>(st, a, B);
 }
 
+template <int MODE, bool BIAS>
+int launch_bwd_dim(hipStream_t st, const BwdArgs& a, int B) {
+  if (a.D == 128) return launch_bwd<MODE, 128, BIAS>(st, a, B);
+  if (a.D == 64) return launch_bwd<MODE, 64, BIAS>(st, a, B);
+  if (a.D <= 48) return launch_bwd_as<MODE, 64, BIAS, false, 48>(st, a, B);
+  if (a.D <= 80) return launch_bwd_as<MODE, 128, BIAS, false, 80>(st, a, B);
+  return launch_bwd_as<MODE, 128, BIAS, false, 96>(st, a, B);
+}
 template <int MODE>
-int launch_bwd_any(hipStream_t st, const BwdArgs& a, int B, int D) {
-  if (D == 128) return a.bias ? launch_bwd<MODE, 128, true>(st, a, B) : launch_bwd<MODE, 128, false>(st, a, B);
-  return a.bias ? launch_bwd<MODE, 64, true>(st, a, B) : launch_bwd<MODE, 64, false>(st, a, B);
+int launch_bwd_any(hipStream_t st, const BwdArgs& a, int B) {
+  return a.bias ? launch_bwd_dim<MODE, true>(st, a, B) : launch_bwd_dim<MODE, false>(st, a, B);
 }
 
-int launch_bwd_reduce(hipStream_t st, const BwdArgs& a, int B, int D) {
+int launch_bwd_reduce(hipStream_t st, const BwdArgs& a, int B) {
   BwdReduceArgs r;
   r.part[0] = a.part; r.part[1] = a.part2;
   r.out[0] = a.out; r.out[1] = a.part2 ? a.out2 : nullptr;
   r.sb[0] = a.o_sb; r.ss[0] = a.o_ss; r.sh[0] = a.o_sh;
   r.sb[1] = a.o2_sb; r.ss[1] = a.o2_ss; r.sh[1] = a.o2_sh;
   r.H = a.H; r.S = a.Se; r.nsplit = a.nsplit;
-  r.chunks = (int64_t)B * a.H * a.Se * (D / 8);
+  r.cpr = a.D / 8;
+  r.chunks = (int64_t)B * a.H * a.Se * r.cpr;
   const dim3 grid((unsigned)((r.chunks + 255) / 256), a.part2 ? 2 : 1);
-  if (D == 128) MDATTN_LAUNCH(bwd_reduce_kernel<128>, grid, dim3(256), 0, st, r);
-  else MDATTN_LAUNCH(bwd_reduce_kernel<64>, grid, dim3(256), 0, st, r);
+  MDATTN_LAUNCH(bwd_reduce_kernel, grid, dim3(256), 0, st, r);
   return launch_status();
 }
 
@@ -649,7 +665,7 @@ extern "C" int64_t mdattn_bwd_workspace_floats(int B, int H, int Sq) {
 }
 
 extern "C" int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D) {
-  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || (D != 128 && D != 64)) return 0;
+  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !native_head_dim(D)) return 0;
   const int64_t BH = (int64_t)B * H;
   return mdattn_bwd_workspace_floats(B, H, Sq) + bwd_split(BH, Sq, Skv, D, 1).floats + 2 * bwd_split(BH, Skv, Sq, D, 2).floats;
 }
@@ -660,7 +676,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
                    int B, int H, int Sq, int Skv, int D,
                    const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                    const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                   const float* key_bias, int64_t bias_stride) {
+                   const float* key_bias, int64_t bias_stride, bool any_head_dim = false) {
   if (!q || !k || !v || !out || !dout || !lse || !dq || !dk || !dv || !workspace) return MDATTN_E_BADARG;
   if (key_bias) {
     if (bias_stride < ((int64_t)Skv + 31) / 32 * 32 || bias_stride % 32 != 0) return MDATTN_E_BADARG;
@@ -669,7 +685,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || D <= 0) return MDATTN_E_BADARG;
   if (!q_strides || !k_strides || !v_strides || !o_strides) return MDATTN_E_BADARG;
   if (!(scale > 0.f) || !(scale < 1e30f)) return MDATTN_E_BADARG;
-  if (D != 128 && D != 64) return MDATTN_E_UNSUPPORTED;
+  if (D != 128 && D != 64 && !(any_head_dim && native_head_dim(D))) return MDATTN_E_UNSUPPORTED;
   if (workspace_floats < mdattn_bwd_workspace_floats(B, H, Sq)) return MDATTN_E_BADARG;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(dout) || !aligned16(dq) ||
       !aligned16(dk) || !aligned16(dv) || !aligned16(workspace) || (reinterpret_cast<uintptr_t>(lse) & 3u))
@@ -698,7 +714,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
     skv = {1, (Sq + kBT - 1) / kBT, 0};
   }
   BwdArgs a;
-  a.lse2 = lse2; a.delta = delta; a.H = H; a.Sp = Sp; a.c = scale * kLog2e; a.scale = scale;
+  a.lse2 = lse2; a.delta = delta; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;
   auto set = [](int64_t& sb, int64_t& ss, int64_t& sh, const mdattn_strides* s) { sb = s->batch; ss = s->seq; sh = s->head; };
   // dq: entity q / dout, stream k (scores), v (dP), k (accumulate)
@@ -708,9 +724,9 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.s1_sb, a.s1_ss, a.s1_sh, k_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, v_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, k_strides);
   set(a.o_sb, a.o_ss, a.o_sh, q_strides);
   a.nsplit = sq.nsplit; a.tps = sq.tps; a.part = workspace + 2 * rows; a.part2 = nullptr;
-  int rc = launch_bwd_any<0>(st, a, B, D);
+  int rc = launch_bwd_any<0>(st, a, B);
   if (rc != MDATTN_OK) return rc;
-  if (sq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B, D)) != MDATTN_OK) return rc;
+  if (sq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B)) != MDATTN_OK) return rc;
   // dk and dv in one pass: entity k / v, stream q (scores, and accumulate for dk), dout (dP, and accumulate for dv)
   a.e1 = (const __bf16*)k; a.e2 = (const __bf16*)v; a.s1 = (const __bf16*)q; a.s2 = (const __bf16*)dout; a.s3 = (const __bf16*)q;
   a.s4 = (const __bf16*)dout;
@@ -720,8 +736,8 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.s4_sb, a.s4_ss, a.s4_sh, o_strides);
   set(a.o_sb, a.o_ss, a.o_sh, k_strides); set(a.o2_sb, a.o2_ss, a.o2_sh, v_strides);
   a.nsplit = skv.nsplit; a.tps = skv.tps; a.part = workspace + 2 * rows + sq.floats; a.part2 = a.part + skv.floats;
-  rc = launch_bwd_any<3>(st, a, B, D);
-  if (rc == MDATTN_OK && skv.nsplit > 1) rc = launch_bwd_reduce(st, a, B, D);
+  rc = launch_bwd_any<3>(st, a, B);
+  if (rc == MDATTN_OK && skv.nsplit > 1) rc = launch_bwd_reduce(st, a, B);
   return rc;
 }
 
@@ -744,6 +760,16 @@ extern "C" int mdattn_bwd_bf16_bias(void* stream, const void* q, const void* k, 
   if (!key_bias) return MDATTN_E_BADARG;
   return bwd_run((hipStream_t)stream, q, k, v, out, dout, lse, dq, dk, dv, workspace, workspace_floats, B, H, Sq, Skv, D,
                  q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride);
+}
+
+extern "C" int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, const void* v, const void* out, const void* dout,
+                                    const float* lse, void* dq, void* dk, void* dv, float* workspace, int64_t workspace_floats,
+                                    int B, int H, int Sq, int Skv, int D,
+                                    const mdattn_strides* q_strides, const mdattn_strides* k_strides,
+                                    const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
+                                    const float* key_bias, int64_t bias_stride) {
+  return bwd_run((hipStream_t)stream, q, k, v, out, dout, lse, dq, dk, dv, workspace, workspace_floats, B, H, Sq, Skv, D,
+                 q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride, true);
 }
 
 // ---------------------------------------------------------------------------------------------------

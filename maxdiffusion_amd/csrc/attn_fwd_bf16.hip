@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "mdattn_common.h"
+#include "mdattn_host.h"
 
 namespace mdattn {
 
@@ -130,12 +131,13 @@ __device__ __forceinline__ void store_row(const AttnArgs& a, const f32x16 (&O)[N
 // the attention itself (75,600 x 40 x 128 outputs: 0.27 ms).  Here the wave's 32 x HD tile is normalised, rounded to
 // bf16 and transposed through LDS, and every store instruction then writes 1 KB of whole rows (4 rows of 256 bytes
 // at head dim 128).  Same values, same rounding as store_row.
-template <int ND>
+// PADDED: the head dim a.D is below ND * 32, and only its columns are stored.
+template <int ND, bool PADDED>
 __device__ __forceinline__ void store_rows_through_lds(const AttnArgs& a, const f32x16 (&O)[ND], float lt, float mc, int b,
                                                        int h, int row0, int lane, char* stage) {
   constexpr int HD = ND * 32;
   constexpr int ROWB = HD * 2 + 16;      // padded row: the 32 lanes of a column write land on 16 different bank groups
-  constexpr int LPR = HD * 2 / 16;       // lanes that share a row in the read-back
+  constexpr int LPR = ND == 3 ? 16 : HD * 2 / 16;  // lanes that share a row in the read-back (a power of two)
   constexpr int RPI = 64 / LPR;          // rows per store instruction
   const int l32 = lane & 31, hh = lane >> 5;
   const float inv = lt > 0.f ? 1.0f / lt : 0.f;  // rows whose keys are all excluded return 0
@@ -157,6 +159,7 @@ __device__ __forceinline__ void store_rows_through_lds(const AttnArgs& a, const 
 #pragma unroll
   for (int j = 0; j < 32 / RPI; ++j) {
     const int r = j * RPI + rr;
+    if (PADDED && cc * 8 >= a.D) continue;
     const uint4 v = *reinterpret_cast<const uint4*>(stage + r * ROWB + cc * 16);
     // streaming store: the output is written once and read by nobody here (1.5 % on the 512-key cross-attention)
     if (row0 + r < a.Sq) st_nt(reinterpret_cast<uint4*>(obase + (int64_t)(row0 + r) * a.o_ss + cc * 8), v);
@@ -452,10 +455,16 @@ constexpr int kKTileS = (kTS / 4) * kGK;              // elements
 constexpr int kStageS = kKTileS + (kTS / 4) * kGV;    // elements per ring slot
 constexpr int kSlotsS = 3;
 
-template <int NW, bool BIAS, int HD, bool PRE>
+// Other head dims (a.D, a multiple of 8 up to DC) run in the layout of the next of the two, HD, with the MFMAs that cover
+// DC columns (DC < HD + 1; 0: a.D == HD): lanes whose 16-byte chunk lies past a.D fetch the row's first chunk instead, which
+// meets zeros in Q (logits) or lands in output columns that are not stored.  A copy of q, k and v padded to 64 or 128
+// columns in front, and one of out cut back behind, are gone: 62 -> 16 us for 16 x 257 tokens x 16 heads of 80 (64 -> 16 us of
+// kernels and the four copies' launches), 626 -> 449 us for 8,192 tokens x 20 heads of 80.
+template <int NW, bool BIAS, int HD, bool PRE, int DC = 0>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 3, HD == 64 ? 4 : 3))) void attn_fwd_bf16_flat_kernel(AttnArgs a) {
-  constexpr int NJ = HD / 16;                                    // QK MFMAs per 32-key tile
-  constexpr int ND = HD / 32;                                    // 32-wide slabs of d = O accumulators
+  constexpr bool PADDED = DC != 0;
+  constexpr int NJ = (PADDED ? DC : HD) / 16;                    // QK MFMAs per 32-key tile
+  constexpr int ND = ((PADDED ? DC : HD) + 31) / 32;             // 32-wide slabs of d = O accumulators
   // Head dim 64: 64-key tiles (two 32-key blocks per ring slot, the LDS of a 32-key tile at head dim 128) in a 2-slot
   // ring: half the barriers and tile bookkeeping per key of a kernel whose softmax already outweighs its MFMAs.
   constexpr int TS = HD == 128 ? kTS : 64;                       // keys per tile
@@ -498,8 +507,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 
   // lane -> (row of the group, logical 16-byte chunk stored at this lane's position)
   const int grow = HD == 128 ? lane >> 4 : lane >> 3;
-  const int kcol = HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8;
-  const int vcol = HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8;
+  auto in_head = [&](int col) __attribute__((always_inline)) { return !PADDED || col < a.D ? col : 0; };
+  const int kcol = in_head(HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8);
+  const int vcol = in_head(HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8);
   constexpr int KGS = HD == 128 ? kGK : 8 * 64;  // group strides in LDS, elements
   constexpr int VGS = HD == 128 ? kGV : 8 * 64;
   const unsigned kofs = (unsigned)(grow * (int)a.k_ss + kcol) * 2u;
@@ -716,13 +726,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     for (int g = 0; g < 32 / RPI; ++g) {
       int row = q0 + RPI * g + grow;
       row = row < a.Sq ? row : a.Sq - 1;
-      const int qcol = HD == 128 ? kcol : ((lane & 7) ^ ((4 * (g & 1) + (grow >> 1)) & 7)) * 8;
+      const int qcol = HD == 128 ? kcol : in_head(((lane & 7) ^ ((4 * (g & 1) + (grow >> 1)) & 7)) * 8);
       lds_dma16(qp + (int64_t)row * a.q_ss + qcol, Qs + (unsigned)(g * KGS) * 2u);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the wave's own Q rows (and its share of tile 0) are in LDS
     const __bf16* qs = smem + STAGE + wave * QTILE;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const bf16x8*>(qs + k_off[j]);
+    for (int j = 0; j < NJ; ++j) {
+      qf[j] = *reinterpret_cast<const bf16x8*>(qs + k_off[j]);
+      if (PADDED && (2 * j + hh) * 8 >= a.D) qf[j] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+    }
   }
   __syncthreads();  // every wave holds its fragments: the staging area is ring slots again
   // SLOTS - 1 tiles are requested ahead of the one being worked on
@@ -756,16 +769,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   __syncthreads();
   tile(nt - 1, (nt - 1) % SLOTS, std::true_type{});
 
-  if (a.o_run) {  // ring step: merged into the f32 carry, row by row
+  if (!PADDED && a.o_run) {  // ring step: merged into the f32 carry, row by row
     store_row<ND>(a, O, xhalf_sum(l), mc, b, h, q0 + l32, hh);
   } else {
-    static_assert(NW * 32 * (HD * 2 + 16) <= SLOTS * STAGE * 2, "the output staging tiles must fit the ring's LDS");
+    static_assert(NW * 32 * (ND * 64 + 16) <= SLOTS * STAGE * 2, "the output staging tiles must fit the ring's LDS");
     __syncthreads();  // every wave has finished reading the ring: its LDS now stages the output tiles
-    store_rows_through_lds<ND>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * 32 * (HD * 2 + 16));
+    store_rows_through_lds<ND, PADDED>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * 32 * (ND * 64 + 16));
   }
 }
 
-template <int NW, bool BIAS, int HD = 128>
+template <int NW, bool BIAS, int HD = 128, int DC = 0>
 static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   constexpr int BM = NW * 32;
   // the ring, or ring slot 0 plus one K-shaped Q staging tile per wave, whichever is larger
@@ -780,8 +793,8 @@ static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   // scale * log2(e) == 1 (to f32 round-off): the caller folded the factor into q; the logits need no multiply.
   // With a key bias the logits are touched after the MFMAs anyway, so that variant keeps its FMA.
   const bool pre = !BIAS && a.c > 1.0f - 1e-6f && a.c < 1.0f + 1e-6f;
-  if (pre) MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, !BIAS>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
-  else MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, false>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
+  if (pre) MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, !BIAS, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
+  else MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, false, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   return launch_status();
 }
 
@@ -810,11 +823,11 @@ using namespace mdattn;
 static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, void* out, float* lse,
                      int B, int H, int Sq, int Skv, int D,
                      const mdattn_strides* q_strides, const mdattn_strides* k_strides,
-                     const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale) {
+                     const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale, bool any_head_dim = false) {
   if (!q || !k || !v || !out || B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || D <= 0) return MDATTN_E_BADARG;
   if (!q_strides || !k_strides || !v_strides || !o_strides) return MDATTN_E_BADARG;
   if (!(scale > 0.f) || !(scale < 1e30f)) return MDATTN_E_BADARG;
-  if (D != kD && D != 64) return MDATTN_E_UNSUPPORTED;
+  if (D != kD && D != 64 && !(any_head_dim && native_head_dim(D))) return MDATTN_E_UNSUPPORTED;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || (reinterpret_cast<uintptr_t>(lse) & 3u))
     return MDATTN_E_ALIGN;
   if (!strides_ok(q_strides, 8) || !strides_ok(k_strides, 8) || !strides_ok(v_strides, 8) || !strides_ok(o_strides, 8))
@@ -823,7 +836,7 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
   // per-lane byte offsets inside one tile are kept in 32 bits
   if (k_strides->seq >= (1 << 23) || v_strides->seq >= (1 << 23)) return MDATTN_E_UNSUPPORTED;
   a.q = (const __bf16*)q; a.k = (const __bf16*)k; a.v = (const __bf16*)v; a.out = (__bf16*)out; a.lse = lse;
-  a.H = H; a.Sq = Sq; a.Skv = Skv;
+  a.H = H; a.Sq = Sq; a.Skv = Skv; a.D = D;
   a.q_sb = q_strides->batch; a.q_ss = q_strides->seq; a.q_sh = q_strides->head;
   a.k_sb = k_strides->batch; a.k_ss = k_strides->seq; a.k_sh = k_strides->head;
   a.v_sb = v_strides->batch; a.v_ss = v_strides->seq; a.v_sh = v_strides->head;
@@ -853,6 +866,35 @@ static int dispatch_fwd(hipStream_t st, const AttnArgs& a, int B, int Sq, int Sk
     case 3: return launch_flat<4, false>(st, a, B);
     default: return MDATTN_E_BADARG;
   }
+}
+
+// Head dims other than 64 and 128: the layout and the MFMAs that cover the next of 48, 80, 96 columns.
+template <bool BIAS>
+static int dispatch_padded(hipStream_t st, const AttnArgs& a, int B) {
+  if (a.D <= 48) return launch_flat<4, BIAS, 64, 48>(st, a, B);
+  if (a.D <= 80) return launch_flat<4, BIAS, 128, 80>(st, a, B);
+  return launch_flat<4, BIAS, 128, 96>(st, a, B);
+}
+
+extern "C" int mdattn_host_head_dim(int D) { return native_head_dim(D); }
+
+extern "C" int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,
+                                    int B, int H, int Sq, int Skv, int D,
+                                    const mdattn_strides* q_strides, const mdattn_strides* k_strides,
+                                    const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
+                                    const float* key_bias, int64_t bias_stride) {
+  if (D == 64 || D == kD)
+    return key_bias ? mdattn_fwd_bf16_bias(stream, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride)
+                    : mdattn_fwd_bf16(stream, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale);
+  AttnArgs a;
+  const int rc = fill_args(a, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale, true);
+  if (rc != MDATTN_OK) return rc;
+  if (!key_bias) return dispatch_padded<false>((hipStream_t)stream, a, B);
+  if (bias_stride < ((Skv + kTS - 1) / kTS) * kTS || bias_stride % kTS != 0) return MDATTN_E_BADARG;
+  if (!aligned16(key_bias)) return MDATTN_E_ALIGN;
+  a.bias = key_bias;
+  a.bias_sb = bias_stride;
+  return dispatch_padded<true>((hipStream_t)stream, a, B);
 }
 
 extern "C" int mdattn_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,

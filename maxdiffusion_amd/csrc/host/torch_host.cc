@@ -87,11 +87,8 @@ Tensor grad_like(const Tensor& g, const Tensor& like) {
 int fwd(const Tensor& q, const Tensor& k, const Tensor& v, const View& vq, const View& vk, const View& vv, const Tensor& out, const Tensor& lse,
         const Tensor& bias, double scale) {
   const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
-  if (bias.defined())
-    return mdattn_fwd_bf16_bias(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st,
-                                &vk.st, &vv.st, &so, (float)scale, f32(bias), bias.stride(0));
-  return mdattn_fwd_bf16(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st, &vk.st,
-                         &vv.st, &so, (float)scale);
+  return mdattn_host_fwd_bf16(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st, &vk.st,
+                              &vv.st, &so, (float)scale, f32(bias), bias.defined() ? bias.stride(0) : 0);
 }
 
 // q, k, v in the caller's own rank; out [B,Sq,H*D]
@@ -119,11 +116,8 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     const int64_t nws = mdattn_bwd_split_workspace_floats(B, H, Sq, Skv, D);
     Tensor ws = at::empty({nws}, lse.options());
     const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
-    const int rc = bias.defined()
-        ? mdattn_bwd_bf16_bias(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq, Skv,
-                               D, &vq.st, &vk.st, &vv.st, &so, (float)scale, f32(bias), bias.stride(0))
-        : mdattn_bwd_bf16(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq, Skv, D,
-                          &vq.st, &vk.st, &vv.st, &so, (float)scale);
+    const int rc = mdattn_host_bwd_bf16(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq,
+                                        Skv, D, &vq.st, &vk.st, &vv.st, &so, (float)scale, f32(bias), bias.defined() ? bias.stride(0) : 0);
     must(rc, "mdattn_bwd_bf16");
     return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
   }
@@ -145,9 +139,10 @@ bool flash_args(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads
                 Tensor& bias) {
   if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q)) return false;
   const auto a = as_view(q, heads), b = as_view(k, heads), c = as_view(v, heads);
-  if (!a || !b || !c || (a->d != 64 && a->d != 128) || a->b != b->b || a->b != c->b || a->h != b->h || a->h != c->h || a->d != b->d || a->d != c->d ||
+  if (!a || !b || !c || a->b != b->b || a->b != c->b || a->h != b->h || a->h != c->h || a->d != b->d || a->d != c->d ||
       b->s != c->s || !(scale > 0))
     return false;
+  if (!mdattn_host_head_dim((int)a->d)) return false;  // padded first
   if (q.numel() == 0 || k.numel() == 0 || std::max(a->s, b->s) >= ((int64_t)1 << 31)) return false;
   if (keep.has_value() && !(bias = mask_bias(*keep, *b, q)).defined()) return false;
   vq = *a; vk = *b; vv = *c;

@@ -132,7 +132,7 @@ struct AttnArgs {
   const __bf16* v;
   __bf16* out;
   float* lse;
-  int H, Sq, Skv;
+  int H, Sq, Skv, D;
   int nqt, total, chunk;
   int64_t q_sb, q_ss, q_sh;
   int64_t k_sb, k_ss, k_sh;
@@ -148,6 +148,10 @@ struct AttnArgs {
 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// Head dims that the attention kernels walk as they are: 64 and 128, and, in the layout of the next of these two with the
+// MFMAs that cover 48, 80 or 96 columns, multiples of 8 up to 48 and from 72 to 96.  (56 saves nothing against 64; 104 to 120
+// save a column of MFMAs at most, spill in the backward, and lose the pipelined forward: they are padded by the caller.)
+inline bool native_head_dim(int D) { return D == 64 || D == 128 || (D > 0 && D % 8 == 0 && (D <= 48 || (D > 64 && D <= 96))); }
 // a rotary table of layout `table` (0: planes, cos and sin; 1: complex; 2: repeated planes; 3: matrices): both pointers or none
 // for the planes, cos alone for the others
 inline bool table_ok(const float* cos, const float* sin, int table) {

@@ -203,3 +203,40 @@ def test_registry_folds_the_scale_into_q_on_long_key_sequences(dev):
     mx, mean = err_stats(hsd(to_np(got), S), ro)
     print(f"Skv={skv} scale={scale:.4f}: max-abs {mx:.3e} mean-abs {mean:.3e}")
     assert mx <= 2e-2 and mean <= 2e-3 and rel_l2(hsd(to_np(got), S), ro) <= 1.5e-2, (skv, mx, mean)
+
+
+@pytest.mark.parametrize("D", [8, 40, 48, 72, 80, 96])
+@pytest.mark.parametrize("sq,skv,masked", [(1, 1, False), (257, 257, False), (130, 333, True), (33, 1100, False)])
+def test_head_dims_the_kernels_walk_unpadded(dev, lib, D, sq, skv, masked):
+  """Every class of unpadded head dims, whole and half-filled last MFMA, both input layouts: forward and gradients against
+  torch autograd on an f32 attention (bars of the padded path, tests/test_gpu_backward.py)."""
+  assert lib.mdattn_host_head_dim(D)
+  B, H = 2, 3
+  gen = torch.Generator(device=dev).manual_seed(D + sq)
+  mk = lambda s: torch.randn((B, s, H * D), generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True)
+  q, k, v = mk(sq), mk(skv), mk(skv)
+  g = torch.randn((B, sq, H * D), generator=gen, device=dev).to(torch.bfloat16)
+  keep = torch.rand((B, skv), generator=gen, device=dev) < 0.7
+  keep[:, 0] = True
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+  args = dict(attention_mask=keep if masked else None)
+  out = op.apply_attention(q, k, v, **args)
+  grads = torch.autograd.grad(out, (q, k, v), g)
+  with torch.no_grad():
+    assert torch.equal(op.apply_attention(q, k, v, **args), out)
+    heads_first = lambda t: t.view(B, -1, H, D).permute(0, 2, 1, 3).contiguous()
+    assert torch.equal(op.apply_attention(heads_first(q), heads_first(k), heads_first(v), **args), out)
+  rq, rk, rv = (t.detach().float().requires_grad_(True) for t in (q, k, v))
+  hf = lambda t: t.view(B, -1, H, D).transpose(1, 2)
+  s = (hf(rq) @ hf(rk).transpose(2, 3)) * D**-0.5
+  if masked:
+    s = s.masked_fill(~keep[:, None, None, :], float("-inf"))
+  ref = (torch.softmax(s, -1) @ hf(rv)).transpose(1, 2).reshape(B, sq, H * D)
+  want = torch.autograd.grad(ref, (rq, rk, rv), g.float())
+  assert rel_l2(to_np(out), ref.detach().cpu().numpy()) <= 6e-3
+  for name, got, r in zip(("dq", "dk", "dv"), grads, want):
+    rn = r.detach().cpu().numpy()
+    if float(np.abs(rn).max()) < 1e-6:  # one key: the exact gradient of q and k is zero
+      assert float(got.float().abs().max()) <= 0.25, name
+      continue
+    assert rel_l2(to_np(got), rn) <= 6e-3, name
