@@ -92,6 +92,8 @@ struct BwdArgs {
   float c, scale;
   const float* bias;   // BIAS: additive per-key bias [B, bias_sb] in natural-log units (mdattn_fwd_bf16_bias)
   int64_t bias_sb;
+  const int* tiles;    // BIAS: TileLists of 32 keys, tiles_sb ints per batch element, or null (see AttnArgs)
+  int tiles_sb;
   // stream split: the tiles of the stream are dealt to nsplit workgroups per entity tile, tps tiles each; with nsplit > 1
   // a workgroup leaves f32 partial sums [split][B*H][Se][D] (part: out's, part2: out2's) for bwd_reduce_kernel
   int nsplit, tps;
@@ -123,8 +125,8 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 #define MDATTN_BWD_LA 4
 #endif
   // fragment look-ahead of the dq pass over its whole read stream (head dim 64, at three waves per SIMD, has room for
-  // two: 1 % on one machine, A/B); the merged pass windows its two MFMA phases separately, LA1 and LA3 below
-  constexpr int LA = MODE == 0 ? (HD == 128 ? MDATTN_BWD_LA : 2) : 0;
+  // two: 1 % on one machine, A/B; not with a key mask's tile list); the merged pass windows its two MFMA phases separately, LA1 and LA3 below
+  constexpr int LA = MODE == 0 ? (HD == 128 ? MDATTN_BWD_LA : BIAS ? 0 : 2) : 0;
   static_assert(LA == 0 || (HAS2 && !BOTH && LA <= 2 * ND), "the window covers the three-product passes");
 #ifndef MDATTN_BWD_LA1
 #define MDATTN_BWD_LA1 2
@@ -149,10 +151,20 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   const int b = bh / a.H, h = bh - b * a.H;
   const int r0 = et * (NW * 32) + wave * 32;
   // this workgroup's stream: rows ss0 .. ss0 + Ss - 1 of the sequence (never empty); everything below counts from ss0
-  const int ss0 = sp * a.tps * kBT;
-  const int Ss = a.Ss - ss0 < a.tps * kBT ? a.Ss - ss0 : a.tps * kBT;
-  const int nt = (Ss + kBT - 1) / kBT;
+  const bool listed = BIAS && MODE == 0 && a.tiles;  // (its tiles are numbered from the sequence's start)
+  const int ss0 = listed ? 0 : sp * a.tps * kBT;
+  const int Ss = listed || a.Ss - ss0 < a.tps * kBT ? a.Ss - ss0 : a.tps * kBT;
+  int nt = (Ss + kBT - 1) / kBT;
   const float c = a.c;
+  // dq pass with a mask: the key tiles that hold a kept key, this workgroup's share of them (perhaps none)
+  [[maybe_unused]] TileList tl{BIAS && MODE == 0 && a.tiles ? a.tiles + (int64_t)b * a.tiles_sb : nullptr};
+  [[maybe_unused]] const int tl_n = tl.count(sp * a.tps + nt);
+  if constexpr (BIAS && MODE == 0) {
+    if (tl.list) {
+      nt = tl_n - sp * a.tps < a.tps ? tl_n - sp * a.tps : a.tps;
+      nt = nt > 0 ? nt : 0;
+    }
+  }
 
   // ---- entity fragments
   int erow = r0 + l32;
@@ -180,7 +192,10 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   // key bias in log2 units: a per-lane scalar when the keys are the entity rows, sixteen values per tile otherwise
   [[maybe_unused]] const float* bias_row = BIAS ? a.bias + b * a.bias_sb + (MODE == 0 ? ss0 : 0) : nullptr;
   [[maybe_unused]] float bias_e = 0.f;
-  if constexpr (BIAS && MODE != 0) bias_e = bias_row[erow] * kLog2e;
+  if constexpr (BIAS && MODE != 0) {
+    bias_e = bias_row[erow] * kLog2e;
+    if (!__syncthreads_or(bias_e > -INFINITY)) nt = 0;  // no kept key among this workgroup's: zero gradients
+  }
 
   // ---- direct global -> LDS loads of one stream tile (layouts and lane maps of the forward kernel)
   const __bf16* s1p = a.s1 + b * a.s1_sb + h * a.s1_sh + ss0 * a.s1_ss;
@@ -291,11 +306,38 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       v_off[sg] = 2 * kBTileA + (4 * hh + vxr) * 64 + (sg ^ vx) * 32 + ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
   }
 
-  dma(0, 0);
+  // LISTED: the tile at position t of this workgroup's share as tile * 2 + (it holds keys with a bias)
+  constexpr bool LISTED = BIAS && MODE == 0;
+  [[maybe_unused]] auto entry = [&](int t) __attribute__((always_inline)) {
+    if (!tl.list) return 2 * t + 1;
+    const int at = sp * a.tps + t;
+    if (t == 0 && (at & 63)) tl.lane_entry = tl.list[1 + ((at & ~63) + lane < tl_n ? (at & ~63) + lane : tl_n - 1)];
+    return tl.at(at, tl_n, lane);
+  };
+  [[maybe_unused]] int ec = 0;
+  if constexpr (LISTED) {
+    if (nt > 0) {
+      ec = entry(0);
+      dma(0, ec >> 1);
+    }
+  } else {
+    if (!BIAS || nt > 0) dma(0, 0);
+  }
   for (int t = 0; t < nt; ++t) {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of tile t has landed
     __syncthreads();                      // ... and everyone's; the other slot (tile t-1) is free
-    if (t + 1 < nt) dma((t + 1) & 1, t + 1);
+    int kt = t;
+    [[maybe_unused]] bool mixed = true;
+    if constexpr (LISTED) {
+      kt = ec >> 1;
+      mixed = ec & 1;
+      if (t + 1 < nt) {
+        ec = entry(t + 1);
+        dma((t + 1) & 1, ec >> 1);
+      }
+    } else {
+      if (t + 1 < nt) dma((t + 1) & 1, t + 1);
+    }
     const __bf16* base = smem + (t & 1) * kBStage;
 
     // Start values of the two MFMA chains: -delta for dP^T, so that the chain ends on dP - delta; and, when the
@@ -365,7 +407,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     // W = P or dS, eight logits (one B operand) at a time
     if constexpr (MODE == 0) {
       if (t == nt - 1) {  // keys past the end of a ragged last tile take no part
-        const int sbase = t * kBT + 4 * hh;
+        const int sbase = kt * kBT + 4 * hh;
 #pragma unroll
         for (int i = 0; i < 16; ++i)
           if (sbase + 8 * (i >> 2) + (i & 3) >= Ss) S[i] = -INFINITY;
@@ -380,10 +422,10 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         if constexpr (MODE == 0) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) nl[e] = nlse_e;
-          if constexpr (BIAS) {
+          if (BIAS && mixed) {
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
-              const int col = t * kBT + 8 * (2 * hb + g) + 4 * hh;
+              const int col = kt * kBT + 8 * (2 * hb + g) + 4 * hh;
               const f32x4 bv = *reinterpret_cast<const f32x4*>(aux + 8 * (2 * hb + g) + 4 * hh);
 #pragma unroll
               for (int e = 0; e < 4; ++e)
@@ -497,7 +539,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 }
 
 template <int MODE, int HD, bool BIAS, bool PRE, int DC>
-__global__ __launch_bounds__((bwd_waves<HD>() * 64)) void attn_bwd_kernel(BwdArgs a) {
+__global__ __launch_bounds__((bwd_waves<HD>() * 64)) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 3 : 2, HD == 64 ? 3 : 2))) void attn_bwd_kernel(BwdArgs a) {
   attn_bwd_body<MODE, HD, BIAS, PRE, DC>(a);
 }
 // The dk / dv pass at head dim 128 wants a few registers more than half the register file (128 accumulators, 64 of
@@ -676,7 +718,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
                    int B, int H, int Sq, int Skv, int D,
                    const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                    const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                   const float* key_bias, int64_t bias_stride, bool any_head_dim = false) {
+                   const float* key_bias, int64_t bias_stride, bool any_head_dim = false, const int* tiles = nullptr) {
   if (!q || !k || !v || !out || !dout || !lse || !dq || !dk || !dv || !workspace) return MDATTN_E_BADARG;
   if (key_bias) {
     if (bias_stride < ((int64_t)Skv + 31) / 32 * 32 || bias_stride % 32 != 0) return MDATTN_E_BADARG;
@@ -716,6 +758,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   BwdArgs a;
   a.lse2 = lse2; a.delta = delta; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;
+  a.tiles = tiles; a.tiles_sb = key_tiles_ints(Skv, 32);
   auto set = [](int64_t& sb, int64_t& ss, int64_t& sh, const mdattn_strides* s) { sb = s->batch; ss = s->seq; sh = s->head; };
   // dq: entity q / dout, stream k (scores), v (dP), k (accumulate)
   a.e1 = (const __bf16*)q; a.e2 = (const __bf16*)dout; a.s1 = (const __bf16*)k; a.s2 = (const __bf16*)v; a.s3 = (const __bf16*)k;
@@ -767,9 +810,9 @@ extern "C" int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, 
                                     int B, int H, int Sq, int Skv, int D,
                                     const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                                     const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                                    const float* key_bias, int64_t bias_stride) {
+                                    const float* key_bias, int64_t bias_stride, const int* tiles) {
   return bwd_run((hipStream_t)stream, q, k, v, out, dout, lse, dq, dk, dv, workspace, workspace_floats, B, H, Sq, Skv, D,
-                 q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride, true);
+                 q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride, true, key_bias ? tiles : nullptr);
 }
 
 // ---------------------------------------------------------------------------------------------------

@@ -496,10 +496,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   const __bf16* kp = a.k + b * a.k_sb + h * a.k_sh;
   const __bf16* vp = a.v + b * a.v_sb + h * a.v_sh;
   const int q0 = qt * BM + wave * 32;
-  const int nt = (a.Skv + TS - 1) / TS;
+  [[maybe_unused]] TileList tl{BIAS && a.tiles ? a.tiles + (int64_t)b * a.tiles_sb : nullptr};
+  int nt = (a.Skv + TS - 1) / TS;  // tiles visited; with a list, 0 when every key is excluded
+  if constexpr (BIAS) nt = tl.count(nt);
   const float c = a.c;
-  // with a bias the logits are brought to log2 units (scale folded, bias added) right after the MFMAs
-  const float cs = BIAS ? 1.0f : c;
   const float* bias_row = BIAS ? a.bias + b * a.bias_sb : nullptr;
   [[maybe_unused]] const int bias_cols = (a.Skv + 31) / 32 * 32;  // entries the caller's bias rows are sure to hold
 
@@ -519,9 +519,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     const unsigned Ks = smem_addr + (unsigned)(slot * STAGE) * 2u;
     const unsigned Vs = Ks + KTILE * 2u;
     // every wave fetches the same values to the same place (a load more per wave and tile, counted in the loop's
-    // s_waitcnt): lane l and lane l + 32 the bias of key l of the tile; the ring runs up to two tiles past the end
+    // s_waitcnt): lane l and lane l + 32 the bias of key l of the tile
     if constexpr (BIAS) {  // (a 64-key tile may reach past the padded bias row, whose length is a multiple of 32)
-      int col = (kt < nt ? kt : nt - 1) * TS + (TS == 64 ? lane : l32);
+      int col = kt * TS + (TS == 64 ? lane : l32);
       col = col < bias_cols ? col : bias_cols - 1;
       lds_dma4(bias_row, (unsigned)col * 4u, Ks + TILES * 2u);
     }
@@ -551,8 +551,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 #pragma unroll
     for (int i = 0; i < 16; ++i) O[db][i] = 0.f;
   float m = -1e30f, l = 0.f;
-  float mc = PRE ? 0.f : m * cs;  // the rows' reference point in log2 units
-  f32x16 negm;                    // PRE (see the pipelined kernel): start value of every score accumulator chain
+  float mc = PRE ? 0.f : BIAS ? m : m * c;  // the rows' reference point in log2 units (its only form with a bias)
+  f32x16 negm;                              // PRE (see the pipelined kernel): start value of every score accumulator chain
 #pragma unroll
   for (int i = 0; i < 16; ++i) negm[i] = 0.f;
 
@@ -583,7 +583,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // waits for every read right before its MFMA.
   constexpr int LA = HD == 128 ? MDATTN_FLAT_LA128 : 0;
   constexpr int FPB = NJ + 2 * ND, NFRAG = NB * FPB;
-  auto tile = [&](int t, auto slot, auto masked) __attribute__((always_inline)) {  // slot: int or integral_constant
+  // t: position in the sequence of visited tiles; kt: the tile itself; mixed: it holds keys with a bias
+  auto tile = [&](int t, int kt, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {  // slot: int or integral_constant
     const __bf16* base = smem + slot * STAGE;
     constexpr int kBlk = 32 * 64;  // a 32-key block of a head-dim-64 tile: 32 rows of 64 elements, in K and in V
     auto frag = [&](int n) __attribute__((always_inline)) {
@@ -618,7 +619,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
         S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[j], (PRE && j == 0) ? negm : S, 0, 0, 0);
       }
     }
-    if constexpr (BIAS) {
+    // the logits of a tile with a bias are brought to log2 units here (scale folded, bias added); those of the others take
+    // the factor in the exponent's FMA
+    const float cs = BIAS && mixed ? 1.0f : c;
+    if (BIAS && mixed) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4 bv = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base + TILES) + 32 * blk + 8 * g + 4 * hh);
@@ -627,7 +631,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       }
     }
     if constexpr (decltype(masked)::value) {
-      const int kv_base = t * TS + 32 * blk + 4 * hh;
+      const int kv_base = kt * TS + 32 * blk + 4 * hh;
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         if (kv_base + 8 * (i >> 2) + (i & 3) >= a.Skv) S[i] = -INFINITY;
@@ -681,6 +685,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
         mc += dm;
 #pragma unroll
         for (int i = 0; i < 16; ++i) { S[i] -= dm; negm[i] -= dm; }
+      } else if constexpr (BIAS) {
+        const float mnew = fmaxf(mc, mloc * cs);
+        alpha = __builtin_amdgcn_exp2f(mc - mnew);
+        mc = mnew;
       } else {
         const float mnew = fmaxf(m, mloc);
         alpha = __builtin_amdgcn_exp2f((m - mnew) * cs);
@@ -719,7 +727,18 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // the wave fetches its 32 rows as a K-shaped tile with the same direct global->LDS loads (whole 256-byte rows per
   // 16 lanes), into a staging area behind ring slot 0 (which receives key tile 0 meanwhile), and reads the fragments
   // with the K fragment offsets.  Each wave stages and reads only its own rows.
-  dma(0, 0);
+  // The tile at position t of the sequence as tile * 2 + mixed, and its loads; without a list position and tile are the same
+  // (positions past the end load rows that are not used).
+  [[maybe_unused]] auto entry = [&](int t) __attribute__((always_inline)) { return tl.at(t < nt ? t : nt - 1, nt, lane); };
+  [[maybe_unused]] int ec = 0, en = 0;  // entries of the tile being worked on and, in a 3-slot ring, of the next
+  if constexpr (BIAS) {
+    if (nt > 0) {
+      ec = entry(0);
+      dma(0, ec >> 1);
+    }
+  } else {
+    dma(0, 0);
+  }
   {
     const unsigned Qs = smem_addr + (unsigned)(STAGE + wave * QTILE) * 2u;
 #pragma unroll
@@ -739,14 +758,29 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   }
   __syncthreads();  // every wave holds its fragments: the staging area is ring slots again
   // SLOTS - 1 tiles are requested ahead of the one being worked on
-#pragma unroll
-  for (int i = 1; i < SLOTS - 1; ++i) dma(i, i);
+  static_assert(SLOTS == 2 || SLOTS == 3, "one tile ahead, or two");
+  if constexpr (SLOTS == 3 && BIAS) {
+    if (nt > 0) {
+      en = entry(1);
+      dma(1, en >> 1);
+    }
+  } else if constexpr (SLOTS == 3) {
+    dma(1, 1);
+  }
   auto step = [&](int t, auto slot, int fill) __attribute__((always_inline)) {
     // vmcnt: this wave's share of tile t has landed (the SLOTS - 2 tiles requested after it may still be in flight)
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((SLOTS - 2) * (2 * GPW + (BIAS ? 1 : 0))));
     __syncthreads();                                  // ... and everyone's; slot `fill` (tile t-1) is free
-    dma(fill, t + SLOTS - 1);
-    tile(t, slot, std::false_type{});
+    if constexpr (BIAS) {
+      const int ef = entry(t + SLOTS - 1);
+      dma(fill, ef >> 1);
+      tile(t, ec >> 1, ec & 1, slot, std::false_type{});
+      ec = SLOTS == 3 ? en : ef;
+      en = ef;
+    } else {
+      dma(fill, t + SLOTS - 1);
+      tile(t, t, false, slot, std::false_type{});
+    }
   };
   if constexpr (HD == 64) {
     // Two copies of the loop body, one per ring slot: the slot is a compile-time constant in each, every fragment
@@ -767,7 +801,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
-  tile(nt - 1, (nt - 1) % SLOTS, std::true_type{});
+  if constexpr (BIAS) {
+    if (nt > 0) tile(nt - 1, ec >> 1, ec & 1, (nt - 1) % SLOTS, std::true_type{});
+  } else {
+    tile(nt - 1, nt - 1, false, (nt - 1) % SLOTS, std::true_type{});
+  }
 
   if (!PADDED && a.o_run) {  // ring step: merged into the f32 carry, row by row
     store_row<ND>(a, O, xhalf_sum(l), mc, b, h, q0 + l32, hh);
@@ -842,7 +880,7 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
   a.v_sb = v_strides->batch; a.v_ss = v_strides->seq; a.v_sh = v_strides->head;
   a.o_sb = o_strides->batch; a.o_ss = o_strides->seq; a.o_sh = o_strides->head;
   a.c = scale * kLog2e;
-  a.bias = nullptr; a.bias_sb = 0;
+  a.bias = nullptr; a.bias_sb = 0; a.tiles = nullptr; a.tiles_sb = 0;
   a.o_run = nullptr; a.lse_run = nullptr;
   return MDATTN_OK;
 }
@@ -882,19 +920,23 @@ extern "C" int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, 
                                     int B, int H, int Sq, int Skv, int D,
                                     const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                                     const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                                    const float* key_bias, int64_t bias_stride) {
-  if (D == 64 || D == kD)
-    return key_bias ? mdattn_fwd_bf16_bias(stream, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride)
-                    : mdattn_fwd_bf16(stream, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale);
+                                    const float* key_bias, int64_t bias_stride, const int* tiles) {
   AttnArgs a;
   const int rc = fill_args(a, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale, true);
   if (rc != MDATTN_OK) return rc;
-  if (!key_bias) return dispatch_padded<false>((hipStream_t)stream, a, B);
+  const hipStream_t st = (hipStream_t)stream;
+  if (!key_bias) return D == 64 || D == kD ? dispatch_fwd(st, a, B, Sq, Skv, D) : dispatch_padded<false>(st, a, B);
   if (bias_stride < ((Skv + kTS - 1) / kTS) * kTS || bias_stride % kTS != 0) return MDATTN_E_BADARG;
-  if (!aligned16(key_bias)) return MDATTN_E_ALIGN;
+  if (!aligned16(key_bias) || (reinterpret_cast<uintptr_t>(tiles) & 3u)) return MDATTN_E_ALIGN;
   a.bias = key_bias;
   a.bias_sb = bias_stride;
-  return dispatch_padded<true>((hipStream_t)stream, a, B);
+  if (tiles) {  // the list for 32-key tiles, or behind it the one for 64-key tiles
+    a.tiles = D > 64 ? tiles : tiles + (int64_t)B * key_tiles_ints(Skv, 32);
+    a.tiles_sb = key_tiles_ints(Skv, D > 64 ? 32 : 64);
+  }
+  if (D == kD) return launch_flat<4, true>(st, a, B);
+  if (D == 64) return launch_flat<4, true, 64>(st, a, B);
+  return dispatch_padded<true>(st, a, B);
 }
 
 extern "C" int mdattn_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,

@@ -84,32 +84,48 @@ Tensor grad_like(const Tensor& g, const Tensor& like) {
 }
 
 // ------------------------------------------------------------------------------------------------ attention
+// A key mask as the kernels take it, in one buffer: the additive bias f32 [B, ceil32(Skv)], then the tile lists
+struct Mask {
+  float* bias = nullptr;
+  int* tiles = nullptr;
+  int64_t stride = 0;
+  static int64_t cols(int64_t skv) { return (skv + 31) / 32 * 32; }
+  Mask(const Tensor& m, const View& vk) {
+    if (!m.defined()) return;
+    stride = cols(vk.s);
+    bias = m.data_ptr<float>();
+    tiles = reinterpret_cast<int*>(bias + vk.b * stride);
+  }
+};
+
 int fwd(const Tensor& q, const Tensor& k, const Tensor& v, const View& vq, const View& vk, const View& vv, const Tensor& out, const Tensor& lse,
-        const Tensor& bias, double scale) {
+        const Tensor& mask, double scale) {
+  const Mask m(mask, vk);
   const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
   return mdattn_host_fwd_bf16(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st, &vk.st,
-                              &vv.st, &so, (float)scale, f32(bias), bias.defined() ? bias.stride(0) : 0);
+                              &vv.st, &so, (float)scale, m.bias, m.stride, m.tiles);
 }
 
 // q, k, v in the caller's own rank; out [B,Sq,H*D]
 struct FlashFn : torch::autograd::Function<FlashFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& bias_, int64_t heads, double scale) {
-    const Tensor bias = value(bias_);
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& mask_, int64_t heads, double scale) {
+    const Tensor mask = value(mask_);
     const View vq = *as_view(q, heads), vk = *as_view(k, heads), vv = *as_view(v, heads);
     Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
     Tensor lse = at::empty({vq.b, vq.h, vq.s}, q.options().dtype(at::kFloat));
-    must(fwd(q, k, v, vq, vk, vv, out, lse, bias, scale), "mdattn_fwd_bf16");
-    ctx->save_for_backward({q, k, v, out, lse, bias});
+    must(fwd(q, k, v, vq, vk, vv, out, lse, mask, scale), "mdattn_fwd_bf16");
+    ctx->save_for_backward({q, k, v, out, lse, mask});
     ctx->saved_data["heads"] = heads;
     ctx->saved_data["scale"] = scale;
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &bias = saved[5];
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &mask = saved[5];
     const int64_t heads = ctx->saved_data["heads"].toInt();
     const double scale = ctx->saved_data["scale"].toDouble();
     const View vq = *as_view(q, heads), vk = *as_view(k, heads), vv = *as_view(v, heads);
+    const Mask m(mask, vk);
     const Tensor dout = grad_like(grads[0], out);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     const int B = (int)vq.b, H = (int)vq.h, Sq = (int)vq.s, Skv = (int)vk.s, D = (int)vq.d;
@@ -117,26 +133,26 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     Tensor ws = at::empty({nws}, lse.options());
     const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
     const int rc = mdattn_host_bwd_bf16(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq,
-                                        Skv, D, &vq.st, &vk.st, &vv.st, &so, (float)scale, f32(bias), bias.defined() ? bias.stride(0) : 0);
+                                        Skv, D, &vq.st, &vk.st, &vv.st, &so, (float)scale, m.bias, m.stride, m.tiles);
     must(rc, "mdattn_bwd_bf16");
     return {dq, dk, dv, Tensor(), Tensor(), Tensor()};
   }
 };
 
-// [B,Skv] keep-mask (bool or uint8) -> additive bias f32 [B, ceil32(Skv)], or undefined when the mask needs the Python path
-Tensor mask_bias(const Tensor& keep, const View& vk, const Tensor& ref) {
+// [B,Skv] keep-mask (bool or uint8) -> Mask, or undefined when it needs the Python path
+Tensor make_mask(const Tensor& keep, const View& vk, const Tensor& ref) {
   if (!keep.is_cuda() || keep.get_device() != ref.get_device() || (keep.scalar_type() != at::kBool && keep.scalar_type() != at::kByte) ||
       keep.dim() != 2 || keep.size(0) != vk.b || keep.size(1) != vk.s || !keep.is_contiguous())
     return Tensor();
-  const int64_t cols = (vk.s + 31) / 32 * 32;
-  Tensor bias = at::empty({vk.b, cols}, keep.options().dtype(at::kFloat));
-  if (mdattn_key_mask_bias(stream(), ptr(keep), f32(bias), (int)vk.b, (int)vk.s, cols, -INFINITY) != MDATTN_OK) return Tensor();
-  return bias;
+  const int B = (int)vk.b, S = (int)vk.s;
+  Tensor m = at::empty({B * Mask::cols(S) + mdattn_host_key_tiles_ints(B, S)}, keep.options().dtype(at::kFloat));
+  const Mask v(m, vk);
+  return mdattn_host_key_tiles(stream(), ptr(keep), v.bias, v.tiles, B, S, v.stride) == MDATTN_OK ? m : Tensor();
 }
 
 // The registry entry's operands, checked: false when the Python path has to take over
 bool flash_args(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep, View& vq, View& vk, View& vv,
-                Tensor& bias) {
+                Tensor& mask) {
   if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q)) return false;
   const auto a = as_view(q, heads), b = as_view(k, heads), c = as_view(v, heads);
   if (!a || !b || !c || a->b != b->b || a->b != c->b || a->h != b->h || a->h != c->h || a->d != b->d || a->d != c->d ||
@@ -144,7 +160,7 @@ bool flash_args(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads
     return false;
   if (!mdattn_host_head_dim((int)a->d)) return false;  // padded first
   if (q.numel() == 0 || k.numel() == 0 || std::max(a->s, b->s) >= ((int64_t)1 << 31)) return false;
-  if (keep.has_value() && !(bias = mask_bias(*keep, *b, q)).defined()) return false;
+  if (keep.has_value() && !(mask = make_mask(*keep, *b, q)).defined()) return false;
   vq = *a; vk = *b; vv = *c;
   return true;
 }
@@ -152,8 +168,8 @@ bool flash_args(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads
 // The registry entry `hip_flash`: [B,S,H*D] or [B,H,S,D] operands -> [B,Sq,H*D]; q_mul is rounded into q first.
 OptTensor flash(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep, double q_mul) {
   View vq, vk, vv;
-  Tensor bias;
-  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, bias)) return std::nullopt;
+  Tensor mask;
+  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, mask)) return std::nullopt;
   at::NoGradGuard guard;
   Tensor qf = q;
   if (q_mul != 1.0) {
@@ -163,17 +179,17 @@ OptTensor flash(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads
     vq = *w;
   }
   Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
-  if (fwd(qf, k, v, vq, vk, vv, out, Tensor(), bias, scale) != MDATTN_OK) return std::nullopt;
+  if (fwd(qf, k, v, vq, vk, vv, out, Tensor(), mask, scale) != MDATTN_OK) return std::nullopt;
   return out;
 }
 
 OptTensor flash_autograd(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep) {
   View vq, vk, vv;
-  Tensor bias;
+  Tensor mask;
   for (const Tensor* t : {&q, &k, &v})
     if (!t->is_non_overlapping_and_dense()) return std::nullopt;  // their gradients take the same strides
-  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, bias)) return std::nullopt;
-  return FlashFn::apply(q, k, v, opt(bias), heads, scale);
+  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, mask)) return std::nullopt;
+  return FlashFn::apply(q, k, v, opt(mask), heads, scale);
 }
 
 // One ring step (ops.flash_attention_merge) on logical [B,S,H,D] views; false: the Python path takes it

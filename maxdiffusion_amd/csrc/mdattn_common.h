@@ -125,6 +125,24 @@ __device__ __forceinline__ unsigned lds_addr_of(const void* p) {
   return (unsigned)(uintptr_t)(const void __attribute__((address_space(3)))*)p;
 }
 
+// The key tiles that a masked pass visits (made by key_tiles_kernel): entry = tile * 2 + (1: the tile holds excluded keys).  A
+// wave keeps 64 entries in a register, one per lane, and reads the wanted one into a scalar: a scalar load per tile would
+// turn every LDS wait around it into a full one.
+struct TileList {
+  const int* list;  // [count, entry 0, entry 1, ..]; null: every tile, the bias applied in each
+  int lane_entry = 0;
+  __device__ __forceinline__ int count(int all) const { return list ? __builtin_amdgcn_readfirstlane(list[0]) : all; }
+  // entry t of n; successive calls go up by one, or repeat
+  __device__ __forceinline__ int at(int t, int n, int lane) {
+    if (!list) return 2 * t + 1;
+    if ((t & 63) == 0) {
+      const int i = t + lane;
+      lane_entry = list[1 + (i < n ? i : n - 1)];
+    }
+    return __builtin_amdgcn_readlane(lane_entry, t & 63);
+  }
+};
+
 // Arguments of the attention-forward kernels (element strides; head_dim contiguous).
 struct AttnArgs {
   const __bf16* q;
@@ -141,6 +159,8 @@ struct AttnArgs {
   float c;  // scale * log2(e)
   const float* bias;   // optional additive per-key bias [B, bias_sb] (natural-log units), flat kernel only
   int64_t bias_sb;
+  const int* tiles;    // with a bias: per batch, the number of key tiles to visit and their entries (see key_tiles_kernel); null: all
+  int tiles_sb;
   float* o_run;    // when set: no `out`; the result is merged in LSE space into this f32 carry (strides o_s*, in floats)
   float* lse_run;  // ... and into its lse [B,H,Sq]
 };
@@ -148,6 +168,8 @@ struct AttnArgs {
 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+// ints per batch of a TileList for tiles of ts keys
+inline int key_tiles_ints(int Skv, int ts) { return 1 + (Skv + ts - 1) / ts; }
 // Head dims that the attention kernels walk as they are: 64 and 128, and, in the layout of the next of these two with the
 // MFMAs that cover 48, 80 or 96 columns, multiples of 8 up to 48 and from 72 to 96.  (56 saves nothing against 64; 104 to 120
 // save a column of MFMAs at most, spill in the backward, and lose the pipelined forward: they are padded by the caller.)

@@ -14,20 +14,25 @@ extern "C" {
  * f32 partial gradients.  With less, the call runs unsplit. */
 int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D);
 
+/* A [B, Skv] keep-mask (bytes) -> the additive bias of mdattn_key_mask_bias (-inf for excluded keys; bias_stride a multiple of
+ * 32) and, in `tiles` (mdattn_host_key_tiles_ints ints), per batch element the lists of key tiles that hold a kept key. */
+int64_t mdattn_host_key_tiles_ints(int B, int Skv);
+int mdattn_host_key_tiles(void* stream, const void* keep, float* bias, int* tiles, int B, int Skv, int64_t bias_stride);
+
 /* Whether mdattn_host_fwd_bf16 and mdattn_host_bwd_bf16 take head dim D. */
 int mdattn_host_head_dim(int D);
 
-/* mdattn_fwd_bf16 / mdattn_fwd_bf16_bias (key_bias null: none) at 64, 128 and the multiples of 8 up to 48 and from
+/* mdattn_fwd_bf16 / mdattn_fwd_bf16_bias (key_bias null: none; tiles: that bias' tile lists, or null: every tile is visited) at 64, 128 and the multiples of 8 up to 48 and from
  * 72 to 96. */
 int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse, int B, int H, int Sq, int Skv, int D,
                          const mdattn_strides* q_strides, const mdattn_strides* k_strides, const mdattn_strides* v_strides,
-                         const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride);
+                         const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride, const int* tiles);
 
-/* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias null: none) at the head dims of mdattn_host_fwd_bf16. */
+/* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias and tiles as above) at the head dims of mdattn_host_fwd_bf16. */
 int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, void* dq,
                          void* dk, void* dv, float* workspace, int64_t workspace_floats, int B, int H, int Sq, int Skv, int D,
                          const mdattn_strides* q_strides, const mdattn_strides* k_strides, const mdattn_strides* v_strides,
-                         const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride);
+                         const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride, const int* tiles);
 
 /* The prologue and its backward with the rotary table in the layout the model made it in:
  *   PLANES    cos, sin f32 [S, D/2] (the layout of mdattn.h's entry points)

@@ -1,6 +1,7 @@
 // HBM-bound helpers around the attention kernel: LSE-space chunk merge, f32->bf16 finalize,
 // per-tensor absmax e4m3 quantisation.
 #include "mdattn_common.h"
+#include "mdattn_host.h"
 
 namespace mdattn {
 
@@ -216,5 +217,95 @@ extern "C" int mdattn_key_mask_bias(void* stream, const void* keep, float* bias,
   const unsigned gx = (unsigned)((bias_stride + 255) / 256 < 1024 ? (bias_stride + 255) / 256 : 1024);
   MDATTN_LAUNCH(mdattn::key_mask_bias_kernel, dim3(gx, B), dim3(256), 0, (hipStream_t)stream,
                      (const uint8_t*)keep, bias, Skv, bias_stride, masked_value);
+  return mdattn::launch_status();
+}
+
+// ------------------------------------------------------------------------------- key mask -> bias and tile lists
+namespace mdattn {
+// The bias of key_mask_bias_kernel (masked value -inf) together with the lists of key tiles that hold a kept key, for
+// tiles of 32 and of 64 keys: a masked attention then costs what its kept keys cost.  One workgroup per batch element; a
+// lane takes two 32-key tiles (one 64-key tile) per turn, ranks come from a ballot per wave and the waves' sums.  Masked calls
+// before (every tile visited, the bias added to every logit) and with the lists: 500 of 2,048 keys x 2,048 queries x 20
+// heads 59 -> 23 us; 3,900 of 4,096 keys 185 -> 170 us at head dim 128, 123 -> 106 us at 64 (x 2 x 10 heads).
+__global__ __launch_bounds__(1024) void key_tiles_kernel(const uint8_t* __restrict__ keep, float* __restrict__ bias, int* __restrict__ tiles,
+                                                         int Skv, int64_t bias_stride, int sb32, int sb64) {
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint8_t* kb = keep + (int64_t)b * Skv;
+  float* bb = bias + b * bias_stride;
+  int* l32 = tiles + (int64_t)b * sb32;
+  int* l64 = tiles + (int64_t)gridDim.x * sb32 + (int64_t)b * sb64;
+  __shared__ unsigned char kept[2][1024];  // keys kept in each half of a lane's tile
+  __shared__ int sums[2][16];
+  const int n64 = (Skv + 63) / 64;
+  int base32 = 0, base64 = 0;
+  for (int t0 = 0; t0 < n64; t0 += 1024) {
+    for (int h = tid; h < 2048; h += 1024) reinterpret_cast<unsigned char*>(kept)[h] = 0;
+    __syncthreads();
+    // the 1024 tiles' keys, neighbouring lanes on neighbouring keys: a wave covers one 64-key tile per trip
+    const int last = t0 + 1024 < n64 ? t0 + 1024 : n64;
+    for (int t = t0 + wave; t < last; t += 16 * 8) {
+      bool k[8];  // eight loads in flight
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = (t + 16 * i) * 64 + lane;
+        k[i] = key < Skv && kb[key];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int ti = t + 16 * i, key = ti * 64 + lane;
+        if (ti >= last) break;
+        if (key < bias_stride) bb[key] = k[i] ? 0.f : -INFINITY;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(k[i]);
+        if (lane == 0) {
+          kept[0][ti - t0] = (unsigned char)__popc((unsigned)m);
+          kept[1][ti - t0] = (unsigned char)__popc((unsigned)(m >> 32));
+        }
+      }
+    }
+    __syncthreads();
+    const int t = t0 + tid;
+    const int k0 = kept[0][tid], k1 = kept[1][tid];
+    const int n32 = (k0 > 0) + (k1 > 0), any = k0 + k1 > 0;
+    // exclusive ranks: of the first / second half's tile among the 32-key tiles, of the tile among the 64-key tiles
+    const unsigned long long lt = (1ull << lane) - 1;
+    const unsigned long long b0 = __builtin_amdgcn_ballot_w64(k0 > 0), b1 = __builtin_amdgcn_ballot_w64(k1 > 0), ba = __builtin_amdgcn_ballot_w64(any);
+    int r32 = __popcll(b0 & lt) + __popcll(b1 & lt), r64 = __popcll(ba & lt);
+    if (lane == 0) {
+      sums[0][wave] = __popcll(b0) + __popcll(b1);
+      sums[1][wave] = __popcll(ba);
+    }
+    __syncthreads();
+    int tot32 = 0, tot64 = 0;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wave) { r32 += sums[0][w]; r64 += sums[1][w]; }
+      tot32 += sums[0][w];
+      tot64 += sums[1][w];
+    }
+    const int left = Skv - t * 64;  // keys of this tile that exist
+    if (n32) {
+      const int e0 = left < 32 ? left : 32, e1 = left - 32 < 32 ? left - 32 : 32;
+      if (k0 > 0) l32[1 + base32 + r32] = 4 * t + (k0 < e0);
+      if (k1 > 0) l32[1 + base32 + r32 + (k0 > 0)] = 4 * t + 2 + (k1 < e1);
+      l64[1 + base64 + r64] = 2 * t + (k0 + k1 < (left < 64 ? left : 64));
+    }
+    base32 += tot32;
+    base64 += tot64;
+    __syncthreads();  // kept and sums are rewritten
+  }
+  if (tid == 0) {
+    l32[0] = base32;
+    l64[0] = base64;
+  }
+}
+}  // namespace mdattn
+
+extern "C" int64_t mdattn_host_key_tiles_ints(int B, int Skv) {
+  return (int64_t)B * (key_tiles_ints(Skv, 32) + key_tiles_ints(Skv, 64));
+}
+
+extern "C" int mdattn_host_key_tiles(void* stream, const void* keep, float* bias, int* tiles, int B, int Skv, int64_t bias_stride) {
+  if (!keep || !bias || !tiles || B <= 0 || Skv <= 0 || bias_stride < Skv || bias_stride % 32) return MDATTN_E_BADARG;
+  MDATTN_LAUNCH(mdattn::key_tiles_kernel, dim3(B), dim3(1024), 0, (hipStream_t)stream, (const uint8_t*)keep, bias, tiles, Skv, bias_stride,
+                key_tiles_ints(Skv, 32), key_tiles_ints(Skv, 64));
   return mdattn::launch_status();
 }

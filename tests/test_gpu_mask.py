@@ -92,3 +92,55 @@ def test_reference_hand_fixture_and_dispatcher(dev):
   # :91-116: everything masked -> zeros
   got = op.apply_attention(q, k, v, attention_mask=torch.tensor([[0, 0]], device=dev))
   assert torch.count_nonzero(got) == 0
+
+
+@pytest.mark.parametrize("D", [128, 64, 80])
+@pytest.mark.parametrize("skv,kind", [(384, "prefix257"), (4500, "prefix100"), (2200, "blocks"), (97, "last"), (333, "none"), (64, "all"), (2111, "holes")])
+def test_masked_attention_visits_the_kept_tiles_only(dev, lib, D, skv, kind):
+  """The registry entry's mask path (tile lists made on the device) against the same attention on the kept keys alone, forward
+  and gradients: lists of one and several registers, tiles dropped in front, between and behind, none kept in one batch
+  element.  f32 accumulation in another order only: bf16 bars of the unmasked kernels."""
+  from maxdiffusion_amd import attention_op as A
+  B, H, sq = 2, 2, 70
+  gen = torch.Generator(device=dev).manual_seed(skv)
+  keep = torch.zeros((B, skv), dtype=torch.bool, device=dev)
+  if kind.startswith("prefix"):
+    keep[:, :int(kind[6:])] = True
+    keep[1, 40:] = False
+  elif kind == "blocks":
+    keep[0, 64:128] = keep[0, 1990:2100] = keep[1, 500:501] = True
+  elif kind == "last":
+    keep[:, skv - 1] = True
+  elif kind == "all":
+    keep[:] = True
+  elif kind == "holes":
+    keep[:] = torch.rand((B, skv), generator=gen, device=dev) < 0.05
+    keep[0, 0] = keep[1, 7] = True
+  else:
+    keep[0, 3:200] = True  # nothing kept in element 1
+  mk = lambda s: torch.randn((B, s, H * D), generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True)
+  q, k, v = mk(sq), mk(skv), mk(skv)
+  g = torch.randn((B, sq, H * D), generator=gen, device=dev).to(torch.bfloat16)
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+  out = op.apply_attention(q, k, v, attention_mask=keep)
+  grads = torch.autograd.grad(out, (q, k, v), g)
+  with torch.no_grad():
+    assert torch.equal(op.apply_attention(q, k, v, attention_mask=keep), out)
+  for b in range(B):
+    idx = keep[b].nonzero()[:, 0]
+    for t in (grads[1], grads[2]):
+      assert not t[b][~keep[b]].any()
+    if idx.numel() == 0:
+      assert not out[b].any() and not grads[0][b].any()
+      continue
+    rq, rk, rv = (t.detach().float().requires_grad_(True) for t in (q[b], k[b, idx], v[b, idx]))
+    hf = lambda t: t.view(-1, H, D).transpose(0, 1)
+    ref = (torch.softmax((hf(rq) @ hf(rk).transpose(1, 2)) * D**-0.5, -1) @ hf(rv)).transpose(0, 1).reshape(sq, H * D)
+    want = torch.autograd.grad(ref, (rq, rk, rv), g[b].float())
+    for name, got, r in (("out", out[b], ref), ("dq", grads[0][b], want[0]), ("dk", grads[1][b, idx], want[1]), ("dv", grads[2][b, idx], want[2])):
+      r = r.detach()
+      if float(r.abs().max()) < 1e-5:  # a single key: the exact gradients of q and k are zero
+        assert float(got.detach().float().abs().max()) <= 0.25, name
+        continue
+      rel = float((got.detach().float() - r).norm() / r.norm())
+      assert rel <= 6e-3, (name, kind, rel)
