@@ -314,9 +314,9 @@ _ROWS_MODES = {"none": 0, "interleaved": 1, "split": 2}
 
 def _norm_rope_rows(x, w, cos, sin, heads, mode, eps):
   if x.is_cuda:
-    out = _lib.host().norm_rope_rows(x, w, cos, sin, heads, _ROWS_MODES[mode], eps)
+    out = _lib.host().norm_rope_rows(x, None, w, None, cos, sin, heads, _ROWS_MODES[mode], eps, 1.0)
     if out is not None:
-      return out
+      return out[0]
   if _wants_grad(x, w):
     return _HipNormRopeRows.apply(x, w, cos, sin, heads, mode, eps)
   return ops.norm_rope_rows(x, w, cos, sin, heads=heads, mode=mode, eps=eps)
@@ -358,6 +358,12 @@ def hip_norm_rope_ltx2(query, key, norm_q_scale, norm_k_scale, heads: int, rotar
   k_tab = k_rotary_emb if k_rotary_emb is not None else (rotary_emb if is_self_attention else None)
   if rotary_emb is None:
     q_tab = k_tab = None
+
+  if key is not None and k_tab is q_tab and query.is_cuda:  # one launch: q and k share every read of the tables
+    cos, sin = (None, None) if q_tab is None else (t.to(torch.float32).contiguous() for t in q_tab)
+    out = _lib.host().norm_rope_rows(query, key, norm_q_scale, norm_k_scale, cos, sin, heads, 0 if q_tab is None else _ROWS_MODES[rope_type], eps, q_mul)
+    if out is not None:
+      return out[0], out[1]
 
   def run(x, scale, tab):
     if tab is None:

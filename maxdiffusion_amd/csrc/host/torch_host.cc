@@ -440,65 +440,78 @@ std::optional<variable_list> norm_rope_qkv(const Tensor& x, const Tensor& bias, 
   return out;
 }
 
-// LTX-2: one tensor, f32 weight, tables of its own size (mode 1) or [B,H,S,D/2] (mode 2)
-Tensor rows_run(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t heads, int64_t mode, double eps) {
-  const int64_t b = x.size(0), s = x.size(1), d = x.size(2) / heads;
-  Tensor out = at::empty({b, s, heads, d}, x.options().dtype(at::kBFloat16));
-  const mdattn_strides so = strides4(out);
-  const int rc = mdattn_norm_rope_rows(stream(), ptr(x), x.scalar_type() == at::kFloat, mut(out), f32(w), mode ? f32(cos) : nullptr,
-                                       mode ? f32(sin) : nullptr, (int)mode, (int)b, (int)s, (int)heads, (int)d, (float)eps, x.stride(0), x.stride(1), &so);
-  return rc == MDATTN_OK ? out : Tensor();
+// LTX-2: q, or q and k with one table; f32 weights; tables of the tensors' own size (mode 1) or [B,H,S,D/2] (mode 2)
+struct Rows {
+  int64_t heads, mode;
+  double eps, w_mul;
+};
+variable_list rows_run(const Tensor& q, const Tensor& k, const Tensor& wq, const Tensor& wk, const Tensor& cos, const Tensor& sin, const Rows& p) {
+  const int64_t b = q.size(0), s = q.size(1), d = q.size(2) / p.heads;
+  Tensor qo = alloc_bshd(q, b, s, p.heads, d, false), ko = k.defined() ? alloc_bshd(q, b, s, p.heads, d, false) : Tensor();
+  const mdattn_strides so = strides4(qo);
+  const int rc = mdattn_host_norm_rope_rows(stream(), ptr(q), ptr(k), q.scalar_type() == at::kFloat, mut(qo), mut(ko), f32(wq), f32(wk), f32(cos), f32(sin),
+                                            (int)p.mode, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps, (float)p.w_mul, q.stride(0), q.stride(1), &so);
+  if (rc != MDATTN_OK) return {};
+  return k.defined() ? variable_list{qo, ko} : variable_list{qo};
 }
 struct RowsFn : torch::autograd::Function<RowsFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const OptTensor& cos_, const OptTensor& sin_, int64_t heads,
-                        int64_t mode, double eps) {
-    const Tensor cos = value(cos_), sin = value(sin_);
-    Tensor out = rows_run(x, w, cos, sin, heads, mode, eps);
-    TORCH_CHECK(out.defined(), "mdattn_norm_rope_rows refused the request");
-    ctx->save_for_backward({x, w, cos, sin});
-    ctx->saved_data["i"] = c10::List<int64_t>({heads, mode});
-    ctx->saved_data["eps"] = eps;
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const OptTensor& k_, const Tensor& wq, const OptTensor& wk_, const OptTensor& cos_,
+                               const OptTensor& sin_, const Rows& p) {
+    const Tensor k = value(k_), wk = value(wk_), cos = value(cos_), sin = value(sin_);
+    variable_list out = rows_run(q, k, wq, wk, cos, sin, p);
+    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_rows refused the request");
+    ctx->save_for_backward({q, k, wq, wk, cos, sin});
+    ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode});
+    ctx->saved_data["f"] = c10::List<double>({p.eps, p.w_mul});
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto sv = ctx->get_saved_variables();
-    const Tensor &x = sv[0], &w = sv[1];
+    const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3];
     const auto iv = ctx->saved_data["i"].toIntVector();
-    const int64_t heads = iv[0], mode = iv[1], b = x.size(0), s = x.size(1), n = x.size(2);
-    const Tensor g = grad_like(grads[0], Tensor());
-    Tensor dx = at::empty_strided(x.sizes(), x.strides(), x.options());
-    Tensor dw = at::empty({n}, w.options());
-    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, n);
-    Tensor ws = at::empty({nws}, w.options());
-    const mdattn_strides sg = strides4(g);
-    must(mdattn_norm_rope_rows_bwd(stream(), ptr(x), x.scalar_type() == at::kFloat, ptr(g), mut(dx), f32(w), f32(dw), mode ? f32(sv[2]) : nullptr,
-                                   mode ? f32(sv[3]) : nullptr, (int)mode, (int)b, (int)s, (int)heads, (int)(n / heads),
-                                   (float)ctx->saved_data["eps"].toDouble(), x.stride(0), x.stride(1), dx.stride(0), dx.stride(1), &sg, f32(ws), nws),
+    const auto fv = ctx->saved_data["f"].toDoubleVector();
+    const int64_t heads = iv[0], mode = iv[1], b = q.size(0), s = q.size(1), n = q.size(2);
+    const bool pair = k.defined();
+    const Tensor gq = grad_like(grads[0], Tensor()), gk = pair ? grad_like(grads[1], gq) : Tensor();
+    Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = pair ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
+    Tensor dwq = at::empty({n}, wq.options()), dwk = pair ? at::empty({n}, wq.options()) : Tensor();
+    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, (pair ? 2 : 1) * n);
+    Tensor ws = at::empty({nws}, wq.options());
+    const mdattn_strides sg = strides4(gq);
+    must(mdattn_host_norm_rope_rows_bwd(stream(), ptr(q), ptr(k), q.scalar_type() == at::kFloat, ptr(gq), ptr(gk), mut(dq), mut(dk), f32(wq), f32(wk),
+                                        f32(dwq), f32(dwk), f32(sv[4]), f32(sv[5]), (int)mode, (int)b, (int)s, (int)heads, (int)(n / heads), (float)fv[0],
+                                        (float)fv[1], q.stride(0), q.stride(1), dq.stride(0), dq.stride(1), &sg, f32(ws), nws),
          "mdattn_norm_rope_rows_bwd");
-    return {dx, dw, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dq, dk, dwq, dwk, Tensor(), Tensor(), Tensor()};
   }
 };
 
-OptTensor norm_rope_rows(const Tensor& x, const Tensor& w, const OptTensor& cos_, const OptTensor& sin_, int64_t heads, int64_t mode, double eps) {
-  const Tensor cos = value(cos_), sin = value(sin_);
-  if (!x.is_cuda() || (x.scalar_type() != at::kFloat && x.scalar_type() != at::kBFloat16) || x.is_neg() || x.dim() != 3 || x.numel() == 0 ||
-      x.stride(2) != 1 || heads <= 0 || x.size(2) % heads)
+std::optional<variable_list> norm_rope_rows(const Tensor& q, const OptTensor& k_, const Tensor& wq, const OptTensor& wk_, const OptTensor& cos_,
+                                            const OptTensor& sin_, int64_t heads, int64_t mode, double eps, double w_mul) {
+  const Tensor k = value(k_), wk = value(wk_), cos = value(cos_), sin = value(sin_);
+  if (!q.is_cuda() || (q.scalar_type() != at::kFloat && q.scalar_type() != at::kBFloat16) || q.is_neg() || q.dim() != 3 || q.numel() == 0 ||
+      q.stride(2) != 1 || heads <= 0 || q.size(2) % heads)
     return std::nullopt;
-  const int64_t b = x.size(0), s = x.size(1), n = x.size(2);
-  if (!in_place(w, at::kFloat, n, x)) return std::nullopt;
+  const int64_t b = q.size(0), s = q.size(1), n = q.size(2);
+  if (!in_place(wq, at::kFloat, n, q)) return std::nullopt;
+  if (k.defined() && (n > 4096 || k.scalar_type() != q.scalar_type() || !k.is_cuda() || k.get_device() != q.get_device() || k.is_neg() ||
+                      k.sizes() != q.sizes() || k.strides() != q.strides() || !wk.defined() || !in_place(wk, at::kFloat, n, q)))
+    return std::nullopt;
   if (mode) {
     const std::array<int64_t, 3> full{b, s, n};
     const std::array<int64_t, 4> half{b, heads, s, n / heads / 2};
     const at::IntArrayRef want = mode == 1 ? at::IntArrayRef(full) : at::IntArrayRef(half);
     for (const Tensor* t : {&cos, &sin})
-      if (!t->defined() || t->sizes() != want || !in_place(*t, at::kFloat, t->numel(), x)) return std::nullopt;
+      if (!t->defined() || t->sizes() != want || !in_place(*t, at::kFloat, t->numel(), q)) return std::nullopt;
   }
-  if (wants_grad({&x, &w})) {
-    if (!x.is_non_overlapping_and_dense()) return std::nullopt;
-    return RowsFn::apply(x, w, opt(cos), opt(sin), heads, mode, eps);
+  const Rows p{heads, mode, eps, w_mul};
+  const Tensor c = mode ? cos : Tensor(), sn = mode ? sin : Tensor();
+  if (wants_grad({&q, &k, &wq, &wk})) {
+    if (!q.is_non_overlapping_and_dense()) return std::nullopt;
+    return RowsFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(c), opt(sn), p);
   }
-  Tensor out = rows_run(x, w, cos, sin, heads, mode, eps);
-  if (!out.defined()) return std::nullopt;
+  variable_list out = rows_run(q, k, wq, wk, c, sn, p);
+  if (out.empty()) return std::nullopt;
   return out;
 }
 

@@ -66,6 +66,18 @@ int mdattn_host_norm_rope_perhead_bwd(void* stream, const void* q_in, const void
                                       const mdattn_strides* dx_strides, const mdattn_strides* g_strides, float* workspace,
                                       int64_t workspace_floats);
 
+/* mdattn_norm_rope_rows and its backward over q and k of one shape at once, the tables shared (k null: one tensor; with k at
+ * most 4,096 channels), the factor w_mul multiplied into q's weight (dwq is the gradient of the weight without it).
+ * workspace: mdattn_norm_rope_bwd_workspace_floats(B*S, H*D times the number of tensors). */
+int mdattn_host_norm_rope_rows(void* stream, const void* q_in, const void* k_in, int x_is_f32, void* q_out, void* k_out, const float* wq,
+                               const float* wk, const float* cos, const float* sin, int rope_mode, int B, int S, int H, int D, float eps,
+                               float w_mul, int64_t in_stride_batch, int64_t in_stride_seq, const mdattn_strides* out_strides);
+int mdattn_host_norm_rope_rows_bwd(void* stream, const void* q_in, const void* k_in, int x_is_f32, const void* gq, const void* gk, void* dq, void* dk,
+                                   const float* wq, const float* wk, float* dwq, float* dwk, const float* cos, const float* sin, int rope_mode,
+                                   int B, int S, int H, int D, float eps, float w_mul, int64_t in_stride_batch, int64_t in_stride_seq,
+                                   int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides, float* workspace,
+                                   int64_t workspace_floats);
+
 #ifdef __cplusplus
 }
 #endif

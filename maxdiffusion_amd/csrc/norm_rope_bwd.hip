@@ -425,29 +425,30 @@ __global__ __launch_bounds__(256) void norm_rope_perhead_bwd_kernel(NormRopeBwdH
 
 // ------------------------------------------------------------------------------------------------ rows (LTX-2)
 struct NormRopeBwdRowsArgs {
-  const void* x_in;
-  const __bf16* g;   // [B,S,H,D] by (g_sb, g_ss, g_sh)
-  void* dx;          // like x_in (bf16 or f32), strides dx_sb, dx_ss
-  const float* w;
+  const void* x_in[2];
+  const __bf16* g[2];  // [B,S,H,D] by (g_sb, g_ss, g_sh)
+  void* dx[2];         // like x_in (bf16 or f32), strides dx_sb, dx_ss
+  const float* w[2];
   const float* cos;
   const float* sin;
-  float* part;       // [nb][N]
+  float* part;         // [nb][tensors * N]
   int S, H, D, N, mode, ntok, nb;
-  float eps, inv_n;
+  float eps, inv_n, w_mul;
   int64_t in_sb, in_ss, dx_sb, dx_ss, g_sb, g_ss, g_sh;
 };
 
 // A lane works on "units" of two 8-element chunks of one head, c and c + D/16 (both partners of either pairing), as
-// the forward kernel does.
-template <int MAXU, bool F32IN>
+// the forward kernel does.  NT tensors per launch: q and k share the table reads (see norm_rope_rows_kernel) and the
+// column sum: 2 x 1,337 tokens x 2,048 channels (f32, split tables) 2 x 18.1 + 2 x 4.6 -> 33.3 + 5.3 us.
+template <int MAXU, bool F32IN, int NT>
 __global__ __launch_bounds__(256) void norm_rope_rows_bwd_kernel(NormRopeBwdRowsArgs a) {
   const int tid = threadIdx.x;
   const int cph = a.D >> 4;
   const int nunits = a.H * cph;
   const int half = a.D >> 1;
-  __shared__ float red[2][2][16];
+  __shared__ float red[2][NT][2][16];
 
-  float accw[MAXU][16];
+  float accw[NT][MAXU][16];
   int xoff[MAXU], goff[MAXU], hh[MAXU], cc8[MAXU];
 #pragma unroll
   for (int i = 0; i < MAXU; ++i) {
@@ -458,35 +459,51 @@ __global__ __launch_bounds__(256) void norm_rope_rows_bwd_kernel(NormRopeBwdRows
     xoff[i] = h * a.D + c * 8;
     goff[i] = (int)(h * a.g_sh) + c * 8;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) accw[i][j] = 0.f;
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) accw[t][i][j] = 0.f;
   }
+  auto weights = [&](int t, int i, float* w) __attribute__((always_inline)) {
+    const float4* wp0 = reinterpret_cast<const float4*>(a.w[t] + xoff[i]);
+    const float4* wp1 = reinterpret_cast<const float4*>(a.w[t] + xoff[i] + half);
+    const float4 w0 = wp0[0], w1 = wp0[1], w2 = wp1[0], w3 = wp1[1];
+    const float f[16] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, w3.x, w3.y, w3.z, w3.w};
+    const float wm = t == 0 ? a.w_mul : 1.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) w[j] = f[j] * wm;
+  };
 
   int par = 0;
   for (int tok = blockIdx.x; tok < a.ntok; tok += a.nb, par ^= 1) {
     const int b = tok / a.S, s = tok - b * a.S;
-    float x[MAXU][16], dy[MAXU][16];
-    float ss = 0.f, sd = 0.f;
+    float x[NT][MAXU][16], dy[NT][MAXU][16];
+    float ss[NT], sd[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) { ss[t] = 0.f; sd[t] = 0.f; }
 #pragma unroll
     for (int i = 0; i < MAXU; ++i) {
       const int u = tid + i * 256;
       if (u < nunits) {
-        const int64_t e0 = b * a.in_sb + s * a.in_ss + xoff[i];
-        if (F32IN) {
-          const float4* p0 = reinterpret_cast<const float4*>(static_cast<const float*>(a.x_in) + e0);
-          const float4* p1 = reinterpret_cast<const float4*>(static_cast<const float*>(a.x_in) + e0 + half);
-          const float4 v0 = ld_nt(p0), v1 = ld_nt(p0 + 1), v2 = ld_nt(p1), v3 = ld_nt(p1 + 1);
-          const float tt[16] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w, v2.x, v2.y, v2.z, v2.w, v3.x, v3.y, v3.z, v3.w};
+        float gf[NT][16];
 #pragma unroll
-          for (int j = 0; j < 16; ++j) x[i][j] = tt[j];
-        } else {
-          const uint4* p = reinterpret_cast<const uint4*>(static_cast<const __bf16*>(a.x_in) + e0);
-          unpack8(ld_nt(p), x[i]);
-          unpack8(ld_nt(p + (a.D >> 4)), x[i] + 8);
+        for (int t = 0; t < NT; ++t) {
+          const int64_t e0 = b * a.in_sb + s * a.in_ss + xoff[i];
+          if (F32IN) {
+            const float4* p0 = reinterpret_cast<const float4*>(static_cast<const float*>(a.x_in[t]) + e0);
+            const float4* p1 = reinterpret_cast<const float4*>(static_cast<const float*>(a.x_in[t]) + e0 + half);
+            const float4 v0 = ld_nt(p0), v1 = ld_nt(p0 + 1), v2 = ld_nt(p1), v3 = ld_nt(p1 + 1);
+            const float tt[16] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w, v2.x, v2.y, v2.z, v2.w, v3.x, v3.y, v3.z, v3.w};
+#pragma unroll
+            for (int j = 0; j < 16; ++j) x[t][i][j] = tt[j];
+          } else {
+            const uint4* p = reinterpret_cast<const uint4*>(static_cast<const __bf16*>(a.x_in[t]) + e0);
+            unpack8(ld_nt(p), x[t][i]);
+            unpack8(ld_nt(p + (a.D >> 4)), x[t][i] + 8);
+          }
+          const uint4* gp = reinterpret_cast<const uint4*>(a.g[t] + b * a.g_sb + s * a.g_ss + goff[i]);
+          unpack8(ld_nt(gp), gf[t]);
+          unpack8(ld_nt(gp + (a.D >> 4)), gf[t] + 8);
         }
-        float gf[16];
-        const uint4* gp = reinterpret_cast<const uint4*>(a.g + b * a.g_sb + s * a.g_ss + goff[i]);
-        unpack8(ld_nt(gp), gf);
-        unpack8(ld_nt(gp + (a.D >> 4)), gf + 8);
         if (a.mode == 1) {
           // out[2j] = y[2j] c[2j] - y[2j+1] s[2j];  out[2j+1] = y[2j+1] c[2j+1] + y[2j] s[2j+1]
           const int64_t t0 = ((int64_t)b * a.S + s) * a.N + xoff[i];
@@ -498,11 +515,13 @@ __global__ __launch_bounds__(256) void norm_rope_rows_bwd_kernel(NormRopeBwdRows
             const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
             const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const float g0 = gf[part * 8 + 2 * j], g1 = gf[part * 8 + 2 * j + 1];
-              dy[i][part * 8 + 2 * j] = g0 * cc[2 * j] + g1 * sv[2 * j + 1];
-              dy[i][part * 8 + 2 * j + 1] = g1 * cc[2 * j + 1] - g0 * sv[2 * j];
-            }
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const float g0 = gf[t][part * 8 + 2 * j], g1 = gf[t][part * 8 + 2 * j + 1];
+                dy[t][i][part * 8 + 2 * j] = g0 * cc[2 * j] + g1 * sv[2 * j + 1];
+                dy[t][i][part * 8 + 2 * j + 1] = g1 * cc[2 * j + 1] - g0 * sv[2 * j];
+              }
           }
         } else if (a.mode == 2) {
           const int64_t t0 = (((int64_t)b * a.H + hh[i]) * a.S + s) * half + cc8[i];
@@ -512,76 +531,90 @@ __global__ __launch_bounds__(256) void norm_rope_rows_bwd_kernel(NormRopeBwdRows
           const float cc[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
           const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            dy[i][j] = gf[j] * cc[j] + gf[8 + j] * sv[j];
-            dy[i][8 + j] = gf[8 + j] * cc[j] - gf[j] * sv[j];
-          }
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              dy[t][i][j] = gf[t][j] * cc[j] + gf[t][8 + j] * sv[j];
+              dy[t][i][8 + j] = gf[t][8 + j] * cc[j] - gf[t][j] * sv[j];
+            }
         } else {
 #pragma unroll
-          for (int j = 0; j < 16; ++j) dy[i][j] = gf[j];
-        }
-        const float4* wp0 = reinterpret_cast<const float4*>(a.w + xoff[i]);
-        const float4* wp1 = reinterpret_cast<const float4*>(a.w + xoff[i] + half);
-        const float4 w0 = wp0[0], w1 = wp0[1], w2 = wp1[0], w3 = wp1[1];
-        const float w[16] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, w3.x, w3.y, w3.z, w3.w};
+          for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          ss = __builtin_fmaf(x[i][j], x[i][j], ss);
-          sd = __builtin_fmaf(x[i][j], w[j] * dy[i][j], sd);
+            for (int j = 0; j < 16; ++j) dy[t][i][j] = gf[t][j];
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          float w[16];
+          weights(t, i, w);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            ss[t] = __builtin_fmaf(x[t][i][j], x[t][i][j], ss[t]);
+            sd[t] = __builtin_fmaf(x[t][i][j], w[j] * dy[t][i][j], sd[t]);
+          }
         }
       }
     }
-    ss = row16_sum(ss);
-    sd = row16_sum(sd);
-    if ((tid & 15) == 0) { red[par][0][tid >> 4] = ss; red[par][1][tid >> 4] = sd; }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      ss[t] = row16_sum(ss[t]);
+      sd[t] = row16_sum(sd[t]);
+      if ((tid & 15) == 0) { red[par][t][0][tid >> 4] = ss[t]; red[par][t][1][tid >> 4] = sd[t]; }
+    }
     __syncthreads();  // one barrier per row: `red` alternates between two halves (see the full-row kernel)
-    float tss = 0.f, tsd = 0.f;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) { tss += red[par][0][j]; tsd += red[par][1][j]; }
-    const float r = rsqrt_newton(tss * a.inv_n + a.eps);
-    const float coef = r * r * r * tsd * a.inv_n;
+    for (int t = 0; t < NT; ++t) {
+      float tss = 0.f, tsd = 0.f;
 #pragma unroll
-    for (int i = 0; i < MAXU; ++i) {
-      const int u = tid + i * 256;
-      if (u < nunits) {
-        const float4* wp0 = reinterpret_cast<const float4*>(a.w + xoff[i]);
-        const float4* wp1 = reinterpret_cast<const float4*>(a.w + xoff[i] + half);
-        const float4 w0 = wp0[0], w1 = wp0[1], w2 = wp1[0], w3 = wp1[1];
-        const float w[16] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, w3.x, w3.y, w3.z, w3.w};
-        float du[16];
+      for (int j = 0; j < 16; ++j)
+        if (j < (int)(blockDim.x >> 4)) { tss += red[par][t][0][j]; tsd += red[par][t][1][j]; }
+      const float r = rsqrt_newton(tss * a.inv_n + a.eps);
+      const float coef = r * r * r * tsd * a.inv_n;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          du[j] = r * w[j] * dy[i][j] - coef * x[i][j];
-          accw[i][j] = __builtin_fmaf(dy[i][j] * r, x[i][j], accw[i][j]);
-        }
-        const int64_t e0 = b * a.dx_sb + s * a.dx_ss + xoff[i];
-        if (F32IN) {
-          float4* p0 = reinterpret_cast<float4*>(static_cast<float*>(a.dx) + e0);
-          float4* p1 = reinterpret_cast<float4*>(static_cast<float*>(a.dx) + e0 + half);
-          p0[0] = make_float4(du[0], du[1], du[2], du[3]);
-          p0[1] = make_float4(du[4], du[5], du[6], du[7]);
-          p1[0] = make_float4(du[8], du[9], du[10], du[11]);
-          p1[1] = make_float4(du[12], du[13], du[14], du[15]);
-        } else {
-          uint4* p = reinterpret_cast<uint4*>(static_cast<__bf16*>(a.dx) + e0);
-          st_nt(p, pack8(du));
-          st_nt(p + (a.D >> 4), pack8(du + 8));
+      for (int i = 0; i < MAXU; ++i) {
+        const int u = tid + i * 256;
+        if (u < nunits) {
+          float w[16], du[16];
+          weights(t, i, w);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            du[j] = r * w[j] * dy[t][i][j] - coef * x[t][i][j];
+            accw[t][i][j] = __builtin_fmaf(dy[t][i][j] * r, x[t][i][j], accw[t][i][j]);
+          }
+          const int64_t e0 = b * a.dx_sb + s * a.dx_ss + xoff[i];
+          if (F32IN) {
+            float4* p0 = reinterpret_cast<float4*>(static_cast<float*>(a.dx[t]) + e0);
+            float4* p1 = reinterpret_cast<float4*>(static_cast<float*>(a.dx[t]) + e0 + half);
+            p0[0] = make_float4(du[0], du[1], du[2], du[3]);
+            p0[1] = make_float4(du[4], du[5], du[6], du[7]);
+            p1[0] = make_float4(du[8], du[9], du[10], du[11]);
+            p1[1] = make_float4(du[12], du[13], du[14], du[15]);
+          } else {
+            uint4* p = reinterpret_cast<uint4*>(static_cast<__bf16*>(a.dx[t]) + e0);
+            st_nt(p, pack8(du));
+            st_nt(p + (a.D >> 4), pack8(du + 8));
+          }
         }
       }
     }
   }
 
-  float* prow = a.part + (int64_t)blockIdx.x * a.N;
 #pragma unroll
-  for (int i = 0; i < MAXU; ++i) {
-    const int u = tid + i * 256;
-    if (u < nunits) {
-      float4* p0 = reinterpret_cast<float4*>(prow + xoff[i]);
-      float4* p1 = reinterpret_cast<float4*>(prow + xoff[i] + half);
-      p0[0] = make_float4(accw[i][0], accw[i][1], accw[i][2], accw[i][3]);
-      p0[1] = make_float4(accw[i][4], accw[i][5], accw[i][6], accw[i][7]);
-      p1[0] = make_float4(accw[i][8], accw[i][9], accw[i][10], accw[i][11]);
-      p1[1] = make_float4(accw[i][12], accw[i][13], accw[i][14], accw[i][15]);
+  for (int t = 0; t < NT; ++t) {
+    float* prow = a.part + (int64_t)blockIdx.x * NT * a.N + (int64_t)t * a.N;
+    const float wm = t == 0 ? a.w_mul : 1.f;  // the gradient of the weight before the factor
+#pragma unroll
+    for (int i = 0; i < MAXU; ++i) {
+      const int u = tid + i * 256;
+      if (u < nunits) {
+        float4* p0 = reinterpret_cast<float4*>(prow + xoff[i]);
+        float4* p1 = reinterpret_cast<float4*>(prow + xoff[i] + half);
+        const float* f = accw[t][i];
+        p0[0] = make_float4(f[0] * wm, f[1] * wm, f[2] * wm, f[3] * wm);
+        p0[1] = make_float4(f[4] * wm, f[5] * wm, f[6] * wm, f[7] * wm);
+        p1[0] = make_float4(f[8] * wm, f[9] * wm, f[10] * wm, f[11] * wm);
+        p1[1] = make_float4(f[12] * wm, f[13] * wm, f[14] * wm, f[15] * wm);
+      }
     }
   }
 }
@@ -784,41 +817,60 @@ extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, cons
                                            g_strides, workspace, workspace_floats);
 }
 
-extern "C" int mdattn_norm_rope_rows_bwd(void* stream, const void* x_in, int x_is_f32, const void* g, void* dx, const float* w,
-                                         float* dw, const float* cos, const float* sin, int rope_mode, int B, int S, int H, int D,
-                                         float eps, int64_t in_stride_batch, int64_t in_stride_seq,
-                                         int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides,
-                                         float* workspace, int64_t workspace_floats) {
-  if (!x_in || !g || !dx || !w || !dw || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !g_strides || !workspace) return MDATTN_E_BADARG;
+extern "C" int mdattn_host_norm_rope_rows_bwd(void* stream, const void* q_in, const void* k_in, int x_is_f32, const void* gq, const void* gk, void* dq,
+                                              void* dk, const float* wq, const float* wk, float* dwq, float* dwk, const float* cos,
+                                              const float* sin, int rope_mode, int B, int S, int H, int D, float eps, float w_mul,
+                                              int64_t in_stride_batch, int64_t in_stride_seq, int64_t dx_stride_batch, int64_t dx_stride_seq,
+                                              const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats) {
+  if (!q_in || !gq || !dq || !wq || !dwq || B <= 0 || S <= 0 || H <= 0 || D <= 0 || !g_strides || !workspace) return MDATTN_E_BADARG;
+  const bool pair = k_in != nullptr;
+  if (pair != (gk != nullptr) || pair != (dk != nullptr) || pair != (dwk != nullptr) || (pair && !wk)) return MDATTN_E_BADARG;
   if (rope_mode < 0 || rope_mode > 2 || (rope_mode != 0 && (!cos || !sin)) || !(eps >= 0.f)) return MDATTN_E_BADARG;
   if (D % 16 != 0) return MDATTN_E_UNSUPPORTED;
   const int64_t N = (int64_t)H * D;
-  if (N / 16 > 2 * 256) return MDATTN_E_UNSUPPORTED;
+  const int64_t units = N / 16;
+  if (units > 2 * 256 || (pair && units > 256)) return MDATTN_E_UNSUPPORTED;
   const int64_t ntok = (int64_t)B * S;
   if (ntok > 0x7FFFFFFF || (int64_t)(H - 1) * g_strides->head + D >= (int64_t)1 << 31) return MDATTN_E_UNSUPPORTED;
   const int in_mult = x_is_f32 ? 4 : 8;
-  if (!aligned16(x_in) || !aligned16(g) || !aligned16(dx) || !aligned16(w) || !aligned16(dw) || !aligned16(cos) || !aligned16(sin) ||
-      !aligned16(workspace))
+  if (!aligned16(q_in) || !aligned16(gq) || !aligned16(dq) || !aligned16(wq) || !aligned16(dwq) || !aligned16(k_in) || !aligned16(gk) ||
+      !aligned16(dk) || !aligned16(wk) || !aligned16(dwk) || !aligned16(cos) || !aligned16(sin) || !aligned16(workspace))
     return MDATTN_E_ALIGN;
   if (in_stride_batch % in_mult || in_stride_seq % in_mult || in_stride_seq < N || dx_stride_batch % in_mult ||
       dx_stride_seq % in_mult || dx_stride_seq < N || !strides_ok(g_strides, 8))
     return MDATTN_E_ALIGN;
   if (g_strides->head < D) return MDATTN_E_BADARG;
-  const bool two = N / 16 > 256;
-  void (*kern)(NormRopeBwdRowsArgs) = x_is_f32 ? (two ? norm_rope_rows_bwd_kernel<2, true> : norm_rope_rows_bwd_kernel<1, true>)
-                                               : (two ? norm_rope_rows_bwd_kernel<2, false> : norm_rope_rows_bwd_kernel<1, false>);
-  static ResidentCache resident[2][2];
-  const int nb = partial_rows(ntok, N, workspace_floats, resident_blocks(resident[x_is_f32 ? 1 : 0][two ? 1 : 0], reinterpret_cast<const void*>(kern), 256, 0));
+  const bool two = units > 256;
+  const int nt = two ? 256 : (int)((units + 63) / 64 * 64);
+  void (*kern)(NormRopeBwdRowsArgs);
+  if (pair) kern = x_is_f32 ? norm_rope_rows_bwd_kernel<1, true, 2> : norm_rope_rows_bwd_kernel<1, false, 2>;
+  else if (two) kern = x_is_f32 ? norm_rope_rows_bwd_kernel<2, true, 1> : norm_rope_rows_bwd_kernel<2, false, 1>;
+  else kern = x_is_f32 ? norm_rope_rows_bwd_kernel<1, true, 1> : norm_rope_rows_bwd_kernel<1, false, 1>;
+  static ResidentCache resident[2][3];
+  const int ncols = (int)((pair ? 2 : 1) * N);
+  const int nb = partial_rows(ntok, ncols, workspace_floats,
+                              resident_blocks(resident[x_is_f32 ? 1 : 0][pair ? 2 : two ? 1 : 0], reinterpret_cast<const void*>(kern), nt, 0));
   if (nb < 1) return MDATTN_E_BADARG;
   NormRopeBwdRowsArgs a;
-  a.x_in = x_in; a.g = (const __bf16*)g; a.dx = dx; a.w = w; a.cos = cos; a.sin = sin; a.part = workspace;
+  a.x_in[0] = q_in; a.x_in[1] = k_in; a.g[0] = (const __bf16*)gq; a.g[1] = (const __bf16*)gk; a.dx[0] = dq; a.dx[1] = dk; a.w[0] = wq; a.w[1] = wk;
+  a.cos = cos; a.sin = sin; a.part = workspace;
   a.S = S; a.H = H; a.D = D; a.N = (int)N; a.mode = rope_mode; a.ntok = (int)ntok; a.nb = nb;
-  a.eps = eps; a.inv_n = 1.0f / (float)N;
+  a.eps = eps; a.inv_n = 1.0f / (float)N; a.w_mul = w_mul;
   a.in_sb = in_stride_batch; a.in_ss = in_stride_seq; a.dx_sb = dx_stride_batch; a.dx_ss = dx_stride_seq;
   a.g_sb = g_strides->batch; a.g_ss = g_strides->seq; a.g_sh = g_strides->head;
   hipStream_t st = (hipStream_t)stream;
-  MDATTN_LAUNCH(kern, dim3(nb), dim3(256), 0, st, a);
+  MDATTN_LAUNCH(kern, dim3(nb), dim3(nt), 0, st, a);
   int rc = launch_status();
   if (rc != MDATTN_OK) return rc;
-  return launch_colsum(st, workspace, nb, (int)N, (int)N, dw, nullptr, nullptr, nullptr);
+  return launch_colsum(st, workspace, nb, ncols, (int)N, dwq, dwk, nullptr, nullptr);
+}
+
+extern "C" int mdattn_norm_rope_rows_bwd(void* stream, const void* x_in, int x_is_f32, const void* g, void* dx, const float* w,
+                                         float* dw, const float* cos, const float* sin, int rope_mode, int B, int S, int H, int D,
+                                         float eps, int64_t in_stride_batch, int64_t in_stride_seq,
+                                         int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides,
+                                         float* workspace, int64_t workspace_floats) {
+  return mdattn_host_norm_rope_rows_bwd(stream, x_in, nullptr, x_is_f32, g, nullptr, dx, nullptr, w, nullptr, dw, nullptr, cos, sin, rope_mode, B, S, H,
+                                        D, eps, 1.0f, in_stride_batch, in_stride_seq, dx_stride_batch, dx_stride_seq, g_strides, workspace,
+                                        workspace_floats);
 }

@@ -86,3 +86,29 @@ def test_golden_ltx2(dev):
     cos, sin = (None if a is None else t(a) for a in cs)
     out = ops.norm_rope_rows(x, t(g["w"]), cos, sin, heads=H, mode=mode)
     _assert_close(to_np(out).reshape(B, S, N), g[f"out_{mode}"], f"ltx2 golden {mode}")
+
+
+@pytest.mark.parametrize("mode,dtype", [("interleaved", torch.float32), ("split", torch.bfloat16), ("none", torch.float32)])
+@pytest.mark.parametrize("H,D,S", [(3, 64, 37), (32, 64, 5), (32, 128, 9)])
+def test_q_and_k_in_one_launch_equal_two_calls(dev, mode, dtype, H, D, S):
+  """Self-attention's q and k go through one launch (shared tables, the query factor in the kernel): outputs and gradients
+  equal, bit for bit, those of one call per tensor with the factor multiplied into the weight; partly filled workgroups."""
+  from maxdiffusion_amd import attention_op as A
+  B, N = 2, H * D
+  gen = torch.Generator(device=dev).manual_seed(N + S)
+  q, k = (torch.randn((B, S, N), generator=gen, device=dev).to(dtype).requires_grad_(True) for _ in range(2))
+  wq, wk = ((1 + 0.1 * torch.randn(N, generator=gen, device=dev)).requires_grad_(True) for _ in range(2))
+  ang = torch.rand((B, S, N) if mode == "interleaved" else (B, H, S, D // 2), generator=gen, device=dev) * 6.28
+  tab = None if mode == "none" else (torch.cos(ang), torch.sin(ang))
+  g = [torch.randn((B, S, H, D), generator=gen, device=dev).to(torch.bfloat16) for _ in range(2)]
+  out = A.hip_norm_rope_ltx2(q, k, wq, wk, H, rotary_emb=tab, rope_type="interleaved" if mode == "none" else mode, q_mul=0.37)
+  got = torch.autograd.grad(out, (q, k, wq, wk), g)
+  f = torch.tensor(0.37, device=dev)
+  cs = (None, None) if tab is None else tab
+  want = (ops.norm_rope_rows(q.detach(), wq.detach() * f, *cs, heads=H, mode=mode), ops.norm_rope_rows(k.detach(), wk.detach(), *cs, heads=H, mode=mode))
+  dq, dwq = ops.norm_rope_rows_backward(q.detach(), wq.detach() * f, g[0], *cs, heads=H, mode=mode)
+  dk, dwk = ops.norm_rope_rows_backward(k.detach(), wk.detach(), g[1], *cs, heads=H, mode=mode)
+  assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
+  assert torch.equal(got[0], dq) and torch.equal(got[1], dk)
+  # the partial sums are the same; the factor meets them before the second stage instead of after it
+  assert torch.allclose(got[2], dwq * f, rtol=2e-6, atol=1e-6 * float(dwq.abs().max())) and torch.equal(got[3], dwk)
