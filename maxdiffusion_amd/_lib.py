@@ -65,8 +65,8 @@ HOST_SIGNATURES = {
     "mdattn_host_norm_rope_fullrow": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _S], _I),
     "mdattn_host_norm_rope_qkv": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _S], _I),
     "mdattn_host_norm_rope_perhead": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _F, _S, _S], _I),
-    "mdattn_host_norm_rope_fullrow_bwd": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _L, _L, _S, _P, _L], _I),
-    "mdattn_host_norm_rope_perhead_bwd": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _S, _S, _S, _P, _L], _I),
+    "mdattn_host_norm_rope_fullrow_bwd": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _L, _L, _S, _P, _L], _I),
+    "mdattn_host_norm_rope_perhead_bwd": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _F, _S, _S, _S, _P, _L], _I),
 }
 
 _lib = None

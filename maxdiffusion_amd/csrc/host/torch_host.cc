@@ -281,16 +281,15 @@ struct FullrowFn : torch::autograd::Function<FullrowFn> {
     const Tensor gq = grad_like(g[0], Tensor());
     const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = has_k ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
-    const auto fo = q.options().dtype(at::kFloat);
-    Tensor dwq = at::empty({n}, fo), dwk = has_k ? at::empty({n}, fo) : Tensor();
+    Tensor dwq = at::empty({n}, q.options()), dwk = has_k ? at::empty({n}, q.options()) : Tensor();
     const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, (has_k ? 2 : 1) * n);
-    Tensor ws = at::empty({nws}, fo);
+    Tensor ws = at::empty({nws}, q.options().dtype(at::kFloat));
     const mdattn_strides sg = strides4(gq);
-    must(mdattn_host_norm_rope_fullrow_bwd(stream(), ptr(q), ptr(k), nullptr, ptr(gq), ptr(gk), mut(dq), mut(dk), ptr(wq), ptr(wk), f32(dwq), f32(dwk),
-                                           nullptr, table_ptr(sv[4]), table_ptr(sv[5]), (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps,
+    must(mdattn_host_norm_rope_fullrow_bwd(stream(), ptr(q), ptr(k), nullptr, ptr(gq), ptr(gk), mut(dq), mut(dk), ptr(wq), ptr(wk), mut(dwq), mut(dwk),
+                                           nullptr, 1, nullptr, nullptr, table_ptr(sv[4]), table_ptr(sv[5]), (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps,
                                            (float)p.q_mul, q.stride(0), q.stride(1), dq.stride(0), dq.stride(1), &sg, f32(ws), nws),
          "mdattn_norm_rope_fullrow_bwd");
-    return {dq, dk, dwq.to(wq.scalar_type()), has_k ? dwk.to(wk.scalar_type()) : Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dq, dk, dwq, dwk, Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -344,19 +343,17 @@ struct PerheadFn : torch::autograd::Function<PerheadFn> {
     const Tensor gq = grad_like(g[0], Tensor());
     const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = has_k ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
-    const auto fo = q.options().dtype(at::kFloat);
-    auto dw = [&](bool want) { return want ? at::empty({d}, fo) : Tensor(); };
+    auto dw = [&](bool want) { return want ? at::empty({d}, q.options()) : Tensor(); };
     Tensor dwq = dw(true), dwk = dw(has_k), dwqt = dw(wqt.defined()), dwkt = dw(wkt.defined() && has_k);
     const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s * h, 4 * d);
-    Tensor ws = at::empty({nws}, fo);
+    Tensor ws = at::empty({nws}, q.options().dtype(at::kFloat));
     const mdattn_strides si = strides4(q), sd = strides4(dq), sg = strides4(gq);
     must(mdattn_host_norm_rope_perhead_bwd(stream(), ptr(q), ptr(k), ptr(gq), ptr(gk), mut(dq), mut(dk), ptr(wq), ptr(wk), ptr(wqt),
-                                           has_k ? ptr(wkt) : nullptr, (int)p.n_txt, f32(dwq), f32(dwk), f32(dwqt), f32(dwkt), table_ptr(sv[6]),
+                                           has_k ? ptr(wkt) : nullptr, (int)p.n_txt, mut(dwq), mut(dwk), mut(dwqt), mut(dwkt), 1, table_ptr(sv[6]),
                                            table_ptr(sv[7]), (int)p.kind, (int)b, (int)s, (int)h, (int)d, (float)p.eps, (float)p.q_mul, &si, &sd, &sg,
                                            f32(ws), nws),
          "mdattn_norm_rope_perhead_bwd");
-    auto cast = [](const Tensor& x, const Tensor& w) { return x.defined() ? x.to(w.scalar_type()) : Tensor(); };
-    return {dq, dk, cast(dwq, wq), cast(dwk, wk), cast(dwqt, wqt), cast(dwkt, wkt), Tensor(), Tensor(), Tensor()};
+    return {dq, dk, dwq, dwk, dwqt, dwkt, Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -407,22 +404,19 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
     const Tensor &x = sv[0], &bias = sv[1], &wq = sv[2], &wk = sv[3];
     const Prologue p = Prologue::saved(ctx);
     const int64_t b = x.size(0), s = x.size(1), n = x.size(2) / 3, d = n / p.heads;
-    const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq);
+    const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq), gv = grad_like(g[2], gq);
     Tensor dx = at::empty({b, s, 3 * n}, x.options());
-    const auto fo = x.options().dtype(at::kFloat);
-    Tensor dwq = at::empty({n}, fo), dwk = at::empty({n}, fo), db = at::empty({2 * n}, fo);
-    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, 4 * n);
-    Tensor ws = at::empty({nws}, fo);
+    Tensor dwq = at::empty({n}, x.options()), dwk = at::empty({n}, x.options()), db = at::empty({3 * n}, x.options());
+    const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, 5 * n);
+    Tensor ws = at::empty({nws}, x.options().dtype(at::kFloat));
     const mdattn_strides sg = strides4(gq);
     const char* xp = static_cast<const char*>(ptr(x));
     char* dp = static_cast<char*>(mut(dx));
-    must(mdattn_host_norm_rope_fullrow_bwd(stream(), xp, xp + 2 * n, ptr(bias), ptr(gq), ptr(gk), dp, dp + 2 * n, ptr(wq), ptr(wk), f32(dwq), f32(dwk),
-                                           f32(db), table_ptr(sv[4]), table_ptr(sv[5]), (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps,
+    must(mdattn_host_norm_rope_fullrow_bwd(stream(), xp, xp + 2 * n, ptr(bias), ptr(gq), ptr(gk), dp, dp + 2 * n, ptr(wq), ptr(wk), mut(dwq), mut(dwk),
+                                           mut(db), 1, ptr(gv), dp + 4 * n, table_ptr(sv[4]), table_ptr(sv[5]), (int)p.kind, (int)b, (int)s, (int)p.heads, (int)d, (float)p.eps,
                                            (float)p.q_mul, x.stride(0), x.stride(1), dx.stride(0), dx.stride(1), &sg, f32(ws), nws),
          "mdattn_norm_rope_fullrow_bwd");
-    dx.narrow(2, 2 * n, n).unflatten(2, {p.heads, d}).copy_(g[2]);
-    Tensor dbias = at::cat({db, g[2].to(at::kFloat).sum(at::IntArrayRef{0, 1}).reshape({n})}).to(bias.scalar_type());
-    return {dx, dbias, dwq.to(wq.scalar_type()), dwk.to(wk.scalar_type()), Tensor(), Tensor(), Tensor()};
+    return {dx, db, dwq, dwk, Tensor(), Tensor(), Tensor()};
   }
 };
 

@@ -39,7 +39,10 @@ int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, const void*
  *   COMPLEX   cos = complex64 [S, D/2], sin null
  *   REPEATED  cos, sin f32 [S, D], each angle for both members of its pair      (per-head forms only)
  *   MATRIX    cos = f32 [S, D/2, 2, 2] = [[cos, -sin], [sin, cos]], sin null     (per-head forms only)
- * No table: cos null, sin null, PLANES. */
+ * No table: cos null, sin null, PLANES.
+ * The backward forms write the weight (and bias) gradients as f32, or (dw_bf16) rounded to bf16.  gv, dv_in (the fused form
+ * with biases; or null): the value block's output gradient, strided like gq, and its place in the fused gradient buffer;
+ * dbias then has 3*H*D entries and the workspace 5*H*D columns. */
 #define MDATTN_TABLE_PLANES 0
 #define MDATTN_TABLE_COMPLEX 1
 #define MDATTN_TABLE_REPEATED 2
@@ -55,13 +58,14 @@ int mdattn_host_norm_rope_perhead(void* stream, const void* q_in, const void* k_
                                   int table, int B, int S, int H, int D, float eps, float q_mul, const mdattn_strides* in_strides,
                                   const mdattn_strides* out_strides);
 int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in, const void* k_in, const void* bias, const void* gq, const void* gk,
-                                      void* dq_in, void* dk_in, const void* wq, const void* wk, float* dwq, float* dwk, float* dbias,
+                                      void* dq_in, void* dk_in, const void* wq, const void* wk, void* dwq, void* dwk, void* dbias,
+                                      int dw_bf16, const void* gv, void* dv_in,
                                       const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps, float q_mul,
                                       int64_t in_stride_batch, int64_t in_stride_seq, int64_t dx_stride_batch, int64_t dx_stride_seq,
                                       const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats);
 int mdattn_host_norm_rope_perhead_bwd(void* stream, const void* q_in, const void* k_in, const void* gq, const void* gk, void* dq_in,
                                       void* dk_in, const void* wq, const void* wk, const void* wq_txt, const void* wk_txt, int n_txt,
-                                      float* dwq, float* dwk, float* dwq_txt, float* dwk_txt, const float* cos, const float* sin,
+                                      void* dwq, void* dwk, void* dwq_txt, void* dwk_txt, int dw_bf16, const float* cos, const float* sin,
                                       int table, int B, int S, int H, int D, float eps, float q_mul, const mdattn_strides* in_strides,
                                       const mdattn_strides* dx_strides, const mdattn_strides* g_strides, float* workspace,
                                       int64_t workspace_floats);

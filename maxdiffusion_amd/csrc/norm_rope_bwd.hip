@@ -256,10 +256,11 @@ __global__ __launch_bounds__(512) void norm_rope_fullrow_bwd_kernel(NormRopeBwdF
 // as a workgroup holds and eight loads are in flight per lane.  Against 64 columns x 16 slices of 256 lanes: 512 columns
 // 21.8 -> 4.7 us, 1,536 columns 17 -> 4.9 us, 10,240 columns 10.0 -> 5.4 us.  Slices are combined inside the wave, then
 // through LDS.  Column col goes to outs[col / seglen][col % seglen].
+// bf16: the outputs are rounded to it here (the gradient of a bf16 weight in its own type; a cast was a launch each).
 struct ColsumArgs {
   const float* part;
-  float* outs[4];
-  int nb, ncols, seglen;
+  void* outs[5];
+  int nb, ncols, seglen, bf16;
 };
 
 __global__ __launch_bounds__(1024) void colsum_kernel(ColsumArgs a) {
@@ -294,7 +295,74 @@ __global__ __launch_bounds__(1024) void colsum_kernel(ColsumArgs a) {
       tot.x += v.x; tot.y += v.y; tot.z += v.z; tot.w += v.w;
     }
     const int seg = col / a.seglen, i = col - seg * a.seglen;  // seglen % 4 == 0: a float4 never straddles segments
-    if (a.outs[seg]) *reinterpret_cast<float4*>(a.outs[seg] + i) = tot;
+    if (!a.outs[seg]) return;
+    if (a.bf16) *reinterpret_cast<uint2*>(static_cast<__bf16*>(a.outs[seg]) + i) = make_uint2(pack2(tot.x, tot.y), pack2(tot.z, tot.w));
+    else *reinterpret_cast<float4*>(static_cast<float*>(a.outs[seg]) + i) = tot;
+  }
+}
+
+// The value block of the fused q|k|v projection: its input gradient is its output gradient, moved from the attention layout
+// into the fused gradient buffer, and the bias gradient is the token sum, as partial rows next to those of q and k.  One
+// read and one write: 18,900 tokens x 2,560 channels 48 us (copy, cast to f32, sum, concatenation and cast back before:
+// 141 us).  A lane owns the chunks tid, tid + 256, ..; four tokens in flight.
+struct ValueBwdArgs {
+  const __bf16* g;
+  uint4* dx;
+  float* part;  // column offset included
+  int S, D, ntok, nb, ncols, nchunks;
+  int64_t g_sb, g_ss, g_sh, dx_sb, dx_ss;
+};
+template <int MAXC>
+__global__ __launch_bounds__(256) void qkv_value_bwd_kernel(ValueBwdArgs a) {
+  const int tid = threadIdx.x;
+  float acc[MAXC][8];
+  int goff[MAXC];
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = tid + i * 256, e = (c < a.nchunks ? c : a.nchunks - 1) << 3;
+    const int h = e / a.D;
+    goff[i] = (int)(h * a.g_sh) + e - h * a.D;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+  }
+  constexpr int kTok = 4;
+  for (int t0 = blockIdx.x; t0 < a.ntok; t0 += kTok * a.nb) {
+    uint4 u[kTok][MAXC];
+#pragma unroll
+    for (int r = 0; r < kTok; ++r) {
+      const int t = min(t0 + r * a.nb, a.ntok - 1);
+      const int b = t / a.S, s = t - b * a.S;
+      const __bf16* row = a.g + b * a.g_sb + s * a.g_ss;
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) u[r][i] = ld_nt(reinterpret_cast<const uint4*>(row + goff[i]));
+    }
+#pragma unroll
+    for (int r = 0; r < kTok; ++r) {
+      const int t = t0 + r * a.nb;
+      if (t >= a.ntok) break;
+      const int b = t / a.S, s = t - b * a.S;
+      uint4* row = a.dx + ((b * a.dx_sb + s * a.dx_ss) >> 3);
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) {
+        const int c = tid + i * 256;
+        if (c < a.nchunks) {
+          float f[8];
+          unpack8(u[r][i], f);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[i][j] += f[j];
+          st_nt(row + c, u[r][i]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = tid + i * 256;
+    if (c < a.nchunks) {
+      float4* p = reinterpret_cast<float4*>(a.part + (int64_t)blockIdx.x * a.ncols + c * 8);
+      p[0] = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+      p[1] = make_float4(acc[i][4], acc[i][5], acc[i][6], acc[i][7]);
+    }
   }
 }
 
@@ -647,10 +715,11 @@ static int resident_blocks(ResidentCache& cache, const void* kernel, int nt, int
   return v;
 }
 
-static int launch_colsum(hipStream_t st, const float* part, int nb, int ncols, int seglen, float* o0, float* o1, float* o2, float* o3) {
+static int launch_colsum(hipStream_t st, const float* part, int nb, int ncols, int seglen, int bf16, void* o0, void* o1, void* o2, void* o3,
+                         void* o4 = nullptr) {
   ColsumArgs c;
-  c.part = part; c.nb = nb; c.ncols = ncols; c.seglen = seglen;
-  c.outs[0] = o0; c.outs[1] = o1; c.outs[2] = o2; c.outs[3] = o3;
+  c.part = part; c.nb = nb; c.ncols = ncols; c.seglen = seglen; c.bf16 = bf16;
+  c.outs[0] = o0; c.outs[1] = o1; c.outs[2] = o2; c.outs[3] = o3; c.outs[4] = o4;
   MDATTN_LAUNCH(colsum_kernel, dim3((ncols + 31) / 32), dim3(1024), 0, st, c);
   return launch_status();
 }
@@ -674,7 +743,8 @@ static int partial_rows(int64_t units, int64_t ncols, int64_t floats, int reside
 
 extern "C" int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in, const void* k_in, const void* bias,
                                             const void* gq, const void* gk, void* dq_in, void* dk_in,
-                                            const void* wq, const void* wk, float* dwq, float* dwk, float* dbias,
+                                            const void* wq, const void* wk, void* dwq, void* dwk, void* dbias, int dw_bf16,
+                                            const void* gv, void* dv_in,
                                             const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps, float q_mul,
                                             int64_t in_stride_batch, int64_t in_stride_seq,
                                             int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides,
@@ -685,6 +755,7 @@ extern "C" int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in,
   if (!table_ok(cos, sin, table)) return MDATTN_E_BADARG;
   if (table != MDATTN_TABLE_PLANES && table != MDATTN_TABLE_COMPLEX) return MDATTN_E_UNSUPPORTED;
   if ((bias == nullptr) != (dbias == nullptr) || (bias && !has_k)) return MDATTN_E_BADARG;  // the fused q|k|v form carries both
+  if ((gv == nullptr) != (dv_in == nullptr) || (gv && !bias)) return MDATTN_E_BADARG;
   if (!(eps >= 0.f) || !(q_mul > 0.f) || !(q_mul < 1e30f)) return MDATTN_E_BADARG;
   const int64_t N = (int64_t)H * D;
   if (D % 8 != 0 || N > 8192) return MDATTN_E_UNSUPPORTED;
@@ -694,11 +765,11 @@ extern "C" int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in,
   if ((int64_t)(H - 1) * g_strides->head + D >= (int64_t)1 << 31) return MDATTN_E_UNSUPPORTED;  // per-lane offsets inside a gradient row are 32-bit
   if (!aligned16(q_in) || !aligned16(k_in) || !aligned16(bias) || !aligned16(gq) || !aligned16(gk) || !aligned16(dq_in) ||
       !aligned16(dk_in) || !aligned16(wq) || !aligned16(wk) || !aligned16(dwq) || !aligned16(dwk) || !aligned16(dbias) ||
-      !aligned16(cos) || !aligned16(sin) || !aligned16(workspace))
+      !aligned16(cos) || !aligned16(sin) || !aligned16(workspace) || !aligned16(gv) || !aligned16(dv_in))
     return MDATTN_E_ALIGN;
   if (in_stride_batch % 8 || in_stride_seq % 8 || dx_stride_batch % 8 || dx_stride_seq % 8 || !strides_ok(g_strides, 8)) return MDATTN_E_ALIGN;
   const int ntens = has_k ? 2 : 1;
-  const int64_t ncols = (int64_t)ntens * (bias ? 2 : 1) * N;
+  const int64_t ncols = (int64_t)ntens * (bias ? 2 : 1) * N + (gv ? N : 0);
   // lanes per workgroup: the row's chunks split evenly over whole waves, at most two chunks per lane up to 8192 channels
   const int nchunks = (int)(N / 8);
   const int maxc = (nchunks + 511) / 512;
@@ -732,14 +803,27 @@ extern "C" int mdattn_host_norm_rope_fullrow_bwd(void* stream, const void* q_in,
   MDATTN_LAUNCH(kern, dim3(nb, ntens), dim3(nt), lds_bytes, st, a);
   int rc = launch_status();
   if (rc != MDATTN_OK) return rc;
-  // columns: [q: dw (, db)] [k: dw (, db)], each N wide
-  if (bias) return launch_colsum(st, workspace, nb, (int)ncols, (int)N, dwq, dbias, dwk, dbias + N);
-  return launch_colsum(st, workspace, nb, (int)ncols, (int)N, dwq, dwk, nullptr, nullptr);
+  if (gv) {
+    ValueBwdArgs v;
+    v.g = (const __bf16*)gv; v.dx = (uint4*)dv_in; v.part = workspace + 4 * N;
+    v.S = S; v.D = D; v.ntok = (int)ntok; v.nb = nb; v.ncols = (int)ncols; v.nchunks = nchunks;
+    v.g_sb = a.g_sb; v.g_ss = a.g_ss; v.g_sh = a.g_sh; v.dx_sb = a.dx_sb; v.dx_ss = a.dx_ss;
+    void (*vk)(ValueBwdArgs) = nchunks <= 256 ? qkv_value_bwd_kernel<1> : nchunks <= 512 ? qkv_value_bwd_kernel<2> : nchunks <= 768 ? qkv_value_bwd_kernel<3> : qkv_value_bwd_kernel<4>;
+    MDATTN_LAUNCH(vk, dim3(nb), dim3(256), 0, st, v);
+    if ((rc = launch_status()) != MDATTN_OK) return rc;
+  }
+  // columns: [q: dw (, db)] [k: dw (, db)] ([v: db]), each N wide
+  if (bias) {
+    char* db = static_cast<char*>(dbias);
+    const int64_t es = dw_bf16 ? 2 : 4;
+    return launch_colsum(st, workspace, nb, (int)ncols, (int)N, dw_bf16, dwq, db, dwk, db + N * es, gv ? db + 2 * N * es : nullptr);
+  }
+  return launch_colsum(st, workspace, nb, (int)ncols, (int)N, dw_bf16, dwq, dwk, nullptr, nullptr);
 }
 
 extern "C" int mdattn_host_norm_rope_perhead_bwd(void* stream, const void* q_in, const void* k_in, const void* gq, const void* gk,
                                             void* dq_in, void* dk_in, const void* wq, const void* wk, const void* wq_txt,
-                                            const void* wk_txt, int n_txt, float* dwq, float* dwk, float* dwq_txt, float* dwk_txt,
+                                            const void* wk_txt, int n_txt, void* dwq, void* dwk, void* dwq_txt, void* dwk_txt, int dw_bf16,
                                             const float* cos, const float* sin, int table, int B, int S, int H, int D, float eps, float q_mul,
                                             const mdattn_strides* in_strides, const mdattn_strides* dx_strides,
                                             const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats) {
@@ -790,7 +874,7 @@ extern "C" int mdattn_host_norm_rope_perhead_bwd(void* stream, const void* q_in,
   int rc = launch_status();
   if (rc != MDATTN_OK) return rc;
   // columns: [q image][q text][k image][k text], each D wide; outputs that do not exist are skipped
-  return launch_colsum(st, workspace, nb, (int)ncols, D, dwq, dwq_txt, dwk, has_k ? dwk_txt : nullptr);
+  return launch_colsum(st, workspace, nb, (int)ncols, D, dw_bf16, dwq, dwq_txt, dwk, has_k ? dwk_txt : nullptr);
 }
 
 // The C ABI's forms take the table as two planes [S, D/2].
@@ -801,7 +885,7 @@ extern "C" int mdattn_norm_rope_fullrow_bwd(void* stream, const void* q_in, cons
                                             int64_t in_stride_batch, int64_t in_stride_seq,
                                             int64_t dx_stride_batch, int64_t dx_stride_seq, const mdattn_strides* g_strides,
                                             float* workspace, int64_t workspace_floats) {
-  return mdattn_host_norm_rope_fullrow_bwd(stream, q_in, k_in, bias, gq, gk, dq_in, dk_in, wq, wk, dwq, dwk, dbias, cos, sin,
+  return mdattn_host_norm_rope_fullrow_bwd(stream, q_in, k_in, bias, gq, gk, dq_in, dk_in, wq, wk, dwq, dwk, dbias, 0, nullptr, nullptr, cos, sin,
                                            MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul, in_stride_batch, in_stride_seq, dx_stride_batch,
                                            dx_stride_seq, g_strides, workspace, workspace_floats);
 }
@@ -813,7 +897,7 @@ extern "C" int mdattn_norm_rope_perhead_bwd(void* stream, const void* q_in, cons
                                             const mdattn_strides* in_strides, const mdattn_strides* dx_strides,
                                             const mdattn_strides* g_strides, float* workspace, int64_t workspace_floats) {
   return mdattn_host_norm_rope_perhead_bwd(stream, q_in, k_in, gq, gk, dq_in, dk_in, wq, wk, wq_txt, wk_txt, n_txt, dwq, dwk, dwq_txt,
-                                           dwk_txt, cos, sin, MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul, in_strides, dx_strides,
+                                           dwk_txt, 0, cos, sin, MDATTN_TABLE_PLANES, B, S, H, D, eps, q_mul, in_strides, dx_strides,
                                            g_strides, workspace, workspace_floats);
 }
 
@@ -862,7 +946,7 @@ extern "C" int mdattn_host_norm_rope_rows_bwd(void* stream, const void* q_in, co
   MDATTN_LAUNCH(kern, dim3(nb), dim3(nt), 0, st, a);
   int rc = launch_status();
   if (rc != MDATTN_OK) return rc;
-  return launch_colsum(st, workspace, nb, ncols, (int)N, dwq, dwk, nullptr, nullptr);
+  return launch_colsum(st, workspace, nb, ncols, (int)N, 0, dwq, dwk, nullptr, nullptr);
 }
 
 extern "C" int mdattn_norm_rope_rows_bwd(void* stream, const void* x_in, int x_is_f32, const void* g, void* dx, const float* w,

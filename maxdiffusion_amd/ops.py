@@ -266,7 +266,7 @@ def norm_rope_fullrow_backward(q, k, wq, wk, cos, sin, heads: int, gq, gk, eps: 
   st = _strides(gq)
   rc = _lib.load().mdattn_host_norm_rope_fullrow_bwd(
       _stream(), _ptr(q), _ptr(k), _ptr(bias), _ptr(gq), _ptr(gk), _ptr(dq), _ptr(dk), _ptr(wq), _ptr(wk), _ptr(dwq), _ptr(dwk),
-      _ptr(dbias), pcos, psin, kind, b, s, heads, d, eps, q_mul, q.stride(0), q.stride(1), dq.stride(0), dq.stride(1),
+      _ptr(dbias), 0, None, None, pcos, psin, kind, b, s, heads, d, eps, q_mul, q.stride(0), q.stride(1), dq.stride(0), dq.stride(1),
       ctypes.byref(st), _ptr(ws), nws)
   _lib.check(rc, "mdattn_norm_rope_fullrow_bwd")
   return (dq, dk, dwq, dwk) if bias is None else (dq, dk, dwq, dwk, dbias)
@@ -302,7 +302,7 @@ def norm_rope_perhead_backward(q, k, wq, wk, cos, sin, gq, gk, eps: float = 1e-6
   si, sd, sg = _strides(q), _strides(dq), _strides(gq)
   rc = _lib.load().mdattn_host_norm_rope_perhead_bwd(
       _stream(), _ptr(q), _ptr(k), _ptr(gq), _ptr(gk), _ptr(dq), _ptr(dk), _ptr(wq), _ptr(wk), _ptr(wq_txt),
-      _ptr(wk_txt if has_k else None), n_txt, _ptr(dwq), _ptr(dwk), _ptr(dwq_t), _ptr(dwk_t), pcos, psin, kind, b, s, h, d, eps, q_mul,
+      _ptr(wk_txt if has_k else None), n_txt, _ptr(dwq), _ptr(dwk), _ptr(dwq_t), _ptr(dwk_t), 0, pcos, psin, kind, b, s, h, d, eps, q_mul,
       ctypes.byref(si), ctypes.byref(sd), ctypes.byref(sg), _ptr(ws), nws)
   _lib.check(rc, "mdattn_norm_rope_perhead_bwd")
   return dq, dk, dwq, dwk, dwq_t, dwk_t

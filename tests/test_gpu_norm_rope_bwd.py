@@ -231,3 +231,28 @@ def test_edges_and_validation(dev, lib):
   assert full(iss=256) == _lib.E_BADARG                      # row stride below H*D
   assert lib.mdattn_norm_rope_bwd_workspace_floats(75600, 10240) == 1024 * 10240
   assert lib.mdattn_norm_rope_bwd_workspace_floats(7, 512) == 7 * 512
+
+
+@pytest.mark.parametrize("B,S,H,D", [(1, 1, 1, 128), (2, 517, 3, 128), (1, 2500, 40, 128), (1, 300, 64, 128), (3, 41, 5, 96)])
+def test_fused_projection_backward_moves_the_value_block(dev, B, S, H, D):
+  """Value block of the fused gradient buffer: the output gradient itself, bit for bit; its bias gradient: the token sum in
+  f32, rounded once (bound: half a bf16 step of the result plus the f32 sum's own error)."""
+  from maxdiffusion_amd import attention_op as A
+  N = H * D
+  gen = torch.Generator(device=dev).manual_seed(S + N)
+  rnd = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16)
+  x, bias = rnd(B, S, 3 * N).requires_grad_(True), rnd(3 * N).requires_grad_(True)
+  w = [(1 + 0.1 * rnd(N).float()).to(torch.bfloat16).requires_grad_(True) for _ in range(2)]
+  g = [rnd(B, S, H, D) for _ in range(3)]
+  out = A.hip_norm_rope_qkv(x, *w, None, H, bias=bias)
+  dx, db, dwq, dwk = torch.autograd.grad(out, (x, bias, *w), g)
+  assert torch.equal(dx[:, :, 2 * N:], g[2].reshape(B, S, N))
+  want = g[2].double().sum(dim=(0, 1)).reshape(N)
+  err = (db[2 * N:].double() - want).abs()
+  assert bool((err <= want.abs() * 2.0**-8 + 2.0**-20 * g[2].double().abs().sum(dim=(0, 1)).reshape(N)).all())
+  # the blocks of q and k: as the plain backward gives them, with the f32 gradients rounded to the parameters' type
+  r = ops.norm_rope_fullrow_backward(x.detach()[:, :, :N], x.detach()[:, :, N:2 * N], w[0].detach(), w[1].detach(), None, None, H, g[0], g[1],
+                                     bias=bias.detach()[:2 * N].contiguous())
+  assert torch.equal(dx[:, :, :N], r[0]) and torch.equal(dx[:, :, N:2 * N], r[1])
+  for got, f in ((dwq, r[2]), (dwk, r[3]), (db[:2 * N], r[4])):
+    assert torch.equal(got, f.to(torch.bfloat16))
