@@ -202,6 +202,10 @@ def hip_flash_fp8_kernel(q, k, v, context):
   if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
     raise NotImplementedError("hip_flash_fp8 has no backward pass: use hip_flash for training, or call it under torch.no_grad()")
   heads = context["heads"]
+  if q.is_cuda:  # one quantisation of q, k and v together
+    out = _lib.host().flash_fp8(q, k, v, heads, context["scale"], context.get("attention_mask"))
+    if out is not None:
+      return out
   qv, kv, vv, d0 = _pad_head_dim(*(_as_bshd(t, heads).to(torch.bfloat16) for t in (q, k, v)))
   qv, kv, vv = qv.contiguous(), kv.contiguous(), vv.contiguous()
   # the softmax scale rides on q's quantisation (one rounding either way) and the q and k scales are powers of two:

@@ -192,6 +192,34 @@ OptTensor flash_autograd(const Tensor& q, const Tensor& k, const Tensor& v, int6
   return FlashFn::apply(q, k, v, opt(mask), heads, scale);
 }
 
+// The registry entry `hip_flash_fp8`: dense bf16 operands of either rank -> [B,Sq,H*D]
+OptTensor flash_fp8(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep) {
+  View vq, vk, vv;
+  Tensor mask;
+  for (const Tensor* t : {&q, &k, &v})  // the quantised copies are dense [B,S,H,D]
+    if (t->dim() == 4 ? !t->permute({0, 2, 1, 3}).is_contiguous() : !t->is_contiguous()) return std::nullopt;
+  if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, mask) || (vq.d != 64 && vq.d != 128)) return std::nullopt;
+  at::NoGradGuard guard;
+  const auto bytes = q.options().dtype(at::kByte);
+  Tensor q8 = at::empty({q.numel()}, bytes), k8 = at::empty({k.numel()}, bytes), v8 = at::empty({v.numel()}, bytes);
+  Tensor ws = at::empty({mdattn_host_quant3_floats()}, q.options().dtype(at::kFloat));
+  if (mdattn_host_quant3_e4m3(stream(), ptr(q), ptr(k), ptr(v), mut(q8), mut(k8), mut(v8), f32(ws), q.numel(), k.numel(),
+                              (float)(scale * 1.4426950408889634)) != MDATTN_OK)
+    return std::nullopt;
+  Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
+  auto dense = [](const View& x) { return mdattn_strides{x.s * x.h * x.d, x.h * x.d, x.d}; };
+  const mdattn_strides sq = dense(vq), skv = dense(vk);
+  const float *s = f32(ws), scale8 = (float)0.6931471805599453;  // q's quantisation carries scale * log2(e)
+  const int B = (int)vq.b, H = (int)vq.h, Sq = (int)vq.s, Skv = (int)vk.s, D = (int)vq.d;
+  const Mask m(mask, vk);
+  const int rc = m.bias ? mdattn_fwd_fp8_bias(stream(), ptr(q8), ptr(k8), ptr(v8), mut(out), nullptr, B, H, Sq, Skv, D, &sq, &skv, &skv, &sq, scale8, s,
+                                              s + 2, s + 4, m.bias, m.stride)
+                        : mdattn_fwd_fp8(stream(), ptr(q8), ptr(k8), ptr(v8), mut(out), nullptr, B, H, Sq, Skv, D, &sq, &skv, &skv, &sq, scale8, s, s + 2,
+                                         s + 4, MDATTN_FP8_SOFTMAX_BYTE_GRID);
+  if (rc != MDATTN_OK) return std::nullopt;
+  return out;
+}
+
 // One ring step (ops.flash_attention_merge) on logical [B,S,H,D] views; false: the Python path takes it
 bool flash_merge(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o_run, const Tensor& lse_run, double scale) {
   if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q) || q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || o_run.dim() != 4)
@@ -518,6 +546,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("build_id", [] { return std::string(kBuildIdRecord + 16); });
   m.def("flash", &flash);
   m.def("flash_autograd", &flash_autograd);
+  m.def("flash_fp8", &flash_fp8);
   m.def("flash_merge", &flash_merge);
   m.def("norm_rope", &norm_rope);
   m.def("norm_rope_perhead", &norm_rope_perhead);

@@ -19,6 +19,13 @@ int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D);
 int64_t mdattn_host_key_tiles_ints(int B, int Skv);
 int mdattn_host_key_tiles(void* stream, const void* keep, float* bias, int* tiles, int B, int Skv, int64_t bias_stride);
 
+/* mdattn_quant_e4m3 of an attention call's q (premul q_premul, power-of-two scale), k (power-of-two scale) and v in two
+ * launches.  ws: mdattn_host_quant3_floats floats, 16-byte aligned, of which [2 t] and [2 t + 1] become scale and absmax of
+ * tensor t. */
+int64_t mdattn_host_quant3_floats(void);
+int mdattn_host_quant3_e4m3(void* stream, const void* q, const void* k, const void* v, void* q8, void* k8, void* v8, float* ws, int64_t nq,
+                            int64_t nkv, float q_premul);
+
 /* Whether mdattn_host_fwd_bf16 and mdattn_host_bwd_bf16 take head dim D. */
 int mdattn_host_head_dim(int D);
 

@@ -347,3 +347,27 @@ def test_fp8_registry_entry_honours_the_mask(dev):
   got, want = op8.apply_attention(q, k, v, attention_mask=keep), op16.apply_attention(q, k, v, attention_mask=keep)
   assert got.shape == want.shape == (B, S, H * 128)
   assert cosine(to_np(got), to_np(want)) >= COS_BAR
+
+
+@pytest.mark.parametrize("b,h,d,sq,skv,rank4,masked", [(1, 1, 64, 1, 1, False, False), (1, 2, 128, 700, 3, False, False), (2, 3, 64, 5, 900, False, True),
+                                                        (1, 1, 128, 63, 65, True, True), (1, 8, 128, 4111, 130, False, False)])
+def test_fp8_entry_quantises_the_three_operands_as_one_by_one(dev, b, h, d, sq, skv, rank4, masked):
+  """Two launches for q, k and v: the same bytes and scales, so the same output bits as three quant_e4m3 calls.  Sizes: a
+  workgroup's worth and less, either side much the longer, and more rows than the maxima have slots (4,111 x 8 x 128)."""
+  shape = lambda s: (b, h, s, d) if rank4 else (b, s, h * d)
+  q, k, v = (to_dev_bf16(O.normal_bf16(shape(s), i) * np.float32(m), dev) for i, (s, m) in enumerate(((sq, 1.0), (skv, 5.0), (skv, 1e-2))))
+  view = (lambda x: x.permute(0, 2, 1, 3).contiguous()) if rank4 else (lambda x: x.view(b, -1, h, d))
+  if rank4:  # the entry's dense form over [B,H,S,D] operands
+    q, k, v = (view(x).permute(0, 2, 1, 3) for x in (q, k, v))
+  keep = None
+  if masked:
+    keep = torch.ones((b, skv), dtype=torch.bool, device=dev)
+    keep[:, skv // 2:] = False
+  got = attention_op.AttentionOp(attention_kernel="hip_flash_fp8", scale=d**-0.5, heads=h, dim_head=d, dtype=torch.bfloat16).apply_attention(
+      q, k, v, attention_mask=keep)
+  q8, s0 = ops.quant_e4m3(view(q), premul=ops.folded_q_mul(d), pow2_scale=True)
+  k8, s1 = ops.quant_e4m3(view(k), pow2_scale=True)
+  v8, s2 = ops.quant_e4m3(view(v))
+  ref = ops.flash_attention_fp8(q8, k8, v8, s0, s1, s2, scale=ops.FOLDED_SCALE, softmax="byte_grid",
+                                key_bias=None if keep is None else ops.key_mask_bias(keep))
+  assert torch.equal(got, ref.reshape(b, sq, h * d))
