@@ -104,8 +104,8 @@ struct BwdArgs {
 // MODE 0: dq (entity = q rows, stream = keys); 3: dk and dv in one pass (entity = key rows, stream = q rows).
 // MODE 1 (dk alone) and 2 (dv alone) are the same body with one accumulator set; the library launches 0 and 3.
 // DC != 0: head dims other than HD (a.D, a multiple of 8 up to DC), as in the forward's flat schedule: the layout of HD, the
-// MFMAs that cover DC columns; chunks past a.D are zero in the entity fragments, any finite data in the stream tiles, and
-// not stored in the gradients.
+// MFMAs that cover DC columns; chunks past a.D are zero in the entity fragments and in the row tiles (written once, no load
+// touches them), the row's first chunk in the transposed tiles, and not stored in the gradients.
 template <int MODE, int HD, bool BIAS, bool PRE, int DC>
 __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   static_assert(!(PRE && BIAS), "a biased logit is touched after the MFMAs anyway");
@@ -206,7 +206,9 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   const int grow = HD == 128 ? lane >> 4 : lane >> 3;
   // lane -> logical 16-byte chunk stored at this lane's position (a wave fills the row groups wave, wave + NW, ...)
   auto in_head = [&](int col) __attribute__((always_inline)) { return !PADDED || col < a.D ? col : 0; };
-  const int acol = in_head(HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8);
+  const int acol0 = HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8;
+  const int acol = in_head(acol0);
+  [[maybe_unused]] const bool ain = !PADDED || acol0 < a.D;
   const int bcol = in_head(HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8);
   const unsigned smem_addr = lds_addr_of(smem);
   // byte offsets of this lane's chunk from the first row of its row group: the same for every full tile.  The merged
@@ -228,6 +230,12 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   // behind the next tile's loads.
   [[maybe_unused]] const unsigned ofs_aux =
       MODE != 0 ? (lane < 32 ? 0u : (unsigned)((a.delta - a.lse2) * 4)) + (unsigned)l32 * 4u : (unsigned)l32 * 4u;
+  [[maybe_unused]] const uint64_t amask = __builtin_amdgcn_ballot_w64(ain);
+  // a row group of a row tile: the lanes whose chunk lies inside the head dim
+  auto dma_a = [&](auto... at) __attribute__((always_inline)) {
+    if constexpr (PADDED) lds_dma16(at..., amask);
+    else lds_dma16(at...);
+  };
   auto dma = [&](int slot, int t) __attribute__((always_inline)) {
     const unsigned A1 = smem_addr + (unsigned)(slot * kBStage) * 2u;
     const unsigned A2 = A1 + kBTileA * 2u;
@@ -257,8 +265,8 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       for (int i = 0; i < (kBT / RPI) / NW; ++i) {
         const int g = wave + NW * i;
         const int64_t r = t * kBT + RPI * g;
-        lds_dma16(s1p + r * a.s1_ss, o1, A1 + (unsigned)(g * kBGK) * 2u);
-        if constexpr (HAS2) lds_dma16(s2p + r * a.s2_ss, o2, A2 + (unsigned)(g * kBGK) * 2u);
+        dma_a(s1p + r * a.s1_ss, o1, A1 + (unsigned)(g * kBGK) * 2u);
+        if constexpr (HAS2) dma_a(s2p + r * a.s2_ss, o2, A2 + (unsigned)(g * kBGK) * 2u);
         lds_dma16(s3p + r * a.s3_ss, o3, Bt + (unsigned)(g * kBGV) * 2u);
         if constexpr (BOTH) lds_dma16(s4p + r * a.s4_ss, o4, Bt + (unsigned)(kBTileB + g * kBGV) * 2u);
       }
@@ -268,8 +276,8 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         const int g = wave + NW * i;
         int rr = t * kBT + RPI * g + grow;
         rr = rr < Ss ? rr : Ss - 1;
-        lds_dma16(s1p + (int64_t)rr * a.s1_ss + acol, A1 + (unsigned)(g * kBGK) * 2u);
-        if constexpr (HAS2) lds_dma16(s2p + (int64_t)rr * a.s2_ss + acol, A2 + (unsigned)(g * kBGK) * 2u);
+        dma_a(s1p + (int64_t)rr * a.s1_ss + acol, A1 + (unsigned)(g * kBGK) * 2u);
+        if constexpr (HAS2) dma_a(s2p + (int64_t)rr * a.s2_ss + acol, A2 + (unsigned)(g * kBGK) * 2u);
         lds_dma16(s3p + (int64_t)rr * a.s3_ss + bcol, Bt + (unsigned)(g * kBGV) * 2u);
         if constexpr (BOTH) lds_dma16(s4p + (int64_t)rr * a.s4_ss + bcol, Bt + (unsigned)(kBTileB + g * kBGV) * 2u);
       }
@@ -304,6 +312,15 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 #pragma unroll
     for (int sg = 0; sg < ND; ++sg)
       v_off[sg] = 2 * kBTileA + (4 * hh + vxr) * 64 + (sg ^ vx) * 32 + ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
+  }
+
+  if (!ain) {  // the chunks past the head dim of this wave's row groups (the loop's first barrier shows them to the others)
+#pragma unroll
+    for (int i = 0; i < 2 * ((kBT / RPI) / NW); ++i) {
+      __bf16* at = smem + (i & 1) * kBStage + (wave + NW * (i >> 1)) * kBGK + lane * 8;
+      *reinterpret_cast<uint4*>(at) = make_uint4(0u, 0u, 0u, 0u);
+      if constexpr (HAS2) *reinterpret_cast<uint4*>(at + kBTileA) = make_uint4(0u, 0u, 0u, 0u);
+    }
   }
 
   // LISTED: the tile at position t of this workgroup's share as tile * 2 + (it holds keys with a bias)

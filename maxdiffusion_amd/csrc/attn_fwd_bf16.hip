@@ -456,8 +456,9 @@ constexpr int kStageS = kKTileS + (kTS / 4) * kGV;    // elements per ring slot
 constexpr int kSlotsS = 3;
 
 // Other head dims (a.D, a multiple of 8 up to DC) run in the layout of the next of the two, HD, with the MFMAs that cover
-// DC columns (DC < HD + 1; 0: a.D == HD): lanes whose 16-byte chunk lies past a.D fetch the row's first chunk instead, which
-// meets zeros in Q (logits) or lands in output columns that are not stored.  A copy of q, k and v padded to 64 or 128
+// DC columns (DC < HD + 1; 0: a.D == HD).  Chunks past a.D: in K's tiles zeros, written once, which no load touches; in V's
+// the row's first chunk, for output columns that are not stored.  (K's pad has to be zero and not only meet zeros in Q: an
+// infinite key would make NaN of its logits.)  A copy of q, k and v padded to 64 or 128
 // columns in front, and one of out cut back behind, are gone: 62 -> 16 us for 16 x 257 tokens x 16 heads of 80 (64 -> 16 us of
 // kernels and the four copies' launches), 626 -> 449 us for 8,192 tokens x 20 heads of 80.
 template <int NW, bool BIAS, int HD, bool PRE, int DC = 0>
@@ -508,7 +509,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // lane -> (row of the group, logical 16-byte chunk stored at this lane's position)
   const int grow = HD == 128 ? lane >> 4 : lane >> 3;
   auto in_head = [&](int col) __attribute__((always_inline)) { return !PADDED || col < a.D ? col : 0; };
-  const int kcol = in_head(HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8);
+  const int kcol0 = HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8;
+  const int kcol = in_head(kcol0);
+  [[maybe_unused]] const bool kin = !PADDED || kcol0 < a.D;  // some lane of every wave is, so the loads count the same in all
+  [[maybe_unused]] const uint64_t kmask = __builtin_amdgcn_ballot_w64(kin);
+  // a K row group: the lanes whose chunk lies inside the head dim
+  auto dma_k = [&](auto... at) __attribute__((always_inline)) {
+    if constexpr (PADDED) lds_dma16(at..., kmask);
+    else lds_dma16(at...);
+  };
   const int vcol = in_head(HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8);
   constexpr int KGS = HD == 128 ? kGK : 8 * 64;  // group strides in LDS, elements
   constexpr int VGS = HD == 128 ? kGV : 8 * 64;
@@ -530,7 +539,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       const __bf16* vt0 = vp + (int64_t)(kt * TS + RPI * wave) * a.v_ss;
 #pragma unroll
       for (int i = 0; i < GPW; ++i) {
-        lds_dma16(kt0 + (int64_t)(RPI * NW * i) * a.k_ss, kofs, Ks + (unsigned)((wave + NW * i) * KGS) * 2u);
+        dma_k(kt0 + (int64_t)(RPI * NW * i) * a.k_ss, kofs, Ks + (unsigned)((wave + NW * i) * KGS) * 2u);
         lds_dma16(vt0 + (int64_t)(RPI * NW * i) * a.v_ss, vofs, Vs + (unsigned)((wave + NW * i) * VGS) * 2u);
       }
     } else {
@@ -539,7 +548,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
         const int g = wave + NW * i;
         int kk = kt * TS + RPI * g + grow;
         kk = kk < a.Skv ? kk : a.Skv - 1;
-        lds_dma16(kp + (int64_t)kk * a.k_ss + kcol, Ks + (unsigned)(g * KGS) * 2u);
+        dma_k(kp + (int64_t)kk * a.k_ss + kcol, Ks + (unsigned)(g * KGS) * 2u);
         lds_dma16(vp + (int64_t)kk * a.v_ss + vcol, Vs + (unsigned)(g * VGS) * 2u);
       }
     }
@@ -757,6 +766,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     }
   }
   __syncthreads();  // every wave holds its fragments: the staging area is ring slots again
+  if (!kin) {       // the chunks past the head dim of this wave's row groups (the loop's first barrier shows them to the others)
+#pragma unroll
+    for (int i = 0; i < SLOTS * GPW; ++i)
+      *reinterpret_cast<uint4*>(smem + (i / GPW) * STAGE + (wave + NW * (i % GPW)) * KGS + lane * 8) = make_uint4(0u, 0u, 0u, 0u);
+  }
   // SLOTS - 1 tiles are requested ahead of the one being worked on
   static_assert(SLOTS == 2 || SLOTS == 3, "one tile ahead, or two");
   if constexpr (SLOTS == 3 && BIAS) {

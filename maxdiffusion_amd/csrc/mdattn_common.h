@@ -117,6 +117,18 @@ __device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, u
 __device__ __forceinline__ void lds_dma16(const void* addr, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_addr), "v"(addr) : "memory", "m0");
 }
+// The same for the lanes of `mask` (at least one).  The mask is applied inside the statement: under an `if` the compiler merges
+// such loads across branches and with that takes the LDS address into a vector register.
+__device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, unsigned lds_addr, uint64_t mask) {
+  uint64_t all;
+  asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %4\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %0"
+               : "=&s"(all) : "s"(lds_addr), "v"(byte_off), "s"(base), "s"(mask) : "memory", "m0", "scc");
+}
+__device__ __forceinline__ void lds_dma16(const void* addr, unsigned lds_addr, uint64_t mask) {
+  uint64_t all;
+  asm volatile("s_mov_b32 m0, %1\n\ts_and_saveexec_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b64 exec, %0"
+               : "=&s"(all) : "s"(lds_addr), "v"(addr), "s"(mask) : "memory", "m0", "scc");
+}
 // The 4-byte form: lane i's dword lands at lds_addr + 4*i.
 __device__ __forceinline__ void lds_dma4(const void* base, unsigned byte_off, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" : : "s"(lds_addr), "v"(byte_off), "s"(base) : "memory", "m0");

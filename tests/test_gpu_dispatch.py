@@ -240,3 +240,28 @@ def test_head_dims_the_kernels_walk_unpadded(dev, lib, D, sq, skv, masked):
       assert float(got.float().abs().max()) <= 0.25, name
       continue
     assert rel_l2(to_np(got), rn) <= 6e-3, name
+
+
+@pytest.mark.parametrize("D", [8, 40, 72, 88])
+def test_an_infinite_key_stays_one_key_at_unpadded_head_dims(dev, D):
+  """A key with an infinite channel whose logits are all -inf takes no part, whatever the kernel keeps past the head dim:
+  output and the gradients that are finite by definition equal those of a call without that key."""
+  B, H, S = 1, 2, 97
+  gen = torch.Generator(device=dev).manual_seed(D)
+  mk = lambda: torch.randn((B, S, H, D), generator=gen, device=dev)
+  q, k, v, g = mk(), mk(), mk(), mk()
+  q[..., 0] = -1 - q[..., 0].abs()
+  k[:, 5, :, 0] = float("inf")
+  flat = lambda t: t.to(torch.bfloat16).reshape(B, S, H * D)
+  keep = (torch.arange(S, device=dev) != 5)[None]
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+
+  def run(kt, **kw):
+    x = [flat(t).requires_grad_(True) for t in (q, kt, v)]
+    out = op.apply_attention(*x, **kw)
+    return out.detach(), [t.view(B, S, H, D) for t in torch.autograd.grad(out, x, flat(g))]
+
+  out, (dq, dk, dv) = run(k)
+  ref, (rq, rk, rv) = run(torch.where(torch.isinf(k), 0.0, k), attention_mask=keep)
+  for name, a, b in (("out", out, ref), ("dq", dq[..., 1:], rq[..., 1:]), ("dk", dk, rk), ("dv", dv, rv)):  # dq[..., 0]: 0 * inf
+    assert rel_l2(to_np(a), to_np(b)) <= 6e-3, name
