@@ -46,6 +46,8 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
   return false;
 }
 // a backward call that the checks of its forward should have made impossible to fail
+// what a saved-tensor hook hands back is read with the form that the forward checked, or refused
+void unpacked(bool ok) { TORCH_CHECK_VALUE(ok, "a tensor saved for the backward pass came back from its hook with another dtype, shape or layout"); }
 void must(int rc, const char* where) { TORCH_CHECK(rc == MDATTN_OK, where, ": mdattn error ", rc, ": ", mdattn_strerror(rc)); }
 
 // [B,S,H,D] as the kernels walk it, over a rank-3 [B,S,H*D] or a rank-4 [B,H,S,D] tensor (attention_op._as_bshd)
@@ -90,6 +92,7 @@ struct Mask {
   int* tiles = nullptr;
   int64_t stride = 0;
   static int64_t cols(int64_t skv) { return (skv + 31) / 32 * 32; }
+  static int64_t floats(const View& vk) { return vk.b * cols(vk.s) + mdattn_host_key_tiles_ints((int)vk.b, (int)vk.s); }
   Mask(const Tensor& m, const View& vk) {
     if (!m.defined()) return;
     stride = cols(vk.s);
@@ -106,6 +109,14 @@ int fwd(const Tensor& q, const Tensor& k, const Tensor& v, const View& vq, const
                               &vv.st, &so, (float)scale, m.bias, m.stride, m.tiles);
 }
 
+bool operands(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, View& vq, View& vk, View& vv) {
+  if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q)) return false;
+  const auto a = as_view(q, heads), b = as_view(k, heads), c = as_view(v, heads);
+  if (!a || !b || !c || a->b != b->b || a->b != c->b || a->h != b->h || a->h != c->h || a->d != b->d || a->d != c->d || b->s != c->s) return false;
+  vq = *a; vk = *b; vv = *c;
+  return true;
+}
+
 // q, k, v in the caller's own rank; out [B,Sq,H*D]
 struct FlashFn : torch::autograd::Function<FlashFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& mask_, int64_t heads, double scale) {
@@ -114,17 +125,23 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
     Tensor lse = at::empty({vq.b, vq.h, vq.s}, q.options().dtype(at::kFloat));
     must(fwd(q, k, v, vq, vk, vv, out, lse, mask, scale), "mdattn_fwd_bf16");
-    ctx->save_for_backward({q, k, v, out, lse, mask});
+    ctx->save_for_backward({q, k, v, out, lse});
+    ctx->saved_data["mask"] = mask;  // not for hooks: its tile lists are indices
     ctx->saved_data["heads"] = heads;
     ctx->saved_data["scale"] = scale;
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4], &mask = saved[5];
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+    const Tensor mask = ctx->saved_data["mask"].toTensor();
     const int64_t heads = ctx->saved_data["heads"].toInt();
     const double scale = ctx->saved_data["scale"].toDouble();
-    const View vq = *as_view(q, heads), vk = *as_view(k, heads), vv = *as_view(v, heads);
+    View vq, vk, vv;
+    unpacked(operands(q, k, v, heads, vq, vk, vv) && q.is_non_overlapping_and_dense() && k.is_non_overlapping_and_dense() &&
+             v.is_non_overlapping_and_dense() && bf16_on(out, q) && out.is_contiguous() && out.sizes() == grads[0].sizes() && out.dim() == 3 &&
+             out.size(0) == vq.b && out.size(1) == vq.s && out.size(2) == vq.h * vq.d && lse.is_cuda() && lse.scalar_type() == at::kFloat &&
+             lse.is_contiguous() && lse.numel() == vq.b * vq.h * vq.s && (!mask.defined() || mask.numel() == Mask::floats(vk)));
     const Mask m(mask, vk);
     const Tensor dout = grad_like(grads[0], out);
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
@@ -145,7 +162,7 @@ Tensor make_mask(const Tensor& keep, const View& vk, const Tensor& ref) {
       keep.dim() != 2 || keep.size(0) != vk.b || keep.size(1) != vk.s || !keep.is_contiguous())
     return Tensor();
   const int B = (int)vk.b, S = (int)vk.s;
-  Tensor m = at::empty({B * Mask::cols(S) + mdattn_host_key_tiles_ints(B, S)}, keep.options().dtype(at::kFloat));
+  Tensor m = at::empty({Mask::floats(vk)}, keep.options().dtype(at::kFloat));
   const Mask v(m, vk);
   return mdattn_host_key_tiles(stream(), ptr(keep), v.bias, v.tiles, B, S, v.stride) == MDATTN_OK ? m : Tensor();
 }
@@ -153,16 +170,10 @@ Tensor make_mask(const Tensor& keep, const View& vk, const Tensor& ref) {
 // The registry entry's operands, checked: false when the Python path has to take over
 bool flash_args(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, double scale, const OptTensor& keep, View& vq, View& vk, View& vv,
                 Tensor& mask) {
-  if (!q.is_cuda() || !bf16_on(q, q) || !bf16_on(k, q) || !bf16_on(v, q)) return false;
-  const auto a = as_view(q, heads), b = as_view(k, heads), c = as_view(v, heads);
-  if (!a || !b || !c || a->b != b->b || a->b != c->b || a->h != b->h || a->h != c->h || a->d != b->d || a->d != c->d ||
-      b->s != c->s || !(scale > 0))
-    return false;
-  if (!mdattn_host_head_dim((int)a->d)) return false;  // padded first
-  if (q.numel() == 0 || k.numel() == 0 || std::max(a->s, b->s) >= ((int64_t)1 << 31)) return false;
-  if (keep.has_value() && !(mask = make_mask(*keep, *b, q)).defined()) return false;
-  vq = *a; vk = *b; vv = *c;
-  return true;
+  if (!operands(q, k, v, heads, vq, vk, vv) || !(scale > 0)) return false;
+  if (!mdattn_host_head_dim((int)vq.d)) return false;  // padded first
+  if (q.numel() == 0 || k.numel() == 0 || std::max(vq.s, vk.s) >= ((int64_t)1 << 31)) return false;
+  return !keep.has_value() || (mask = make_mask(*keep, vk, q)).defined();
 }
 
 // The registry entry `hip_flash`: [B,S,H*D] or [B,H,S,D] operands -> [B,Sq,H*D]; q_mul is rounded into q first.
@@ -265,6 +276,24 @@ std::optional<Table> as_table(const OptTensor& a, const OptTensor& b, int64_t s,
 const float* table_ptr(const Tensor& t) { return t.defined() ? static_cast<const float*>(t.data_ptr()) : nullptr; }
 bool weight_ok(const Tensor& w, int64_t n, const Tensor& ref) { return bf16_on(w, ref) && w.is_contiguous() && w.numel() == n; }
 
+// a saved q (or fused q|k|v), the k beside it, their weights and table in the form that the forward took
+bool rows_back(const Tensor& q, const Tensor& k, int64_t dim, bool dense) {
+  return bf16_on(q, q) && q.dim() == dim && q.stride(-1) == 1 && (!dense || q.is_non_overlapping_and_dense()) &&
+         (!k.defined() || (bf16_on(k, q) && k.sizes() == q.sizes() && k.strides() == q.strides()));
+}
+bool weights_back(std::initializer_list<const Tensor*> ws, int64_t n, const Tensor& ref) {
+  for (const Tensor* w : ws)
+    if (w->defined() && !weight_ok(*w, n, ref)) return false;
+  return true;
+}
+bool table_back(const Tensor& cos, const Tensor& sin, int64_t kind, int64_t s, int64_t d, const Tensor& ref) {
+  if (!cos.defined()) return true;
+  if (kind == MDATTN_TABLE_COMPLEX) return in_place(cos, at::kComplexFloat, s * d / 2, ref);
+  if (kind == MDATTN_TABLE_MATRIX) return in_place(cos, at::kFloat, s * d * 2, ref);
+  const int64_t n = kind == MDATTN_TABLE_REPEATED ? s * d : s * d / 2;
+  return in_place(cos, at::kFloat, n, ref) && in_place(sin, at::kFloat, n, ref);
+}
+
 struct Prologue {
   int64_t heads, kind, n_txt = 0;
   double eps, q_mul;
@@ -304,7 +333,9 @@ struct FullrowFn : torch::autograd::Function<FullrowFn> {
     const auto sv = ctx->get_saved_variables();
     const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3];
     const Prologue p = Prologue::saved(ctx);
+    unpacked(rows_back(q, k, 3, true) && q.numel() == g[0].numel());
     const int64_t b = q.size(0), s = q.size(1), n = q.size(2), d = n / p.heads;
+    unpacked(weights_back({&wq, &wk}, n, q) && table_back(sv[4], sv[5], p.kind, s, d, q) && g[0].sizes() == at::IntArrayRef({b, s, p.heads, d}));
     const bool has_k = k.defined();
     const Tensor gq = grad_like(g[0], Tensor());
     const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
@@ -366,7 +397,9 @@ struct PerheadFn : torch::autograd::Function<PerheadFn> {
     const auto sv = ctx->get_saved_variables();
     const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3], &wqt = sv[4], &wkt = sv[5];
     const Prologue p = Prologue::saved(ctx);
+    unpacked(rows_back(q, k, 4, true) && q.sizes() == g[0].sizes());
     const int64_t b = q.size(0), s = q.size(1), h = q.size(2), d = q.size(3);
+    unpacked(weights_back({&wq, &wk, &wqt, &wkt}, d, q) && table_back(sv[6], sv[7], p.kind, s, d, q));
     const bool has_k = k.defined();
     const Tensor gq = grad_like(g[0], Tensor());
     const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
@@ -431,8 +464,13 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
     const auto sv = ctx->get_saved_variables();
     const Tensor &x = sv[0], &bias = sv[1], &wq = sv[2], &wk = sv[3];
     const Prologue p = Prologue::saved(ctx);
+    unpacked(rows_back(x, Tensor(), 3, false));
     const int64_t b = x.size(0), s = x.size(1), n = x.size(2) / 3, d = n / p.heads;
-    const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq), gv = grad_like(g[2], gq);
+    unpacked(weights_back({&wq, &wk}, n, x) && weight_ok(bias, 3 * n, x) && table_back(sv[4], sv[5], p.kind, s, d, x) &&
+             g[0].sizes() == at::IntArrayRef({b, s, p.heads, d}));
+    const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq);
+    Tensor gv = grad_like(g[2], gq);
+    if (reinterpret_cast<uintptr_t>(gv.data_ptr()) & 15) gv = gv.clone(at::MemoryFormat::Preserve);  // the value block took any view
     Tensor dx = at::empty({b, s, 3 * n}, x.options());
     Tensor dwq = at::empty({n}, x.options()), dwk = at::empty({n}, x.options()), db = at::empty({3 * n}, x.options());
     const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, 5 * n);
@@ -483,7 +521,7 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     variable_list out = rows_run(q, k, wq, wk, cos, sin, p);
     TORCH_CHECK(!out.empty(), "mdattn_norm_rope_rows refused the request");
     ctx->save_for_backward({q, k, wq, wk, cos, sin});
-    ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode});
+    ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode, (int64_t)q.scalar_type()});
     ctx->saved_data["f"] = c10::List<double>({p.eps, p.w_mul});
     return out;
   }
@@ -492,8 +530,13 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3];
     const auto iv = ctx->saved_data["i"].toIntVector();
     const auto fv = ctx->saved_data["f"].toDoubleVector();
-    const int64_t heads = iv[0], mode = iv[1], b = q.size(0), s = q.size(1), n = q.size(2);
+    const int64_t heads = iv[0], mode = iv[1];
     const bool pair = k.defined();
+    unpacked(q.is_cuda() && (int64_t)q.scalar_type() == iv[2] && q.dim() == 3 && q.stride(2) == 1 && q.is_non_overlapping_and_dense() &&
+             (!pair || (k.get_device() == q.get_device() && k.scalar_type() == q.scalar_type() && k.sizes() == q.sizes() && k.strides() == q.strides())));
+    const int64_t b = q.size(0), s = q.size(1), n = q.size(2);
+    unpacked(grads[0].sizes() == at::IntArrayRef({b, s, heads, n / heads}) && in_place(wq, at::kFloat, n, q) && (!pair || in_place(wk, at::kFloat, n, q)));
+    for (const Tensor& t : {sv[4], sv[5]}) unpacked(!mode || in_place(t, at::kFloat, mode == 1 ? q.numel() : q.numel() / 2, q));
     const Tensor gq = grad_like(grads[0], Tensor()), gk = pair ? grad_like(grads[1], gq) : Tensor();
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = pair ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
     Tensor dwq = at::empty({n}, wq.options()), dwk = pair ? at::empty({n}, wq.options()) : Tensor();

@@ -206,3 +206,40 @@ def test_no_grad_path_is_unchanged(dev):
     assert not op.apply_attention(qg, k, v).requires_grad
   tracked = op.apply_attention(qg, k, v)
   assert tracked.requires_grad and torch.equal(tracked.detach(), plain)
+
+
+def test_saved_tensor_hooks_around_the_backward(dev):
+  """What a hook hands back is used (a copy with the same layout, as an offloading hook returns it; a mask's tile lists do
+  not pass through hooks) or refused with a ValueError (another dtype): never read as something it is not."""
+  B, H, D, S = 1, 2, 128, 70
+  N = H * D
+  gen = torch.Generator(device=dev).manual_seed(3)
+  mk = lambda *s, dt=torch.bfloat16: torch.randn(s, generator=gen, device=dev).to(dt).requires_grad_(True)
+  g = torch.randn((B, S, N), generator=gen, device=dev).to(torch.bfloat16)
+  keep = torch.arange(S, device=dev)[None] < 41
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+  q, k, v, wq, wk = mk(B, S, N), mk(B, S, N), mk(B, S, N), mk(N), mk(N)
+  qkv, bias = mk(B, S, 3 * N), mk(3 * N)
+  hq, hk, hw = mk(B, S, H, D), mk(B, S, H, D), mk(D)
+  rq, rk, rw = mk(B, S, N, dt=torch.float32), mk(B, S, N, dt=torch.float32), mk(N, dt=torch.float32)
+  gh = g.view(B, S, H, D)
+  freqs = torch.polar(torch.ones(S, D // 2, device=dev), torch.rand(S, D // 2, generator=gen, device=dev))[None, None]
+  calls = {
+      "attention": (lambda: (op.apply_attention(q, k, v, attention_mask=keep),), (q, k, v), (g,)),
+      "full row": (lambda: A.hip_norm_rope(q, k, wq, wk, freqs, H), (q, k, wq, wk), (gh, gh)),
+      "fused": (lambda: A.hip_norm_rope_qkv(qkv, wq, wk, freqs, H, bias=bias), (qkv, bias, wq, wk), (gh, gh, gh)),
+      "per head": (lambda: A.hip_norm_rope(hq, hk, hw, hw, freqs, H, per_head=True), (hq, hk, hw), (gh, gh)),
+      "rows": (lambda: A.hip_norm_rope_ltx2(rq, rk, rw, rw, H), (rq, rk, rw), (gh, gh)),
+  }
+  lossy = lambda t: t.to(torch.bfloat16) if t.dtype == torch.float32 else t.to(torch.float32)
+  for name, (call, leaves, gs) in calls.items():
+    print(name, flush=True)
+    want = torch.autograd.grad(call(), leaves, gs)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(dev)):
+      out = call()
+    for a, b in zip(torch.autograd.grad(out, leaves, gs), want):
+      assert torch.equal(a, b), name
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lossy):
+      out = call()
+    with pytest.raises(ValueError):
+      torch.autograd.grad(out, leaves, gs)
