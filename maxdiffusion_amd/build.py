@@ -183,6 +183,9 @@ def build_library(verbose: bool = True) -> str:
   except BaseException:
     if host is not None:
       host[1].kill()
+      host[1].wait()
+      if os.path.exists(host[0]):
+        os.remove(host[0])
     raise
   if host is not None:
     _finish_host_extension(host, verbose)
