@@ -125,6 +125,22 @@ __device__ __forceinline__ void store_row(const AttnArgs& a, const f32x16 (&O)[N
   if (a.lse && hh == 0) a.lse[lidx] = (mc + __log2f(lt)) * kLn2;
 }
 
+// The epilogue of a workgroup that walked only a share of the keys: O, the row's sum of P and its reference point as they are.
+template <int ND, bool PADDED>
+__device__ __forceinline__ void store_partial(const AttnArgs& a, const f32x16 (&O)[ND], float lt, float mc, int sp, int bh, int row, int hh) {
+  if (row >= a.Sq) return;
+  const int64_t r = ((int64_t)sp * a.BH + bh) * a.Sq + row;
+  float* p = a.part + r * (PADDED ? a.D : ND * 32) + 4 * hh;
+#pragma unroll
+  for (int db = 0; db < ND; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (PADDED && db * 32 + 8 * g >= a.D) continue;
+      *reinterpret_cast<f32x4*>(p + db * 32 + 8 * g) = f32x4{O[db][4 * g], O[db][4 * g + 1], O[db][4 * g + 2], O[db][4 * g + 3]};
+    }
+  if (hh == 0) a.ml[r] = make_float2(mc, lt);
+}
+
 // The same epilogue with whole-row stores, for a wave that may use `stage` (32 rows of HD * 2 + 16 bytes of LDS that
 // nobody else touches any more).  store_row writes, per instruction, 16 bytes of each of 32 rows that lie a whole
 // token apart; at short key sequences, where the output is a large part of the launch's work, that costs as much as
@@ -490,15 +506,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   const int wg = blockIdx.x;
   const int w = (wg & 7) * a.chunk + (wg >> 3);
   if (w >= a.total) return;
-  const int bh = w / a.nqt, qt = w - bh * a.nqt;
+  const int bhs = w / a.nqt, qt = w - bhs * a.nqt;  // query tiles fastest: neighbouring workgroups walk the same keys
+  const int bh = BIAS ? bhs : bhs / a.nsplit, sp = BIAS ? 0 : bhs - bh * a.nsplit;
   const int b = bh / a.H, h = bh - b * a.H;
+  // this workgroup's keys: kv0 .. kv0 + Skv - 1 (never empty); everything below counts from kv0
+  const int kv0 = BIAS ? 0 : sp * a.tps * TS;
+  const int Skv = BIAS || a.Skv - kv0 < a.tps * TS ? a.Skv - kv0 : a.tps * TS;
 
   const __bf16* qp = a.q + b * a.q_sb + h * a.q_sh;
-  const __bf16* kp = a.k + b * a.k_sb + h * a.k_sh;
-  const __bf16* vp = a.v + b * a.v_sb + h * a.v_sh;
+  const __bf16* kp = a.k + b * a.k_sb + h * a.k_sh + kv0 * a.k_ss;
+  const __bf16* vp = a.v + b * a.v_sb + h * a.v_sh + kv0 * a.v_ss;
   const int q0 = qt * BM + wave * 32;
   [[maybe_unused]] TileList tl{BIAS && a.tiles ? a.tiles + (int64_t)b * a.tiles_sb : nullptr};
-  int nt = (a.Skv + TS - 1) / TS;  // tiles visited; with a list, 0 when every key is excluded
+  int nt = (Skv + TS - 1) / TS;  // tiles visited; with a list, 0 when every key is excluded
   if constexpr (BIAS) nt = tl.count(nt);
   const float c = a.c;
   const float* bias_row = BIAS ? a.bias + b * a.bias_sb : nullptr;
@@ -534,7 +554,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       col = col < bias_cols ? col : bias_cols - 1;
       lds_dma4(bias_row, (unsigned)col * 4u, Ks + TILES * 2u);
     }
-    if (kt * TS + TS <= a.Skv) {
+    if (kt * TS + TS <= Skv) {
       const __bf16* kt0 = kp + (int64_t)(kt * TS + RPI * wave) * a.k_ss;
       const __bf16* vt0 = vp + (int64_t)(kt * TS + RPI * wave) * a.v_ss;
 #pragma unroll
@@ -547,7 +567,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       for (int i = 0; i < GPW; ++i) {
         const int g = wave + NW * i;
         int kk = kt * TS + RPI * g + grow;
-        kk = kk < a.Skv ? kk : a.Skv - 1;
+        kk = kk < Skv ? kk : Skv - 1;
         dma_k(kp + (int64_t)kk * a.k_ss + kcol, Ks + (unsigned)(g * KGS) * 2u);
         lds_dma16(vp + (int64_t)kk * a.v_ss + vcol, Vs + (unsigned)(g * VGS) * 2u);
       }
@@ -643,7 +663,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       const int kv_base = kt * TS + 32 * blk + 4 * hh;
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (kv_base + 8 * (i >> 2) + (i & 3) >= a.Skv) S[i] = -INFINITY;
+        if (kv_base + 8 * (i >> 2) + (i & 3) >= Skv) S[i] = -INFINITY;
     }
     // ---- online softmax.  The hot path takes no row maximum: P and its sum are formed against the row's
     // current reference point, and only a partial sum above kTrig (a logit far above the reference, or
@@ -821,7 +841,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     tile(nt - 1, nt - 1, false, (nt - 1) % SLOTS, std::true_type{});
   }
 
-  if (!PADDED && a.o_run) {  // ring step: merged into the f32 carry, row by row
+  if (!BIAS && a.part) {
+    store_partial<ND, PADDED>(a, O, xhalf_sum(l), mc, sp, bh, q0 + l32, hh);
+  } else if (!PADDED && a.o_run) {  // ring step: merged into the f32 carry, row by row
     store_row<ND>(a, O, xhalf_sum(l), mc, b, h, q0 + l32, hh);
   } else {
     static_assert(NW * 32 * (ND * 64 + 16) <= SLOTS * STAGE * 2, "the output staging tiles must fit the ring's LDS");
@@ -838,7 +860,11 @@ static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   constexpr int stage_el = (HD == 128 ? kStageS : 2 * 64 * 64) + (BIAS ? 128 : 0), qtile_el = HD == 128 ? kKTileS : 32 * 64;
   constexpr int lds_bytes = (slots * stage_el > stage_el + NW * qtile_el ? slots * stage_el : stage_el + NW * qtile_el) * 2;
   a.nqt = (a.Sq + BM - 1) / BM;
-  const int64_t total = (int64_t)B * a.H * a.nqt;
+  if (!a.part) {
+    a.nsplit = 1;
+    a.tps = (a.Skv + (HD == 128 ? kTS : 64) - 1) / (HD == 128 ? kTS : 64);
+  }
+  const int64_t total = (int64_t)B * a.H * a.nqt * a.nsplit;
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
@@ -848,6 +874,37 @@ static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   if (pre) MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, !BIAS, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   else MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, false, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   return launch_status();
+}
+
+// The shares of a split call brought to one reference point and summed, in the order of the splits: one 16-byte store per lane.
+// Bound by the partials, which come back from beyond the other XCDs' L2s: about 2.8 TB/s written and read (a layout with
+// whole 1 KB stores, as the lanes hold the accumulators, measured the same).
+__global__ __launch_bounds__(256) void fwd_combine_kernel(AttnArgs a, int cpr, int64_t chunks) {  // cpr: 16-byte chunks per row, D/8
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= chunks) return;
+  const int64_t row = i / cpr, rows = (int64_t)a.BH * a.Sq;
+  const int c = (int)(i - row * cpr);
+  float m = -INFINITY;
+  for (int k = 0; k < a.nsplit; ++k) {
+    const float2 u = a.ml[k * rows + row];
+    if (u.y != 0.f) m = fmaxf(m, u.x);  // (a share without weight carries no reference point)
+  }
+  const float4* p = reinterpret_cast<const float4*>(a.part) + 2 * i;
+  float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, l = 0.f;
+  for (int k = 0; k < a.nsplit; ++k, p += 2 * chunks) {
+    const float2 u = a.ml[k * rows + row];
+    const float w = u.y != 0.f ? __builtin_amdgcn_exp2f(u.x - m) : 0.f;
+    const float4 x = p[0], y = p[1];
+    l += w * u.y;
+    f[0] += w * x.x; f[1] += w * x.y; f[2] += w * x.z; f[3] += w * x.w; f[4] += w * y.x; f[5] += w * y.y; f[6] += w * y.z; f[7] += w * y.w;
+  }
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] *= inv;
+  const int s = (int)(row % a.Sq);
+  const int64_t bh = row / a.Sq, b = bh / a.H, h = bh - b * a.H;
+  *reinterpret_cast<uint4*>(a.out + b * a.o_sb + (int64_t)s * a.o_ss + h * a.o_sh + c * 8) = pack8(f);
+  if (a.lse && c == 0) a.lse[row] = (m + __log2f(l)) * kLn2;
 }
 
 template <int NW>
@@ -896,6 +953,7 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
   a.c = scale * kLog2e;
   a.bias = nullptr; a.bias_sb = 0; a.tiles = nullptr; a.tiles_sb = 0;
   a.o_run = nullptr; a.lse_run = nullptr;
+  a.nsplit = 1; a.tps = 0; a.BH = B * H; a.part = nullptr; a.ml = nullptr;
   return MDATTN_OK;
 }
 
@@ -928,18 +986,65 @@ static int dispatch_padded(hipStream_t st, const AttnArgs& a, int B) {
   return launch_flat<4, BIAS, 128, 96>(st, a, B);
 }
 
+// Into how many shares a call's keys are cut.  A query tile is one workgroup that walks every key: few heads times few
+// queries leave most of the chip idle meanwhile.  The cost of n shares in us: a workgroup's tiles at the rate that
+// workgroups sharing a CU leave each other, and for n > 1 the second launch, its serial loop and the partials.  Fitted to
+// 4 .. 512 query tiles x 256 .. 4,096 keys x 1 .. 16 shares, within 15 %.  4 query tiles x 2,048 keys 39.3 -> 17.2 us, 32 x
+// 1,024 22.1 -> 17.9, 128 x 4,096 76.6 -> 48.6 (head dim 128); 32 x 2,048 27.9 -> 16.7 (64), 36.7 -> 20.1 (80).
+struct FwdSplit {
+  int nsplit, tps;
+  int64_t rows;  // of partials
+};
+static FwdSplit fwd_split(int64_t BH, int Sq, int Skv, int D) {
+  const int ts = D > 64 ? kTS : 64, nt = (Skv + ts - 1) / ts;
+  const int64_t tiles = BH * ((Sq + 127) / 128);
+  FwdSplit best{1, nt, 0};
+  if (D == kD && Skv > 3072 && BH * ((Sq + 255) / 256) >= 128) return best;  // the pipelined kernel's
+  const double tile_us = D > 64 ? 0.55 : 0.75, partial_us = 3.0e-4 * D;     // a tile of keys; a workgroup's partials
+  auto walk = [&](int64_t wgs, int tps) {
+    const double load = 0.5 + 0.58 * (double)wgs / 256;
+    return tile_us * tps * (load > 1.0 ? load : 1.0);
+  };
+  double best_cost = 0.9 * walk(tiles, nt);
+  for (int n = 2; n <= 16 && nt / n >= 4; ++n) {
+    const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
+    const double cost = walk(tiles * ns, tps) + 4.0 + 0.45 * ns + partial_us * (double)(tiles * ns);
+    if (cost < best_cost) { best_cost = cost; best = {ns, tps, ns * BH * Sq}; }
+  }
+  return best;
+}
+
+extern "C" int64_t mdattn_host_fwd_workspace_floats(int B, int H, int Sq, int Skv, int D) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !native_head_dim(D)) return 0;
+  return fwd_split((int64_t)B * H, Sq, Skv, D).rows * (D + 2);
+}
+
 extern "C" int mdattn_host_head_dim(int D) { return native_head_dim(D); }
 
 extern "C" int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,
                                     int B, int H, int Sq, int Skv, int D,
                                     const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                                     const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                                    const float* key_bias, int64_t bias_stride, const int* tiles) {
+                                    const float* key_bias, int64_t bias_stride, const int* tiles, float* workspace, int64_t workspace_floats) {
   AttnArgs a;
   const int rc = fill_args(a, q, k, v, out, lse, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale, true);
   if (rc != MDATTN_OK) return rc;
   const hipStream_t st = (hipStream_t)stream;
-  if (!key_bias) return D == 64 || D == kD ? dispatch_fwd(st, a, B, Sq, Skv, D) : dispatch_padded<false>(st, a, B);
+  if (!key_bias) {
+    const FwdSplit s = fwd_split((int64_t)B * H, Sq, Skv, D);
+    if (s.nsplit == 1 || !workspace || workspace_floats < s.rows * (D + 2) || forced_fwd_schedule() != 0)
+      return D == 64 || D == kD ? dispatch_fwd(st, a, B, Sq, Skv, D) : dispatch_padded<false>(st, a, B);
+    if (!aligned16(workspace)) return MDATTN_E_ALIGN;
+    a.nsplit = s.nsplit;
+    a.tps = s.tps;
+    a.part = workspace;
+    a.ml = reinterpret_cast<float2*>(workspace + s.rows * D);
+    const int split_rc = D == kD ? launch_flat<4, false>(st, a, B) : D == 64 ? launch_flat<4, false, 64>(st, a, B) : dispatch_padded<false>(st, a, B);
+    if (split_rc != MDATTN_OK) return split_rc;
+    const int64_t chunks = (int64_t)B * H * Sq * (D / 8);  // at most a few million: split calls are small ones
+    MDATTN_LAUNCH(fwd_combine_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a, D / 8, chunks);
+    return launch_status();
+  }
   if (bias_stride < ((Skv + kTS - 1) / kTS) * kTS || bias_stride % kTS != 0) return MDATTN_E_BADARG;
   if (!aligned16(key_bias) || (reinterpret_cast<uintptr_t>(tiles) & 3u)) return MDATTN_E_ALIGN;
   a.bias = key_bias;

@@ -105,8 +105,10 @@ int fwd(const Tensor& q, const Tensor& k, const Tensor& v, const View& vq, const
         const Tensor& mask, double scale) {
   const Mask m(mask, vk);
   const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
+  const int64_t nws = m.bias ? 0 : mdattn_host_fwd_workspace_floats((int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d);
+  const Tensor ws = nws ? at::empty({nws}, q.options().dtype(at::kFloat)) : Tensor();
   return mdattn_host_fwd_bf16(stream(), ptr(q), ptr(k), ptr(v), mut(out), f32(lse), (int)vq.b, (int)vq.h, (int)vq.s, (int)vk.s, (int)vq.d, &vq.st, &vk.st,
-                              &vv.st, &so, (float)scale, m.bias, m.stride, m.tiles);
+                              &vv.st, &so, (float)scale, m.bias, m.stride, m.tiles, f32(ws), nws);
 }
 
 bool operands(const Tensor& q, const Tensor& k, const Tensor& v, int64_t heads, View& vq, View& vk, View& vv) {

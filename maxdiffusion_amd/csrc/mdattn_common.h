@@ -175,6 +175,12 @@ struct AttnArgs {
   int tiles_sb;
   float* o_run;    // when set: no `out`; the result is merged in LSE space into this f32 carry (strides o_s*, in floats)
   float* lse_run;  // ... and into its lse [B,H,Sq]
+  // key split (flat kernel without a bias): the key tiles are dealt to nsplit workgroups per query tile, tps each; with part
+  // set, each leaves its un-normalised f32 output [split][B*H][Sq][D] and (reference point, sum of P) per row for
+  // fwd_combine_kernel
+  int nsplit, tps, BH;
+  float* part;
+  float2* ml;
 };
 
 

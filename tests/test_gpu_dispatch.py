@@ -265,3 +265,31 @@ def test_an_infinite_key_stays_one_key_at_unpadded_head_dims(dev, D):
   ref, (rq, rk, rv) = run(torch.where(torch.isinf(k), 0.0, k), attention_mask=keep)
   for name, a, b in (("out", out, ref), ("dq", dq[..., 1:], rq[..., 1:]), ("dk", dk, rk), ("dv", dv, rv)):  # dq[..., 0]: 0 * inf
     assert rel_l2(to_np(a), to_np(b)) <= 6e-3, name
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,D", [(1, 1, 1, 2048, 128), (1, 4, 126, 1025, 128), (2, 3, 200, 4100, 128), (1, 2, 257, 3000, 64),
+                                          (1, 3, 65, 1300, 40), (2, 2, 130, 2049, 72), (1, 4, 127, 2048, 96)])
+def test_keys_split_over_workgroups(dev, lib, B, H, Sq, Skv, D):
+  """Few query tiles against many keys: the shares meet in the combine kernel.  Ragged last tiles and shares, an output row
+  stride of its own, shares whose logits lie far apart, and the lse through the gradients; against f32 attention on the same
+  bf16 operands (bars of the unsplit path)."""
+  assert lib.mdattn_host_fwd_workspace_floats(B, H, Sq, Skv, D) > 0
+  gen = torch.Generator(device=dev).manual_seed(Sq + Skv + D)
+  mk = lambda s: torch.randn((B, s, H * D), generator=gen, device=dev)
+  k = mk(Skv)
+  k[:, Skv // 3:Skv // 2] *= 6  # one share holds the large logits
+  q, k, v = (t.to(torch.bfloat16).requires_grad_(True) for t in (mk(Sq), k, mk(Skv)))
+  g = mk(Sq).to(torch.bfloat16)
+  for scale in (D**-0.5, float(np.log(2.0)) * 0.1, float(np.log(2.0))):  # the last: the kernels' form without the multiply
+    op = A.AttentionOp(attention_kernel="hip_flash", scale=scale, heads=H, dim_head=D, dtype=torch.bfloat16)
+    if scale > 0.5:
+      q = (q.detach() * 0.1).requires_grad_(True)
+    out = op.apply_attention(q, k, v)
+    grads = torch.autograd.grad(out, (q, k, v), g)
+    rq, rk, rv = (t.detach().float().requires_grad_(True) for t in (q, k, v))
+    hf = lambda t: t.view(B, -1, H, D).transpose(1, 2)
+    ref = (torch.softmax((hf(rq) @ hf(rk).transpose(2, 3)) * scale, -1) @ hf(rv)).transpose(1, 2).reshape(B, Sq, H * D)
+    want = torch.autograd.grad(ref, (rq, rk, rv), g.float())
+    assert rel_l2(to_np(out), ref.detach().cpu().numpy()) <= 6e-3, scale
+    for name, got, r in zip(("dq", "dk", "dv"), grads, want):
+      assert rel_l2(to_np(got), r.detach().cpu().numpy()) <= 1e-2, (name, scale)
