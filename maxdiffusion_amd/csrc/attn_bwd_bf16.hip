@@ -82,8 +82,11 @@ struct BwdArgs {
   const __bf16* s4;  // MODE 3: second stream tensor to accumulate with (dout, for dv); s3 is q (for dk)
   __bf16* out2;      // MODE 3: dv
   int64_t s4_sb, s4_ss, s4_sh, o2_sb, o2_ss, o2_sh;
-  const float* lse2;   // [B,H,Sp] -lse * log2(e), -inf on padded rows
-  const float* delta;  // [B,H,Sp] -rowsum(dout * out)
+  // Written by the dq pass for the dk / dv pass, both negated (they start the MFMA chains that they are subtracted from)
+  float* lse2;         // [B,H,Sp] -lse * log2(e), -inf on padded rows
+  float* delta;        // [B,H,Sp] -rowsum(dout * out), 0 on padded rows
+  const __bf16* fwd;   // MODE 0: the forward's out, with the strides of dout (e2)
+  const float* lse;    // MODE 0: the forward's lse [B,H,Se]
   int H, Se, Ss, Sp, D;
   int net, total, chunk;
   int64_t e1_sb, e1_ss, e1_sh, e2_sb, e2_ss, e2_sh;
@@ -182,12 +185,28 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       for (int s = 0; s < NJ; ++s) ef2[s] = in_row(s) ? *reinterpret_cast<const bf16x8*>(p2 + s * 16) : zero8;
     }
   }
-  const float* lrow = a.lse2 + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
-  const float* drow = a.delta + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
-  float nlse_e = 0.f, ndelta_e = 0.f;  // the workspace holds both negated
+  float* lrow = a.lse2 + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
+  float* drow = a.delta + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
+  float nlse_e = 0.f, ndelta_e = 0.f;  // both negated
   if constexpr (MODE == 0) {
-    nlse_e = lrow[erow];
-    ndelta_e = drow[erow];
+    // rowsum(dout * out) from the dout fragments that the pass holds anyway.  In a launch in front of it dout was read once
+    // more (40 us at 32,760 rows x 12 heads): a training pass there against 512 keys 656 -> 644 us, 24 x 4,608 1094 -> 1076.
+    const __bf16* po = a.fwd + b * a.e2_sb + h * a.e2_sh + (int64_t)erow * a.e2_ss + hh * 8;
+#pragma unroll
+    for (int s = 0; s < NJ; ++s) {
+      const bf16x8 o = in_row(s) ? *reinterpret_cast<const bf16x8*>(po + s * 16) : zero8;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ndelta_e = __builtin_fmaf(-(float)o[e], (float)ef2[s][e], ndelta_e);
+    }
+    ndelta_e = xhalf_sum(ndelta_e);
+    // rows whose keys were all masked (the forward wrote lse = -inf, out = 0) take no part: p = 0
+    const float lv = a.lse[(int64_t)bh * a.Se + erow];
+    nlse_e = lv > -INFINITY ? -lv * kLog2e : -INFINITY;
+    const int row = r0 + l32;
+    if (sp == 0 && hh == 0 && row < a.Sp) {
+      lrow[row] = row < a.Se ? nlse_e : -INFINITY;
+      drow[row] = row < a.Se ? ndelta_e : 0.f;
+    }
   }
   // key bias in log2 units: a per-lane scalar when the keys are the entity rows, sixteen values per tile otherwise
   [[maybe_unused]] const float* bias_row = BIAS ? a.bias + b * a.bias_sb + (MODE == 0 ? ss0 : 0) : nullptr;
@@ -568,37 +587,6 @@ __global__ __launch_bounds__((bwd_waves<HD>() * 64)) __attribute__((amdgpu_waves
   attn_bwd_body<3, HD, BIAS, PRE, DC>(a);
 }
 
-// The workspace, both negated (they start the MFMA chains that they are subtracted from):
-// delta[b,h,q] = -sum_d dout*out, lse2 = -lse*log2(e); rows q in [Sq, Sp) get delta 0, lse2 -inf.  16 lanes per row
-// (head dim 64: the upper 8 stay idle).
-__global__ __launch_bounds__(256) void bwd_prep_kernel(const __bf16* out, const __bf16* dout, const float* lse,
-                                                       float* lse2, float* delta, int H, int Sq, int Sp, int D,
-                                                       int64_t rows, int64_t o_sb, int64_t o_ss, int64_t o_sh) {
-  const int64_t r = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  if (r >= rows) return;
-  const int lane = threadIdx.x & 15;
-  const int q = (int)(r % Sp);
-  const int64_t bh = r / Sp;
-  const int h = (int)(bh % H);
-  const int64_t b = bh / H;
-  float acc = 0.f;
-  if (q < Sq && lane * 8 < D) {
-    const int64_t off = b * o_sb + (int64_t)q * o_ss + h * o_sh + lane * 8;
-    float x[8], y[8];
-    unpack8(*reinterpret_cast<const uint4*>(out + off), x);
-    unpack8(*reinterpret_cast<const uint4*>(dout + off), y);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc = __builtin_fmaf(x[j], y[j], acc);
-  }
-  acc = row16_sum(acc);
-  if (lane == 0) {
-    delta[r] = q < Sq ? -acc : 0.f;
-    // padded rows, and rows whose keys were all masked (the forward wrote lse = -inf, out = 0), take no part: p = 0
-    const float lv = q < Sq ? lse[bh * Sq + q] : -INFINITY;
-    lse2[r] = lv > -INFINITY ? -lv * kLog2e : -INFINITY;
-  }
-}
-
 // Sums the partial gradients of a split pass in the order of the splits and rounds them to bf16: one 16-byte store per
 // lane, blockIdx.y = tensor.  Bound by the partials' bytes: 12.8 us for 63 MB (4.9 TB/s).
 struct BwdReduceArgs {
@@ -729,7 +717,7 @@ extern "C" int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int S
   return mdattn_bwd_workspace_floats(B, H, Sq) + bwd_split(BH, Sq, Skv, D, 1).floats + 2 * bwd_split(BH, Skv, Sq, D, 2).floats;
 }
 
-// Shared body of mdattn_bwd_bf16 and mdattn_bwd_bf16_static: validation, the preparation kernel and the two passes.
+// Shared body of mdattn_bwd_bf16 and mdattn_bwd_bf16_static: validation and the two passes.
 static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, const void* out, const void* dout,
                    const float* lse, void* dq, void* dk, void* dv, float* workspace, int64_t workspace_floats,
                    int B, int H, int Sq, int Skv, int D,
@@ -760,10 +748,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   float* lse2 = workspace;
   float* delta = workspace + (int64_t)B * H * Sp;
   const int64_t rows = (int64_t)B * H * Sp;
-  if ((rows + 15) / 16 > 0x7FFFFFFF || rows >= (1 << 29)) return MDATTN_E_UNSUPPORTED;  // delta - lse2 as a 32-bit byte offset
-  MDATTN_LAUNCH(bwd_prep_kernel, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, (const __bf16*)out,
-                     (const __bf16*)dout, lse, lse2, delta, H, Sq, Sp, D, rows, o_strides->batch, o_strides->seq, o_strides->head);
-  if (launch_status() != MDATTN_OK) return MDATTN_E_LAUNCH;
+  if (rows >= (1 << 29)) return MDATTN_E_UNSUPPORTED;  // delta - lse2 as a 32-bit byte offset
 
   // stream splits, when the caller's workspace holds their partials (it always holds lse2 and delta)
   const int64_t BH = (int64_t)B * H;
@@ -773,7 +758,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
     skv = {1, (Sq + kBT - 1) / kBT, 0};
   }
   BwdArgs a;
-  a.lse2 = lse2; a.delta = delta; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
+  a.lse2 = lse2; a.delta = delta; a.fwd = (const __bf16*)out; a.lse = lse; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;
   a.tiles = tiles; a.tiles_sb = key_tiles_ints(Skv, 32);
   auto set = [](int64_t& sb, int64_t& ss, int64_t& sh, const mdattn_strides* s) { sb = s->batch; ss = s->seq; sh = s->head; };
@@ -837,7 +822,7 @@ extern "C" int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, 
 // forbid hipMalloc).  The workspace (-lse in log2 units and -delta, one float each per padded query row) lives in a
 // file-scope device array instead of a caller's buffer.  Every GPU holds its own copy of the array at its own
 // address: that address is looked up once per device with hipGetSymbolAddress and kept; host code never uses the
-// array's name as a pointer.  bwd_prep_kernel writes every element the passes read, so nothing has to be cleared
+// array's name as a pointer.  The dq pass writes every element of it that the dk / dv pass reads, so nothing has to be cleared
 // between calls; calls that overlap on one GPU share the array and race.
 static __device__ __align__(256) float scratch[MDATTN_BWD_STATIC_MAX_FLOATS];
 
