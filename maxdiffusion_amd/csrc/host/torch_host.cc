@@ -71,6 +71,13 @@ std::optional<View> as_view(const Tensor& t, int64_t heads) {
   }
   return v;
 }
+bool aligned(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+// Whether the kernels read this place and these strides (their own checks refuse the others): the padding of a head dim makes
+// a copy, and with it takes views at any address, so head dims walked unpadded have to fall back to it before a node exists.
+bool walkable(const Tensor& t, const View& v) {
+  const int64_t m = v.st.batch | v.st.seq | v.st.head;
+  return aligned(t) && m % 8 == 0 && v.st.seq >= v.d && v.st.seq < (1 << 23) && v.st.head > 0;
+}
 // a logical [B,S,H,D] tensor
 mdattn_strides strides4(const Tensor& t) { return {t.stride(0), t.stride(1), t.stride(2)}; }
 
@@ -145,7 +152,8 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
              out.size(0) == vq.b && out.size(1) == vq.s && out.size(2) == vq.h * vq.d && lse.is_cuda() && lse.scalar_type() == at::kFloat &&
              lse.is_contiguous() && lse.numel() == vq.b * vq.h * vq.s && (!mask.defined() || mask.numel() == Mask::floats(vk)));
     const Mask m(mask, vk);
-    const Tensor dout = grad_like(grads[0], out);
+    Tensor dout = grad_like(grads[0], out);
+    if (vq.d != 64 && vq.d != 128 && !aligned(dout)) dout = dout.clone();  // (a padded call's backward copies it as well)
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     const int B = (int)vq.b, H = (int)vq.h, Sq = (int)vq.s, Skv = (int)vk.s, D = (int)vq.d;
     const int64_t nws = mdattn_bwd_split_workspace_floats(B, H, Sq, Skv, D);
@@ -201,6 +209,7 @@ OptTensor flash_autograd(const Tensor& q, const Tensor& k, const Tensor& v, int6
   Tensor mask;
   for (const Tensor* t : {&q, &k, &v})
     if (!t->is_non_overlapping_and_dense()) return std::nullopt;  // their gradients take the same strides
+  if (!operands(q, k, v, heads, vq, vk, vv) || !walkable(q, vq) || !walkable(k, vk) || !walkable(v, vv)) return std::nullopt;
   if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, mask)) return std::nullopt;
   return FlashFn::apply(q, k, v, opt(mask), heads, scale);
 }

@@ -243,3 +243,25 @@ def test_saved_tensor_hooks_around_the_backward(dev):
       out = call()
     with pytest.raises(ValueError):
       torch.autograd.grad(out, leaves, gs)
+
+
+@pytest.mark.parametrize("rank4", [False, True])
+def test_unpadded_head_dim_at_any_address(dev, rank4):
+  """A head dim that the kernels walk unpadded (80), with operands and an output gradient that start 2 bytes past an aligned
+  address: taken as the padding copy takes them, and the same result as for aligned copies within two bf16 roundings
+  (the padded kernels sum in another order)."""
+  B, H, D, S = 1, 2, 80, 70
+  N = H * D
+  shape = (B, H, S, D) if rank4 else (B, S, N)
+  gen = torch.Generator(device=dev).manual_seed(4)
+  base = [torch.randn(B * S * N + 1, generator=gen, device=dev).to(torch.bfloat16) for _ in range(4)]
+  odd = [t[1:].view(shape).requires_grad_(True) for t in base[:3]]
+  even = [t.detach().clone().requires_grad_(True) for t in odd]
+  g = base[3][1:].view(B, S, N)
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+  want = op.apply_attention(*even)
+  want_grads = torch.autograd.grad(want, even, g.clone())
+  for leaves in (odd, even):  # operands and gradient at odd addresses, then the gradient alone
+    out = op.apply_attention(*leaves)
+    for a, b in zip((out, *torch.autograd.grad(out, leaves, g)), (want, *want_grads)):
+      assert rel_l2(a.detach().float().cpu().numpy(), b.detach().float().cpu().numpy()) <= 8e-3
