@@ -18,9 +18,9 @@
 //   acc^T += stream3^T . W          (A = the tile through the transposing LDS read)
 // lse and delta belong to the q rows: per-lane scalars for dq; for dk / dv sixteen values per lane and tile, which
 // ride through the ring next to the tile (a register load inside the loop would be waited for in issue order, i.e.
-// behind the next tile's loads).  They come from a workspace that a small kernel fills first (-delta and -lse in log2
-// units, padded to a multiple of 32 rows with -lse = -inf so that padded q rows get p = 0).  Both are stored negated
-// because they start the MFMA chains they are subtracted from: dP^T - delta comes out of the chain, and so does
+// behind the next tile's loads).  The dq pass forms them and leaves them in a workspace for the dk / dv pass (-delta and
+// -lse in log2 units, padded to a multiple of 32 rows with -lse = -inf so that padded q rows get p = 0).  Both are stored
+// negated because they start the MFMA chains they are subtracted from: dP^T - delta comes out of the chain, and so does
 // S^T - lse when the caller's q already carries scale * log2(e) (the factor c is then 1).
 #include <atomic>
 #include <mutex>
