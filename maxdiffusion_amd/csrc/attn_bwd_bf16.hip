@@ -104,6 +104,39 @@ struct BwdArgs {
   float* part2;
 };
 
+// A wave's 32 rows of a gradient, rounded to bf16 and stored as pieces of 128 bytes of a row (8 rows per instruction), 64 columns
+// at a time through `stage` (kStageRows bytes of LDS that nobody else touches any more; 64 columns and not the row, so that
+// eight waves fit the ring).  As the accumulators lie, an instruction wrote 16 bytes of each of 32 rows a whole token apart:
+// a training pass with 32,760 queries x 512 keys x 12 heads 638 -> 622 us, Flux 24 x 4,608 1076 -> 1062, 2 x 1,337 x 32 heads of 64
+// 214 -> 209 (the longer the stream, the smaller the share: 18,900 x 20 heads 13.28 ms both ways).
+constexpr int kStageRowB = 64 * 2 + 16, kStageRows = 32 * kStageRowB;
+template <int ND, bool PADDED>
+__device__ __forceinline__ void store_rows(const f32x16 (&acc)[ND], float mul, __bf16* base, int64_t ss, int row0, int rows, int D, int lane,
+                                           char* stage) {
+  const int l32 = lane & 31, hh = lane >> 5, rr = lane >> 3, cc = lane & 7;
+#pragma unroll
+  for (int d0 = 0; d0 < ND; d0 += 2) {
+    // LDS accesses of one wave execute in order: the reads see the writes above them, and the next round's writes follow
+#pragma unroll
+    for (int db = d0; db < (d0 + 2 < ND ? d0 + 2 : ND); ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        uint2 u;
+        u.x = pack2(acc[db][4 * g] * mul, acc[db][4 * g + 1] * mul);
+        u.y = pack2(acc[db][4 * g + 2] * mul, acc[db][4 * g + 3] * mul);
+        *reinterpret_cast<uint2*>(stage + l32 * kStageRowB + ((db - d0) * 32 + 8 * g + 4 * hh) * 2) = u;
+      }
+    const int col = d0 * 32 + cc * 8;
+    if (col >= (PADDED ? D : ND * 32)) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = row0 + 8 * j + rr;
+      const uint4 v = *reinterpret_cast<const uint4*>(stage + (8 * j + rr) * kStageRowB + cc * 16);
+      if (row < rows) *reinterpret_cast<uint4*>(base + (int64_t)row * ss + col) = v;
+    }
+  }
+}
+
 // MODE 0: dq (entity = q rows, stream = keys); 3: dk and dv in one pass (entity = key rows, stream = q rows).
 // MODE 1 (dk alone) and 2 (dv alone) are the same body with one accumulator set; the library launches 0 and 3.
 // DC != 0: head dims other than HD (a.D, a multiple of 8 up to DC), as in the forward's flat schedule: the layout of HD, the
@@ -546,32 +579,13 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     }
     return;
   }
-  if (row < a.Se) {
-    __bf16* orow = a.out + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_ss + 4 * hh;
-#pragma unroll
-    for (int db = 0; db < ND; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        if (PADDED && db * 32 + 8 * g >= a.D) continue;
-        uint2 u;
-        u.x = pack2(acc[db][4 * g] * osc, acc[db][4 * g + 1] * osc);
-        u.y = pack2(acc[db][4 * g + 2] * osc, acc[db][4 * g + 3] * osc);
-        *reinterpret_cast<uint2*>(orow + db * 32 + 8 * g) = u;
-      }
-    if constexpr (BOTH) {
-      __bf16* orow2 = a.out2 + b * a.o2_sb + h * a.o2_sh + (int64_t)row * a.o2_ss + 4 * hh;
-#pragma unroll
-      for (int db = 0; db < ND; ++db)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          if (PADDED && db * 32 + 8 * g >= a.D) continue;
-          uint2 u;
-          u.x = pack2(acc2[db][4 * g], acc2[db][4 * g + 1]);
-          u.y = pack2(acc2[db][4 * g + 2], acc2[db][4 * g + 3]);
-          *reinterpret_cast<uint2*>(orow2 + db * 32 + 8 * g) = u;
-        }
-    }
-  }
+  static_assert(NW * kStageRows <= 2 * kBStage * 2, "the output staging tiles must fit the ring's LDS");
+  // the lane number once more: the loop has no register for it (spills at head dim 128)
+  const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  __syncthreads();  // every wave has finished reading the ring, and no load into it is in flight: it now stages the outputs
+  char* stage = smem_raw_b + wave * kStageRows;
+  store_rows<ND, PADDED>(acc, osc, a.out + b * a.o_sb + h * a.o_sh, a.o_ss, r0, a.Se, a.D, ln, stage);
+  if constexpr (BOTH) store_rows<ND, PADDED>(acc2, 1.0f, a.out2 + b * a.o2_sb + h * a.o2_sh, a.o2_ss, r0, a.Se, a.D, ln, stage);
 }
 
 template <int MODE, int HD, bool BIAS, bool PRE, int DC>
