@@ -582,6 +582,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   float m = -1e30f, l = 0.f;
   float mc = PRE ? 0.f : BIAS ? m : m * c;  // the rows' reference point in log2 units (its only form with a bias)
   f32x16 negm;                              // PRE (see the pipelined kernel): start value of every score accumulator chain
+  // PRE: the lanes whose row has met no key with a logit above -inf yet, and with that no reference point.  A key with an
+  // infinite channel has such a logit, and a share of the keys may start with 32 of them.
+  [[maybe_unused]] uint64_t fresh = ~0ull;
 #pragma unroll
   for (int i = 0; i < 16; ++i) negm[i] = 0.f;
 
@@ -629,7 +632,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     }
 #pragma unroll
    for (int blk = 0; blk < NB; ++blk) {
-    const bool first = t == 0 && blk == 0;
     // ---- S^T = K.Q^T: one chain of MFMAs; the other waves of the SIMD fill the gaps between them.  A wave in an
     // MFMA phase issues ahead of the SIMD's waves in their softmax phase (1-2 % on short key sequences).
     __builtin_amdgcn_s_setprio(1);
@@ -702,18 +704,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       return lsum;
     };
     float lsum = soft(mc);
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(lsum <= kTrig)) != 0 || (PRE && first), 0)) {
+    if (__builtin_expect((__builtin_amdgcn_ballot_w64(!(lsum <= kTrig)) | (PRE ? fresh : 0ull)) != 0, 0)) {
       float mloc = S[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) mloc = fmaxf(mloc, S[i]);
       mloc = xhalf_max(mloc);
       float alpha;
       if constexpr (PRE) {  // S holds logits minus the old reference: shift them and the chains' start value
-        const float dm = first ? mloc : fmaxf(mloc, 0.f);
-        alpha = first ? 0.f : __builtin_amdgcn_exp2f(-dm);
+        const bool f = (fresh >> lane) & 1;
+        const float dm = f ? (mloc == -INFINITY ? 0.f : mloc) : fmaxf(mloc, 0.f);
+        alpha = f ? 0.f : __builtin_amdgcn_exp2f(-dm);
         mc += dm;
 #pragma unroll
         for (int i = 0; i < 16; ++i) { S[i] -= dm; negm[i] -= dm; }
+        fresh = __builtin_amdgcn_ballot_w64(f && mloc == -INFINITY);
       } else if constexpr (BIAS) {
         const float mnew = fmaxf(mc, mloc * cs);
         alpha = __builtin_amdgcn_exp2f(mc - mnew);

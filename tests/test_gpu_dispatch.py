@@ -293,3 +293,35 @@ def test_keys_split_over_workgroups(dev, lib, B, H, Sq, Skv, D):
     assert rel_l2(to_np(out), ref.detach().cpu().numpy()) <= 6e-3, scale
     for name, got, r in zip(("dq", "dk", "dv"), grads, want):
       assert rel_l2(to_np(got), r.detach().cpu().numpy()) <= 1e-2, (name, scale)
+
+
+@pytest.mark.parametrize("D", [128, 64, 40, 80])
+def test_infinite_keys_at_the_start_of_a_share(dev, lib, D):
+  """Split keys in the form without the multiply: a share (and the whole call) that starts with keys whose logits are all -inf
+  takes its reference point from the first key that has a finite one, however low (odd rows: around -300 in log2 units)."""
+  B, H, Sq, Skv = 1, 4, 126, 2048
+  assert lib.mdattn_host_fwd_workspace_floats(B, H, Sq, Skv, D) > 0
+  gen = torch.Generator(device=dev).manual_seed(D)
+  mk = lambda s: torch.randn((B, s, H, D), generator=gen, device=dev)
+  q, k, v = 0.1 * mk(Sq), mk(Skv), mk(Skv)
+  q[..., 0] = -1 - q[..., 0].abs()
+  q[..., 1] = torch.arange(Sq, device=dev).view(1, Sq, 1) % 2 * 20.0
+  k[..., 1] = -15.0
+  gone = torch.zeros(Skv, dtype=torch.bool, device=dev)
+  gone[:40] = gone[512:1100] = True  # whole first tiles of shares, one share altogether
+  k[:, gone, :, 0] = float("inf")
+  q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=float(np.log(2.0)), heads=H, dim_head=D, dtype=torch.bfloat16)
+  x = [t.reshape(B, -1, H * D).requires_grad_(True) for t in (q, k, v)]
+  out = op.apply_attention(*x)
+  dk, dv = (t.view(B, Skv, H, D) for t in torch.autograd.grad(out, x, torch.ones_like(out))[1:])
+  hf = lambda t: t.double().transpose(1, 2)
+  rk, rv = (hf(t[:, ~gone]).requires_grad_(True) for t in (k, v))
+  ref = (torch.softmax((hf(q) @ rk.transpose(2, 3)) * float(np.log(2.0)), -1) @ rv).transpose(1, 2).reshape(B, Sq, H * D)
+  wk, wv = torch.autograd.grad(ref, (rk, rv), torch.ones_like(ref))
+  assert rel_l2(to_np(out), ref.detach().cpu().numpy()) <= 6e-3
+  with torch.no_grad():
+    assert torch.equal(op.apply_attention(*x), out)
+  assert not dk[:, gone].any() and not dv[:, gone].any()
+  for name, a, b in (("dk", dk, wk), ("dv", dv, wv)):  # bars of the split test
+    assert rel_l2(to_np(a[:, ~gone].transpose(1, 2)), b.cpu().numpy()) <= 1e-2, name
