@@ -481,7 +481,8 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
              g[0].sizes() == at::IntArrayRef({b, s, p.heads, d}));
     const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq);
     Tensor gv = grad_like(g[2], gq);
-    if (reinterpret_cast<uintptr_t>(gv.data_ptr()) & 15) gv = gv.clone(at::MemoryFormat::Preserve);  // the value block took any view
+    // the value block took a view at any address; the copy has gq's strides also where these leave gaps (a clone would close them)
+    if (!aligned(gv)) gv = at::empty_strided(gq.sizes(), gq.strides(), gq.options()).copy_(gv);
     Tensor dx = at::empty({b, s, 3 * n}, x.options());
     Tensor dwq = at::empty({n}, x.options()), dwk = at::empty({n}, x.options()), db = at::empty({3 * n}, x.options());
     const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, 5 * n);

@@ -265,3 +265,29 @@ def test_unpadded_head_dim_at_any_address(dev, rank4):
     out = op.apply_attention(*leaves)
     for a, b in zip((out, *torch.autograd.grad(out, leaves, g)), (want, *want_grads)):
       assert rel_l2(a.detach().float().cpu().numpy(), b.detach().float().cpu().numpy()) <= 8e-3
+
+
+def _fused_prologue(dev, B, S, H, D, bias=True):
+  """Leaves of the fused prologue and a call of it."""
+  N = H * D
+  gen = torch.Generator(device=dev).manual_seed(B + S + H)
+  mk = lambda *s: torch.randn(s, generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True)
+  freqs = torch.polar(torch.ones(S, D // 2, device=dev), torch.rand(S, D // 2, generator=gen, device=dev))[None, None]
+  leaves = (mk(B, S, 3 * N), mk(N), mk(N)) + ((mk(3 * N),) if bias else ())
+  return leaves, lambda: A.hip_norm_rope_qkv(*leaves[:3], freqs, H, bias=leaves[3] if bias else None), gen
+
+
+@pytest.mark.parametrize("gaps,at", [(8, 4), (0, 4), (24, 0)])
+def test_value_gradient_at_any_address(dev, gaps, at):
+  """The value block's gradient as a view that starts `at` columns into wider rows, next to gradients of q and k with the same
+  strides: the result of dense copies, bit for bit (the same values in the same order)."""
+  B, S, H, D = 2, 37, 3, 64
+  leaves, call, gen = _fused_prologue(dev, B, S, H, D)
+  wide = [torch.randn((B, S, H, D + gaps), generator=gen, device=dev).to(torch.bfloat16) for _ in range(2)]
+  edge = torch.randn(B * S * H * (D + gaps) + 8, generator=gen, device=dev).to(torch.bfloat16)
+  gq, gk = (t[..., :D] for t in wide)
+  gv = edge.as_strided(gq.shape, gq.stride(), at)
+  got = torch.autograd.grad(call(), leaves, (gq, gk, gv))
+  want = torch.autograd.grad(call(), leaves, (gq.contiguous(), gk.contiguous(), gv.contiguous()))
+  for a, b in zip(got, want):
+    assert torch.equal(a, b)
