@@ -91,6 +91,26 @@ Tensor grad_like(const Tensor& g, const Tensor& like) {
   if (like.defined()) return x.strides() == like.strides() ? x : at::empty_strided(like.sizes(), like.strides(), x.options()).copy_(x);
   return x.stride(-1) == 1 ? x : x.contiguous();
 }
+// The gradients of a prologue's outputs, all with the strides of the first: the kernels walk them with one set.  A first one
+// that is expanded (stride 0, as the sum over an axis hands it back) is read in place only when the others are too: nothing
+// can be copied into its layout.
+bool repeats(const Tensor& t) {
+  for (int64_t i = 0; i < t.dim(); ++i)
+    if (t.size(i) > 1 && t.stride(i) == 0) return true;
+  return false;
+}
+void grads_alike(std::initializer_list<Tensor*> gs) {
+  Tensor& first = **gs.begin();
+  first = grad_like(first, Tensor());
+  if (repeats(first))
+    for (const Tensor* g : gs)
+      if (g->defined() && (g->strides() != first.strides() || !aligned(*g) || g->scalar_type() != at::kBFloat16)) {
+        first = first.contiguous();
+        break;
+      }
+  for (Tensor* g : gs)
+    if (g->defined() && g != &first) *g = grad_like(*g, first);
+}
 
 // ------------------------------------------------------------------------------------------------ attention
 // A key mask as the kernels take it, in one buffer: the additive bias f32 [B, ceil32(Skv)], then the tile lists
@@ -348,8 +368,8 @@ struct FullrowFn : torch::autograd::Function<FullrowFn> {
     const int64_t b = q.size(0), s = q.size(1), n = q.size(2), d = n / p.heads;
     unpacked(weights_back({&wq, &wk}, n, q) && table_back(sv[4], sv[5], p.kind, s, d, q) && g[0].sizes() == at::IntArrayRef({b, s, p.heads, d}));
     const bool has_k = k.defined();
-    const Tensor gq = grad_like(g[0], Tensor());
-    const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
+    Tensor gq = g[0], gk = has_k ? g[1] : Tensor();
+    grads_alike({&gq, &gk});
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = has_k ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
     Tensor dwq = at::empty({n}, q.options()), dwk = has_k ? at::empty({n}, q.options()) : Tensor();
     const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, (has_k ? 2 : 1) * n);
@@ -412,8 +432,8 @@ struct PerheadFn : torch::autograd::Function<PerheadFn> {
     const int64_t b = q.size(0), s = q.size(1), h = q.size(2), d = q.size(3);
     unpacked(weights_back({&wq, &wk, &wqt, &wkt}, d, q) && table_back(sv[6], sv[7], p.kind, s, d, q));
     const bool has_k = k.defined();
-    const Tensor gq = grad_like(g[0], Tensor());
-    const Tensor gk = has_k ? grad_like(g[1], gq) : Tensor();
+    Tensor gq = g[0], gk = has_k ? g[1] : Tensor();
+    grads_alike({&gq, &gk});
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = has_k ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
     auto dw = [&](bool want) { return want ? at::empty({d}, q.options()) : Tensor(); };
     Tensor dwq = dw(true), dwk = dw(has_k), dwqt = dw(wqt.defined()), dwkt = dw(wkt.defined() && has_k);
@@ -479,8 +499,8 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
     const int64_t b = x.size(0), s = x.size(1), n = x.size(2) / 3, d = n / p.heads;
     unpacked(weights_back({&wq, &wk}, n, x) && weight_ok(bias, 3 * n, x) && table_back(sv[4], sv[5], p.kind, s, d, x) &&
              g[0].sizes() == at::IntArrayRef({b, s, p.heads, d}));
-    const Tensor gq = grad_like(g[0], Tensor()), gk = grad_like(g[1], gq);
-    Tensor gv = grad_like(g[2], gq);
+    Tensor gq = g[0], gk = g[1], gv = g[2];
+    grads_alike({&gq, &gk, &gv});
     // the value block took a view at any address; the copy has gq's strides also where these leave gaps (a clone would close them)
     if (!aligned(gv)) gv = at::empty_strided(gq.sizes(), gq.strides(), gq.options()).copy_(gv);
     Tensor dx = at::empty({b, s, 3 * n}, x.options());
@@ -549,7 +569,8 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     const int64_t b = q.size(0), s = q.size(1), n = q.size(2);
     unpacked(grads[0].sizes() == at::IntArrayRef({b, s, heads, n / heads}) && in_place(wq, at::kFloat, n, q) && (!pair || in_place(wk, at::kFloat, n, q)));
     for (const Tensor& t : {sv[4], sv[5]}) unpacked(!mode || in_place(t, at::kFloat, mode == 1 ? q.numel() : q.numel() / 2, q));
-    const Tensor gq = grad_like(grads[0], Tensor()), gk = pair ? grad_like(grads[1], gq) : Tensor();
+    Tensor gq = grads[0], gk = pair ? grads[1] : Tensor();
+    grads_alike({&gq, &gk});
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = pair ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
     Tensor dwq = at::empty({n}, wq.options()), dwk = pair ? at::empty({n}, wq.options()) : Tensor();
     const int64_t nws = mdattn_norm_rope_bwd_workspace_floats(b * s, (pair ? 2 : 1) * n);

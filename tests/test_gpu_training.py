@@ -291,3 +291,16 @@ def test_value_gradient_at_any_address(dev, gaps, at):
   want = torch.autograd.grad(call(), leaves, (gq.contiguous(), gk.contiguous(), gv.contiguous()))
   for a, b in zip(got, want):
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which", [(0, 1), (0,), (0, 2), (0, 1, 2)])
+def test_expanded_output_gradients(dev, which):
+  """Output gradients expanded over the batch (what a sum over it hands back) beside dense ones."""
+  B, S, H, D = 2, 21, 2, 64
+  leaves, call, gen = _fused_prologue(dev, B, S, H, D)
+  mk = lambda b: torch.randn((b, S, H, D), generator=gen, device=dev).to(torch.bfloat16)
+  gs = [mk(1).expand(B, S, H, D) if i in which else mk(B) for i in range(3)]
+  got = torch.autograd.grad(call(), leaves, gs)
+  want = torch.autograd.grad(call(), leaves, [g.contiguous() for g in gs])
+  for a, b in zip(got, want):
+    assert torch.equal(a, b)
