@@ -246,7 +246,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   [[maybe_unused]] float bias_e = 0.f;
   if constexpr (BIAS && MODE != 0) {
     bias_e = bias_row[erow] * kLog2e;
-    if (!__syncthreads_or(bias_e > -INFINITY)) nt = 0;  // no kept key among this workgroup's: zero gradients
+    if (!__syncthreads_or(bias_e != -INFINITY)) nt = 0;  // only excluded keys in this workgroup: zero gradients (a NaN excludes none)
   }
 
   // ---- direct global -> LDS loads of one stream tile (layouts and lane maps of the forward kernel)

@@ -144,3 +144,17 @@ def test_masked_attention_visits_the_kept_tiles_only(dev, lib, D, skv, kind):
         continue
       rel = float((got.detach().float() - r).norm() / r.norm())
       assert rel <= 6e-3, (name, kind, rel)
+
+
+def test_nan_in_a_key_bias_reaches_the_gradients(dev):
+  """A NaN bias between excluded keys is not taken for another excluded key: the rows' outputs and the gradients of that key
+  are NaN."""
+  B, S, H, D = 1, 70, 2, 128
+  gen = torch.Generator(device=dev).manual_seed(1)
+  q, k, v, g = (torch.randn((B, S, H, D), generator=gen, device=dev).to(torch.bfloat16) for _ in range(4))
+  bias = torch.full((B, 96), float("-inf"), device=dev)
+  bias[0, 3] = float("nan")
+  out, lse = ops.flash_attention(q, k, v, return_lse=True, key_bias=bias)
+  dq, dk, dv = ops.flash_attention_backward(q, k, v, out, g, lse, key_bias=bias)
+  for t in (out, lse, dq, dk[:, 3], dv[:, 3]):
+    assert t.isnan().all()
