@@ -233,8 +233,9 @@ class _HipNormRopeFullrow(torch.autograd.Function):
   @staticmethod
   def forward(ctx, q, k, wq, wk, table, heads, eps, out_layout, q_mul):
     q_out, k_out = ops.norm_rope_fullrow(q, k, wq, wk, table, None, heads, eps, out_layout, q_mul)
-    ctx.save_for_backward(q, k, wq, wk, *_saved_table(table)[:2])
-    ctx.cfg = (heads, eps, q_mul, _saved_table(table)[2])
+    cos, sin, kind = _saved_table(table)
+    ctx.save_for_backward(q, k, wq, wk, cos, sin)
+    ctx.cfg = (heads, eps, q_mul, kind)
     return q_out, k_out
 
   @staticmethod
@@ -254,8 +255,9 @@ class _HipNormRopeQkv(torch.autograd.Function):
   @staticmethod
   def forward(ctx, qkv, bias, wq, wk, table, heads, eps, out_layout, q_mul):
     q_out, k_out, v_out = ops.norm_rope_qkv(qkv, wq, wk, table, None, heads, bias, eps, out_layout, q_mul)
-    ctx.save_for_backward(qkv, bias, wq, wk, *_saved_table(table)[:2])
-    ctx.cfg = (heads, eps, q_mul, _saved_table(table)[2])
+    cos, sin, kind = _saved_table(table)
+    ctx.save_for_backward(qkv, bias, wq, wk, cos, sin)
+    ctx.cfg = (heads, eps, q_mul, kind)
     return q_out, k_out, v_out
 
   @staticmethod
@@ -281,8 +283,9 @@ class _HipNormRopePerhead(torch.autograd.Function):
   @staticmethod
   def forward(ctx, q, k, wq, wk, wq_txt, wk_txt, table, eps, n_txt, out_layout, q_mul):
     q_out, k_out = ops.norm_rope_perhead(q, k, wq, wk, table, None, eps, wq_txt, wk_txt, n_txt, out_layout, q_mul)
-    ctx.save_for_backward(q, k, wq, wk, wq_txt, wk_txt, *_saved_table(table)[:2])
-    ctx.cfg = (eps, n_txt, q_mul, _saved_table(table)[2])
+    cos, sin, kind = _saved_table(table)
+    ctx.save_for_backward(q, k, wq, wk, wq_txt, wk_txt, cos, sin)
+    ctx.cfg = (eps, n_txt, q_mul, kind)
     return q_out, k_out
 
   @staticmethod
@@ -581,7 +584,12 @@ def _table_pair(freqs_cis):
 
 
 def _saved_table(table):
-  return (None, None, 0) if table is None else (table.cos, table.sin, table.kind)
+  """The table as a node keeps it, with its kind: a copy of one that is read in place, which is the caller's own (made in
+  inference mode, or rewritten before the backward)."""
+  if table is None:
+    return None, None, 0
+  copy = lambda t: t.clone() if t is not None and table.kind else t
+  return copy(table.cos), copy(table.sin), table.kind
 
 
 def hip_norm_rope(q, k, wq, wk, freqs_cis, heads: int, eps: float = 1e-6, per_head: bool = False,

@@ -304,6 +304,15 @@ std::optional<Table> as_table(const OptTensor& a, const OptTensor& b, int64_t s,
   t.cos = *a;
   return t;
 }
+// The table as a node keeps it.  One that is read in place belongs to the caller, who may have made it in inference mode (autograd
+// refuses to save such a tensor) or may rewrite it before the backward: a dense copy of it, one launch (two for two planes),
+// where it was split into planes of its own before.  Half planes [S, D/2] were always saved as they are.
+void own_table(Table& t) {
+  if (!t.cos.defined() || t.kind == MDATTN_TABLE_PLANES) return;
+  at::NoGradGuard guard;
+  t.cos = t.cos.clone();
+  if (t.sin.defined()) t.sin = t.sin.clone();
+}
 const float* table_ptr(const Tensor& t) { return t.defined() ? static_cast<const float*>(t.data_ptr()) : nullptr; }
 bool weight_ok(const Tensor& w, int64_t n, const Tensor& ref) { return bf16_on(w, ref) && w.is_contiguous() && w.numel() == n; }
 
@@ -390,11 +399,12 @@ std::optional<variable_list> norm_rope(const Tensor& q, const OptTensor& k_, con
   const int64_t n = q.size(2);
   if (!weight_ok(wq, n, q)) return std::nullopt;
   if (k.defined() && (!bf16_on(k, q) || k.sizes() != q.sizes() || k.strides() != q.strides() || !wk.defined() || !weight_ok(wk, n, q))) return std::nullopt;
-  const auto t = as_table(fa, fb, q.size(1), n / heads, false, q);
+  auto t = as_table(fa, fb, q.size(1), n / heads, false, q);
   if (!t) return std::nullopt;
   const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
   if (wants_grad({&q, &k, &wq, &wk})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
+    own_table(*t);
     return FullrowFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(t->cos), opt(t->sin), p);
   }
   variable_list out = fullrow_run(q, k, wq, wk, t->cos, t->sin, p);
@@ -458,11 +468,12 @@ std::optional<variable_list> norm_rope_perhead(const Tensor& q, const OptTensor&
   if (!weight_ok(wq, d, q) || (wqt.defined() && !weight_ok(wqt, d, q)) || (wkt.defined() && !weight_ok(wkt, d, q))) return std::nullopt;
   if (k.defined() ? (!bf16_on(k, q) || k.sizes() != q.sizes() || k.strides() != q.strides() || !wk.defined() || !weight_ok(wk, d, q)) : wkt.defined())
     return std::nullopt;
-  const auto t = as_table(fa, fb, q.size(1), d, true, q);
+  auto t = as_table(fa, fb, q.size(1), d, true, q);
   if (!t) return std::nullopt;
   const Prologue p{q.size(2), t->kind, n_txt, eps, q_mul, bhsd};
   if (wants_grad({&q, &k, &wq, &wk, &wqt, &wkt})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
+    own_table(*t);
     return PerheadFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(wqt), opt(wkt), opt(t->cos), opt(t->sin), p);
   }
   variable_list out = perhead_run(q, k, wq, wk, wqt, wkt, t->cos, t->sin, p);
@@ -523,10 +534,13 @@ std::optional<variable_list> norm_rope_qkv(const Tensor& x, const Tensor& bias, 
   if (!x.is_cuda() || !bf16_on(x, x) || x.dim() != 3 || x.numel() == 0 || x.stride(2) != 1 || heads <= 0 || x.size(2) % (3 * heads)) return std::nullopt;
   const int64_t n = x.size(2) / 3;
   if (!weight_ok(wq, n, x) || !weight_ok(wk, n, x) || !weight_ok(bias, 3 * n, x)) return std::nullopt;
-  const auto t = as_table(fa, fb, x.size(1), n / heads, false, x);
+  auto t = as_table(fa, fb, x.size(1), n / heads, false, x);
   if (!t) return std::nullopt;
   const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
-  if (wants_grad({&x, &bias, &wq, &wk})) return QkvFn::apply(x, bias, wq, wk, opt(t->cos), opt(t->sin), p);
+  if (wants_grad({&x, &bias, &wq, &wk})) {
+    own_table(*t);
+    return QkvFn::apply(x, bias, wq, wk, opt(t->cos), opt(t->sin), p);
+  }
   variable_list out = qkv_run(x, bias, wq, wk, t->cos, t->sin, p);
   if (out.empty()) return std::nullopt;
   return out;

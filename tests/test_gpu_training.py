@@ -304,3 +304,59 @@ def test_expanded_output_gradients(dev, which):
   want = torch.autograd.grad(call(), leaves, [g.contiguous() for g in gs])
   for a, b in zip(got, want):
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("form,table", [(f, "complex") for f in ("full row", "fused", "fused, no bias", "slices")] +
+                         [(f, t) for f in ("per head", "per head slices") for t in ("complex", "repeated", "matrix")])
+def test_table_made_in_inference_mode_and_rewritten(dev, form, table):
+  """The backward uses the table that the forward read: one made in inference mode (a cache that sampling filled) is taken,
+  and one rewritten in between changes nothing.  `slices`: q and k as column blocks of one buffer, and the fused form
+  without biases, which go through the Python nodes."""
+  B, S, H, D = 1, 35, 2, 64
+  N = H * D
+  leaves, fused, gen = _fused_prologue(dev, B, S, H, D, bias=form != "fused, no bias")
+  per_head = form.startswith("per head")
+  ang = torch.rand(S, D // 2, generator=gen, device=dev)
+  c, s = torch.cos(ang), torch.sin(ang)
+
+  def make():
+    if table == "complex":
+      return (torch.polar(torch.ones_like(ang), ang)[None, None],)
+    if table == "repeated":
+      return c.repeat_interleave(2, 1), s.repeat_interleave(2, 1)
+    return (torch.stack([torch.stack([c, -s], -1), torch.stack([s, c], -1)], -2),)
+
+  qkv, wq, wk = leaves[:3]
+  wide = qkv.detach()
+  q, k = (wide[..., i * N:(i + 1) * N] for i in (0, 1))
+  w = (wq, wk)
+  if per_head:
+    q, k = q.unflatten(2, (H, D)), k.unflatten(2, (H, D))
+    w = tuple(t.detach()[:D].requires_grad_(True) for t in w)
+  if "slices" not in form:
+    q, k = q.contiguous(), k.contiguous()
+  q, k = (t.detach().requires_grad_(True) for t in (q, k))
+
+  def run(rewrite, make):
+    t = make()
+    f = t[0] if len(t) == 1 else t
+    if form.startswith("fused"):
+      x = leaves
+      out = A.hip_norm_rope_qkv(qkv, wq, wk, f, H, bias=leaves[3] if len(leaves) == 4 else None)
+    else:
+      x = (q, k) + w
+      out = A.hip_norm_rope(q, k, *w, f, H, per_head=per_head)
+    if rewrite:
+      for a in t:
+        a.zero_()
+    g = torch.ones((B, S, H, D), dtype=torch.bfloat16, device=dev)
+    return torch.autograd.grad(out, x, (g,) * len(out))
+
+  def sampled():
+    with torch.inference_mode():
+      return make()
+
+  want = run(False, make)
+  for got in (run(False, sampled), run(True, make)):
+    for a, b in zip(got, want):
+      assert torch.equal(a, b)
