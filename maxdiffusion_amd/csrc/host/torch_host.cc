@@ -566,7 +566,9 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     const Tensor k = value(k_), wk = value(wk_), cos = value(cos_), sin = value(sin_);
     variable_list out = rows_run(q, k, wq, wk, cos, sin, p);
     TORCH_CHECK(!out.empty(), "mdattn_norm_rope_rows refused the request");
-    ctx->save_for_backward({q, k, wq, wk, cos, sin});
+    // a weight with a factor is saved as a copy, as its product with the factor was: the caller's may be an inference tensor, or
+    // be updated before the backward
+    ctx->save_for_backward({q, k, p.w_mul == 1.0 ? wq : wq.clone(), wk, cos, sin});
     ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode, (int64_t)q.scalar_type()});
     ctx->saved_data["f"] = c10::List<double>({p.eps, p.w_mul});
     return out;

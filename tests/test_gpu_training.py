@@ -360,3 +360,27 @@ def test_table_made_in_inference_mode_and_rewritten(dev, form, table):
   for got in (run(False, sampled), run(True, make)):
     for a, b in zip(got, want):
       assert torch.equal(a, b)
+
+
+def _ltx2(dev):
+  B, S, H, D = 1, 23, 2, 64
+  gen = torch.Generator(device=dev).manual_seed(6)
+  mk = lambda *s: torch.randn(s, generator=gen, device=dev).requires_grad_(True)
+  g = torch.randn((B, S, H, D), generator=gen, device=dev).to(torch.bfloat16)
+  return mk(B, S, H * D), mk(B, S, H * D), mk(H * D), mk(H * D), H, g
+
+
+def test_ltx2_query_weight_under_a_factor(dev):
+  """With q_mul the backward uses the query weight that the forward read: rewritten in between, or made in inference mode."""
+  q, k, wq, wk, H, g = _ltx2(dev)
+  want = torch.autograd.grad(A.hip_norm_rope_ltx2(q, k, wq, wk, H, q_mul=0.5), (q, k, wq, wk), (g, g))
+  w = wq.detach().clone().requires_grad_(True)
+  out = A.hip_norm_rope_ltx2(q, k, w, wk, H, q_mul=0.5)
+  with torch.no_grad():
+    w.zero_()
+  for a, b in zip(torch.autograd.grad(out, (q, k, w, wk), (g, g)), want):
+    assert torch.equal(a, b)
+  with torch.inference_mode():
+    w = wq.detach().clone()
+  for a, b in zip(torch.autograd.grad(A.hip_norm_rope_ltx2(q, k, w, wk, H, q_mul=0.5), (q, k, wk), (g, g)), (want[0], want[1], want[3])):
+    assert torch.equal(a, b)
