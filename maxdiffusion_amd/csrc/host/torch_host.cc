@@ -1,7 +1,8 @@
 // The torch-side host path in C++: what ops.py and attention_op.py do around a C-ABI call (checks, strides, allocation,
 // the stream, the autograd node), for the inputs that need nothing unusual.  Every function returns None for any other
 // input -- another dtype, a CPU tensor, a shape the kernels refuse -- and the Python path beside the call takes over and
-// raises or converts as it always did; nothing is computed here that the kernels do not compute.
+// raises or converts as it always did; nothing is computed here that the kernels do not compute.  A backward call that a kernel
+// refuses (a gradient at an unaligned address) raises the MdattnError that the Python nodes raise.
 //
 // Why native: a call of the smallest size is host time (4 heads x 126 tokens: 10 us of kernels).  The Python path took
 // 36.7 us for prologue + attention (ctypes' conversion of twenty arguments, four stride structs, the checks), this one
@@ -9,6 +10,7 @@
 // step become 91-108.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <pybind11/stl.h>
 #include <torch/csrc/utils/pybind.h>
@@ -45,10 +47,31 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
     if (t->defined() && t->requires_grad()) return true;
   return false;
 }
-// a backward call that the checks of its forward should have made impossible to fail
 // what a saved-tensor hook hands back is read with the form that the forward checked, or refused
 void unpacked(bool ok) { TORCH_CHECK_VALUE(ok, "a tensor saved for the backward pass came back from its hook with another dtype, shape or layout"); }
-void must(int rc, const char* where) { TORCH_CHECK(rc == MDATTN_OK, where, ": mdattn error ", rc, ": ", mdattn_strerror(rc)); }
+// a backward call: _lib.check(rc, where), whose MdattnError autograd's engine carries back to the thread that waits for it
+void must(int rc, const char* where) {
+  if (rc == MDATTN_OK) return;
+  py::gil_scoped_acquire gil;
+  try {
+    py::module_::import("maxdiffusion_amd._lib").attr("check")(rc, where);
+  } catch (py::error_already_set& e) {
+    e.restore();
+  }
+  python_error err;
+  err.persist();
+  throw err;
+}
+// thrown by a node's forward when a kernel refuses the request, before anything was saved: the Python path takes the call
+struct Refused {};
+template <class F>
+auto unless_refused(F&& apply) -> std::optional<decltype(apply())> {
+  try {
+    return apply();
+  } catch (const Refused&) {
+    return std::nullopt;
+  }
+}
 
 // [B,S,H,D] as the kernels walk it, over a rank-3 [B,S,H*D] or a rank-4 [B,H,S,D] tensor (attention_op._as_bshd)
 struct View {
@@ -153,7 +176,7 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     const View vq = *as_view(q, heads), vk = *as_view(k, heads), vv = *as_view(v, heads);
     Tensor out = at::empty({vq.b, vq.s, vq.h * vq.d}, q.options());
     Tensor lse = at::empty({vq.b, vq.h, vq.s}, q.options().dtype(at::kFloat));
-    must(fwd(q, k, v, vq, vk, vv, out, lse, mask, scale), "mdattn_fwd_bf16");
+    if (fwd(q, k, v, vq, vk, vv, out, lse, mask, scale) != MDATTN_OK) throw Refused{};
     ctx->save_for_backward({q, k, v, out, lse});
     ctx->saved_data["mask"] = mask;  // not for hooks: its tile lists are indices
     ctx->saved_data["heads"] = heads;
@@ -231,7 +254,7 @@ OptTensor flash_autograd(const Tensor& q, const Tensor& k, const Tensor& v, int6
     if (!t->is_non_overlapping_and_dense()) return std::nullopt;  // their gradients take the same strides
   if (!operands(q, k, v, heads, vq, vk, vv) || !walkable(q, vq) || !walkable(k, vk) || !walkable(v, vv)) return std::nullopt;
   if (!flash_args(q, k, v, heads, scale, keep, vq, vk, vv, mask)) return std::nullopt;
-  return FlashFn::apply(q, k, v, opt(mask), heads, scale);
+  return unless_refused([&] { return FlashFn::apply(q, k, v, opt(mask), heads, scale); });
 }
 
 // The registry entry `hip_flash_fp8`: dense bf16 operands of either rank -> [B,Sq,H*D]
@@ -364,7 +387,7 @@ struct FullrowFn : torch::autograd::Function<FullrowFn> {
                                const OptTensor& cos_, const OptTensor& sin_, const Prologue& p) {
     const Tensor k = value(k_), wk = value(wk_), cos = value(cos_), sin = value(sin_);
     variable_list out = fullrow_run(q, k, wq, wk, cos, sin, p);
-    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_fullrow refused the request");
+    if (out.empty()) throw Refused{};
     ctx->save_for_backward({q, k, wq, wk, cos, sin});
     p.save(ctx);
     return out;
@@ -405,7 +428,7 @@ std::optional<variable_list> norm_rope(const Tensor& q, const OptTensor& k_, con
   if (wants_grad({&q, &k, &wq, &wk})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
     own_table(*t);
-    return FullrowFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(t->cos), opt(t->sin), p);
+    return unless_refused([&] { return FullrowFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(t->cos), opt(t->sin), p); });
   }
   variable_list out = fullrow_run(q, k, wq, wk, t->cos, t->sin, p);
   if (out.empty()) return std::nullopt;
@@ -429,7 +452,7 @@ struct PerheadFn : torch::autograd::Function<PerheadFn> {
                                const OptTensor& wkt_, const OptTensor& cos_, const OptTensor& sin_, const Prologue& p) {
     const Tensor k = value(k_), wk = value(wk_), wqt = value(wqt_), wkt = value(wkt_), cos = value(cos_), sin = value(sin_);
     variable_list out = perhead_run(q, k, wq, wk, wqt, wkt, cos, sin, p);
-    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_perhead refused the request");
+    if (out.empty()) throw Refused{};
     ctx->save_for_backward({q, k, wq, wk, wqt, wkt, cos, sin});
     p.save(ctx);
     return out;
@@ -474,7 +497,7 @@ std::optional<variable_list> norm_rope_perhead(const Tensor& q, const OptTensor&
   if (wants_grad({&q, &k, &wq, &wk, &wqt, &wkt})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
     own_table(*t);
-    return PerheadFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(wqt), opt(wkt), opt(t->cos), opt(t->sin), p);
+    return unless_refused([&] { return PerheadFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(wqt), opt(wkt), opt(t->cos), opt(t->sin), p); });
   }
   variable_list out = perhead_run(q, k, wq, wk, wqt, wkt, t->cos, t->sin, p);
   if (out.empty()) return std::nullopt;
@@ -497,7 +520,7 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
                                const OptTensor& sin_, const Prologue& p) {
     const Tensor cos = value(cos_), sin = value(sin_);
     variable_list out = qkv_run(x, bias, wq, wk, cos, sin, p);
-    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_qkv refused the request");
+    if (out.empty()) throw Refused{};
     ctx->save_for_backward({x, bias, wq, wk, cos, sin});
     p.save(ctx);
     return out;
@@ -539,7 +562,7 @@ std::optional<variable_list> norm_rope_qkv(const Tensor& x, const Tensor& bias, 
   const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
   if (wants_grad({&x, &bias, &wq, &wk})) {
     own_table(*t);
-    return QkvFn::apply(x, bias, wq, wk, opt(t->cos), opt(t->sin), p);
+    return unless_refused([&] { return QkvFn::apply(x, bias, wq, wk, opt(t->cos), opt(t->sin), p); });
   }
   variable_list out = qkv_run(x, bias, wq, wk, t->cos, t->sin, p);
   if (out.empty()) return std::nullopt;
@@ -565,7 +588,7 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
                                const OptTensor& sin_, const Rows& p) {
     const Tensor k = value(k_), wk = value(wk_), cos = value(cos_), sin = value(sin_);
     variable_list out = rows_run(q, k, wq, wk, cos, sin, p);
-    TORCH_CHECK(!out.empty(), "mdattn_norm_rope_rows refused the request");
+    if (out.empty()) throw Refused{};
     // a weight with a factor is saved as a copy, as its product with the factor was: the caller's may be an inference tensor, or
     // be updated before the backward
     ctx->save_for_backward({q, k, p.w_mul == 1.0 ? wq : wq.clone(), wk, cos, sin});
@@ -622,7 +645,7 @@ std::optional<variable_list> norm_rope_rows(const Tensor& q, const OptTensor& k_
   const Tensor c = mode ? cos : Tensor(), sn = mode ? sin : Tensor();
   if (wants_grad({&q, &k, &wq, &wk})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
-    return RowsFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(c), opt(sn), p);
+    return unless_refused([&] { return RowsFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(c), opt(sn), p); });
   }
   variable_list out = rows_run(q, k, wq, wk, c, sn, p);
   if (out.empty()) return std::nullopt;

@@ -12,6 +12,7 @@ import torch
 
 import oracle as O
 from helpers import cosine, rel_l2, to_dev_bf16
+from maxdiffusion_amd import _lib
 from maxdiffusion_amd import attention_op as A
 from maxdiffusion_amd import ops
 
@@ -384,3 +385,27 @@ def test_ltx2_query_weight_under_a_factor(dev):
     w = wq.detach().clone()
   for a, b in zip(torch.autograd.grad(A.hip_norm_rope_ltx2(q, k, w, wk, H, q_mul=0.5), (q, k, wk), (g, g)), (want[0], want[1], want[3])):
     assert torch.equal(a, b)
+
+
+def test_a_refused_training_call_raises_the_library_error(dev):
+  """What a kernel refuses in training raises MdattnError with its code: in the forward as without gradients, and in the backward."""
+  mk = lambda *s, dtype=torch.bfloat16: torch.ones(s, dtype=dtype, device=dev).requires_grad_(True)
+  wide, small = mk(1, 4, 65 * 128), mk(1, 4, 2, 32)  # more than 8,192 channels; a head dim that the per-head kernels do not have
+  calls = [lambda: A.hip_norm_rope(wide, None, mk(65 * 128), None, None, 65),
+           lambda: A.hip_norm_rope_qkv(mk(1, 4, 3 * 65 * 128), mk(65 * 128), mk(65 * 128), None, 65, bias=mk(3 * 65 * 128)),
+           lambda: A.hip_norm_rope(small, None, mk(32), None, None, 2, per_head=True),
+           lambda: A.hip_norm_rope_ltx2(wide, None, mk(65 * 128, dtype=torch.float32), None, 65)]
+  for call in calls:
+    with torch.no_grad(), pytest.raises(_lib.MdattnError) as plain:
+      call()
+    with pytest.raises(_lib.MdattnError) as e:
+      call()
+    assert e.value.code == plain.value.code == -2
+
+  q, k, v = (mk(1, 8, 2 * 128) for _ in range(3))
+  off = torch.ones(8 * 256 + 8, dtype=torch.bfloat16, device=dev)[4:-4]  # 8 bytes off a 16-byte address
+  op = A.AttentionOp(attention_kernel="hip_flash", heads=2, dim_head=128, scale=0.1)
+  for out in (op.apply_attention(q, k, v), A.hip_norm_rope(q, None, mk(256), None, None, 2)[0]):
+    with pytest.raises(_lib.MdattnError) as e:
+      out.backward(off.view(out.shape))
+    assert e.value.code == -3
