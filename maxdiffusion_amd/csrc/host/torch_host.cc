@@ -659,12 +659,15 @@ const char kBuildIdRecord[] = "mdattn-build-id:" MDATTN_BUILD_ID;
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("build_id", [] { return std::string(kBuildIdRecord + 16); });
-  m.def("flash", &flash);
-  m.def("flash_autograd", &flash_autograd);
-  m.def("flash_fp8", &flash_fp8);
-  m.def("flash_merge", &flash_merge);
-  m.def("norm_rope", &norm_rope);
-  m.def("norm_rope_perhead", &norm_rope_perhead);
-  m.def("norm_rope_qkv", &norm_rope_qkv);
-  m.def("norm_rope_rows", &norm_rope_rows);
+  // Other Python threads run meanwhile, as they do during a call through ctypes: a launch may wait for room in its queue, an
+  // allocation for memory.
+  using Unlocked = py::call_guard<py::gil_scoped_release>;
+  m.def("flash", &flash, Unlocked());
+  m.def("flash_autograd", &flash_autograd, Unlocked());
+  m.def("flash_fp8", &flash_fp8, Unlocked());
+  m.def("flash_merge", &flash_merge, Unlocked());
+  m.def("norm_rope", &norm_rope, Unlocked());
+  m.def("norm_rope_perhead", &norm_rope_perhead, Unlocked());
+  m.def("norm_rope_qkv", &norm_rope_qkv, Unlocked());
+  m.def("norm_rope_rows", &norm_rope_rows, Unlocked());
 }

@@ -1,6 +1,9 @@
 """`hip_flash` behind the reference-shaped dispatcher: rank-3 and rank-4 inputs, cross-attention,
 compared with a restated `dot_product` registered by the test (the reference's own integration
 test compares flash against dot_product the same way, tests/attention_test.py:90-147)."""
+import sys
+import threading
+import time
 from unittest import mock
 
 import numpy as np
@@ -9,6 +12,7 @@ import torch
 
 import oracle as O
 from helpers import err_stats, rel_l2, to_dev_bf16, to_np
+from maxdiffusion_amd import _lib
 from maxdiffusion_amd import attention_op as A
 
 pytestmark = pytest.mark.gpu
@@ -325,3 +329,34 @@ def test_infinite_keys_at_the_start_of_a_share(dev, lib, D):
   assert not dk[:, gone].any() and not dv[:, gone].any()
   for name, a, b in (("dk", dk, wk), ("dv", dv, wv)):  # bars of the split test
     assert rel_l2(to_np(a[:, ~gone].transpose(1, 2)), b.cpu().numpy()) <= 1e-2, name
+
+
+def test_other_threads_run_during_a_call(dev):
+  """A call leaves the interpreter lock to other threads, as a call through ctypes does.  With a switch interval that never ends a
+  waiting thread gets the lock only where the running one lets go of it, and between the calls below it does not."""
+  x = torch.randn(1, 128, 2 * 128, device=dev).to(torch.bfloat16)
+  flash = _lib.host().flash
+  keep = [flash(x, x, x, 2, 0.1, None, 1.0) for _ in range(3)]  # (nothing is freed inside the loop)
+  go, ran = threading.Lock(), []
+  go.acquire()
+
+  def other():
+    with go:
+      ran.append(True)
+
+  interval = sys.getswitchinterval()
+  t = threading.Thread(target=other)
+  t.start()
+  time.sleep(0.2)  # it waits for `go`
+  sys.setswitchinterval(1000.0)
+  try:
+    go.release()
+    for _ in range(4000):
+      keep.append(flash(x, x, x, 2, 0.1, None, 1.0))
+      if ran:
+        break
+    seen = bool(ran)
+  finally:
+    sys.setswitchinterval(interval)
+    t.join()
+  assert seen
