@@ -594,21 +594,52 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     ctx->save_for_backward({q, k, p.w_mul == 1.0 ? wq : wq.clone(), wk, cos, sin});
     ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode, (int64_t)q.scalar_type()});
     ctx->saved_data["f"] = c10::List<double>({p.eps, p.w_mul});
+    ctx->set_materialize_grads(false);  // an output that the loss does not reach: no gradient for its input and weight
     return out;
   }
+  // A backward through one output frees what both have saved; the other output's is kept beside, with its versions, so that a
+  // second backward through that one runs as it would through a node of its own.
+  static void leave(AutogradContext* ctx, const variable_list& sv, int64_t which) {
+    variable_list left(6);
+    for (const int64_t i : {which, 2 + which, (int64_t)4, (int64_t)5}) left[i] = sv[i];
+    c10::List<int64_t> versions;
+    for (const Tensor& t : left) versions.push_back(!t.defined() || t.is_inference() ? 0 : t._version());
+    ctx->saved_data["left"] = left;
+    ctx->saved_data["versions"] = versions;
+  }
+  static variable_list saved(AutogradContext* ctx, int64_t one, bool pair) {
+    try {
+      return ctx->get_saved_variables();
+    } catch (const c10::Error&) {
+      const auto at = ctx->saved_data.find("left");
+      if (pair || at == ctx->saved_data.end()) throw;
+      const variable_list left = at->second.toTensorVector();
+      const auto versions = ctx->saved_data["versions"].toIntVector();
+      if (!left[one].defined()) throw;
+      for (size_t i = 0; i < left.size(); ++i)
+        TORCH_CHECK(!left[i].defined() || left[i].is_inference() || left[i]._version() == versions[i],
+                    "one of the variables needed for gradient computation has been modified by an inplace operation");
+      ctx->saved_data.erase(at);
+      return left;
+    }
+  }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const auto sv = ctx->get_saved_variables();
-    const Tensor &q = sv[0], &k = sv[1], &wq = sv[2], &wk = sv[3];
+    const bool has[2] = {grads[0].defined(), grads.size() > 1 && grads[1].defined()};
+    if (!has[0] && !has[1]) return variable_list(7);
+    const bool pair = has[0] && has[1];
+    const int one = has[0] ? 0 : 1;  // the tensor of a backward of one
+    const variable_list sv = saved(ctx, one, pair);
+    if (!pair && sv[1 - one].defined()) leave(ctx, sv, 1 - one);
+    const Tensor q = sv[one], k = pair ? sv[1] : Tensor(), wq = sv[2 + one], wk = pair ? sv[3] : Tensor();
     const auto iv = ctx->saved_data["i"].toIntVector();
     const auto fv = ctx->saved_data["f"].toDoubleVector();
     const int64_t heads = iv[0], mode = iv[1];
-    const bool pair = k.defined();
     unpacked(q.is_cuda() && (int64_t)q.scalar_type() == iv[2] && q.dim() == 3 && q.stride(2) == 1 && q.is_non_overlapping_and_dense() &&
              (!pair || (k.get_device() == q.get_device() && k.scalar_type() == q.scalar_type() && k.sizes() == q.sizes() && k.strides() == q.strides())));
     const int64_t b = q.size(0), s = q.size(1), n = q.size(2);
-    unpacked(grads[0].sizes() == at::IntArrayRef({b, s, heads, n / heads}) && in_place(wq, at::kFloat, n, q) && (!pair || in_place(wk, at::kFloat, n, q)));
+    unpacked(grads[one].sizes() == at::IntArrayRef({b, s, heads, n / heads}) && in_place(wq, at::kFloat, n, q) && (!pair || in_place(wk, at::kFloat, n, q)));
     for (const Tensor& t : {sv[4], sv[5]}) unpacked(!mode || in_place(t, at::kFloat, mode == 1 ? q.numel() : q.numel() / 2, q));
-    Tensor gq = grads[0], gk = pair ? grads[1] : Tensor();
+    Tensor gq = grads[one], gk = pair ? grads[1] : Tensor();
     grads_alike({&gq, &gk});
     Tensor dq = at::empty_strided(q.sizes(), q.strides(), q.options()), dk = pair ? at::empty_strided(q.sizes(), q.strides(), q.options()) : Tensor();
     Tensor dwq = at::empty({n}, wq.options()), dwk = pair ? at::empty({n}, wq.options()) : Tensor();
@@ -617,8 +648,9 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     const mdattn_strides sg = strides4(gq);
     must(mdattn_host_norm_rope_rows_bwd(stream(), ptr(q), ptr(k), q.scalar_type() == at::kFloat, ptr(gq), ptr(gk), mut(dq), mut(dk), f32(wq), f32(wk),
                                         f32(dwq), f32(dwk), f32(sv[4]), f32(sv[5]), (int)mode, (int)b, (int)s, (int)heads, (int)(n / heads), (float)fv[0],
-                                        (float)fv[1], q.stride(0), q.stride(1), dq.stride(0), dq.stride(1), &sg, f32(ws), nws),
+                                        one ? 1.0f : (float)fv[1], q.stride(0), q.stride(1), dq.stride(0), dq.stride(1), &sg, f32(ws), nws),
          "mdattn_norm_rope_rows_bwd");
+    if (one) return {Tensor(), dq, Tensor(), dwq, Tensor(), Tensor(), Tensor()};
     return {dq, dk, dwq, dwk, Tensor(), Tensor(), Tensor()};
   }
 };
@@ -643,7 +675,9 @@ std::optional<variable_list> norm_rope_rows(const Tensor& q, const OptTensor& k_
   }
   const Rows p{heads, mode, eps, w_mul};
   const Tensor c = mode ? cos : Tensor(), sn = mode ? sin : Tensor();
-  if (wants_grad({&q, &k, &wq, &wk})) {
+  const bool grad_q = wants_grad({&q, &wq}), grad_k = k.defined() ? wants_grad({&k, &wk}) : grad_q;
+  if (grad_q != grad_k) return std::nullopt;  // one call each: the other output needs no gradient
+  if (grad_q) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
     return unless_refused([&] { return RowsFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(c), opt(sn), p); });
   }

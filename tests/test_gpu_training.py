@@ -409,3 +409,38 @@ def test_a_refused_training_call_raises_the_library_error(dev):
     with pytest.raises(_lib.MdattnError) as e:
       out.backward(off.view(out.shape))
     assert e.value.code == -3
+
+
+def test_ltx2_gradient_of_the_query_alone(dev):
+  """A loss that reaches one of q and k leaves the other and its weight without a gradient, and operands that need none get none."""
+  q, k, wq, wk, H, g = _ltx2(dev)
+  both = torch.autograd.grad(A.hip_norm_rope_ltx2(q, k, wq, wk, H, q_mul=0.5), (q, k, wq, wk), (g, g))
+  for i in (0, 1):
+    got = torch.autograd.grad(A.hip_norm_rope_ltx2(q, k, wq, wk, H, q_mul=0.5)[i], (q, k, wq, wk), g, allow_unused=True)
+    for j in range(4):
+      assert torch.equal(got[j], both[j]) if j % 2 == i else got[j] is None
+  qo, ko = A.hip_norm_rope_ltx2(q, k.detach(), wq, wk.detach(), H)
+  assert qo.requires_grad and not ko.requires_grad
+  qo, ko = A.hip_norm_rope_ltx2(q.detach(), k, wq.detach(), wk, H)
+  assert ko.requires_grad and not qo.requires_grad
+
+
+def test_ltx2_backward_through_the_query_then_the_key(dev):
+  """Two losses with a backward each, as through two nodes: the second one takes what the first left, once, and refuses it when
+  it was rewritten."""
+  q, k, wq, wk, H, g = _ltx2(dev)
+  both = torch.autograd.grad(A.hip_norm_rope_ltx2(q, k, wq, wk, H, q_mul=0.5), (q, k, wq, wk), (g, g))
+  for order in ((0, 1), (1, 0)):
+    out = A.hip_norm_rope_ltx2(q, k, wq, wk, H, q_mul=0.5)
+    for i in order:
+      for got, want in zip(torch.autograd.grad(out[i], (q, wq) if i == 0 else (k, wk), g), both[i::2]):
+        assert torch.equal(got, want)
+    for i in order:
+      with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out[i], (q, wq) if i == 0 else (k, wk), g)
+  out = A.hip_norm_rope_ltx2(q, k, wq, wk, H)
+  torch.autograd.grad(out[0], q, g)
+  with torch.no_grad():
+    k.mul_(2)
+  with pytest.raises(RuntimeError, match="inplace"):
+    torch.autograd.grad(out[1], k, g)
