@@ -303,78 +303,94 @@ extern "C" int mdattn_key_mask_bias(void* stream, const void* keep, float* bias,
 // ------------------------------------------------------------------------------- key mask -> bias and tile lists
 namespace mdattn {
 // The bias of key_mask_bias_kernel (masked value -inf) together with the lists of key tiles that hold a kept key, for
-// tiles of 32 and of 64 keys: a masked attention then costs what its kept keys cost.  One workgroup per batch element; a
-// lane takes two 32-key tiles (one 64-key tile) per turn, ranks come from a ballot per wave and the waves' sums.  Masked calls
-// before (every tile visited, the bias added to every logit) and with the lists: 500 of 2,048 keys x 2,048 queries x 20
-// heads 59 -> 23 us; 3,900 of 4,096 keys 185 -> 170 us at head dim 128, 123 -> 106 us at 64 (x 2 x 10 heads).
+// tiles of 32 and of 64 keys: a masked attention then costs what its kept keys cost.  A workgroup takes kTileSlice tiles of 64
+// keys of one batch element, as many as its waves load in one trip; where its entries start it finds by counting the kept tiles
+// of all the slices before it, 64 bytes per lane (one workgroup per element took one slice after the other: 42 us for 75,600
+// keys, now 5.0; 4.9 and 5.0 us for 4,096).  Masked calls before (every tile visited, the bias added to every logit) and with the
+// lists: 500 of 2,048 keys x 2,048 queries x 20 heads 59 -> 23 us; 3,900 of 4,096 keys 185 -> 170 us at head dim 128, 123 ->
+// 106 us at 64 (x 2 x 10 heads).
+constexpr int kTileSlice = 128;
 __global__ __launch_bounds__(1024) void key_tiles_kernel(const uint8_t* __restrict__ keep, float* __restrict__ bias, int* __restrict__ tiles,
-                                                         int Skv, int64_t bias_stride, int sb32, int sb64) {
-  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+                                                         int Skv, int64_t bias_stride, int B, int slices, int sb32, int sb64) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x / slices, slice = blockIdx.x - b * slices;
   const uint8_t* kb = keep + (int64_t)b * Skv;
   float* bb = bias + b * bias_stride;
   int* l32 = tiles + (int64_t)b * sb32;
-  int* l64 = tiles + (int64_t)gridDim.x * sb32 + (int64_t)b * sb64;
-  __shared__ unsigned char kept[2][1024];  // keys kept in each half of a lane's tile
-  __shared__ int sums[2][16];
-  const int n64 = (Skv + 63) / 64;
-  int base32 = 0, base64 = 0;
-  for (int t0 = 0; t0 < n64; t0 += 1024) {
-    for (int h = tid; h < 2048; h += 1024) reinterpret_cast<unsigned char*>(kept)[h] = 0;
-    __syncthreads();
-    // the 1024 tiles' keys, neighbouring lanes on neighbouring keys: a wave covers one 64-key tile per trip
-    const int last = t0 + 1024 < n64 ? t0 + 1024 : n64;
-    for (int t = t0 + wave; t < last; t += 16 * 8) {
-      bool k[8];  // eight loads in flight
+  int* l64 = tiles + (int64_t)B * sb32 + (int64_t)b * sb64;
+  __shared__ int kept[2][kTileSlice];  // keys kept in each half of a tile
+  __shared__ int sums[2][16], mine[2][kTileSlice / 64];
+  const int n64 = (Skv + 63) / 64, t0 = slice * kTileSlice, last = t0 + kTileSlice < n64 ? t0 + kTileSlice : n64;
+
+  // this slice's keys, neighbouring lanes on neighbouring keys: a wave covers one tile per load, eight loads in flight
+  // (the address of a key past the end is that of the last one: under a condition the loads would wait for one another)
+  uint8_t k[kTileSlice / 16];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int key = (t + 16 * i) * 64 + lane;
-        k[i] = key < Skv && kb[key];
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int ti = t + 16 * i, key = ti * 64 + lane;
-        if (ti >= last) break;
-        if (key < bias_stride) bb[key] = k[i] ? 0.f : -INFINITY;
-        const unsigned long long m = __builtin_amdgcn_ballot_w64(k[i]);
-        if (lane == 0) {
-          kept[0][ti - t0] = (unsigned char)__popc((unsigned)m);
-          kept[1][ti - t0] = (unsigned char)__popc((unsigned)(m >> 32));
-        }
-      }
-    }
-    __syncthreads();
-    const int t = t0 + tid;
-    const int k0 = kept[0][tid], k1 = kept[1][tid];
-    const int n32 = (k0 > 0) + (k1 > 0), any = k0 + k1 > 0;
-    // exclusive ranks: of the first / second half's tile among the 32-key tiles, of the tile among the 64-key tiles
-    const unsigned long long lt = (1ull << lane) - 1;
-    const unsigned long long b0 = __builtin_amdgcn_ballot_w64(k0 > 0), b1 = __builtin_amdgcn_ballot_w64(k1 > 0), ba = __builtin_amdgcn_ballot_w64(any);
-    int r32 = __popcll(b0 & lt) + __popcll(b1 & lt), r64 = __popcll(ba & lt);
-    if (lane == 0) {
-      sums[0][wave] = __popcll(b0) + __popcll(b1);
-      sums[1][wave] = __popcll(ba);
-    }
-    __syncthreads();
-    int tot32 = 0, tot64 = 0;
-    for (int w = 0; w < 16; ++w) {
-      if (w < wave) { r32 += sums[0][w]; r64 += sums[1][w]; }
-      tot32 += sums[0][w];
-      tot64 += sums[1][w];
-    }
-    const int left = Skv - t * 64;  // keys of this tile that exist
-    if (n32) {
-      const int e0 = left < 32 ? left : 32, e1 = left - 32 < 32 ? left - 32 : 32;
-      if (k0 > 0) l32[1 + base32 + r32] = 4 * t + (k0 < e0);
-      if (k1 > 0) l32[1 + base32 + r32 + (k0 > 0)] = 4 * t + 2 + (k1 < e1);
-      l64[1 + base64 + r64] = 2 * t + (k0 + k1 < (left < 64 ? left : 64));
-    }
-    base32 += tot32;
-    base64 += tot64;
-    __syncthreads();  // kept and sums are rewritten
+  for (int i = 0; i < kTileSlice / 16; ++i) {
+    const int64_t key = (int64_t)(t0 + wave + 16 * i) * 64 + lane;
+    k[i] = kb[key < Skv ? key : Skv - 1];
   }
-  if (tid == 0) {
-    l32[0] = base32;
-    l64[0] = base64;
+  // the tiles in front of it, all of 64 keys
+  typedef unsigned u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+  int c32 = 0, c64 = 0;
+  for (int t = tid; t - lane < t0; t += 1024) {
+    unsigned h0 = 0, h1 = 0;
+    if (t < t0) {
+      const u32x4_any* p = reinterpret_cast<const u32x4_any*>(kb + (int64_t)t * 64);
+      const u32x4_any w = p[0] | p[1], x = p[2] | p[3];
+      h0 = w.x | w.y | w.z | w.w;
+      h1 = x.x | x.y | x.z | x.w;
+    }
+    const unsigned long long b0 = __builtin_amdgcn_ballot_w64(h0 != 0), b1 = __builtin_amdgcn_ballot_w64(h1 != 0);
+    c32 += __popcll(b0) + __popcll(b1);
+    c64 += __popcll(b0 | b1);
+  }
+  if (lane == 0) { sums[0][wave] = c32; sums[1][wave] = c64; }
+#pragma unroll
+  for (int i = 0; i < kTileSlice / 16; ++i) {
+    const int at = wave + 16 * i;
+    const int64_t key = (int64_t)(t0 + at) * 64 + lane;
+    const bool kp = key < Skv && k[i];
+    if (key < bias_stride) bb[key] = kp ? 0.f : -INFINITY;
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(kp);
+    if (lane == 0) {
+      kept[0][at] = __popc((unsigned)m);
+      kept[1][at] = __popc((unsigned)(m >> 32));
+    }
+  }
+  __syncthreads();
+  // a lane per tile.  Exclusive ranks: of the first / second half's tile among the 32-key tiles, of the tile among the 64-key tiles
+  const int t = t0 + tid;
+  const int k0 = tid < kTileSlice ? kept[0][tid] : 0, k1 = tid < kTileSlice ? kept[1][tid] : 0;
+  const unsigned long long lt = (1ull << lane) - 1;
+  const unsigned long long b0 = __builtin_amdgcn_ballot_w64(k0 > 0), b1 = __builtin_amdgcn_ballot_w64(k1 > 0);
+  if (lane == 0 && wave < kTileSlice / 64) {
+    mine[0][wave] = __popcll(b0) + __popcll(b1);
+    mine[1][wave] = __popcll(b0 | b1);
+  }
+  __syncthreads();
+  if (tid >= kTileSlice) return;
+  int r32 = __popcll(b0 & lt) + __popcll(b1 & lt), r64 = __popcll((b0 | b1) & lt), n32 = 0, n = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) { n32 += sums[0][w]; n += sums[1][w]; }
+  r32 += n32;
+  r64 += n;
+#pragma unroll
+  for (int w = 0; w < kTileSlice / 64; ++w) {
+    if (w < wave) { r32 += mine[0][w]; r64 += mine[1][w]; }
+    n32 += mine[0][w];
+    n += mine[1][w];
+  }
+  const int left = Skv - t * 64;  // keys of this tile that exist
+  if (k0 + k1 > 0) {
+    const int e0 = left < 32 ? left : 32, e1 = left - 32 < 32 ? left - 32 : 32;
+    if (k0 > 0) l32[1 + r32] = 4 * t + (k0 < e0);
+    if (k1 > 0) l32[1 + r32 + (k0 > 0)] = 4 * t + 2 + (k1 < e1);
+    l64[1 + r64] = 2 * t + (k0 + k1 < (left < 64 ? left : 64));
+  }
+  if (last == n64 && tid == 0) {
+    l32[0] = n32;
+    l64[0] = n;
   }
 }
 }  // namespace mdattn
@@ -385,7 +401,9 @@ extern "C" int64_t mdattn_host_key_tiles_ints(int B, int Skv) {
 
 extern "C" int mdattn_host_key_tiles(void* stream, const void* keep, float* bias, int* tiles, int B, int Skv, int64_t bias_stride) {
   if (!keep || !bias || !tiles || B <= 0 || Skv <= 0 || bias_stride < Skv || bias_stride % 32) return MDATTN_E_BADARG;
-  MDATTN_LAUNCH(mdattn::key_tiles_kernel, dim3(B), dim3(1024), 0, (hipStream_t)stream, (const uint8_t*)keep, bias, tiles, Skv, bias_stride,
-                key_tiles_ints(Skv, 32), key_tiles_ints(Skv, 64));
+  const int slices = (int)(((int64_t)Skv + 64 * mdattn::kTileSlice - 1) / (64 * mdattn::kTileSlice));
+  if ((int64_t)B * slices > 0x7FFFFFFF) return MDATTN_E_UNSUPPORTED;
+  MDATTN_LAUNCH(mdattn::key_tiles_kernel, dim3(B * slices), dim3(1024), 0, (hipStream_t)stream, (const uint8_t*)keep, bias, tiles, Skv, bias_stride, B,
+                slices, key_tiles_ints(Skv, 32), key_tiles_ints(Skv, 64));
   return mdattn::launch_status();
 }

@@ -3,6 +3,7 @@
 Oracle: dense softmax with the masked keys excluded; rows without a kept key return 0
 (models/attention_flax.py:1552-1554).  Hand fixtures follow the reference's own mask tests
 (tests/ltx2/test_attention_ltx2.py:38-116)."""
+import ctypes
 import math
 
 import numpy as np
@@ -158,3 +159,35 @@ def test_nan_in_a_key_bias_reaches_the_gradients(dev):
   dq, dk, dv = ops.flash_attention_backward(q, k, v, out, g, lse, key_bias=bias)
   for t in (out, lse, dq, dk[:, 3], dv[:, 3]):
     assert t.isnan().all()
+
+
+@pytest.mark.parametrize("B,skv", [(1, 1), (3, 33), (2, 8191), (3, 8192), (2, 8193), (2, 24631), (1, 75600)])
+@pytest.mark.parametrize("density", [1.0, 0.02, 0.0])
+def test_key_tile_lists(dev, lib, B, skv, density):
+  """The bias and the tile lists of a mask, against numpy: one slice of 8,192 keys and several, rows at any address."""
+  rng = np.random.default_rng(skv)
+  keep = rng.random((B, skv)) < density
+  keep[B - 1, skv // 2:] = density > 0.5 and skv % 2 == 1  # an element that ends in dropped (or mixed and kept) tiles
+  cols, ints = (skv + 31) // 32 * 32, lib.mdattn_host_key_tiles_ints
+  ints.restype = ctypes.c_int64
+  n = ints(B, skv)
+  bias = torch.full((B, cols), 7.0, device=dev)
+  tiles = torch.full((n,), -1, dtype=torch.int32, device=dev)
+  kd = torch.from_numpy(keep).to(dev)
+  rc = lib.mdattn_host_key_tiles(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), ctypes.c_void_p(kd.data_ptr()), ctypes.c_void_p(bias.data_ptr()),
+                                 ctypes.c_void_p(tiles.data_ptr()), B, skv, ctypes.c_int64(cols))
+  assert rc == 0
+  want = np.full((B, cols), -np.inf, np.float32)
+  want[:, :skv][keep] = 0
+  assert np.array_equal(bias.cpu().numpy(), want)
+  got, at = tiles.cpu().numpy(), 0
+  for ts in (32, 64):
+    nt = (skv + ts - 1) // ts
+    for b in range(B):
+      kept = np.add.reduceat(keep[b].astype(int), np.arange(0, skv, ts))
+      size = np.minimum(ts, skv - ts * np.arange(nt))
+      entries = [2 * t + int(kept[t] < size[t]) for t in range(nt) if kept[t]]
+      assert got[at] == len(entries) and list(got[at + 1:at + 1 + len(entries)]) == entries
+      assert (got[at + 1 + len(entries):at + 1 + nt] == -1).all()
+      at += 1 + nt
+  assert at == n
