@@ -477,7 +477,13 @@ constexpr int kSlotsS = 3;
 // infinite key would make NaN of its logits.)  A copy of q, k and v padded to 64 or 128
 // columns in front, and one of out cut back behind, are gone: 62 -> 16 us for 16 x 257 tokens x 16 heads of 80 (64 -> 16 us of
 // kernels and the four copies' launches), 626 -> 449 us for 8,192 tokens x 20 heads of 80.
-template <int NW, bool BIAS, int HD, bool PRE, int DC = 0>
+// BIAS: kNoBias; kKeyBias, an additive bias per key, every tile visited; kKeyMask, a keep-mask as a bias of 0 and -inf with the list of
+// the tiles that hold a kept key.  In one form for both, the list and the choice per tile cost an additive bias 10 to 20 %, and a
+// mask with a dropped key in every tile as much: 4,096 keys and queries x 10 heads 109 us before the lists, 122 in one form, 110 now
+// (nothing dropped: 109, 105, 100); 512 queries x 75,600 keys x 40 heads 1,575, 1,929, 1,693 (1,575, 1,647, 1,505).  There a SIMD has one
+// wave, and what stands between two tiles is the time.
+enum { kNoBias, kKeyBias, kKeyMask };
+template <int NW, int BIAS, int HD, bool PRE, int DC = 0>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 3, HD == 64 ? 4 : 3))) void attn_fwd_bf16_flat_kernel(AttnArgs a) {
   constexpr bool PADDED = DC != 0;
   constexpr int NJ = (PADDED ? DC : HD) / 16;                    // QK MFMAs per 32-key tile
@@ -517,9 +523,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   const __bf16* kp = a.k + b * a.k_sb + h * a.k_sh + kv0 * a.k_ss;
   const __bf16* vp = a.v + b * a.v_sb + h * a.v_sh + kv0 * a.v_ss;
   const int q0 = qt * BM + wave * 32;
-  [[maybe_unused]] TileList tl{BIAS && a.tiles ? a.tiles + (int64_t)b * a.tiles_sb : nullptr};
+  [[maybe_unused]] TileList tl{BIAS == kKeyMask ? a.tiles + (int64_t)b * a.tiles_sb : nullptr};
   int nt = (Skv + TS - 1) / TS;  // tiles visited; with a list, 0 when every key is excluded
-  if constexpr (BIAS) nt = tl.count(nt);
+  if constexpr (BIAS == kKeyMask) nt = tl.count(nt);
   const float c = a.c;
   const float* bias_row = BIAS ? a.bias + b * a.bias_sb : nullptr;
   [[maybe_unused]] const int bias_cols = (a.Skv + 31) / 32 * 32;  // entries the caller's bias rows are sure to hold
@@ -544,23 +550,33 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   const unsigned kofs = (unsigned)(grow * (int)a.k_ss + kcol) * 2u;
   const unsigned vofs = (unsigned)(grow * (int)a.v_ss + vcol) * 2u;
   const unsigned smem_addr = lds_addr_of(smem);
-  auto dma = [&](int slot, int kt) __attribute__((always_inline)) {
+  // the first rows of this wave's row groups of tile kt (a row number and a stride below 2^23 multiply without their signs)
+  struct Rows {
+    const __bf16 *k, *v;
+  };
+  auto rows = [&](int kt) __attribute__((always_inline)) -> Rows {
+    if constexpr (BIAS == kKeyMask) {
+      const uint64_t r = (unsigned)(kt * TS + RPI * wave);
+      return {kp + r * (unsigned)a.k_ss, vp + r * (unsigned)a.v_ss};
+    } else {
+      return {kp + (int64_t)(kt * TS + RPI * wave) * a.k_ss, vp + (int64_t)(kt * TS + RPI * wave) * a.v_ss};
+    }
+  };
+  auto dma = [&](int slot, int kt, const Rows& at) __attribute__((always_inline)) {
     const unsigned Ks = smem_addr + (unsigned)(slot * STAGE) * 2u;
     const unsigned Vs = Ks + KTILE * 2u;
     // every wave fetches the same values to the same place (a load more per wave and tile, counted in the loop's
     // s_waitcnt): lane l and lane l + 32 the bias of key l of the tile
     if constexpr (BIAS) {  // (a 64-key tile may reach past the padded bias row, whose length is a multiple of 32)
-      int col = kt * TS + (TS == 64 ? lane : l32);
+      int col = (BIAS == kKeyMask || kt < nt ? kt : nt - 1) * TS + (TS == 64 ? lane : l32);  // the loads run past the end
       col = col < bias_cols ? col : bias_cols - 1;
       lds_dma4(bias_row, (unsigned)col * 4u, Ks + TILES * 2u);
     }
     if (kt * TS + TS <= Skv) {
-      const __bf16* kt0 = kp + (int64_t)(kt * TS + RPI * wave) * a.k_ss;
-      const __bf16* vt0 = vp + (int64_t)(kt * TS + RPI * wave) * a.v_ss;
 #pragma unroll
       for (int i = 0; i < GPW; ++i) {
-        dma_k(kt0 + (int64_t)(RPI * NW * i) * a.k_ss, kofs, Ks + (unsigned)((wave + NW * i) * KGS) * 2u);
-        lds_dma16(vt0 + (int64_t)(RPI * NW * i) * a.v_ss, vofs, Vs + (unsigned)((wave + NW * i) * VGS) * 2u);
+        dma_k(at.k + (int64_t)(RPI * NW * i) * a.k_ss, kofs, Ks + (unsigned)((wave + NW * i) * KGS) * 2u);
+        lds_dma16(at.v + (int64_t)(RPI * NW * i) * a.v_ss, vofs, Vs + (unsigned)((wave + NW * i) * VGS) * 2u);
       }
     } else {
 #pragma unroll
@@ -580,8 +596,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 #pragma unroll
     for (int i = 0; i < 16; ++i) O[db][i] = 0.f;
   float m = -1e30f, l = 0.f;
-  float mc = PRE ? 0.f : BIAS ? m : m * c;  // the rows' reference point in log2 units (its only form with a bias)
-  f32x16 negm;                              // PRE (see the pipelined kernel): start value of every score accumulator chain
+  // a biased logit is in log2 units before the exponent, the others take the factor in the exponent's FMA
+  const float cs = BIAS == kKeyBias ? 1.0f : c;
+  float mc = PRE ? 0.f : m * cs;  // the rows' reference point in log2 units
+  f32x16 negm;                    // PRE (see the pipelined kernel): start value of every score accumulator chain
   // PRE: the lanes whose row has met no key with a logit above -inf yet, and with that no reference point.  A key with an
   // infinite channel has such a logit, and a share of the keys may start with 32 of them.
   [[maybe_unused]] uint64_t fresh = ~0ull;
@@ -615,8 +633,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // waits for every read right before its MFMA.
   constexpr int LA = HD == 128 ? MDATTN_FLAT_LA128 : 0;
   constexpr int FPB = NJ + 2 * ND, NFRAG = NB * FPB;
-  // t: position in the sequence of visited tiles; kt: the tile itself; mixed: it holds keys with a bias
-  auto tile = [&](int t, int kt, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {  // slot: int or integral_constant
+  // kt: the tile; mixed (kKeyMask): it holds excluded keys; slot: int or integral_constant
+  auto tile = [&](int kt, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {
     const __bf16* base = smem + slot * STAGE;
     constexpr int kBlk = 32 * 64;  // a 32-key block of a head-dim-64 tile: 32 rows of 64 elements, in K and in V
     auto frag = [&](int n) __attribute__((always_inline)) {
@@ -650,15 +668,22 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
         S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[j], (PRE && j == 0) ? negm : S, 0, 0, 0);
       }
     }
-    // the logits of a tile with a bias are brought to log2 units here (scale folded, bias added); those of the others take
-    // the factor in the exponent's FMA
-    const float cs = BIAS && mixed ? 1.0f : c;
-    if (BIAS && mixed) {
+    auto bias4 = [&](int g) __attribute__((always_inline)) {
+      return *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base + TILES) + 32 * blk + 8 * g + 4 * hh);
+    };
+    if constexpr (BIAS == kKeyBias) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const f32x4 bv = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base + TILES) + 32 * blk + 8 * g + 4 * hh);
+        const f32x4 bv = bias4(g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[4 * g + e] = __builtin_fmaf(S[4 * g + e], c, bv[e] * kLog2e);
+      }
+    } else if (BIAS == kKeyMask && mixed) {  // 0 or -inf: in any unit
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 bv = bias4(g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[4 * g + e] += bv[e];
       }
     }
     if constexpr (decltype(masked)::value) {
@@ -718,10 +743,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 #pragma unroll
         for (int i = 0; i < 16; ++i) { S[i] -= dm; negm[i] -= dm; }
         fresh = __builtin_amdgcn_ballot_w64(f && mloc == -INFINITY);
-      } else if constexpr (BIAS) {
-        const float mnew = fmaxf(mc, mloc * cs);
-        alpha = __builtin_amdgcn_exp2f(mc - mnew);
-        mc = mnew;
       } else {
         const float mnew = fmaxf(m, mloc);
         alpha = __builtin_amdgcn_exp2f((m - mnew) * cs);
@@ -760,17 +781,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // the wave fetches its 32 rows as a K-shaped tile with the same direct global->LDS loads (whole 256-byte rows per
   // 16 lanes), into a staging area behind ring slot 0 (which receives key tile 0 meanwhile), and reads the fragments
   // with the K fragment offsets.  Each wave stages and reads only its own rows.
-  // The tile at position t of the sequence as tile * 2 + mixed, and its loads; without a list position and tile are the same
-  // (positions past the end load rows that are not used).
+  // kKeyMask: the visited tile at position t as tile * 2 + mixed (positions past the end load rows that are not used)
   [[maybe_unused]] auto entry = [&](int t) __attribute__((always_inline)) { return tl.at(t < nt ? t : nt - 1, nt, lane); };
   [[maybe_unused]] int ec = 0, en = 0;  // entries of the tile being worked on and, in a 3-slot ring, of the next
-  if constexpr (BIAS) {
+  if constexpr (BIAS == kKeyMask) {
     if (nt > 0) {
       ec = entry(0);
-      dma(0, ec >> 1);
+      dma(0, ec >> 1, rows(ec >> 1));
     }
   } else {
-    dma(0, 0);
+    dma(0, 0, rows(0));
   }
   {
     const unsigned Qs = smem_addr + (unsigned)(STAGE + wave * QTILE) * 2u;
@@ -797,27 +817,38 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   }
   // SLOTS - 1 tiles are requested ahead of the one being worked on
   static_assert(SLOTS == 2 || SLOTS == 3, "one tile ahead, or two");
-  if constexpr (SLOTS == 3 && BIAS) {
+  if constexpr (SLOTS == 3 && BIAS == kKeyMask) {
     if (nt > 0) {
       en = entry(1);
-      dma(1, en >> 1);
+      dma(1, en >> 1, rows(en >> 1));
     }
   } else if constexpr (SLOTS == 3) {
-    dma(1, 1);
+    dma(1, 1, rows(1));
+  }
+  // kKeyMask: the tile to be requested next and its rows, known before the barrier: their arithmetic behind it would hold up the
+  // request
+  [[maybe_unused]] int ef = 0;
+  [[maybe_unused]] Rows rf{kp, vp};
+  if constexpr (BIAS == kKeyMask) {
+    if (nt > 1) {
+      ef = entry(SLOTS - 1);
+      rf = rows(ef >> 1);
+    }
   }
   auto step = [&](int t, auto slot, int fill) __attribute__((always_inline)) {
     // vmcnt: this wave's share of tile t has landed (the SLOTS - 2 tiles requested after it may still be in flight)
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((SLOTS - 2) * (2 * GPW + (BIAS ? 1 : 0))));
     __syncthreads();                                  // ... and everyone's; slot `fill` (tile t-1) is free
-    if constexpr (BIAS) {
-      const int ef = entry(t + SLOTS - 1);
-      dma(fill, ef >> 1);
-      tile(t, ec >> 1, ec & 1, slot, std::false_type{});
+    if constexpr (BIAS == kKeyMask) {
+      dma(fill, ef >> 1, rf);
+      tile(ec >> 1, ec & 1, slot, std::false_type{});
       ec = SLOTS == 3 ? en : ef;
       en = ef;
+      ef = entry(t + SLOTS);
+      rf = rows(ef >> 1);
     } else {
-      dma(fill, t + SLOTS - 1);
-      tile(t, t, false, slot, std::false_type{});
+      dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
+      tile(t, false, slot, std::false_type{});
     }
   };
   if constexpr (HD == 64) {
@@ -839,10 +870,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
-  if constexpr (BIAS) {
-    if (nt > 0) tile(nt - 1, ec >> 1, ec & 1, (nt - 1) % SLOTS, std::true_type{});
+  if constexpr (BIAS == kKeyMask) {
+    if (nt > 0) tile(ec >> 1, ec & 1, (nt - 1) % SLOTS, std::true_type{});
   } else {
-    tile(nt - 1, nt - 1, false, (nt - 1) % SLOTS, std::true_type{});
+    tile(nt - 1, false, (nt - 1) % SLOTS, std::true_type{});
   }
 
   if (!BIAS && a.part) {
@@ -856,7 +887,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   }
 }
 
-template <int NW, bool BIAS, int HD = 128, int DC = 0>
+template <int NW, int BIAS, int HD = 128, int DC = 0>
 static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   constexpr int BM = NW * 32;
   // the ring, or ring slot 0 plus one K-shaped Q staging tile per wave, whichever is larger
@@ -962,7 +993,7 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
 }
 
 static int dispatch_fwd(hipStream_t st, const AttnArgs& a, int B, int Sq, int Skv, int D) {
-  if (D == 64) return launch_flat<4, false, 64>(st, a, B);  // head dim 64: the flat schedule only
+  if (D == 64) return launch_flat<4, kNoBias, 64>(st, a, B);  // head dim 64: the flat schedule only
 
   // Two schedules.  The software-pipelined kernel (8 waves x 32 query rows, two waves per SIMD) is the faster one
   // on long key sequences; its prologue and epilogue (three tiles of look-ahead, one virtual block at each end)
@@ -977,13 +1008,13 @@ static int dispatch_fwd(hipStream_t st, const AttnArgs& a, int B, int Sq, int Sk
   switch (variant) {
     case 1: return launch_fwd<8>(st, a, B);
     case 2: return launch_fwd<4>(st, a, B);
-    case 3: return launch_flat<4, false>(st, a, B);
+    case 3: return launch_flat<4, kNoBias>(st, a, B);
     default: return MDATTN_E_BADARG;
   }
 }
 
 // Head dims other than 64 and 128: the layout and the MFMAs that cover the next of 48, 80, 96 columns.
-template <bool BIAS>
+template <int BIAS>
 static int dispatch_padded(hipStream_t st, const AttnArgs& a, int B) {
   if (a.D <= 48) return launch_flat<4, BIAS, 64, 48>(st, a, B);
   if (a.D <= 80) return launch_flat<4, BIAS, 128, 80>(st, a, B);
@@ -1037,29 +1068,28 @@ extern "C" int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, 
   if (!key_bias) {
     const FwdSplit s = fwd_split((int64_t)B * H, Sq, Skv, D);
     if (s.nsplit == 1 || !workspace || workspace_floats < s.rows * (D + 2) || forced_fwd_schedule() != 0)
-      return D == 64 || D == kD ? dispatch_fwd(st, a, B, Sq, Skv, D) : dispatch_padded<false>(st, a, B);
+      return D == 64 || D == kD ? dispatch_fwd(st, a, B, Sq, Skv, D) : dispatch_padded<kNoBias>(st, a, B);
     if (!aligned16(workspace)) return MDATTN_E_ALIGN;
     a.nsplit = s.nsplit;
     a.tps = s.tps;
     a.part = workspace;
     a.ml = reinterpret_cast<float2*>(workspace + s.rows * D);
-    const int split_rc = D == kD ? launch_flat<4, false>(st, a, B) : D == 64 ? launch_flat<4, false, 64>(st, a, B) : dispatch_padded<false>(st, a, B);
+    const int split_rc = D == kD ? launch_flat<4, kNoBias>(st, a, B) : D == 64 ? launch_flat<4, kNoBias, 64>(st, a, B) : dispatch_padded<kNoBias>(st, a, B);
     if (split_rc != MDATTN_OK) return split_rc;
     const int64_t chunks = (int64_t)B * H * Sq * (D / 8);  // at most a few million: split calls are small ones
     MDATTN_LAUNCH(fwd_combine_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a, D / 8, chunks);
     return launch_status();
   }
   if (bias_stride < ((Skv + kTS - 1) / kTS) * kTS || bias_stride % kTS != 0) return MDATTN_E_BADARG;
+  if (!tiles) return MDATTN_E_BADARG;
   if (!aligned16(key_bias) || (reinterpret_cast<uintptr_t>(tiles) & 3u)) return MDATTN_E_ALIGN;
   a.bias = key_bias;
   a.bias_sb = bias_stride;
-  if (tiles) {  // the list for 32-key tiles, or behind it the one for 64-key tiles
-    a.tiles = D > 64 ? tiles : tiles + (int64_t)B * key_tiles_ints(Skv, 32);
-    a.tiles_sb = key_tiles_ints(Skv, D > 64 ? 32 : 64);
-  }
-  if (D == kD) return launch_flat<4, true>(st, a, B);
-  if (D == 64) return launch_flat<4, true, 64>(st, a, B);
-  return dispatch_padded<true>(st, a, B);
+  a.tiles = D > 64 ? tiles : tiles + (int64_t)B * key_tiles_ints(Skv, 32);  // the list for 32-key tiles, or behind it the one for 64
+  a.tiles_sb = key_tiles_ints(Skv, D > 64 ? 32 : 64);
+  if (D == kD) return launch_flat<4, kKeyMask>(st, a, B);
+  if (D == 64) return launch_flat<4, kKeyMask, 64>(st, a, B);
+  return dispatch_padded<kKeyMask>(st, a, B);
 }
 
 extern "C" int mdattn_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse,
@@ -1100,6 +1130,6 @@ extern "C" int mdattn_fwd_bf16_bias(void* stream, const void* q, const void* k, 
   if (!aligned16(key_bias)) return MDATTN_E_ALIGN;
   a.bias = key_bias;
   a.bias_sb = bias_stride;
-  if (D == 64) return launch_flat<4, true, 64>((hipStream_t)stream, a, B);
-  return launch_flat<4, true>((hipStream_t)stream, a, B);
+  if (D == 64) return launch_flat<4, kKeyBias, 64>((hipStream_t)stream, a, B);
+  return launch_flat<4, kKeyBias>((hipStream_t)stream, a, B);
 }

@@ -141,15 +141,17 @@ __device__ __forceinline__ unsigned lds_addr_of(const void* p) {
 // wave keeps 64 entries in a register, one per lane, and reads the wanted one into a scalar: a scalar load per tile would
 // turn every LDS wait around it into a full one.
 struct TileList {
-  const int* list;  // [count, entry 0, entry 1, ..]; null: every tile, the bias applied in each
+  const int* list;  // [count, entry 0, entry 1, ..]; null: none, every tile is visited
   int lane_entry = 0;
   __device__ __forceinline__ int count(int all) const { return list ? __builtin_amdgcn_readfirstlane(list[0]) : all; }
   // entry t of n; successive calls go up by one, or repeat
   __device__ __forceinline__ int at(int t, int n, int lane) {
-    if (!list) return 2 * t + 1;
     if ((t & 63) == 0) {
       const int i = t + lane;
       lane_entry = list[1 + (i < n ? i : n - 1)];
+      // waited for here, once in 64 tiles: a load still pending where the branch ends would be waited for at every tile, and with
+      // it every tile that is on its way into LDS
+      asm volatile("" : "+v"(lane_entry));
     }
     return __builtin_amdgcn_readlane(lane_entry, t & 63);
   }
@@ -171,7 +173,7 @@ struct AttnArgs {
   float c;  // scale * log2(e)
   const float* bias;   // optional additive per-key bias [B, bias_sb] (natural-log units), flat kernel only
   int64_t bias_sb;
-  const int* tiles;    // with a bias: per batch, the number of key tiles to visit and their entries (see key_tiles_kernel); null: all
+  const int* tiles;    // kKeyMask: per batch element, the number of key tiles to visit and their entries (see key_tiles_kernel)
   int tiles_sb;
   float* o_run;    // when set: no `out`; the result is merged in LSE space into this f32 carry (strides o_s*, in floats)
   float* lse_run;  // ... and into its lse [B,H,Sq]

@@ -29,8 +29,8 @@ int mdattn_host_quant3_e4m3(void* stream, const void* q, const void* k, const vo
 /* Whether mdattn_host_fwd_bf16 and mdattn_host_bwd_bf16 take head dim D. */
 int mdattn_host_head_dim(int D);
 
-/* mdattn_fwd_bf16 / mdattn_fwd_bf16_bias (key_bias null: none; tiles: that bias' tile lists, or null: every tile is visited) at 64, 128 and the multiples of 8 up to 48 and from
- * 72 to 96.  workspace: mdattn_host_fwd_workspace_floats floats, 16-byte aligned, with which a call without a bias whose query
+/* mdattn_fwd_bf16, or (key_bias and tiles of mdattn_host_key_tiles) the same under a key mask, at head dims 64, 128 and the multiples
+ * of 8 up to 48 and from 72 to 96.  workspace: mdattn_host_fwd_workspace_floats floats, 16-byte aligned, with which a call without a bias whose query
  * tiles leave the chip idle is split over its keys; 0: it would not be.  With less, the call runs unsplit. */
 int64_t mdattn_host_fwd_workspace_floats(int B, int H, int Sq, int Skv, int D);
 int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void* v, void* out, float* lse, int B, int H, int Sq, int Skv, int D,
@@ -38,7 +38,7 @@ int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void*
                          const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride, const int* tiles,
                          float* workspace, int64_t workspace_floats);
 
-/* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias and tiles as above) at the head dims of mdattn_host_fwd_bf16. */
+/* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias with or without tiles) at the head dims of mdattn_host_fwd_bf16. */
 int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, void* dq,
                          void* dk, void* dv, float* workspace, int64_t workspace_floats, int B, int H, int Sq, int Skv, int D,
                          const mdattn_strides* q_strides, const mdattn_strides* k_strides, const mdattn_strides* v_strides,
