@@ -118,9 +118,9 @@ def built_library_id(path: str | None = None) -> str | None:
 
 
 def library_is_current() -> bool:
-  """True when libmdattn.so (and, where torch is installed, the host extension) exists and was built from the sources in
+  """True when libmdattn.so (and, where torch is installed for ROCm, the host extension) exists and was built from the sources in
   this tree."""
-  return built_library_id() == source_id() and (built_library_id(HOST_EXT_PATH) == source_id() or not _has_torch())
+  return built_library_id() == source_id() and (built_library_id(HOST_EXT_PATH) == source_id() or not _has_rocm_torch())
 
 
 def ensure_built(verbose: bool = True) -> str:
@@ -131,15 +131,22 @@ def ensure_built(verbose: bool = True) -> str:
   return LIB_PATH
 
 
-def _has_torch() -> bool:
+def _torch_dir() -> str | None:
   import importlib.util
 
-  return importlib.util.find_spec("torch") is not None
+  spec = importlib.util.find_spec("torch")
+  return os.path.dirname(spec.origin) if spec is not None and spec.origin else None
+
+
+def _has_rocm_torch() -> bool:
+  """Whether the host extension can be linked: a torch for CPUs, beside JAX for instance, has no use for it."""
+  d = _torch_dir()
+  return d is not None and os.path.exists(os.path.join(d, "lib", "libc10_hip.so"))
 
 
 def _start_host_extension():
-  """Starts the compiler on csrc/host/torch_host.cc (host code only: g++); None where torch is absent."""
-  if not _has_torch():
+  """Starts the compiler on csrc/host/torch_host.cc (host code only: g++); None without a torch for ROCm."""
+  if not _has_rocm_torch():
     return None
   import sysconfig
 

@@ -98,6 +98,18 @@ def test_stale_library_is_refused(monkeypatch):
   assert not build.library_is_current()
 
 
+def test_torch_without_rocm_needs_no_host_extension(monkeypatch, tmp_path):
+  """Beside a torch for CPUs the library builds and is current without the torch side."""
+  from maxdiffusion_amd import build
+
+  monkeypatch.setattr(build, "HOST_EXT_PATH", str(tmp_path / "none.so"))
+  assert not build.library_is_current()
+  (tmp_path / "lib").mkdir()
+  monkeypatch.setattr(build, "_torch_dir", lambda: str(tmp_path))
+  assert build._start_host_extension() is None
+  assert build.library_is_current()
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
   from maxdiffusion_amd import _lib
 
