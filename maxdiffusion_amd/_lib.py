@@ -112,10 +112,12 @@ def host():
 
     import torch  # noqa: F401  (its libraries before ours)
 
-    ext = importlib.import_module("." + build.HOST_EXT_NAME, __package__)
-    if ext.build_id() != lib.mdattn_build_id().decode():
-      raise RuntimeError(f"{build.HOST_EXT_PATH} was built from other sources than libmdattn.so: rebuild with `python -m maxdiffusion_amd.build`")
-    _host = ext
+    # read from the file: an extension for another torch does not load
+    have, want = build.built_library_id(build.HOST_EXT_PATH), build.host_build_id(lib.mdattn_build_id().decode())
+    if have != want:
+      raise RuntimeError(f"{build.HOST_EXT_PATH} was built from other sources than libmdattn.so, or for another torch ({have}; needed: {want}): "
+                         "rebuild with `python -m maxdiffusion_amd.build`")
+    _host = importlib.import_module("." + build.HOST_EXT_NAME, __package__)
   return _host
 
 

@@ -101,6 +101,13 @@ def source_id() -> str:
   return h.hexdigest()[:16]
 
 
+def host_build_id(sources: str) -> str:
+  """The id of the host extension: its sources', and the torch and the Python whose C++ interfaces it is compiled against."""
+  import importlib.metadata
+
+  return f"{sources} torch {importlib.metadata.version('torch')} python {sys.version_info[0]}.{sys.version_info[1]}"
+
+
 def built_library_id(path: str | None = None) -> str | None:
   """The source id a built library carries, read from the file (nothing is loaded), or None."""
   path = path or LIB_PATH
@@ -118,9 +125,9 @@ def built_library_id(path: str | None = None) -> str | None:
 
 
 def library_is_current() -> bool:
-  """True when libmdattn.so (and, where torch is installed for ROCm, the host extension) exists and was built from the sources in
-  this tree."""
-  return built_library_id() == source_id() and (built_library_id(HOST_EXT_PATH) == source_id() or not _has_rocm_torch())
+  """True when libmdattn.so (and, where torch is installed for ROCm, the host extension for this torch) exists and was built from
+  the sources in this tree."""
+  return built_library_id() == source_id() and (not _has_rocm_torch() or built_library_id(HOST_EXT_PATH) == host_build_id(source_id()))
 
 
 def ensure_built(verbose: bool = True) -> str:
@@ -154,7 +161,7 @@ def _start_host_extension():
 
   obj = HOST_EXT_PATH + f".{os.getpid()}.o"
   cmd = [shutil.which("g++") or "g++", "-c", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
-         f"-DTORCH_EXTENSION_NAME={HOST_EXT_NAME}", f'-DMDATTN_BUILD_ID="{source_id()}"', f"-I{INCLUDE}", f"-I{CSRC}", "-I/opt/rocm/include",
+         f"-DTORCH_EXTENSION_NAME={HOST_EXT_NAME}", f'-DMDATTN_BUILD_ID="{host_build_id(source_id())}"', f"-I{INCLUDE}", f"-I{CSRC}", "-I/opt/rocm/include",
          *[f"-isystem{p}" for p in include_paths()], f"-I{sysconfig.get_paths()['include']}",
          os.path.join(CSRC, "host", "torch_host.cc"), "-o", obj]
   return obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

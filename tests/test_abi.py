@@ -98,6 +98,21 @@ def test_stale_library_is_refused(monkeypatch):
   assert not build.library_is_current()
 
 
+def test_host_extension_for_another_torch_is_refused(lib, monkeypatch):
+  """An extension that was compiled against another torch is rebuilt, and said to be stale, instead of failing to load."""
+  import importlib.metadata
+
+  from maxdiffusion_amd import _lib, build
+
+  assert build.library_is_current()
+  real = importlib.metadata.version
+  monkeypatch.setattr(importlib.metadata, "version", lambda name: "0.0" if name == "torch" else real(name))
+  assert not build.library_is_current()
+  monkeypatch.setattr(_lib, "_host", None)
+  with pytest.raises(RuntimeError, match="another torch"):
+    _lib.host()
+
+
 def test_torch_without_rocm_needs_no_host_extension(monkeypatch, tmp_path):
   """Beside a torch for CPUs the library builds and is current without the torch side."""
   from maxdiffusion_amd import build
