@@ -444,3 +444,35 @@ def test_ltx2_backward_through_the_query_then_the_key(dev):
     k.mul_(2)
   with pytest.raises(RuntimeError, match="inplace"):
     torch.autograd.grad(out[1], k, g)
+
+
+@pytest.mark.parametrize("form", ["slices", "per head slices", "fused, no bias"])
+def test_gradients_of_the_python_nodes(dev, form):
+  """Calls that the C++ nodes leave to the Python ones -- q and k as column blocks of one buffer, the fused form without biases --
+  against the dense call on the same values, with a table that is read in place.  The slices: the same kernels on the same
+  values, bit for bit.  Without biases: the kernel without them against one that adds zeros, where sums may round in another
+  order: half a unit in the last place of bf16 on either side, 2 * 2^-9."""
+  B, S, H, D = 2, 37, 3, 64
+  N = H * D
+  per_head = form.startswith("per head")
+  (qkv, wq, wk, bias), _, gen = _fused_prologue(dev, B, S, H, D)
+  table = torch.polar(torch.ones(S, D // 2, device=dev), torch.rand(S, D // 2, generator=gen, device=dev))
+  gs = [torch.randn((B, S, H, D), generator=gen, device=dev).to(torch.bfloat16) for _ in range(3)]
+  if form == "fused, no bias":
+    with torch.no_grad():
+      bias.zero_()
+    got = torch.autograd.grad(A.hip_norm_rope_qkv(qkv, wq, wk, table, H), (qkv, wq, wk), gs)
+    want = torch.autograd.grad(A.hip_norm_rope_qkv(qkv, wq, wk, table, H, bias=bias), (qkv, wq, wk), gs)
+    for a, b in zip(got, want):
+      assert rel_l2(a.float().cpu().numpy(), b.float().cpu().numpy()) <= 2**-8
+    return
+  w = tuple(t.detach()[:D if per_head else N].clone().requires_grad_(True) for t in (wq, wk))
+  cut = [qkv.detach()[..., i * N:(i + 1) * N] for i in (0, 1)]
+  if per_head:
+    cut = [t.unflatten(2, (H, D)) for t in cut]
+  grads = []
+  for q, k in (cut, [t.contiguous() for t in cut]):
+    q, k = (t.detach().requires_grad_(True) for t in (q, k))
+    grads.append(torch.autograd.grad(A.hip_norm_rope(q, k, *w, table, H, per_head=per_head), (q, k) + w, gs[:2]))
+  for a, b in zip(*grads):
+    assert torch.equal(a, b)
