@@ -354,8 +354,8 @@ int mdattn_bwd_bf16_bias(void* stream, const void* q, const void* k, const void*
 /*
  * mdattn_bwd_bf16 for callers that cannot allocate device memory and have no workspace to hand over: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.
- * Same arguments and results as mdattn_bwd_bf16 without `workspace`: the lse / delta scratch lives in a device array
- * that is part of the library image (MDATTN_BWD_STATIC_MAX_FLOATS floats = 32 MiB, held by every GPU the library runs
+ * Same arguments and results as mdattn_bwd_bf16 without `workspace`: the scratch (lse / delta and, where they fit behind them,
+ * the partial gradients of a split pass) lives in a device array that is part of the library image (MDATTN_BWD_STATIC_MAX_FLOATS floats = 32 MiB, held by every GPU the library runs
  * on until the process ends).  Requests with mdattn_bwd_workspace_floats(B,H,Sq) above that limit (more than
  * 4,194,304 padded query rows over all batches and heads) return MDATTN_E_TOOBIG and launch nothing.  The call
  * allocates nothing and frees nothing.  All calls on one GPU share the array: calls that may overlap on one GPU (two

@@ -99,8 +99,8 @@ def _folds_scale(keys: int, d: int, scale: float) -> bool:
 
 
 def _pad_head_dim(qv, kv, vv):
-  """Head dims below 128 that the kernels do not walk as they are (csrc/mdattn_common.h: native_head_dim) are zero-padded to the next size the kernels take (64 or 128), as the
-  reference's flash wrappers pad them to 128 (attention_flax.py:223-259, `_pad_data_for_flash`): zero columns of q and
+  """Head dims below 128 that the kernels do not walk as they are (csrc/mdattn_common.h: native_head_dim) are zero-padded to
+  the next size the kernels take (64 or 128), as the reference's flash wrappers pad them to 128 (attention_flax.py:223-259, `_pad_data_for_flash`): zero columns of q and
   k add nothing to a logit, zero columns of v give output columns that the caller of this helper slices off.  Returns
   the (possibly padded) views and the original head dim.  One more pass over each tensor; gradients flow through the
   pad.  Head dims above 128 are left alone: the kernel entry rejects them."""
@@ -358,7 +358,7 @@ def hip_norm_rope_ltx2(query, key, norm_q_scale, norm_k_scale, heads: int, rotar
   by `rotary_emb`, the key by `k_rotary_emb` if given, else by `rotary_emb` when this is self-attention, else not
   at all.  Tables are (cos, sin) as LTX2RotaryPosEmbed returns them: [B,S,H*D] (interleaved) or [B,H,S,D/2] (split).
   Returns (q, k) bf16 [B,S,H,D], ready for `hip_flash`.  `key` None (cached K/V): only the query is processed.
-  `q_mul` (see hip_norm_rope) is folded into the f32 query scale on the host."""
+  `q_mul` (see hip_norm_rope) is folded into the f32 query scale."""
   if rope_type not in ("interleaved", "split"):
     raise ValueError(f"{rope_type=} not supported. Choose between 'interleaved' and 'split'.")  # :145-146
   q_tab = rotary_emb

@@ -833,7 +833,8 @@ extern "C" int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, 
 
 // ---------------------------------------------------------------------------------------------------
 // mdattn_bwd_bf16_static: the same backward for callers that cannot allocate (HIP graph capture, serving loops that
-// forbid hipMalloc).  The workspace (-lse in log2 units and -delta, one float each per padded query row) lives in a
+// forbid hipMalloc).  The workspace (-lse in log2 units and -delta, one float each per padded query row, and behind them the
+// partial gradients of a split pass where the array has room) lives in a
 // file-scope device array instead of a caller's buffer.  Every GPU holds its own copy of the array at its own
 // address: that address is looked up once per device with hipGetSymbolAddress and kept; host code never uses the
 // array's name as a pointer.  The dq pass writes every element of it that the dk / dv pass reads, so nothing has to be cleared

@@ -307,8 +307,8 @@ namespace mdattn {
 // keys of one batch element, as many as its waves load in one trip; where its entries start it finds by counting the kept tiles
 // of all the slices before it, 64 bytes per lane (one workgroup per element took one slice after the other: 42 us for 75,600
 // keys, now 5.0; 4.9 and 5.0 us for 4,096).  Masked calls before (every tile visited, the bias added to every logit) and with the
-// lists: 500 of 2,048 keys x 2,048 queries x 20 heads 59 -> 23 us; 3,900 of 4,096 keys 185 -> 170 us at head dim 128, 123 ->
-// 106 us at 64 (x 2 x 10 heads).
+// lists: 500 of 2,048 keys x 2,048 queries x 20 heads 61 -> 23 us; 3,900 of 4,096 keys 188 -> 171 us at head dim 128, 126 ->
+// 107 us at 64 (x 2 x 10 heads).  With a dropped key in every tile the lists give nothing (attn_fwd_bf16.hip: kKeyMask).
 constexpr int kTileSlice = 128;
 __global__ __launch_bounds__(1024) void key_tiles_kernel(const uint8_t* __restrict__ keep, float* __restrict__ bias, int* __restrict__ tiles,
                                                          int Skv, int64_t bias_stride, int B, int slices, int sb32, int sb64) {

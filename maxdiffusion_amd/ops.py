@@ -439,8 +439,8 @@ def flash_attention_backward(q, k, v, out, dout, lse, scale: float | None = None
 
 def flash_attention_backward_static(q, k, v, out, dout, lse, dq, dk, dv, scale: float | None = None):
   """`flash_attention_backward` into caller-provided dq, dk, dv (strides of q, k, v) through the entry point that
-  allocates nothing: its lse / delta scratch is a static device array of the library (32 MiB per GPU), so the call can
-  sit in code that must not allocate (HIP graph capture).  Raises MdattnError (code E_TOOBIG) when B*H*ceil32(Sq)
+  allocates nothing: its scratch (lse / delta and, where they fit, the partial gradients of a split pass) is a static
+  device array of the library (32 MiB per GPU), so the call can sit in code that must not allocate (HIP graph capture).  Raises MdattnError (code E_TOOBIG) when B*H*ceil32(Sq)
   exceeds 4,194,304 rows.  Calls that overlap on one GPU share the scratch and race."""
   _check_dev(q, k, v, out, dout, lse, dq, dk, dv)
   if not all(t.dtype == torch.bfloat16 for t in (q, k, v, out, dout, dq, dk, dv)):
