@@ -341,6 +341,7 @@ def hip_norm_rope_qkv(qkv, wq, wk, freqs_cis, heads: int, bias=None, eps: float 
     if out is not None:
       return tuple(out)
   b, s, n3 = qkv.shape
+  wq, wk = _dense_weight(wq), _dense_weight(wk)
   table = _rope_table(freqs_cis, s, n3 // 3 // heads)
   if _wants_grad(qkv, wq, wk, bias):
     if inplace:
@@ -579,6 +580,11 @@ def _rope_table(freqs_cis, seq: int, d: int, per_head: bool = False):
 _LAYOUTS = ("bshd", "bhsd")
 
 
+def _dense_weight(w):
+  """A norm weight as the prologue kernels read it; the gradient of another form flows through the conversion."""
+  return None if w is None else w.to(torch.bfloat16).contiguous()
+
+
 def _table_pair(freqs_cis):
   return freqs_cis if isinstance(freqs_cis, (tuple, list)) else (freqs_cis, None)
 
@@ -613,6 +619,7 @@ def hip_norm_rope(q, k, wq, wk, freqs_cis, heads: int, eps: float = 1e-6, per_he
       out = host.norm_rope(q, k, wq, wk, *_table_pair(freqs_cis), heads, eps, q_mul, bhsd)
     if out is not None:
       return (out[0], out[1] if k is not None else None)
+  wq, wk, wq_txt, wk_txt = (_dense_weight(w) for w in (wq, wk, wq_txt, wk_txt))
   if per_head:
     b, s, h, d = q.shape
     table = _rope_table(freqs_cis, s, d, per_head=True)

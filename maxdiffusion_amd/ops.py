@@ -103,6 +103,12 @@ def _table_args(cos, sin, s, d):
   return _ptr(_table(cos, s, d, "cos")), _ptr(_table(sin, s, d, "sin")), 0
 
 
+def _check_weights(n, **weights):
+  for name, w in weights.items():
+    if w is not None and (w.dtype != torch.bfloat16 or w.numel() != n or not w.is_contiguous()):
+      raise ValueError(f"{name} must be a contiguous bf16 tensor of {n} elements, got {tuple(w.shape)} {w.dtype} strides {w.stride()}")
+
+
 def norm_rope_fullrow(q, k, wq, wk, cos, sin, heads: int, eps: float = 1e-6, out_layout: str = "bshd", q_mul: float = 1.0):
   """q, k: bf16 [B, S, H*D] (k may be None) -> (q_out, k_out) logical [B,S,H,D] views in `out_layout`.
 
@@ -118,6 +124,7 @@ def norm_rope_fullrow(q, k, wq, wk, cos, sin, heads: int, eps: float = 1e-6, out
   d = n // heads
   if k is not None and (k.shape != q.shape or k.dtype != q.dtype or k.stride() != q.stride()):
     raise ValueError("k must match q in shape, dtype and strides")
+  _check_weights(n, wq=wq, wk=wk if k is not None else None)
   pcos, psin, kind = _table_args(cos, sin, s, d)
   q_out = _alloc_like_layout(b, s, heads, d, out_layout, torch.bfloat16, q.device)
   k_out = _alloc_like_layout(b, s, heads, d, out_layout, torch.bfloat16, q.device) if k is not None else None
@@ -142,6 +149,7 @@ def norm_rope_qkv(qkv, wq, wk, cos, sin, heads: int, bias=None, eps: float = 1e-
   b, s, n3 = qkv.shape
   n = n3 // 3
   d = n // heads
+  _check_weights(n, wq=wq, wk=wk)
   pcos, psin, kind = _table_args(cos, sin, s, d)
   if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != n3 or not bias.is_contiguous()):
     raise ValueError("bias must be a contiguous bf16 [3*H*D] tensor")
@@ -200,6 +208,7 @@ def norm_rope_perhead(q, k, wq, wk, cos, sin, eps: float = 1e-6, wq_txt=None, wk
   b, s, h, d = q.shape
   if k is not None and (k.shape != q.shape or k.stride() != q.stride() or k.dtype != q.dtype):
     raise ValueError("k must match q in shape, dtype and strides")
+  _check_weights(d, wq=wq, wk=wk if k is not None else None, wq_txt=wq_txt, wk_txt=wk_txt if k is not None else None)
   pcos, psin, kind = _table_args(cos, sin, s, d)
   q_out = _alloc_like_layout(b, s, h, d, out_layout, torch.bfloat16, q.device)
   k_out = _alloc_like_layout(b, s, h, d, out_layout, torch.bfloat16, q.device) if k is not None else None
@@ -244,6 +253,7 @@ def norm_rope_fullrow_backward(q, k, wq, wk, cos, sin, heads: int, gq, gk, eps: 
     raise ValueError("k must match q in shape, dtype and strides")
   if has_k != (gk is not None):
     raise ValueError("gk must be given exactly when k is")
+  _check_weights(n, wq=wq, wk=wk if has_k else None)
   pcos, psin, kind = _table_args(cos, sin, s, d)
   gq = _grad_view(gq, (b, s, heads, d), "gq")
   if has_k:
@@ -286,6 +296,7 @@ def norm_rope_perhead_backward(q, k, wq, wk, cos, sin, gq, gk, eps: float = 1e-6
     raise ValueError("k must match q in shape, dtype and strides")
   if has_k != (gk is not None):
     raise ValueError("gk must be given exactly when k is")
+  _check_weights(d, wq=wq, wk=wk if has_k else None, wq_txt=wq_txt, wk_txt=wk_txt if has_k else None)
   pcos, psin, kind = _table_args(cos, sin, s, d)
   gq = _grad_view(gq, q.shape, "gq")
   if has_k:

@@ -8,7 +8,7 @@ import torch
 
 import oracle as O
 from helpers import bits_to_dev, bits_to_f32, err_stats, golden, to_dev_bf16, to_np
-from maxdiffusion_amd import ops
+from maxdiffusion_amd import attention_op, ops
 
 pytestmark = pytest.mark.gpu
 MAX_ABS, MEAN_ABS = 2e-2, 2e-3
@@ -255,3 +255,36 @@ def test_rotary_tables_are_read_in_the_layout_the_model_made(dev, form, D, S):
       want, back = ops.norm_rope_fullrow(*x, *w, cos, sin, H), ops.norm_rope_fullrow_backward(*x, *w, cos, sin, H, *g)
     assert all(torch.equal(a, b) for a, b in zip(out, want))
     assert all(torch.equal(a, b.to(torch.bfloat16)) for a, b in zip(got, back))
+
+
+@pytest.mark.parametrize("form", ["full row", "fused", "per head"])
+def test_norm_weights_of_another_type_or_layout(dev, form):
+  """f32 and strided norm weights are read as their bf16 values, with gradients in their own type; another size is refused."""
+  B, S, H, D = 1, 9, 2, 64
+  N = D if form == "per head" else H * D
+  gen = torch.Generator(device=dev).manual_seed(3)
+  x = [torch.randn((B, S, H * D), generator=gen, device=dev).to(torch.bfloat16) for _ in range(3)]
+  w = [(1 + torch.rand(N, generator=gen, device=dev)).to(torch.bfloat16) for _ in range(2)]
+  g = torch.randn((B, S, H, D), generator=gen, device=dev).to(torch.bfloat16)
+
+  def run(ws):
+    ws = [t.detach().requires_grad_(True) for t in ws]
+    if form == "fused":
+      out = attention_op.hip_norm_rope_qkv(torch.cat(x, 2), *ws, None, H)[:2]
+    elif form == "per head":
+      out = attention_op.hip_norm_rope(*(t.view(B, S, H, D) for t in x[:2]), *ws, None, H, per_head=True)
+    else:
+      out = attention_op.hip_norm_rope(*x[:2], *ws, None, H)
+    return out, torch.autograd.grad(out, ws, (g, g))
+
+  out, grads = run(w)
+  for make in (lambda t: t.float(), lambda t: t.repeat_interleave(2)[::2]):
+    ws = [make(t) for t in w]
+    o, gr = run(ws)
+    for a, b in zip(o, out):
+      assert torch.equal(a, b)
+    for a, b, t in zip(gr, grads, ws):
+      assert a.dtype == t.dtype and torch.equal(a.to(torch.bfloat16), b)
+  for bad in ([w[0][:8], w[1]], [w[0], w[1].repeat(2)]):
+    with pytest.raises(ValueError, match="contiguous bf16 tensor of"):
+      run(bad)
