@@ -478,10 +478,10 @@ constexpr int kSlotsS = 3;
 // columns in front, and one of out cut back behind, are gone: 62 -> 16 us for 16 x 257 tokens x 16 heads of 80 (64 -> 16 us of
 // kernels and the four copies' launches), 626 -> 449 us for 8,192 tokens x 20 heads of 80.
 // BIAS: kNoBias; kKeyBias, an additive bias per key, every tile visited; kKeyMask, a keep-mask as a bias of 0 and -inf with the list of
-// the tiles that hold a kept key.  In one form for both, the list and the choice per tile cost an additive bias 10 to 20 %, and a
-// mask with a dropped key in every tile as much: 4,096 keys and queries x 10 heads 109 us before the lists, 122 in one form, 110 now
-// (nothing dropped: 109, 105, 100); 512 queries x 75,600 keys x 40 heads 1,575, 1,929, 1,693 (1,575, 1,647, 1,505).  There a SIMD has one
-// wave, and what stands between two tiles is the time.
+// the tiles that hold a kept key.  In one form for both, the list and a choice per tile cost an additive bias 10 to 20 %, and a mask with
+// a dropped key in every tile as much: 4,096 keys and queries x 10 heads of 128 109 us before the lists, 122 in one form, 110 now
+// (nothing dropped: 109, 105, 100), of 64 81, 90, 72 (81, 73, 72); 512 queries x 75,600 keys x 40 heads of 128 1,575, 1,929, 1,693 (1,575,
+// 1,647, 1,505), of 64 1,072, 1,332, 1,021 (1,063, 1,051, 1,009): there a SIMD has one wave, and what stands between two tiles is the time.
 enum { kNoBias, kKeyBias, kKeyMask };
 template <int NW, int BIAS, int HD, bool PRE, int DC = 0>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 3, HD == 64 ? 4 : 3))) void attn_fwd_bf16_flat_kernel(AttnArgs a) {
@@ -633,6 +633,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // waits for every read right before its MFMA.
   constexpr int LA = HD == 128 ? MDATTN_FLAT_LA128 : 0;
   constexpr int FPB = NJ + 2 * ND, NFRAG = NB * FPB;
+  // kKeyMask: the chain of a logit's MFMAs starts from the bias, whose reads go out with the first fragments' and which no instruction
+  // adds.  Four 32-wide slabs keep the LDS too busy for reads in every tile: there the bias is added behind the chain, in the tiles
+  // that hold excluded keys.  4,096 keys and queries x 10 heads, nothing dropped / a key in every tile, from the bias: 106 / 106 us at head
+  // dim 128, 72 / 71 at 64, 93 / 93 at 80; behind the chain: 100 / 110, 70 / 80, 89 / 99.
+  constexpr bool kBiasFirst = BIAS == kKeyMask && ND < 4;
   // kt: the tile; mixed (kKeyMask): it holds excluded keys; slot: int or integral_constant
   auto tile = [&](int kt, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {
     const __bf16* base = smem + slot * STAGE;
@@ -653,9 +658,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     // ---- S^T = K.Q^T: one chain of MFMAs; the other waves of the SIMD fill the gaps between them.  A wave in an
     // MFMA phase issues ahead of the SIMD's waves in their softmax phase (1-2 % on short key sequences).
     __builtin_amdgcn_s_setprio(1);
+    auto bias4 = [&](int g) __attribute__((always_inline)) {
+      return *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base + TILES) + 32 * blk + 8 * g + 4 * hh);
+    };
     f32x16 S;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) S[i] = 0.f;
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 bv = kBiasFirst ? bias4(g) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[4 * g + e] = bv[e];
+    }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       if constexpr (LA > 0) {
@@ -668,9 +680,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
         S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[j], (PRE && j == 0) ? negm : S, 0, 0, 0);
       }
     }
-    auto bias4 = [&](int g) __attribute__((always_inline)) {
-      return *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base + TILES) + 32 * blk + 8 * g + 4 * hh);
-    };
     if constexpr (BIAS == kKeyBias) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -678,7 +687,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[4 * g + e] = __builtin_fmaf(S[4 * g + e], c, bv[e] * kLog2e);
       }
-    } else if (BIAS == kKeyMask && mixed) {  // 0 or -inf: in any unit
+    } else if (BIAS == kKeyMask && !kBiasFirst && mixed) {  // 0 or -inf: in any unit
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4 bv = bias4(g);
