@@ -170,15 +170,21 @@ __device__ __forceinline__ void store_rows_through_lds(const AttnArgs& a, const 
   const int row = row0 + l32;
   if (a.lse && hh == 0 && row < a.Sq) a.lse[((int64_t)b * a.H + h) * a.Sq + row] = (mc + __log2f(lt)) * kLn2;
   // LDS accesses of one wave execute in order: the reads below see the writes above
-  __bf16* obase = a.out + b * a.o_sb + h * a.o_sh;
   const int rr = lane / LPR, cc = lane % LPR;
+  if (PADDED && cc * 8 >= a.D) return;
+  __bf16* p = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(row0 + rr) * a.o_ss + cc * 8;
+  const int64_t step = (int64_t)RPI * a.o_ss;
+  // streaming stores: the output is written once and read by nobody here (1.5 % on the 512-key cross-attention)
+  if (row0 + 32 <= a.Sq) {  // every read before the first store: one wait, no condition per row
+    uint4 v[32 / RPI];
 #pragma unroll
-  for (int j = 0; j < 32 / RPI; ++j) {
-    const int r = j * RPI + rr;
-    if (PADDED && cc * 8 >= a.D) continue;
-    const uint4 v = *reinterpret_cast<const uint4*>(stage + r * ROWB + cc * 16);
-    // streaming store: the output is written once and read by nobody here (1.5 % on the 512-key cross-attention)
-    if (row0 + r < a.Sq) st_nt(reinterpret_cast<uint4*>(obase + (int64_t)(row0 + r) * a.o_ss + cc * 8), v);
+    for (int j = 0; j < 32 / RPI; ++j) v[j] = *reinterpret_cast<const uint4*>(stage + (j * RPI + rr) * ROWB + cc * 16);
+#pragma unroll
+    for (int j = 0; j < 32 / RPI; ++j, p += step) st_nt(reinterpret_cast<uint4*>(p), v[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 32 / RPI; ++j, p += step)
+      if (row0 + j * RPI + rr < a.Sq) st_nt(reinterpret_cast<uint4*>(p), *reinterpret_cast<const uint4*>(stage + (j * RPI + rr) * ROWB + cc * 16));
   }
 }
 
@@ -568,7 +574,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     // every wave fetches the same values to the same place (a load more per wave and tile, counted in the loop's
     // s_waitcnt): lane l and lane l + 32 the bias of key l of the tile
     if constexpr (BIAS) {  // (a 64-key tile may reach past the padded bias row, whose length is a multiple of 32)
-      int col = (BIAS == kKeyMask || kt < nt ? kt : nt - 1) * TS + (TS == 64 ? lane : l32);  // the loads run past the end
+      int col = kt * TS + (TS == 64 ? lane : l32);
       col = col < bias_cols ? col : bias_cols - 1;
       lds_dma4(bias_row, (unsigned)col * 4u, Ks + TILES * 2u);
     }
@@ -602,7 +608,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   f32x16 negm;                    // PRE (see the pipelined kernel): start value of every score accumulator chain
   // PRE: the lanes whose row has met no key with a logit above -inf yet, and with that no reference point.  A key with an
   // infinite channel has such a logit, and a share of the keys may start with 32 of them.
-  [[maybe_unused]] uint64_t fresh = ~0ull;
+  [[maybe_unused]] uint64_t fresh = 0;
 #pragma unroll
   for (int i = 0; i < 16; ++i) negm[i] = 0.f;
 
@@ -638,8 +644,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // that hold excluded keys.  4,096 keys and queries x 10 heads, nothing dropped / a key in every tile, from the bias: 106 / 106 us at head
   // dim 128, 72 / 71 at 64, 93 / 93 at 80; behind the chain: 100 / 110, 70 / 80, 89 / 99.
   constexpr bool kBiasFirst = BIAS == kKeyMask && ND < 4;
-  // kt: the tile; mixed (kKeyMask): it holds excluded keys; slot: int or integral_constant
-  auto tile = [&](int kt, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {
+  // kt: the tile; first: of this workgroup; mixed (kKeyMask): it holds excluded keys; slot: int or integral_constant
+  auto tile = [&](int kt, bool first, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {
     const __bf16* base = smem + slot * STAGE;
     constexpr int kBlk = 32 * 64;  // a 32-key block of a head-dim-64 tile: 32 rows of 64 elements, in K and in V
     auto frag = [&](int n) __attribute__((always_inline)) {
@@ -655,6 +661,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     }
 #pragma unroll
    for (int blk = 0; blk < NB; ++blk) {
+    if (decltype(masked)::value && blk > 0 && kt * TS + 32 * blk >= Skv) break;  // past the end
     // ---- S^T = K.Q^T: one chain of MFMAs; the other waves of the SIMD fill the gaps between them.  A wave in an
     // MFMA phase issues ahead of the SIMD's waves in their softmax phase (1-2 % on short key sequences).
     __builtin_amdgcn_s_setprio(1);
@@ -696,10 +703,35 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       }
     }
     if constexpr (decltype(masked)::value) {
-      const int kv_base = kt * TS + 32 * blk + 4 * hh;
+      if (kt * TS + 32 * blk + 32 > Skv) {
+        asm volatile("" ::: "memory");  // keeps the branch
+        const int kv_base = kt * TS + 32 * blk + 4 * hh;
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (kv_base + 8 * (i >> 2) + (i & 3) >= Skv) S[i] = -INFINITY;
+        for (int i = 0; i < 16; ++i)
+          if (kv_base + 8 * (i >> 2) + (i & 3) >= Skv) S[i] = -INFINITY;
+      }
+    }
+    // ---- the rows' reference points start at the maximum of their first keys: formed in front of the softmax, which in the cold
+    // branch below would be done twice, with a rescale of accumulators that hold zeros.  With a few hundred keys the vector
+    // instructions a workgroup runs once weigh as much as seven tiles'; this, the tail's -inf only where there is a tail, no request
+    // past the last tile, scalar bases for Q's rows and unconditional output stores took 75,600 queries x 40 heads against 512 keys
+    // from 783 to 769 us, 40,000 x 40 against 256 from 269 to 251 and against 126 from 205 to 190, and 75,600 x 40 against a mask's
+    // 257 keys from 612 to 570.
+    if (first && blk == 0) {
+      asm volatile("" ::: "memory");
+      float mloc = S[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) mloc = fmaxf(mloc, S[i]);
+      mloc = xhalf_max(mloc);
+      if constexpr (PRE) {
+        fresh = __builtin_amdgcn_ballot_w64(mloc == -INFINITY);
+        mc = mloc == -INFINITY ? 0.f : mloc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { S[i] -= mc; negm[i] -= mc; }
+      } else {
+        m = fmaxf(m, mloc);
+        mc = m * cs;
+      }
     }
     // ---- online softmax.  The hot path takes no row maximum: P and its sum are formed against the row's
     // current reference point, and only a partial sum above kTrig (a logit far above the reference, or
@@ -803,12 +835,20 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   }
   {
     const unsigned Qs = smem_addr + (unsigned)(STAGE + wave * QTILE) * 2u;
+    auto qcol = [&](int g) __attribute__((always_inline)) {
+      return HD == 128 ? kcol : in_head(((lane & 7) ^ ((4 * (g & 1) + (grow >> 1)) & 7)) * 8);
+    };
+    if (q0 + 32 <= a.Sq && a.q_ss < (1 << 23)) {  // uniform bases and one or two lane offsets
 #pragma unroll
-    for (int g = 0; g < 32 / RPI; ++g) {
-      int row = q0 + RPI * g + grow;
-      row = row < a.Sq ? row : a.Sq - 1;
-      const int qcol = HD == 128 ? kcol : in_head(((lane & 7) ^ ((4 * (g & 1) + (grow >> 1)) & 7)) * 8);
-      lds_dma16(qp + (int64_t)row * a.q_ss + qcol, Qs + (unsigned)(g * KGS) * 2u);
+      for (int g = 0; g < 32 / RPI; ++g)
+        lds_dma16(qp + (int64_t)(q0 + RPI * g) * a.q_ss, (unsigned)(grow * (int)a.q_ss + qcol(g)) * 2u, Qs + (unsigned)(g * KGS) * 2u);
+    } else {
+#pragma unroll
+      for (int g = 0; g < 32 / RPI; ++g) {
+        int row = q0 + RPI * g + grow;
+        row = row < a.Sq ? row : a.Sq - 1;
+        lds_dma16(qp + (int64_t)row * a.q_ss + qcol(g), Qs + (unsigned)(g * KGS) * 2u);
+      }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the wave's own Q rows (and its share of tile 0) are in LDS
     const __bf16* qs = smem + STAGE + wave * QTILE;
@@ -827,12 +867,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // SLOTS - 1 tiles are requested ahead of the one being worked on
   static_assert(SLOTS == 2 || SLOTS == 3, "one tile ahead, or two");
   if constexpr (SLOTS == 3 && BIAS == kKeyMask) {
-    if (nt > 0) {
+    if (nt > 1) {
       en = entry(1);
       dma(1, en >> 1, rows(en >> 1));
     }
   } else if constexpr (SLOTS == 3) {
-    dma(1, 1, rows(1));
+    if (nt > 1) dma(1, 1, rows(1));
   }
   // kKeyMask: the tile to be requested next and its rows, known before the barrier: their arithmetic behind it would hold up the
   // request
@@ -849,15 +889,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((SLOTS - 2) * (2 * GPW + (BIAS ? 1 : 0))));
     __syncthreads();                                  // ... and everyone's; slot `fill` (tile t-1) is free
     if constexpr (BIAS == kKeyMask) {
-      dma(fill, ef >> 1, rf);
-      tile(ec >> 1, ec & 1, slot, std::false_type{});
+      if (t + SLOTS - 1 < nt) dma(fill, ef >> 1, rf);
+      tile(ec >> 1, t == 0, ec & 1, slot, std::false_type{});
       ec = SLOTS == 3 ? en : ef;
       en = ef;
       ef = entry(t + SLOTS);
       rf = rows(ef >> 1);
     } else {
-      dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
-      tile(t, false, slot, std::false_type{});
+      if (t + SLOTS - 1 < nt) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
+      tile(t, t == 0, false, slot, std::false_type{});
     }
   };
   if constexpr (HD == 64) {
@@ -880,9 +920,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
   if constexpr (BIAS == kKeyMask) {
-    if (nt > 0) tile(ec >> 1, ec & 1, (nt - 1) % SLOTS, std::true_type{});
+    if (nt > 0) tile(ec >> 1, nt == 1, ec & 1, (nt - 1) % SLOTS, std::true_type{});
   } else {
-    tile(nt - 1, false, (nt - 1) % SLOTS, std::true_type{});
+    tile(nt - 1, nt == 1, false, (nt - 1) % SLOTS, std::true_type{});
   }
 
   if (!BIAS && a.part) {
