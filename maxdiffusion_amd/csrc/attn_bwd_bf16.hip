@@ -56,12 +56,6 @@ constexpr int bwd_slot_elems() {  // bf16 elements per ring slot
   return BwdLayout<HD>::Stage + (MODE == 3 ? BwdLayout<HD>::TileB : 0) + ((MODE != 0 || BIAS) ? 2 * kAuxFloats : 0);
 }
 
-// Waves per workgroup, 32 entity rows each.  Head dim 128: eight, one workgroup per CU at two waves per SIMD, so that
-// the CU's eight waves share one stream ring (half the global->LDS traffic of two workgroups of four; 3-6 % faster).
-// Head dim 64: four, three workgroups per CU.
-template <int HD>
-constexpr int bwd_waves() { return HD == 128 ? 8 : 4; }
-
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr_b;
 typedef __attribute__((ext_vector_type(8))) short s16x8_b;
 
@@ -102,6 +96,7 @@ struct BwdArgs {
   int nsplit, tps;
   float* part;
   float* part2;
+  int waves;  // per workgroup (head dim 128: 8 or 4)
 };
 
 // A wave's 32 rows of a gradient, rounded to bf16 and stored as pieces of 128 bytes of a row (8 rows per instruction), 64 columns
@@ -142,12 +137,11 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[ND], float mul, _
 // DC != 0: head dims other than HD (a.D, a multiple of 8 up to DC), as in the forward's flat schedule: the layout of HD, the
 // MFMAs that cover DC columns; chunks past a.D are zero in the entity fragments and in the row tiles (written once, no load
 // touches them), the row's first chunk in the transposed tiles, and not stored in the gradients.
-template <int MODE, int HD, bool BIAS, bool PRE, int DC>
+template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
 __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   static_assert(!(PRE && BIAS), "a biased logit is touched after the MFMAs anyway");
   extern __shared__ __attribute__((aligned(16))) char smem_raw_b[];
   __bf16* smem = reinterpret_cast<__bf16*>(smem_raw_b);
-  constexpr int NW = bwd_waves<HD>();
   constexpr bool HAS2 = MODE != 2;
   constexpr bool BOTH = MODE == 3;
   using L = BwdLayout<HD>;
@@ -241,12 +235,15 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       drow[row] = row < a.Se ? ndelta_e : 0.f;
     }
   }
+  // a wave without rows, or with excluded keys only, brings its share of the tiles and computes nothing
+  bool idle = r0 >= a.Se;
   // key bias in log2 units: a per-lane scalar when the keys are the entity rows, sixteen values per tile otherwise
   [[maybe_unused]] const float* bias_row = BIAS ? a.bias + b * a.bias_sb + (MODE == 0 ? ss0 : 0) : nullptr;
   [[maybe_unused]] float bias_e = 0.f;
   if constexpr (BIAS && MODE != 0) {
     bias_e = bias_row[erow] * kLog2e;
     if (!__syncthreads_or(bias_e != -INFINITY)) nt = 0;  // only excluded keys in this workgroup: zero gradients (a NaN excludes none)
+    idle = idle || __builtin_amdgcn_ballot_w64(bias_e != -INFINITY) == 0;
   }
 
   // ---- direct global -> LDS loads of one stream tile (layouts and lane maps of the forward kernel)
@@ -407,6 +404,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     } else {
       if (t + 1 < nt) dma((t + 1) & 1, t + 1);
     }
+    if (idle) continue;
     const __bf16* base = smem + (t & 1) * kBStage;
 
     // Start values of the two MFMA chains: -delta for dP^T, so that the chain ends on dP - delta; and, when the
@@ -588,17 +586,17 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   if constexpr (BOTH) store_rows<ND, PADDED>(acc2, 1.0f, a.out2 + b * a.o2_sb + h * a.o2_sh, a.o2_ss, r0, a.Se, a.D, ln, stage);
 }
 
-template <int MODE, int HD, bool BIAS, bool PRE, int DC>
-__global__ __launch_bounds__((bwd_waves<HD>() * 64)) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 3 : 2, HD == 64 ? 3 : 2))) void attn_bwd_kernel(BwdArgs a) {
-  attn_bwd_body<MODE, HD, BIAS, PRE, DC>(a);
+template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
+__global__ __launch_bounds__((NW * 64)) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 3 : 2, HD == 64 ? 3 : 2))) void attn_bwd_kernel(BwdArgs a) {
+  attn_bwd_body<MODE, HD, BIAS, PRE, DC, NW>(a);
 }
 // The dk / dv pass at head dim 128 wants a few registers more than half the register file (128 accumulators, 64 of
 // entity fragments, 32 of S and dP): held to two waves per SIMD, which the schedule needs to overlap one wave's
 // exponentials with the other's MFMAs; at one wave per SIMD it measured 28 % slower.  Head dim 64 fits three waves
 // per SIMD (3 % faster than two).
-template <int HD, bool BIAS, bool PRE, int DC>
-__global__ __launch_bounds__((bwd_waves<HD>() * 64)) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 3 : 2, HD == 64 ? 3 : 2))) void attn_bwd_both_kernel(BwdArgs a) {
-  attn_bwd_body<3, HD, BIAS, PRE, DC>(a);
+template <int HD, bool BIAS, bool PRE, int DC, int NW>
+__global__ __launch_bounds__((NW * 64)) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 3 : 2, HD == 64 ? 3 : 2))) void attn_bwd_both_kernel(BwdArgs a) {
+  attn_bwd_body<3, HD, BIAS, PRE, DC, NW>(a);
 }
 
 // Sums the partial gradients of a split pass in the order of the splits and rounds them to bf16: one 16-byte store per
@@ -622,6 +620,7 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
   const int64_t b = bh / a.H, h = bh - b * a.H;
   const float4* p = reinterpret_cast<const float4*>(a.part[t]) + 2 * i;
   float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
   for (int k = 0; k < a.nsplit; ++k, p += 2 * a.chunks) {
     const float4 u = ld_nt(p), v = ld_nt(p + 1);
     f[0] += u.x; f[1] += u.y; f[2] += u.z; f[3] += u.w; f[4] += v.x; f[5] += v.y; f[6] += v.z; f[7] += v.w;
@@ -629,51 +628,77 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
   *reinterpret_cast<uint4*>(a.out[t] + b * a.sb[t] + (int64_t)s * a.ss[t] + h * a.sh[t] + c * 8) = pack8(f);
 }
 
-// Into how many pieces a pass cuts its stream.  A pass has one workgroup per (batch, head, entity tile); cross-attention's
-// dk / dv pass (512 keys: two tiles per head) would leave most of the chip idle while each workgroup walks every query
-// row.  The cost of n pieces, in tiles: rounds of workgroups times (tiles per workgroup + 2 for a workgroup's start), the
-// write and read-back of n f32 partials, and the launch that sums them.  12 heads x 32,760 queries x 512 keys: the dk / dv
-// pass takes 1312 us in one piece (24 workgroups) and 201 us in ten, + 13 us of bwd_reduce_kernel.  Pieces under 16
-// tiles (512 rows) spend as long starting and writing partials as walking.
-constexpr int kMinSplitTiles = 16, kMaxSplit = 32;
-struct BwdSplit {
-  int nsplit, tps;
+// How a pass is launched: the waves of a workgroup and into how many pieces it cuts its stream, by the lowest cost in us of
+//   rounds of workgroups x (stream tiles per workgroup x time per tile + a workgroup's start and end)
+//   + for a cut stream the partials written and read back at 5 TB/s and the launch that sums them.
+// Head dims above 64: eight waves (256 entity rows, one workgroup per CU) share each tile, which a full chip walks 4 % faster;
+// four (128 rows, two workgroups per CU) leave less of a tile empty, and hide one workgroup's start behind the other's tiles, which
+// in the dq pass, whose start reads three rows for every one it will write, counts against a few hundred keys; alone on a CU
+// a workgroup of four is a third faster per tile.  Measured (dq / dk, dv pass, us, eight waves -> four): 69,319 queries x 512 keys x 40
+// heads 1,421 / 1,259 -> 1,251 / 1,360, 512 x 512 x 32 24.8 / 28.5 -> 18.6 / 22.7, 2,000 x 2,000 x 40 153 / 201 -> 130 / 181, 18,900 x
+// 18,900 x 20 4,345 / 6,039 -> 4,495 / 6,328.
+// The stream is cut where its own rows leave a pass without workgroups: 12 heads x 32,760 queries x 512 keys: the dk / dv pass takes
+// 1312 us in one piece (24 workgroups) and 201 us in ten, + 13 us of bwd_reduce_kernel.
+constexpr int kMinSplitTiles = 8, kMaxSplit = 32;
+struct BwdPlan {
+  int waves, nsplit, tps;
   int64_t floats;  // of one tensor's partials
 };
-// entity rows Se, stream rows Ss; tensors: gradients the pass produces (2 in the dk / dv pass)
-inline BwdSplit bwd_split(int64_t BH, int Se, int Ss, int D, int tensors) {
-  const int rows = D > 64 ? bwd_waves<128>() * 32 : bwd_waves<64>() * 32;
-  const int slots = D > 64 ? 256 : 3 * 256;                // workgroups the chip holds at once
-  const double tile_us = tensors == 2 ? 1.7 : 1.2;         // a workgroup's time per stream tile
-  const int64_t entities = BH * ((Se + rows - 1) / rows), floats = BH * Se * D;
-  const double partial = 2.0 * tensors * (double)floats * 4 / 5e6 / tile_us;  // written and read at 5 TB/s
+inline double bwd_pass_us(int D, int tensors, int waves, int64_t wgs, int tps) {
+  if (D <= 64) return (double)((wgs + 767) / 768) * (tps + 2) * (tensors == 2 ? 1.7 : 1.2);
+  const int slots = waves == 8 ? 256 : 512;
+  const int64_t rounds = wgs / slots, rest = wgs % slots;
+  const double tile = tensors == 2 ? (waves == 8 ? 1.65 : 1.75) : (waves == 8 ? 1.2 : 1.25);
+  const double alone = waves == 8 ? tile : tensors == 2 ? 1.3 : 0.8;       // with the CU to itself
+  const double full = tensors == 2 ? 0.0 : waves == 8 ? 10.0 : 5.5;        // of a start, when every CU reads its rows at once
+  double us = (double)rounds * (tps * tile + 4.0 + full);
+  if (rest) us += tps * (rest <= 256 ? alone : tile) + 4.0 + full * (double)rest / slots;
+  return us;
+}
+// entity rows Se, stream rows Ss; tensors: gradients the pass produces (2 in the dk / dv pass); room: floats for partials
+inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t room) {
   const int nt = (Ss + kBT - 1) / kBT;
-  BwdSplit best{1, nt, 0};
-  double best_cost = (double)((entities + slots - 1) / slots) * (nt + 2);
-  for (int n = 2; n <= kMaxSplit && nt / n >= kMinSplitTiles; ++n) {
-    const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
-    const double cost = (double)((entities * ns + slots - 1) / slots) * (tps + 2) + partial * ns + 5.0 / tile_us;
-    if (cost < best_cost * 0.95) { best_cost = cost; best = {ns, tps, ns * floats}; }
+  const int64_t floats = BH * Se * D;
+  const double partial = 2.0 * tensors * (double)floats * 4 / 5e6;
+  BwdPlan best{D > 64 ? 8 : 4, 1, nt, 0};
+  double best_cost = 1e300;
+  for (int waves = best.waves; waves >= 4; waves -= 4) {
+    const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)), nt);
+    if (cost < best_cost) { best_cost = cost; best.waves = waves; }
   }
+  for (int waves = D > 64 ? 8 : 4; waves >= 4; waves -= 4)
+    for (int n = 2; n <= kMaxSplit && nt / n >= kMinSplitTiles; ++n) {
+      const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
+      if (ns * floats * tensors > room) break;
+      const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)) * ns, tps) + partial * ns + 8.0;
+      if (cost < best_cost * 0.95) { best_cost = cost; best = {waves, ns, tps, ns * floats}; }
+    }
   return best;
 }
 
-template <int MODE, int HD, bool BIAS, bool PRE, int DC = 0>
-int launch_bwd_as(hipStream_t st, BwdArgs a, int B) {
+template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
+int launch_bwd_nw(hipStream_t st, BwdArgs a, int B) {
   constexpr int lds_bytes = 2 * bwd_slot_elems<MODE, HD, BIAS>() * 2;
-  constexpr int NW = bwd_waves<HD>();
   a.net = (a.Se + NW * 32 - 1) / (NW * 32);
   const int64_t total = (int64_t)B * a.H * a.net * a.nsplit;
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
   void (*kern)(BwdArgs);
-  if constexpr (MODE == 3) kern = attn_bwd_both_kernel<HD, BIAS, PRE, DC>;
-  else kern = attn_bwd_kernel<MODE, HD, BIAS, PRE, DC>;
+  if constexpr (MODE == 3) kern = attn_bwd_both_kernel<HD, BIAS, PRE, DC, NW>;
+  else kern = attn_bwd_kernel<MODE, HD, BIAS, PRE, DC, NW>;
   static LdsOptIn opted;
   if (lds_opt_in(opted, reinterpret_cast<const void*>(kern), lds_bytes) != MDATTN_OK) return MDATTN_E_LAUNCH;
   MDATTN_LAUNCH(kern, dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   return launch_status();
+}
+
+template <int MODE, int HD, bool BIAS, bool PRE, int DC = 0>
+int launch_bwd_as(hipStream_t st, const BwdArgs& a, int B) {
+  if constexpr (HD == 128) {
+    if (a.waves == 8) return launch_bwd_nw<MODE, HD, BIAS, PRE, DC, 8>(st, a, B);
+  }
+  return launch_bwd_nw<MODE, HD, BIAS, PRE, DC, 4>(st, a, B);
 }
 
 // scale * log2(e) == 1 (to f32 round-off: the caller's q carries the factor, as for the forward): the logits leave the
@@ -728,7 +753,9 @@ extern "C" int64_t mdattn_bwd_workspace_floats(int B, int H, int Sq) {
 extern "C" int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !native_head_dim(D)) return 0;
   const int64_t BH = (int64_t)B * H;
-  return mdattn_bwd_workspace_floats(B, H, Sq) + bwd_split(BH, Sq, Skv, D, 1).floats + 2 * bwd_split(BH, Skv, Sq, D, 2).floats;
+  // the two passes run one after the other and their partials share the space
+  const int64_t dq = bwd_plan(BH, Sq, Skv, D, 1, INT64_MAX).floats, dkv = 2 * bwd_plan(BH, Skv, Sq, D, 2, INT64_MAX).floats;
+  return mdattn_bwd_workspace_floats(B, H, Sq) + (dq > dkv ? dq : dkv);
 }
 
 // Shared body of mdattn_bwd_bf16 and mdattn_bwd_bf16_static: validation and the two passes.
@@ -764,13 +791,9 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   const int64_t rows = (int64_t)B * H * Sp;
   if (rows >= (1 << 29)) return MDATTN_E_UNSUPPORTED;  // delta - lse2 as a 32-bit byte offset
 
-  // stream splits, when the caller's workspace holds their partials (it always holds lse2 and delta)
+  // a stream is cut as far as the caller's workspace holds the partials (it always holds lse2 and delta)
   const int64_t BH = (int64_t)B * H;
-  BwdSplit sq = bwd_split(BH, Sq, Skv, D, 1), skv = bwd_split(BH, Skv, Sq, D, 2);
-  if (workspace_floats < 2 * rows + sq.floats + 2 * skv.floats) {
-    sq = {1, (Skv + kBT - 1) / kBT, 0};
-    skv = {1, (Sq + kBT - 1) / kBT, 0};
-  }
+  const BwdPlan pq = bwd_plan(BH, Sq, Skv, D, 1, workspace_floats - 2 * rows), pkv = bwd_plan(BH, Skv, Sq, D, 2, workspace_floats - 2 * rows);
   BwdArgs a;
   a.lse2 = lse2; a.delta = delta; a.fwd = (const __bf16*)out; a.lse = lse; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;
@@ -782,10 +805,10 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.e1_sb, a.e1_ss, a.e1_sh, q_strides); set(a.e2_sb, a.e2_ss, a.e2_sh, o_strides);
   set(a.s1_sb, a.s1_ss, a.s1_sh, k_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, v_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, k_strides);
   set(a.o_sb, a.o_ss, a.o_sh, q_strides);
-  a.nsplit = sq.nsplit; a.tps = sq.tps; a.part = workspace + 2 * rows; a.part2 = nullptr;
+  a.waves = pq.waves; a.nsplit = pq.nsplit; a.tps = pq.tps; a.part = workspace + 2 * rows; a.part2 = nullptr;
   int rc = launch_bwd_any<0>(st, a, B);
   if (rc != MDATTN_OK) return rc;
-  if (sq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B)) != MDATTN_OK) return rc;
+  if (pq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B)) != MDATTN_OK) return rc;
   // dk and dv in one pass: entity k / v, stream q (scores, and accumulate for dk), dout (dP, and accumulate for dv)
   a.e1 = (const __bf16*)k; a.e2 = (const __bf16*)v; a.s1 = (const __bf16*)q; a.s2 = (const __bf16*)dout; a.s3 = (const __bf16*)q;
   a.s4 = (const __bf16*)dout;
@@ -794,9 +817,9 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.s1_sb, a.s1_ss, a.s1_sh, q_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, o_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, q_strides);
   set(a.s4_sb, a.s4_ss, a.s4_sh, o_strides);
   set(a.o_sb, a.o_ss, a.o_sh, k_strides); set(a.o2_sb, a.o2_ss, a.o2_sh, v_strides);
-  a.nsplit = skv.nsplit; a.tps = skv.tps; a.part = workspace + 2 * rows + sq.floats; a.part2 = a.part + skv.floats;
+  a.waves = pkv.waves; a.nsplit = pkv.nsplit; a.tps = pkv.tps; a.part2 = a.part + pkv.floats;
   rc = launch_bwd_any<3>(st, a, B);
-  if (rc == MDATTN_OK && skv.nsplit > 1) rc = launch_bwd_reduce(st, a, B);
+  if (rc == MDATTN_OK && pkv.nsplit > 1) rc = launch_bwd_reduce(st, a, B);
   return rc;
 }
 

@@ -322,3 +322,27 @@ def test_backward_split_over_the_other_sequence(dev, lib, D, sq, skv, masked):
   assert not dk[:, ~keep[0]].any() and not dv[:, ~keep[0]].any()
   for g, r, name in ((to_np(got[0]), rq, "dq"), (dk[:, keep[0]], rk, "dk"), (dv[:, keep[0]], rv, "dv")):
     _check(hsd(g), r, f"{name} Sq={sq} Skv={skv} D={D} masked={masked}")
+
+
+@pytest.mark.parametrize("D", [128, 80])
+@pytest.mark.parametrize("H,sq,skv,masked", [(2, 129, 33, False), (2, 127, 97, True), (2, 33, 160, True), (200, 250, 255, False), (200, 250, 255, True)])
+def test_backward_workgroups_of_four_and_eight_waves(dev, D, H, sq, skv, masked):
+  """Workgroups of four waves (few rows: tiles of 128 with empty waves) and, for dk / dv of 200 heads, of eight; a mask that
+  leaves whole waves of 32 keys without a kept one."""
+  from maxdiffusion_amd import attention_op as A
+
+  q, do = O.normal_bf16((1, sq, H, D), 0), O.normal_bf16((1, sq, H, D), 3)
+  k, v = O.normal_bf16((1, skv, H, D), 1), O.normal_bf16((1, skv, H, D), 2)
+  keep = np.ones((1, skv), bool)
+  if masked:
+    keep[:, 32:64] = False
+    keep[:, 70::3] = False
+  flat = lambda x: to_dev_bf16(x, dev).reshape(1, x.shape[1], H * D)
+  leaves = [flat(x).requires_grad_(True) for x in (q, k, v)]
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+  out = op.apply_attention(*leaves, attention_mask=torch.from_numpy(keep).to(dev) if masked else None)
+  got = [to_np(g).reshape(1, -1, H, D) for g in torch.autograd.grad(out, leaves, flat(do))]
+  assert not got[1][:, ~keep[0]].any() and not got[2][:, ~keep[0]].any()
+  ref = O.attention_bwd(hsd(q), hsd(k[:, keep[0]]), hsd(v[:, keep[0]]), hsd(do), D**-0.5)
+  for g, r, name in ((got[0], ref[0], "dq"), (got[1][:, keep[0]], ref[1], "dk"), (got[2][:, keep[0]], ref[2], "dv")):
+    _check(hsd(g), r, f"{name} H={H} Sq={sq} Skv={skv} D={D} masked={masked}")
