@@ -274,6 +274,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
   f32x16 negm;
 #pragma unroll
   for (int i = 0; i < 16; ++i) negm[i] = 0.f;
+  // PRE: the lanes whose row has met no key with a logit above -inf yet (see the flat kernel); from block 0 on
+  [[maybe_unused]] uint64_t fresh = 0;
 
   // lane-constant LDS offsets
   // K fragment j (logical chunk 2j + hh) of row l32 sits at chunk position (2j + hh) ^ (l32 & 3): pair j ^ x1,
@@ -352,7 +354,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
       }                                                                                                       \
       __builtin_amdgcn_sched_barrier(0);                                                                      \
     }                                                                                                         \
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(lsum <= kTrig)) != 0 || (PRE && (BLK) == 0), 0)) {     \
+    if (__builtin_expect((__builtin_amdgcn_ballot_w64(!(lsum <= kTrig)) | (PRE ? fresh : 0ull)) != 0, 0)) {   \
       float mloc = SC[0];                                                                                     \
       _Pragma("unroll") for (int i = 1; i < 16; ++i) mloc = fmaxf(mloc, SC[i]);                               \
       mloc = xhalf_max(mloc);                                                                                 \
@@ -360,8 +362,10 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
       /* 16, so a row can trigger again only when its maximum has grown by another 20 log2 units          */  \
       float alpha;                                                                                            \
       if (PRE) { /* SC and SN hold logits minus the old reference: shift them, and the chains' start value */ \
-        const float dm = (BLK) == 0 ? mloc : fmaxf(mloc, 0.f);                                                \
-        alpha = (BLK) == 0 ? 0.f : __builtin_amdgcn_exp2f(-dm);                                               \
+        const bool f = (fresh >> lane) & 1;                                                                   \
+        const float dm = f ? (mloc == -INFINITY ? 0.f : mloc) : fmaxf(mloc, 0.f);                             \
+        alpha = f ? 0.f : __builtin_amdgcn_exp2f(-dm);                                                        \
+        fresh = __builtin_amdgcn_ballot_w64(f && mloc == -INFINITY);                                          \
         mc += dm;                                                                                             \
         _Pragma("unroll") for (int i = 0; i < 16; ++i) { SC[i] -= dm; SN[i] -= dm; negm[i] -= dm; }           \
       } else {                                                                                                \
@@ -438,6 +442,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
     }
     kdma += kBN * a.k_ss;
     vdma += kBN * a.v_ss;
+    if (PRE && t == 0) fresh = ~0ull;  // block 0 is next
     // iteration 2t: softmax(2t), PV(2t-1), QK(2t+1)
     MDATTN_ITER(Sb, Sa, Pb, Pa, Kc1, Kn0, Vc1, Vn0, 2 * t)
   };
@@ -1041,19 +1046,39 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
   return MDATTN_OK;
 }
 
+// The schedule of a call at head dim 128 (1: pipelined, eight waves; 2: pipelined, four; 3: flat) by the lowest time in us; nt: 32-key
+// tiles.  Fitted to 1 .. 40 heads x 126 .. 40,000 queries x 126 .. 8,192 keys, within 10 % from 1,024 keys on:
+//   pipelined, eight waves: one workgroup of 256 queries per CU, 0.55 us per tile while half of the CUs are busy, 0.82 (the power
+//     limit) when all are, rounds of 256;
+//   pipelined, four waves: 128 queries, one workgroup per CU, 0.41 to 0.47: the fastest where there is one for each CU at most;
+//   flat: 128 queries, three workgroups per CU, 0.55 / 0.92 / 1.34 with one, two, three of them; its start is the shortest.
+// Measured (pipelined 8 / pipelined 4 / flat): 20 heads x 1,024 queries x 4,096 keys 80 / 62 / 76, 4 x 8,192 x 4,096 80 / 69 / 80,
+// 40 x 2,048 x 4,096 188 / 193 / 164, 12 x 8,192 x 4,096 190 / 202 / 178, 20 x 16,384 x 4,096 553 / 662 / 567, 40 x 512 x 512 20.5 / 15.6 / 13.8.
+struct FwdSchedule {
+  int variant;
+  double us;
+};
+static FwdSchedule fwd_schedule(int64_t BH, int Sq, int Skv) {
+  const double nt = (Skv + 31) / 32;
+  const int64_t w8 = BH * ((Sq + 255) / 256), w4 = BH * ((Sq + 127) / 128);
+  const int64_t rest8 = w8 % 256, rest4 = w4 % 768;
+  const double last8 = rest8 <= 128 ? 0.55 : 0.55 + 0.27 * (double)(rest8 - 128) / 128;
+  const double us8 = 4.0 + (double)(w8 / 256) * (0.82 * nt + 7.5) + (rest8 ? last8 * nt + 7.5 : 0.0);
+  double last = rest4 == 0 ? 0.0 : rest4 <= 256 ? 0.55 : rest4 <= 512 ? 0.62 + 0.3 * (double)(rest4 - 256) / 256 : 1.22 + 0.1 * (double)(rest4 - 512) / 256;
+  if (w4 > 768 && rest4 > 0 && rest4 <= 512) last = rest4 <= 256 ? 0.48 : last < 0.8 ? 0.8 : last;  // the rounds before have not ended together
+  FwdSchedule best{3, 4.0 + ((double)(w4 / 768) * 1.34 + last) * nt};
+  if (us8 < best.us) best = {1, us8};
+  if (w4 <= 256) {
+    const double us4 = 9.5 + (w4 <= 128 ? 0.41 : 0.41 + 0.06 * (double)(w4 - 128) / 128) * nt;
+    if (us4 < best.us) best = {2, us4};
+  }
+  return best;
+}
+
 static int dispatch_fwd(hipStream_t st, const AttnArgs& a, int B, int Sq, int Skv, int D) {
   if (D == 64) return launch_flat<4, kNoBias, 64>(st, a, B);  // head dim 64: the flat schedule only
-
-  // Two schedules.  The software-pipelined kernel (8 waves x 32 query rows, two waves per SIMD) is the faster one
-  // on long key sequences; its prologue and epilogue (three tiles of look-ahead, one virtual block at each end)
-  // weigh on short ones, where the flat kernel (4 waves x 32 rows, three workgroups per CU) wins: measured
-  // cross-over between 2048 and 4608 keys.  The flat kernel also yields twice the workgroups on tiny grids.
-  // mdattn_set_fwd_schedule (1: pipelined 8 waves, 2: pipelined 4 waves, 3: flat) overrides the choice, for tests.
-  int variant = forced_fwd_schedule();
-  if (variant == 0) {
-    const int64_t wg256 = (int64_t)B * a.H * ((Sq + 255) / 256);
-    variant = (Skv <= 3072 || wg256 < 128) ? 3 : 1;
-  }
+  // mdattn_set_fwd_schedule overrides the choice, for tests
+  const int forced = forced_fwd_schedule(), variant = forced ? forced : fwd_schedule((int64_t)B * a.H, Sq, Skv).variant;
   switch (variant) {
     case 1: return launch_fwd<8>(st, a, B);
     case 2: return launch_fwd<4>(st, a, B);
@@ -1083,13 +1108,17 @@ static FwdSplit fwd_split(int64_t BH, int Sq, int Skv, int D) {
   const int ts = D > 64 ? kTS : 64, nt = (Skv + ts - 1) / ts;
   const int64_t tiles = BH * ((Sq + 127) / 128);
   FwdSplit best{1, nt, 0};
-  if (D == kD && Skv > 3072 && BH * ((Sq + 255) / 256) >= 128) return best;  // the pipelined kernel's
   const double tile_us = D > 64 ? 0.55 : 0.75, partial_us = 3.0e-4 * D;     // a tile of keys; a workgroup's partials
   auto walk = [&](int64_t wgs, int tps) {
     const double load = 0.5 + 0.58 * (double)wgs / 256;
     return tile_us * tps * (load > 1.0 ? load : 1.0);
   };
   double best_cost = 0.9 * walk(tiles, nt);
+  if (D == kD) {  // (the costs here leave out a workgroup's start, and are a tenth too high for 100 workgroups and more)
+    const FwdSchedule s = fwd_schedule(BH, Sq, Skv);
+    const double whole = (s.variant == 2 ? 1.12 : 0.9) * (s.us - 4.0);
+    best_cost = whole < best_cost ? whole : best_cost;
+  }
   for (int n = 2; n <= 16 && nt / n >= 4; ++n) {
     const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
     const double cost = walk(tiles * ns, tps) + 4.0 + 0.45 * ns + partial_us * (double)(tiles * ns);

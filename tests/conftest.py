@@ -32,6 +32,15 @@ def pytest_collection_modifyitems(config, items):
       item.add_marker(skip)
 
 
+def pytest_runtest_setup(item):
+  # tests that compare the allocator's counts: garbage of earlier tests (tensors in reference cycles) is collected before them and
+  # not in their middle
+  if "no_alloc" in item.module.__name__:
+    import gc
+
+    gc.collect()
+
+
 @pytest.fixture(scope="session", autouse=True)
 def _current_library():
   """Before the first test of a session touches the library: make sure that what is built comes from the sources in the

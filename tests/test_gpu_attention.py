@@ -421,3 +421,27 @@ def test_seeded_sweep_of_shapes_layouts_and_paths(dev, variant):
     assert bool(torch.isfinite(out.float()).all()), what
     assert float(d.max()) <= 2.5e-2 and float((lse - rl).abs().max()) <= 2e-3, what   # x8 logits: |out| up to ~4, one bf16 ulp is 1.6e-2
     assert float((out.float() - ref).norm() / ref.norm()) <= REL_L2, what
+
+
+@pytest.mark.parametrize("folded", [False, True])
+@pytest.mark.parametrize("H,sq,skv", [(2, 130, 2100), (3, 128, 1291), (1, 1, 4097), (12, 2690, 1420)])
+def test_few_query_tiles_against_many_keys(dev, folded, H, sq, skv):
+  """A workgroup per CU at most: the pipelined schedule of four waves, also as a ring step, and where a row's first 32 keys have
+  logits of -inf (a key with an infinite channel takes no part, like any key that is left out)."""
+  q, k, v = O.normal_bf16((1, sq, H, 128), 0), O.normal_bf16((1, skv, H, 128), 1), O.normal_bf16((1, skv, H, 128), 2)
+  q[..., 0] = -np.abs(q[..., 0]) - np.float32(0.5)
+  scale = ops.FOLDED_SCALE if folded else 128**-0.5
+  if folded:
+    q = O.bf16_round(q * np.float32(ops.folded_q_mul(128)))
+  gone = np.zeros(skv, bool)
+  gone[:min(40, skv - 1)] = True
+  kg = k.copy()
+  kg[:, gone, :, 0] = np.inf
+  rows = slice(0, min(sq, 300))
+  for keys, kept in ((k, ~np.zeros(skv, bool)), (kg, ~gone)):
+    out, lse = _run_np(q, keys, v, dev, scale=scale)
+    ro, rl = O.attention(hsd(q[:, rows]), hsd(k[:, kept]), hsd(v[:, kept]), scale)
+    _check(hsd(out[:, rows]), lse[0][:, rows], ro, rl, f"H={H} Sq={sq} Skv={skv} folded={folded} {int((~kept).sum())} infinite")
+    o_run, l_run = ops.new_merge_state(1, sq, H, 128, dev)
+    ops.flash_attention_merge(to_dev_bf16(q, dev), to_dev_bf16(keys, dev), to_dev_bf16(v, dev), o_run, l_run, scale=scale)
+    _check(hsd(to_np(o_run)[:, rows]), to_np(l_run)[0][:, rows], ro, rl, "as a ring step")
