@@ -56,6 +56,11 @@ constexpr int bwd_slot_elems() {  // bf16 elements per ring slot
   return BwdLayout<HD>::Stage + (MODE == 3 ? BwdLayout<HD>::TileB : 0) + ((MODE != 0 || BIAS) ? 2 * kAuxFloats : 0);
 }
 
+// Tensors whose entity rows go through LDS: of the dq pass's three, at head dim 128 two, whose areas of two workgroups of four waves fit
+// a CU.
+template <int MODE, int HD>
+constexpr int bwd_staged() { return MODE != 0 ? 0 : HD == 64 ? 3 : 2; }
+
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr_b;
 typedef __attribute__((ext_vector_type(8))) short s16x8_b;
 
@@ -196,52 +201,15 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     }
   }
 
-  // ---- entity fragments
-  int erow = r0 + l32;
-  erow = erow < a.Se ? erow : a.Se - 1;
-  bf16x8 ef1[NJ], ef2[NJ];
-  const bf16x8 zero8 = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-  auto in_row = [&](int s) __attribute__((always_inline)) { return !PADDED || s * 16 + hh * 8 < a.D; };
-  {
-    const __bf16* p = a.e1 + b * a.e1_sb + h * a.e1_sh + (int64_t)erow * a.e1_ss + hh * 8;
-#pragma unroll
-    for (int s = 0; s < NJ; ++s) ef1[s] = in_row(s) ? *reinterpret_cast<const bf16x8*>(p + s * 16) : zero8;
-    if constexpr (HAS2) {
-      const __bf16* p2 = a.e2 + b * a.e2_sb + h * a.e2_sh + (int64_t)erow * a.e2_ss + hh * 8;
-#pragma unroll
-      for (int s = 0; s < NJ; ++s) ef2[s] = in_row(s) ? *reinterpret_cast<const bf16x8*>(p2 + s * 16) : zero8;
-    }
-  }
   float* lrow = a.lse2 + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
   float* drow = a.delta + ((int64_t)b * a.H + h) * a.Sp + (MODE != 0 ? ss0 : 0);
-  float nlse_e = 0.f, ndelta_e = 0.f;  // both negated
-  if constexpr (MODE == 0) {
-    // rowsum(dout * out) from the dout fragments that the pass holds anyway.  In a launch in front of it dout was read once
-    // more (40 us at 32,760 rows x 12 heads): a training pass there against 512 keys 656 -> 644 us, 24 x 4,608 1094 -> 1076.
-    const __bf16* po = a.fwd + b * a.e2_sb + h * a.e2_sh + (int64_t)erow * a.e2_ss + hh * 8;
-#pragma unroll
-    for (int s = 0; s < NJ; ++s) {
-      const bf16x8 o = in_row(s) ? *reinterpret_cast<const bf16x8*>(po + s * 16) : zero8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ndelta_e = __builtin_fmaf(-(float)o[e], (float)ef2[s][e], ndelta_e);
-    }
-    ndelta_e = xhalf_sum(ndelta_e);
-    // rows whose keys were all masked (the forward wrote lse = -inf, out = 0) take no part: p = 0
-    const float lv = a.lse[(int64_t)bh * a.Se + erow];
-    nlse_e = lv > -INFINITY ? -lv * kLog2e : -INFINITY;
-    const int row = r0 + l32;
-    if (sp == 0 && hh == 0 && row < a.Sp) {
-      lrow[row] = row < a.Se ? nlse_e : -INFINITY;
-      drow[row] = row < a.Se ? ndelta_e : 0.f;
-    }
-  }
   // a wave without rows, or with excluded keys only, brings its share of the tiles and computes nothing
   bool idle = r0 >= a.Se;
   // key bias in log2 units: a per-lane scalar when the keys are the entity rows, sixteen values per tile otherwise
   [[maybe_unused]] const float* bias_row = BIAS ? a.bias + b * a.bias_sb + (MODE == 0 ? ss0 : 0) : nullptr;
   [[maybe_unused]] float bias_e = 0.f;
   if constexpr (BIAS && MODE != 0) {
-    bias_e = bias_row[erow] * kLog2e;
+    bias_e = bias_row[r0 + l32 < a.Se ? r0 + l32 : a.Se - 1] * kLog2e;
     if (!__syncthreads_or(bias_e != -INFINITY)) nt = 0;  // only excluded keys in this workgroup: zero gradients (a NaN excludes none)
     idle = idle || __builtin_amdgcn_ballot_w64(bias_e != -INFINITY) == 0;
   }
@@ -363,6 +331,56 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       v_off[sg] = 2 * kBTileA + (4 * hh + vxr) * 64 + (sg ^ vx) * 32 + ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
   }
 
+  // ---- entity fragments.  As lanes hold them they are 16-byte pieces of one row: a load from global memory touches 32 bytes of each of
+  // 32 rows.  The dq pass, which reads three rows for every one it writes, stages them instead: a wave's rows arrive like a
+  // stream tile, whole rows per load, in an area that then becomes the ring, and the fragments are read with a row tile's offsets
+  // (32,530 queries x 77 keys x 20 heads 172 -> 147 us, 69,319 x 512 x 40 1,231 -> 1,156, 18,900 x 18,900 x 20 4,235 -> 4,202).
+  // The dk / dv pass, with two tensors and a long stream, would only see its first tile requested later (512 x 512 x 32 22.4 -> 23.2 us).
+  constexpr int NST = bwd_staged<MODE, HD>();
+  bf16x8 ef1[NJ], ef2[NJ];
+  [[maybe_unused]] bf16x8 ef3[MODE == 0 ? NJ : 1];  // MODE 0: the forward's out, for delta
+  const bf16x8 zero8 = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+  auto in_row = [&](int s) __attribute__((always_inline)) { return !PADDED || s * 16 + hh * 8 < a.D; };
+  auto direct = [&](bf16x8 (&f)[NJ], const __bf16* p, int64_t ss) __attribute__((always_inline)) {
+    p += (int64_t)(r0 + l32 < a.Se ? r0 + l32 : a.Se - 1) * ss + hh * 8;
+#pragma unroll
+    for (int s = 0; s < NJ; ++s) f[s] = in_row(s) ? *reinterpret_cast<const bf16x8*>(p + s * 16) : zero8;
+  };
+  if constexpr (NST == 0) {
+    direct(ef1, a.e1 + b * a.e1_sb + h * a.e1_sh, a.e1_ss);
+    if constexpr (HAS2) direct(ef2, a.e2 + b * a.e2_sb + h * a.e2_sh, a.e2_ss);
+  } else {
+    const unsigned stage0 = smem_addr + (unsigned)(wave * NST * kBTileA) * 2u;
+    const bool whole = r0 + 32 <= a.Se;
+    auto stage = [&](const __bf16* p, int64_t ss, int n) __attribute__((always_inline)) {
+#pragma unroll
+      for (int g = 0; g < 32 / RPI; ++g) {
+        const int col = in_head(HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (g & 1) + (grow >> 1)) & 7)) * 8);
+        const unsigned at = stage0 + (unsigned)(n * kBTileA + g * kBGK) * 2u;
+        if (whole) {
+          lds_dma16(p + (int64_t)(r0 + RPI * g) * ss, (__umul24((unsigned)grow, (unsigned)ss) + (unsigned)col) * 2u, at);
+        } else {
+          const int row = r0 + RPI * g + grow;
+          lds_dma16(p + (int64_t)(row < a.Se ? row : a.Se - 1) * ss + col, at);
+        }
+      }
+    };
+    const __bf16* po = a.fwd + b * a.e2_sb + h * a.e2_sh;
+    if constexpr (NST < 3) direct(ef3, po, a.e2_ss);
+    stage(a.e1 + b * a.e1_sb + h * a.e1_sh, a.e1_ss, 0);
+    stage(a.e2 + b * a.e2_sb + h * a.e2_sh, a.e2_ss, 1);
+    if constexpr (NST == 3) stage(po, a.e2_ss, 2);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the wave's own rows
+    const __bf16* at = smem + wave * NST * kBTileA;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      ef1[j] = in_row(j) ? *reinterpret_cast<const bf16x8*>(at + k_off[j]) : zero8;
+      ef2[j] = in_row(j) ? *reinterpret_cast<const bf16x8*>(at + kBTileA + k_off[j]) : zero8;
+      if constexpr (NST == 3) ef3[j] = in_row(j) ? *reinterpret_cast<const bf16x8*>(at + 2 * kBTileA + k_off[j]) : zero8;
+    }
+    __syncthreads();  // every wave holds its fragments: the staging area is the ring now
+  }
+
   if (!ain) {  // the chunks past the head dim of this wave's row groups (the loop's first barrier shows them to the others)
 #pragma unroll
     for (int i = 0; i < 2 * ((kBT / RPI) / NW); ++i) {
@@ -388,6 +406,25 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     }
   } else {
     if (!BIAS || nt > 0) dma(0, 0);
+  }
+  // Beside the first tile's way: rowsum(dout * out) from the dout fragments that the pass holds anyway.  In a launch in front of it
+  // dout was read once more (40 us at 32,760 rows x 12 heads): a training pass there against 512 keys 656 -> 644 us, 24 x 4,608
+  // 1094 -> 1076.
+  float nlse_e = 0.f, ndelta_e = 0.f;  // both negated
+  if constexpr (MODE == 0) {
+#pragma unroll
+    for (int s = 0; s < NJ; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ndelta_e = __builtin_fmaf(-(float)ef3[s][e], (float)ef2[s][e], ndelta_e);
+    ndelta_e = xhalf_sum(ndelta_e);
+    // rows whose keys were all masked (the forward wrote lse = -inf, out = 0) take no part: p = 0
+    const int row = r0 + l32;
+    const float lv = a.lse[(int64_t)bh * a.Se + (row < a.Se ? row : a.Se - 1)];
+    nlse_e = lv > -INFINITY ? -lv * kLog2e : -INFINITY;
+    if (sp == 0 && hh == 0 && row < a.Sp) {
+      lrow[row] = row < a.Se ? nlse_e : -INFINITY;
+      drow[row] = row < a.Se ? ndelta_e : 0.f;
+    }
   }
   for (int t = 0; t < nt; ++t) {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of tile t has landed
@@ -630,7 +667,7 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
 
 // How a pass is launched: the waves of a workgroup and into how many pieces it cuts its stream, by the lowest cost in us of
 //   rounds of workgroups x (stream tiles per workgroup x time per tile + a workgroup's start and end)
-//   + for a cut stream the partials written and read back at 5 TB/s and the launch that sums them.
+//   + for a cut stream the partials, read back at 5 TB/s, and the launch that sums them.
 // Head dims above 64: eight waves (256 entity rows, one workgroup per CU) share each tile, which a full chip walks 4 % faster;
 // four (128 rows, two workgroups per CU) leave less of a tile empty, and hide one workgroup's start behind the other's tiles, which
 // in the dq pass, whose start reads three rows for every one it will write, counts against a few hundred keys; alone on a CU
@@ -645,7 +682,11 @@ struct BwdPlan {
   int64_t floats;  // of one tensor's partials
 };
 inline double bwd_pass_us(int D, int tensors, int waves, int64_t wgs, int tps) {
-  if (D <= 64) return (double)((wgs + 767) / 768) * (tps + 2) * (tensors == 2 ? 1.7 : 1.2);
+  if (D <= 64) {  // workgroups of four waves, three per CU
+    const double tile[3] = {tensors == 2 ? 0.74 : 0.54, tensors == 2 ? 1.15 : 0.8, tensors == 2 ? 1.45 : 1.1};  // with one, two, three of them
+    const int64_t rest = wgs % 768;
+    return (double)(wgs / 768) * (tps * tile[2] + 4.0) + (rest ? tps * tile[(rest - 1) / 256] + 4.0 : 0.0);
+  }
   const int slots = waves == 8 ? 256 : 512;
   const int64_t rounds = wgs / slots, rest = wgs % slots;
   const double tile = tensors == 2 ? (waves == 8 ? 1.65 : 1.75) : (waves == 8 ? 1.2 : 1.25);
@@ -659,7 +700,7 @@ inline double bwd_pass_us(int D, int tensors, int waves, int64_t wgs, int tps) {
 inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t room) {
   const int nt = (Ss + kBT - 1) / kBT;
   const int64_t floats = BH * Se * D;
-  const double partial = 2.0 * tensors * (double)floats * 4 / 5e6;
+  const double partial = 1.5 * tensors * (double)floats * 4 / 5e6;  // (writing them is half hidden)
   BwdPlan best{D > 64 ? 8 : 4, 1, nt, 0};
   double best_cost = 1e300;
   for (int waves = best.waves; waves >= 4; waves -= 4) {
@@ -670,7 +711,7 @@ inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t 
     for (int n = 2; n <= kMaxSplit && nt / n >= kMinSplitTiles; ++n) {
       const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
       if (ns * floats * tensors > room) break;
-      const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)) * ns, tps) + partial * ns + 8.0;
+      const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)) * ns, tps) + partial * ns + 6.0;
       if (cost < best_cost * 0.95) { best_cost = cost; best = {waves, ns, tps, ns * floats}; }
     }
   return best;
@@ -678,7 +719,9 @@ inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t 
 
 template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
 int launch_bwd_nw(hipStream_t st, BwdArgs a, int B) {
-  constexpr int lds_bytes = 2 * bwd_slot_elems<MODE, HD, BIAS>() * 2;
+  // the ring, or in front of it the waves' staged rows
+  constexpr int ring = 2 * bwd_slot_elems<MODE, HD, BIAS>() * 2, staged = NW * bwd_staged<MODE, HD>() * BwdLayout<HD>::TileA * 2;
+  constexpr int lds_bytes = ring > staged ? ring : staged;
   a.net = (a.Se + NW * 32 - 1) / (NW * 32);
   const int64_t total = (int64_t)B * a.H * a.net * a.nsplit;
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
