@@ -137,6 +137,27 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[ND], float mul, _
   }
 }
 
+// The same for the f32 partial sums of a wave's rows [rows][D]: 32 columns at a time, 128 bytes of each of 8 rows per instruction
+// instead of 32 bytes of each of 32 (dk / dv pass of 32,760 queries x 512 keys x 12 heads 236 -> 227 us).
+template <int ND, bool PADDED>
+__device__ __forceinline__ void store_partial_rows(const f32x16 (&acc)[ND], float mul, float* base, int row0, int rows, int D, int lane, char* stage) {
+  const int l32 = lane & 31, hh = lane >> 5, rr = lane >> 3, cc = lane & 7;
+#pragma unroll
+  for (int db = 0; db < ND; ++db) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(stage + l32 * kStageRowB + (8 * g + 4 * hh) * 4) =
+          f32x4{acc[db][4 * g] * mul, acc[db][4 * g + 1] * mul, acc[db][4 * g + 2] * mul, acc[db][4 * g + 3] * mul};
+    const int col = db * 32 + cc * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = row0 + 8 * j + rr;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(stage + (8 * j + rr) * kStageRowB + cc * 16);
+      if (row < rows && (!PADDED || col < D)) *reinterpret_cast<f32x4*>(base + (int64_t)row * (PADDED ? D : ND * 32) + col) = v;
+    }
+  }
+}
+
 // MODE 0: dq (entity = q rows, stream = keys); 3: dk and dv in one pass (entity = key rows, stream = q rows).
 // MODE 1 (dk alone) and 2 (dv alone) are the same body with one accumulator set; the library launches 0 and 3.
 // DC != 0: head dims other than HD (a.D, a multiple of 8 up to DC), as in the forward's flat schedule: the layout of HD, the
@@ -594,31 +615,18 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     }
   }
 
-  const int row = r0 + l32;
   const float osc = HAS2 ? a.scale : 1.0f;  // dq = scale * dS k, dk = scale * dS^T q
-  if (a.nsplit > 1) {  // partial sums over this workgroup's share of the stream, in f32
-    if (row < a.Se) {
-      const int64_t nbh = a.total / (a.net * a.nsplit);
-      const int64_t o = (((int64_t)sp * nbh + bh) * a.Se + row) * (PADDED ? a.D : HD) + 4 * hh;
-#pragma unroll
-      for (int db = 0; db < ND; ++db)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          if (PADDED && db * 32 + 8 * g >= a.D) continue;
-          *reinterpret_cast<f32x4*>(a.part + o + db * 32 + 8 * g) =
-              f32x4{acc[db][4 * g] * osc, acc[db][4 * g + 1] * osc, acc[db][4 * g + 2] * osc, acc[db][4 * g + 3] * osc};
-          if constexpr (BOTH)
-            *reinterpret_cast<f32x4*>(a.part2 + o + db * 32 + 8 * g) =
-                f32x4{acc2[db][4 * g], acc2[db][4 * g + 1], acc2[db][4 * g + 2], acc2[db][4 * g + 3]};
-        }
-    }
-    return;
-  }
   static_assert(NW * kStageRows <= 2 * kBStage * 2, "the output staging tiles must fit the ring's LDS");
   // the lane number once more: the loop has no register for it (spills at head dim 128)
   const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   __syncthreads();  // every wave has finished reading the ring, and no load into it is in flight: it now stages the outputs
   char* stage = smem_raw_b + wave * kStageRows;
+  if (a.nsplit > 1) {  // partial sums over this workgroup's share of the stream, in f32
+    const int64_t nbh = a.total / (a.net * a.nsplit), o = ((int64_t)sp * nbh + bh) * a.Se * (PADDED ? a.D : HD);
+    store_partial_rows<ND, PADDED>(acc, osc, a.part + o, r0, a.Se, a.D, ln, stage);
+    if constexpr (BOTH) store_partial_rows<ND, PADDED>(acc2, 1.0f, a.part2 + o, r0, a.Se, a.D, ln, stage);
+    return;
+  }
   store_rows<ND, PADDED>(acc, osc, a.out + b * a.o_sb + h * a.o_sh, a.o_ss, r0, a.Se, a.D, ln, stage);
   if constexpr (BOTH) store_rows<ND, PADDED>(acc2, 1.0f, a.out2 + b * a.o2_sb + h * a.o2_sh, a.o2_ss, r0, a.Se, a.D, ln, stage);
 }

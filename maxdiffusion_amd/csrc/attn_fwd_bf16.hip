@@ -75,54 +75,62 @@ __device__ __forceinline__ bf16x8 read_vt(const __bf16* p0, const __bf16* p1) {
   return __builtin_bit_cast(bf16x8, r);
 }
 
-// Epilogue of both schedules for one query row: lane (row, hh) holds, for each 32-wide block db of the head dim, the
-// values d = 32 db + 8 g + 4 hh + 0..3 (g = 0..3) of the un-normalised output, `lt` is the row's sum of P and `mc` its
-// reference point in log2 units.  Either out = O / lt as bf16 and lse = ln 2 * (mc + log2 lt), or, with a running
-// (o_run, lse_run) pair, the LSE-space merge of that result into the pair (ring_attention_kernel.py:1062-1073 of the
-// reference, with (0, -1e30) as the neutral start): the attention result of this call never goes to memory.
+// Epilogue of a ring step: the LSE-space merge of a wave's 32 rows into the running f32 pair (o_run, lse_run)
+// (ring_attention_kernel.py:1062-1073 of the reference, with (0, -1e30) as the neutral start): the attention result of this call never
+// goes to memory.  Lane (row, hh) holds, for each 32-wide block db of the head dim, the values d = 32 db + 8 g + 4 hh + 0..3 (g = 0..3) of
+// the un-normalised output, `lt` is the row's sum of P and `mc` its reference point in log2 units.  The rows pass through `stage`
+// (kMergeStage bytes of LDS that nobody else touches any more), 64 columns at a time, so that the carry is read and written 256 bytes of
+// each of 4 rows per instruction; as the lanes hold it an instruction touched 32 bytes of each of 32 rows (40 heads x 1,000 x 1,000
+// 37.1 -> 34.1 us, 2 x 12 x 2,720 x 2,720 115 -> 110, 40 x 9,450 x 9,450 1,479 -> 1,466).
+constexpr int kMergeRowB = 64 * 4 + 16, kMergeStage = 32 * kMergeRowB;
 template <int ND>
-__device__ __forceinline__ void store_row(const AttnArgs& a, const f32x16 (&O)[ND], float lt, float mc, int b, int h,
-                                          int row, int hh) {
-  if (row >= a.Sq) return;
-  const int64_t lidx = ((int64_t)b * a.H + h) * a.Sq + row;
-  if (a.o_run) {
-    const float l2 = lt > 0.f ? (mc + __log2f(lt)) * kLn2 : -INFINITY;
-    const float l1 = a.lse_run[lidx];  // both lanes of the row read it before lane hh = 0 writes it back
-    const float L = fmaxf(l1, l2);
-    float w1 = 0.f, w2 = 0.f;
-    if (L > -INFINITY) { w1 = expf(l1 - L); w2 = expf(l2 - L); }
-    const float den = w1 + w2;
-    const float invd = den > 0.f ? 1.0f / den : 0.f;
-    w1 *= invd;
-    w2 = lt > 0.f ? w2 * invd / lt : 0.f;
-    float* orow = a.o_run + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_ss + 4 * hh;
+__device__ __forceinline__ void merge_rows_through_lds(const AttnArgs& a, const f32x16 (&O)[ND], float lt, float mc, int b, int h, int row0,
+                                                       int lane, char* stage) {
+  static_assert(ND % 2 == 0, "64 columns at a time");
+  const int l32 = lane & 31, hh = lane >> 5, rr = lane >> 4, cc = lane & 15;
+  const int64_t lidx = ((int64_t)b * a.H + h) * a.Sq + row0 + l32;
+  const bool mine = row0 + l32 < a.Sq;
+  const float l2 = lt > 0.f ? (mc + __log2f(lt)) * kLn2 : -INFINITY;
+  const float l1 = mine ? a.lse_run[lidx] : -INFINITY;  // both lanes of the row read it before lane hh = 0 writes it back
+  const float L = fmaxf(l1, l2);
+  float w1 = 0.f, w2 = 0.f;
+  if (L > -INFINITY) { w1 = expf(l1 - L); w2 = expf(l2 - L); }
+  const float den = w1 + w2;
+  const float invd = den > 0.f ? 1.0f / den : 0.f;
+  w1 *= invd;
+  w2 = lt > 0.f ? w2 * invd / lt : 0.f;
+  if (mine && hh == 0) a.lse_run[lidx] = den > 0.f ? L + logf(den) : L;
+  float* base = a.o_run + b * a.o_sb + h * a.o_sh + (int64_t)(row0 + rr) * a.o_ss + cc * 4;
+  const int64_t step = 4 * a.o_ss;
+  float u1[8], u2[8];
 #pragma unroll
-    for (int db = 0; db < ND; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        float4* p = reinterpret_cast<float4*>(orow + db * 32 + 8 * g);
-        float4 r = *p;
-        r.x = w1 * r.x + w2 * O[db][4 * g];
-        r.y = w1 * r.y + w2 * O[db][4 * g + 1];
-        r.z = w1 * r.z + w2 * O[db][4 * g + 2];
-        r.w = w1 * r.w + w2 * O[db][4 * g + 3];
-        *p = r;
-      }
-    if (hh == 0) a.lse_run[lidx] = den > 0.f ? L + logf(den) : L;
-    return;
+  for (int j = 0; j < 8; ++j) {
+    u1[j] = __shfl(w1, 4 * j + rr);
+    u2[j] = __shfl(w2, 4 * j + rr);
   }
-  const float inv = lt > 0.f ? 1.0f / lt : 0.f;  // rows whose keys are all excluded return 0
-  __bf16* orow = a.out + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_ss + 4 * hh;
 #pragma unroll
-  for (int db = 0; db < ND; ++db)
+  for (int d0 = 0; d0 < ND; d0 += 2) {
+    float4 r[8];
+    float* p = base + d0 * 32;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      uint2 u;
-      u.x = pack2(O[db][4 * g] * inv, O[db][4 * g + 1] * inv);
-      u.y = pack2(O[db][4 * g + 2] * inv, O[db][4 * g + 3] * inv);
-      *reinterpret_cast<uint2*>(orow + db * 32 + 8 * g) = u;
+    for (int j = 0; j < 8; ++j, p += step)
+      if (row0 + 4 * j + rr < a.Sq) r[j] = *reinterpret_cast<const float4*>(p);
+    // LDS accesses of one wave execute in order: the reads see the writes above them, and the next round's writes follow
+#pragma unroll
+    for (int db = d0; db < d0 + 2; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(stage + l32 * kMergeRowB + ((db - d0) * 32 + 8 * g + 4 * hh) * 4) =
+            f32x4{O[db][4 * g], O[db][4 * g + 1], O[db][4 * g + 2], O[db][4 * g + 3]};
+    p = base + d0 * 32;
+#pragma unroll
+    for (int j = 0; j < 8; ++j, p += step) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(stage + (4 * j + rr) * kMergeRowB + cc * 16);
+      if (row0 + 4 * j + rr < a.Sq)
+        *reinterpret_cast<float4*>(p) = make_float4(u1[j] * r[j].x + u2[j] * x[0], u1[j] * r[j].y + u2[j] * x[1], u1[j] * r[j].z + u2[j] * x[2],
+                                                    u1[j] * r[j].w + u2[j] * x[3]);
     }
-  if (a.lse && hh == 0) a.lse[lidx] = (mc + __log2f(lt)) * kLn2;
+  }
 }
 
 // The epilogue of a workgroup that walked only a share of the keys: O, the row's sum of P and its reference point as they are.
@@ -141,12 +149,13 @@ __device__ __forceinline__ void store_partial(const AttnArgs& a, const f32x16 (&
   if (hh == 0) a.ml[r] = make_float2(mc, lt);
 }
 
-// The same epilogue with whole-row stores, for a wave that may use `stage` (32 rows of HD * 2 + 16 bytes of LDS that
-// nobody else touches any more).  store_row writes, per instruction, 16 bytes of each of 32 rows that lie a whole
-// token apart; at short key sequences, where the output is a large part of the launch's work, that costs as much as
-// the attention itself (75,600 x 40 x 128 outputs: 0.27 ms).  Here the wave's 32 x HD tile is normalised, rounded to
-// bf16 and transposed through LDS, and every store instruction then writes 1 KB of whole rows (4 rows of 256 bytes
-// at head dim 128).  Same values, same rounding as store_row.
+// The epilogue of a whole call: out = O / lt as bf16 and lse = ln 2 * (mc + log2 lt), in whole rows, for a wave that may use `stage` (32
+// rows of HD * 2 + 16 bytes of LDS that nobody else touches any more).  As the lanes hold the output an instruction would write 16
+// bytes of each of 32 rows that lie a whole token apart; at short key sequences, where the output is a large part of the launch's
+// work, that costs as much as the attention itself (75,600 x 40 x 128 outputs: 0.27 ms).  Here the wave's 32 x HD tile is
+// normalised, rounded to bf16 and transposed through LDS, and every store instruction then writes 1 KB of whole rows (4 rows of
+// 256 bytes at head dim 128).  In the pipelined schedule, which took the lanes' layout until then: 12 heads x 4,680 x 4,680 128 -> 126
+// us, 4 x 4,096 x 2,048 35.1 -> 33.6, 40 x 9,450 x 9,450 1,394 -> 1,382.
 // PADDED: the head dim a.D is below ND * 32, and only its columns are stored.
 template <int ND, bool PADDED>
 __device__ __forceinline__ void store_rows_through_lds(const AttnArgs& a, const f32x16 (&O)[ND], float lt, float mc, int b,
@@ -458,7 +467,11 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
 #undef MDATTN_ITER
 
   // ---- epilogue: normalise, convert, store; lse = m*scale + ln(l)
-  store_row<4>(a, O, xhalf_sum(l), mc, b, h, q0 + l32, hh);
+  static_assert(32 * (4 * 64 + 16) <= 4 * kStage * 2 / NW && kMergeStage <= 4 * kStage * 2 / NW, "the staged rows must fit the ring's LDS");
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();  // every wave has finished reading the ring, and no load into it is in flight: it now stages the output
+  if (a.o_run) merge_rows_through_lds<4>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * kMergeStage);
+  else store_rows_through_lds<4, false>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * 32 * (4 * 64 + 16));
 }
 
 #ifndef MDATTN_FLAT_PAIRWISE
@@ -932,13 +945,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 
   if (!BIAS && a.part) {
     store_partial<ND, PADDED>(a, O, xhalf_sum(l), mc, sp, bh, q0 + l32, hh);
-  } else if (!PADDED && a.o_run) {  // ring step: merged into the f32 carry, row by row
-    store_row<ND>(a, O, xhalf_sum(l), mc, b, h, q0 + l32, hh);
-  } else {
-    static_assert(NW * 32 * (ND * 64 + 16) <= SLOTS * STAGE * 2, "the output staging tiles must fit the ring's LDS");
-    __syncthreads();  // every wave has finished reading the ring: its LDS now stages the output tiles
-    store_rows_through_lds<ND, PADDED>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * 32 * (ND * 64 + 16));
+    return;
   }
+  static_assert(NW * 32 * (ND * 64 + 16) <= SLOTS * STAGE * 2, "the output staging tiles must fit the ring's LDS");
+  __syncthreads();  // every wave has finished reading the ring: its LDS now stages the output tiles
+  if constexpr (!PADDED) {
+    if (a.o_run) {  // ring step: merged into the f32 carry
+      merge_rows_through_lds<ND>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * kMergeStage);
+      return;
+    }
+  }
+  store_rows_through_lds<ND, PADDED>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * 32 * (ND * 64 + 16));
 }
 
 template <int NW, int BIAS, int HD = 128, int DC = 0>
@@ -947,7 +964,8 @@ static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   // the ring, or ring slot 0 plus one K-shaped Q staging tile per wave, whichever is larger
   constexpr int slots = HD == 128 ? kSlotsS : 2;
   constexpr int stage_el = (HD == 128 ? kStageS : 2 * 64 * 64) + (BIAS ? 128 : 0), qtile_el = HD == 128 ? kKTileS : 32 * 64;
-  constexpr int lds_bytes = (slots * stage_el > stage_el + NW * qtile_el ? slots * stage_el : stage_el + NW * qtile_el) * 2;
+  constexpr int ring_bytes = (slots * stage_el > stage_el + NW * qtile_el ? slots * stage_el : stage_el + NW * qtile_el) * 2;
+  constexpr int lds_bytes = ring_bytes > NW * kMergeStage ? ring_bytes : NW * kMergeStage;
   a.nqt = (a.Sq + BM - 1) / BM;
   if (!a.part) {
     a.nsplit = 1;
@@ -1052,7 +1070,7 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
 //     limit) when all are, rounds of 256;
 //   pipelined, four waves: 128 queries, one workgroup per CU, 0.41 to 0.47: the fastest where there is one for each CU at most;
 //   flat: 128 queries, three workgroups per CU, 0.55 / 0.92 / 1.34 with one, two, three of them; its start is the shortest.
-// Measured (pipelined 8 / pipelined 4 / flat): 20 heads x 1,024 queries x 4,096 keys 80 / 62 / 76, 4 x 8,192 x 4,096 80 / 69 / 80,
+// Measured (pipelined 8 / pipelined 4 / flat): 20 heads x 1,024 queries x 4,096 keys 80 / 61 / 76, 4 x 8,192 x 4,096 80 / 67 / 80,
 // 40 x 2,048 x 4,096 188 / 193 / 164, 12 x 8,192 x 4,096 190 / 202 / 178, 20 x 16,384 x 4,096 553 / 662 / 567, 40 x 512 x 512 20.5 / 15.6 / 13.8.
 struct FwdSchedule {
   int variant;
@@ -1063,13 +1081,13 @@ static FwdSchedule fwd_schedule(int64_t BH, int Sq, int Skv) {
   const int64_t w8 = BH * ((Sq + 255) / 256), w4 = BH * ((Sq + 127) / 128);
   const int64_t rest8 = w8 % 256, rest4 = w4 % 768;
   const double last8 = rest8 <= 128 ? 0.55 : 0.55 + 0.27 * (double)(rest8 - 128) / 128;
-  const double us8 = 4.0 + (double)(w8 / 256) * (0.82 * nt + 7.5) + (rest8 ? last8 * nt + 7.5 : 0.0);
+  const double us8 = 3.0 + (double)(w8 / 256) * (0.82 * nt + 7.5) + (rest8 ? last8 * nt + 7.5 : 0.0);
   double last = rest4 == 0 ? 0.0 : rest4 <= 256 ? 0.55 : rest4 <= 512 ? 0.62 + 0.3 * (double)(rest4 - 256) / 256 : 1.22 + 0.1 * (double)(rest4 - 512) / 256;
   if (w4 > 768 && rest4 > 0 && rest4 <= 512) last = rest4 <= 256 ? 0.48 : last < 0.8 ? 0.8 : last;  // the rounds before have not ended together
   FwdSchedule best{3, 4.0 + ((double)(w4 / 768) * 1.34 + last) * nt};
   if (us8 < best.us) best = {1, us8};
   if (w4 <= 256) {
-    const double us4 = 9.5 + (w4 <= 128 ? 0.41 : 0.41 + 0.06 * (double)(w4 - 128) / 128) * nt;
+    const double us4 = 8.0 + (w4 <= 128 ? 0.41 : 0.41 + 0.06 * (double)(w4 - 128) / 128) * nt;
     if (us4 < best.us) best = {2, us4};
   }
   return best;
