@@ -24,6 +24,7 @@
 // S^T - lse when the caller's q already carries scale * log2(e) (the factor c is then 1).
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "mdattn_common.h"
 #include "mdattn_host.h"
@@ -32,29 +33,23 @@ namespace mdattn {
 namespace {
 
 constexpr int kBT = 32;                  // stream rows per tile
-// Tile layouts of the forward's flat schedule (see attn_fwd_bf16.hip).  Head dim 128: groups of 4 rows, row-read
-// layout padded by 64 B per group (chunk c of row r at c ^ (r & 3)), transposed-read layout with 64-byte segments at
-// s ^ (r & 3).  Head dim 64 (LTX-2's audio stream): 128-byte rows, groups of 8 rows, chunk c at c ^ ((r >> 1) & 7) for
-// the row reads and at c ^ 4*((r >> 1) & 1) for the transposing reads, both unpadded.
+// A tile: 32 rows of HD elements, filled by loads of 1 KB (4 rows at head dim 128, 8 at 64, LTX-2's audio stream).  One copy serves the row
+// reads (ds_read_b128, 16 rows x one 16-byte chunk at a time) and the transposing reads (ds_read_b64_tr_b16, 4 rows x 64
+// bytes): chunk c of row r sits at position c ^ swizzle(r), whose upper part, distinct within 4 rows that follow each other, moves
+// the 64-byte segment (the 4 rows x 64 bytes cover every bank once) and whose lower part makes all positions of 16 rows distinct.  With
+// a copy in a layout for each kind of read every tensor that is read both ways went from the L2 to LDS twice.
 template <int HD>
-struct BwdLayout {
-  static constexpr int RPI = HD == 128 ? 4 : 8;                          // rows one load instruction fills
-  static constexpr int GA = HD == 128 ? 4 * 128 + 32 : 8 * 64;           // group stride, row-read layout (elements)
-  static constexpr int GB = HD == 128 ? 4 * 128 : 8 * 64;                // group stride, transposed-read layout
-  static constexpr int TileA = (kBT / RPI) * GA;
-  static constexpr int TileB = (kBT / RPI) * GB;
-  static constexpr int Stage = 2 * TileA + TileB;                        // elements per ring slot
-  static constexpr int V8 = HD == 128 ? 2 * GB : 8 * 64;                 // second transposing read: rows + 8
-  static constexpr int VH = HD == 128 ? 4 * GB : 16 * 64;                // second 16-row half of the tile
+struct BwdTile {
+  static constexpr int RPI = HD == 128 ? 4 : 8;        // rows one load instruction fills
+  static constexpr int Row = HD * 2, Bytes = 32 * Row;
+  static __device__ __forceinline__ int swizzle(int r) { return HD == 128 ? 4 * (r & 3) + ((r >> 2) & 3) : 4 * ((r >> 1) & 1) + ((r >> 2) & 3); }
 };
 
 // Per-row f32 values of a stream tile (lse and delta of its q rows, or the bias of its keys) travel through the ring as
 // well: 64 floats behind the tiles of a slot.
 constexpr int kAuxFloats = 64;
 template <int MODE, int HD, bool BIAS>
-constexpr int bwd_slot_elems() {  // bf16 elements per ring slot
-  return BwdLayout<HD>::Stage + (MODE == 3 ? BwdLayout<HD>::TileB : 0) + ((MODE != 0 || BIAS) ? 2 * kAuxFloats : 0);
-}
+constexpr int bwd_slot_bytes() { return 2 * BwdTile<HD>::Bytes + ((MODE != 0 || BIAS) ? 4 * kAuxFloats : 0); }
 
 // Tensors whose entity rows go through LDS: of the dq pass's three, at head dim 128 two, whose areas of two workgroups of four waves fit
 // a CU.
@@ -64,23 +59,26 @@ constexpr int bwd_staged() { return MODE != 0 ? 0 : HD == 64 ? 3 : 2; }
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr_b;
 typedef __attribute__((ext_vector_type(8))) short s16x8_b;
 
-__device__ __forceinline__ bf16x8 read_vt_b(const __bf16* p0, const __bf16* p1) {
-  s16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr_b)p0);
-  s16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr_b)p1);
+typedef const bf16x8 __attribute__((address_space(3))) * lds_bf16x8_ptr;
+typedef const f32x4 __attribute__((address_space(3))) * lds_f32x4_ptr;
+
+// LDS addresses
+__device__ __forceinline__ bf16x8 read_row(unsigned at) { return *(lds_bf16x8_ptr)at; }
+__device__ __forceinline__ bf16x8 read_vt_b(unsigned at0, unsigned at1) {
+  s16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr_b)at0);
+  s16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr_b)at1);
   s16x8_b r = __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(bf16x8, r);
 }
 
 struct BwdArgs {
   const __bf16* e1;  // entity tensor of the score contraction
-  const __bf16* e2;  // entity tensor of the dP contraction (unused for dv)
-  const __bf16* s1;  // stream tensor of the score contraction
-  const __bf16* s2;  // stream tensor of the dP contraction (unused for dv)
-  const __bf16* s3;  // stream tensor the gradient accumulates with
+  const __bf16* e2;  // entity tensor of the dP contraction
+  const __bf16* s1;  // stream tensor of the score contraction, which the gradient (MODE 3: dk) accumulates with
+  const __bf16* s2;  // stream tensor of the dP contraction; MODE 3: dv accumulates with it
   __bf16* out;       // gradient of the entity rows
-  const __bf16* s4;  // MODE 3: second stream tensor to accumulate with (dout, for dv); s3 is q (for dk)
   __bf16* out2;      // MODE 3: dv
-  int64_t s4_sb, s4_ss, s4_sh, o2_sb, o2_ss, o2_sh;
+  int64_t o2_sb, o2_ss, o2_sh;
   // Written by the dq pass for the dk / dv pass, both negated (they start the MFMA chains that they are subtracted from)
   float* lse2;         // [B,H,Sp] -lse * log2(e), -inf on padded rows
   float* delta;        // [B,H,Sp] -rowsum(dout * out), 0 on padded rows
@@ -89,7 +87,7 @@ struct BwdArgs {
   int H, Se, Ss, Sp, D;
   int net, total, chunk;
   int64_t e1_sb, e1_ss, e1_sh, e2_sb, e2_ss, e2_sh;
-  int64_t s1_sb, s1_ss, s1_sh, s2_sb, s2_ss, s2_sh, s3_sb, s3_ss, s3_sh;
+  int64_t s1_sb, s1_ss, s1_sh, s2_sb, s2_ss, s2_sh;
   int64_t o_sb, o_ss, o_sh;
   float c, scale;
   const float* bias;   // BIAS: additive per-key bias [B, bias_sb] in natural-log units (mdattn_fwd_bf16_bias)
@@ -159,23 +157,20 @@ __device__ __forceinline__ void store_partial_rows(const f32x16 (&acc)[ND], floa
 }
 
 // MODE 0: dq (entity = q rows, stream = keys); 3: dk and dv in one pass (entity = key rows, stream = q rows).
-// MODE 1 (dk alone) and 2 (dv alone) are the same body with one accumulator set; the library launches 0 and 3.
 // DC != 0: head dims other than HD (a.D, a multiple of 8 up to DC), as in the forward's flat schedule: the layout of HD, the
-// MFMAs that cover DC columns; chunks past a.D are zero in the entity fragments and in the row tiles (written once, no load
-// touches them), the row's first chunk in the transposed tiles, and not stored in the gradients.
+// MFMAs that cover DC columns; chunks past a.D are zero in the entity fragments and in the tiles (written once, no load
+// touches them), and not stored in the gradients.
 template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
 __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   static_assert(!(PRE && BIAS), "a biased logit is touched after the MFMAs anyway");
-  extern __shared__ __attribute__((aligned(16))) char smem_raw_b[];
-  __bf16* smem = reinterpret_cast<__bf16*>(smem_raw_b);
-  constexpr bool HAS2 = MODE != 2;
+  extern __shared__ __attribute__((aligned(1024))) char smem_raw_b[];  // (fragment addresses are formed by xor)
+  static_assert(MODE == 0 || MODE == 3, "dq, or dk and dv");
   constexpr bool BOTH = MODE == 3;
-  using L = BwdLayout<HD>;
+  using T = BwdTile<HD>;
   constexpr bool PADDED = DC != 0;
   constexpr int NJ = (PADDED ? DC : HD) / 16;         // MFMAs per 32 x 32 block of a contraction over the head dim
   constexpr int ND = ((PADDED ? DC : HD) + 31) / 32;  // 32-wide slabs of d = accumulators
-  constexpr int kBD = HD, kBGK = L::GA, kBGV = L::GB, kBTileA = L::TileA, kBTileB = L::TileB;
-  constexpr int kBStage = bwd_slot_elems<MODE, HD, BIAS>();  // MODE 3: a second transposed-read tile (dout)
+  constexpr int kSlot = bwd_slot_bytes<MODE, HD, BIAS>(), kAux = 2 * T::Bytes;  // a slot: two tiles, the f32 values
   constexpr bool AUX = MODE != 0 || BIAS;
 #ifndef MDATTN_BWD_LA
 #define MDATTN_BWD_LA 4
@@ -183,7 +178,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   // fragment look-ahead of the dq pass over its whole read stream (head dim 64, at three waves per SIMD, has room for
   // two: 1 % on one machine, A/B; not with a key mask's tile list); the merged pass windows its two MFMA phases separately, LA1 and LA3 below
   constexpr int LA = MODE == 0 ? (HD == 128 ? MDATTN_BWD_LA : BIAS ? 0 : 2) : 0;
-  static_assert(LA == 0 || (HAS2 && !BOTH && LA <= 2 * ND), "the window covers the three-product passes");
+  static_assert(LA == 0 || (!BOTH && LA <= 2 * ND), "the window covers the three-product pass");
 #ifndef MDATTN_BWD_LA1
 #define MDATTN_BWD_LA1 2
 #endif
@@ -192,7 +187,6 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 #endif
   constexpr int LA3 = BOTH && HD == 128 ? (BIAS ? 4 : MDATTN_BWD_LA3) : 0;
   constexpr int LA1 = BOTH && HD == 128 ? MDATTN_BWD_LA1 : 0;  // merged pass: look-ahead over the chains' row reads only
-  constexpr int kBAux = L::Stage + (BOTH ? L::TileB : 0);    // where a slot's f32 values start (elements)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,47 +231,39 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 
   // ---- direct global -> LDS loads of one stream tile (layouts and lane maps of the forward kernel)
   const __bf16* s1p = a.s1 + b * a.s1_sb + h * a.s1_sh + ss0 * a.s1_ss;
-  const __bf16* s2p = HAS2 ? a.s2 + b * a.s2_sb + h * a.s2_sh + ss0 * a.s2_ss : nullptr;
-  const __bf16* s3p = a.s3 + b * a.s3_sb + h * a.s3_sh + ss0 * a.s3_ss;
-  [[maybe_unused]] const __bf16* s4p = BOTH ? a.s4 + b * a.s4_sb + h * a.s4_sh + ss0 * a.s4_ss : nullptr;
-  constexpr int RPI = L::RPI;
+  const __bf16* s2p = a.s2 + b * a.s2_sb + h * a.s2_sh + ss0 * a.s2_ss;
+  constexpr int RPI = T::RPI;
   const int grow = HD == 128 ? lane >> 4 : lane >> 3;
-  // lane -> logical 16-byte chunk stored at this lane's position (a wave fills the row groups wave, wave + NW, ...)
+  // lane -> logical 16-byte chunk stored at this lane's position of row group g (a wave fills the groups wave, wave + NW, ...: the
+  // swizzle sees the same g)
   auto in_head = [&](int col) __attribute__((always_inline)) { return !PADDED || col < a.D ? col : 0; };
-  const int acol0 = HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (wave & 1) + (grow >> 1)) & 7)) * 8;
+  auto chunk_col = [&](int g) __attribute__((always_inline)) { return ((lane & (HD / 8 - 1)) ^ T::swizzle(RPI * g + grow)) * 8; };
+  const int acol0 = chunk_col(wave);
   const int acol = in_head(acol0);
   [[maybe_unused]] const bool ain = !PADDED || acol0 < a.D;
-  const int bcol = in_head(HD == 128 ? ((lane & 15) ^ (grow << 2)) * 8 : ((lane & 7) ^ (((grow >> 1) & 1) << 2)) * 8);
-  const unsigned smem_addr = lds_addr_of(smem);
-  // byte offsets of this lane's chunk from the first row of its row group: the same for every full tile.  The merged
-  // pass at head dim 128 has no registers to keep them in (spilled, every reload would wait for the load issued
-  // before it): it forms them again per tile from the lane number, a dozen full-rate instructions.
+  const unsigned smem_addr = lds_addr_of(smem_raw_b);
+  // byte offset of a lane's chunk from the first row of its row group: the same for every full tile (strides are below 2^23).  The
+  // merged pass at head dim 128 has no registers to keep the two offsets in (spilled, every reload would wait for the load
+  // issued before it): it forms them again per tile from the lane number, half a dozen full-rate instructions.
   constexpr bool REFORM = BOTH && HD == 128;
-  auto chunk_ofs = [&](int ln, int64_t ss, bool transposed) __attribute__((always_inline)) {
+  auto chunk_ofs = [&](int ln, int64_t ss) __attribute__((always_inline)) {
     const int gr = HD == 128 ? ln >> 4 : ln >> 3;
-    const int col = in_head(transposed ? (HD == 128 ? ((ln & 15) ^ (gr << 2)) * 8 : ((ln & 7) ^ (((gr >> 1) & 1) << 2)) * 8)
-                                       : (HD == 128 ? ((ln & 15) ^ gr) * 8 : ((ln & 7) ^ ((4 * (wave & 1) + (gr >> 1)) & 7)) * 8));
-    return (__umul24((unsigned)gr, (unsigned)ss) + (unsigned)col) * 2u;  // strides are below 2^23
+    return (__umul24((unsigned)gr, (unsigned)ss) + (unsigned)in_head(((ln & (HD / 8 - 1)) ^ T::swizzle(RPI * wave + gr)) * 8)) * 2u;
   };
-  [[maybe_unused]] const unsigned ofs1 = REFORM ? 0u : chunk_ofs(lane, a.s1_ss, false);
-  [[maybe_unused]] const unsigned ofs2 = HAS2 && !REFORM ? chunk_ofs(lane, a.s2_ss, false) : 0u;
-  [[maybe_unused]] const unsigned ofs3 = REFORM ? 0u : chunk_ofs(lane, a.s3_ss, true);
-  [[maybe_unused]] const unsigned ofs4 = BOTH && !REFORM ? chunk_ofs(lane, a.s4_ss, true) : 0u;
+  [[maybe_unused]] const unsigned ofs1 = REFORM ? 0u : chunk_ofs(lane, a.s1_ss), ofs2 = REFORM ? 0u : chunk_ofs(lane, a.s2_ss);
   // wave 0 brings a tile's f32 values: lanes 0-31 the lse of its 32 q rows and lanes 32-63 their delta, or (dq pass)
   // every lane the bias of key lane % 32.  Through LDS because a register load here would be waited for in order
   // behind the next tile's loads.
   [[maybe_unused]] const unsigned ofs_aux =
       MODE != 0 ? (lane < 32 ? 0u : (unsigned)((a.delta - a.lse2) * 4)) + (unsigned)l32 * 4u : (unsigned)l32 * 4u;
   [[maybe_unused]] const uint64_t amask = __builtin_amdgcn_ballot_w64(ain);
-  // a row group of a row tile: the lanes whose chunk lies inside the head dim
+  // a row group: the lanes whose chunk lies inside the head dim
   auto dma_a = [&](auto... at) __attribute__((always_inline)) {
     if constexpr (PADDED) lds_dma16(at..., amask);
     else lds_dma16(at...);
   };
   auto dma = [&](int slot, int t) __attribute__((always_inline)) {
-    const unsigned A1 = smem_addr + (unsigned)(slot * kBStage) * 2u;
-    const unsigned A2 = A1 + kBTileA * 2u;
-    const unsigned Bt = A2 + kBTileA * 2u;
+    const unsigned A1 = smem_addr + (unsigned)(slot * kSlot), A2 = A1 + T::Bytes;
     if constexpr (AUX) {
       if (wave == 0) {
         unsigned oa = ofs_aux;
@@ -286,27 +272,23 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
           asm volatile("" : "+v"(ln));
           oa = (ln < 32 ? 0u : (unsigned)((a.delta - a.lse2) * 4)) + (unsigned)(ln & 31) * 4u;
         }
-        lds_dma4((MODE != 0 ? lrow : bias_row) + t * kBT, oa, A1 + kBAux * 2u);
+        lds_dma4((MODE != 0 ? lrow : bias_row) + t * kBT, oa, A1 + kAux);
       }
     }
     if (t * kBT + kBT <= Ss) {  // a full tile: uniform row-group bases, one per-lane offset per stream
-      unsigned o1 = ofs1, o2 = ofs2, o3 = ofs3, o4 = ofs4;
+      unsigned o1 = ofs1, o2 = ofs2;
       if constexpr (REFORM) {
         int ln = lane;
-        asm volatile("" : "+v"(ln));  // opaque: keeps the four offsets from being hoisted out of the loop
-        o1 = chunk_ofs(ln, a.s1_ss, false);
-        o2 = chunk_ofs(ln, a.s2_ss, false);
-        o3 = chunk_ofs(ln, a.s3_ss, true);
-        o4 = chunk_ofs(ln, a.s4_ss, true);
+        asm volatile("" : "+v"(ln));  // opaque: keeps the two offsets from being hoisted out of the loop
+        o1 = chunk_ofs(ln, a.s1_ss);
+        o2 = chunk_ofs(ln, a.s2_ss);
       }
 #pragma unroll
       for (int i = 0; i < (kBT / RPI) / NW; ++i) {
         const int g = wave + NW * i;
         const int64_t r = t * kBT + RPI * g;
-        dma_a(s1p + r * a.s1_ss, o1, A1 + (unsigned)(g * kBGK) * 2u);
-        if constexpr (HAS2) dma_a(s2p + r * a.s2_ss, o2, A2 + (unsigned)(g * kBGK) * 2u);
-        lds_dma16(s3p + r * a.s3_ss, o3, Bt + (unsigned)(g * kBGV) * 2u);
-        if constexpr (BOTH) lds_dma16(s4p + r * a.s4_ss, o4, Bt + (unsigned)(kBTileB + g * kBGV) * 2u);
+        dma_a(s1p + r * a.s1_ss, o1, A1 + (unsigned)g * 1024u);
+        dma_a(s2p + r * a.s2_ss, o2, A2 + (unsigned)g * 1024u);
       }
     } else {  // the ragged last tile: rows past the end repeat the last row
 #pragma unroll
@@ -314,10 +296,8 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         const int g = wave + NW * i;
         int rr = t * kBT + RPI * g + grow;
         rr = rr < Ss ? rr : Ss - 1;
-        dma_a(s1p + (int64_t)rr * a.s1_ss + acol, A1 + (unsigned)(g * kBGK) * 2u);
-        if constexpr (HAS2) dma_a(s2p + (int64_t)rr * a.s2_ss + acol, A2 + (unsigned)(g * kBGK) * 2u);
-        lds_dma16(s3p + (int64_t)rr * a.s3_ss + bcol, Bt + (unsigned)(g * kBGV) * 2u);
-        if constexpr (BOTH) lds_dma16(s4p + (int64_t)rr * a.s4_ss + bcol, Bt + (unsigned)(kBTileB + g * kBGV) * 2u);
+        dma_a(s1p + (int64_t)rr * a.s1_ss + acol, A1 + (unsigned)g * 1024u);
+        dma_a(s2p + (int64_t)rr * a.s2_ss + acol, A2 + (unsigned)g * 1024u);
       }
     }
   };
@@ -332,25 +312,23 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       if constexpr (BOTH) acc2[db][i] = 0.f;
     }
 
-  // per-lane fragment offsets (elements)
-  int k_off[NJ], v_off[ND];
+  // Fragment addresses from the first byte of a tile, a multiple of 256: row read j (logical chunk 2 j + hh of row l32) at k_at ^ 32 j;
+  // transposing read of 32-column slab sg at v_at ^ 64 sg for the rows 4 hh + 0..3 and, eight rows on, at that ^ 32.
   const int vxr = (lane & 15) >> 2;
-  if constexpr (HD == 128) {
-    const int kx0 = l32 & 1, kx1 = (l32 >> 1) & 1;
-    const int k_base = (l32 >> 2) * kBGK + (l32 & 3) * kBD + (hh ^ kx0) * 8;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) k_off[j] = k_base + ((j & 1) ? -16 : 16) * kx1 + j * 16;
-#pragma unroll
-    for (int sg = 0; sg < ND; ++sg)
-      v_off[sg] = 2 * kBTileA + hh * kBGV + vxr * kBD + (sg ^ vxr) * 32 + ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
-  } else {
-    const int kx = (l32 >> 1) & 7, vx = (vxr >> 1) & 1;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) k_off[j] = l32 * 64 + (((2 * j + hh) ^ kx) * 8);
-#pragma unroll
-    for (int sg = 0; sg < ND; ++sg)
-      v_off[sg] = 2 * kBTileA + (4 * hh + vxr) * 64 + (sg ^ vx) * 32 + ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
-  }
+  const unsigned k_at = (unsigned)(l32 * T::Row + ((hh ^ T::swizzle(l32)) * 16));
+  const unsigned v_at = (unsigned)((4 * hh + vxr) * T::Row + ((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ T::swizzle(4 * hh + vxr)) * 16 + (lane & 1) * 8);
+  // CONST, the dq pass with eight waves: the two copies of the loop body know their slot, and what the xors give is a lane constant plus
+  // an immediate offset.  Elsewhere they are formed again for every tile: the merged pass at head dim 128 has no registers for
+  // them, and a short stream walks two copies slower than one (32,760 queries x 512 keys x 12 heads 176 us, 199 with two copies;
+  // 18,900 x 18,900 x 20 4,470 and 4,266).
+  constexpr bool CONST = MODE == 0 && NW == 8;
+  auto row_frag = [&](unsigned tile, int j, int ofs) __attribute__((always_inline)) {
+    return (((CONST ? smem_addr : tile) + k_at) ^ (unsigned)(32 * j)) + (CONST ? tile - smem_addr + ofs : (unsigned)ofs);
+  };
+  auto vt_frag = [&](unsigned slot_at, int jv, int second) __attribute__((always_inline)) {  // second: of the slot's second tile
+    const unsigned at = ((CONST ? smem_addr : slot_at) + v_at) ^ (unsigned)(64 * (jv % ND)), add = (CONST ? slot_at - smem_addr : 0u) + second * T::Bytes;
+    return read_vt_b(at + (add + (jv / ND) * 16 * T::Row), (at ^ 32u) + (add + (8 + (jv / ND) * 16) * T::Row));
+  };
 
   // ---- entity fragments.  As lanes hold them they are 16-byte pieces of one row: a load from global memory touches 32 bytes of each of
   // 32 rows.  The dq pass, which reads three rows for every one it writes, stages them instead: a wave's rows arrive like a
@@ -369,15 +347,15 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   };
   if constexpr (NST == 0) {
     direct(ef1, a.e1 + b * a.e1_sb + h * a.e1_sh, a.e1_ss);
-    if constexpr (HAS2) direct(ef2, a.e2 + b * a.e2_sb + h * a.e2_sh, a.e2_ss);
+    direct(ef2, a.e2 + b * a.e2_sb + h * a.e2_sh, a.e2_ss);
   } else {
-    const unsigned stage0 = smem_addr + (unsigned)(wave * NST * kBTileA) * 2u;
+    const unsigned stage0 = smem_addr + (unsigned)(wave * NST * T::Bytes);
     const bool whole = r0 + 32 <= a.Se;
     auto stage = [&](const __bf16* p, int64_t ss, int n) __attribute__((always_inline)) {
 #pragma unroll
       for (int g = 0; g < 32 / RPI; ++g) {
-        const int col = in_head(HD == 128 ? ((lane & 15) ^ grow) * 8 : ((lane & 7) ^ ((4 * (g & 1) + (grow >> 1)) & 7)) * 8);
-        const unsigned at = stage0 + (unsigned)(n * kBTileA + g * kBGK) * 2u;
+        const int col = in_head(chunk_col(g));
+        const unsigned at = stage0 + (unsigned)(n * T::Bytes + g * 1024);
         if (whole) {
           lds_dma16(p + (int64_t)(r0 + RPI * g) * ss, (__umul24((unsigned)grow, (unsigned)ss) + (unsigned)col) * 2u, at);
         } else {
@@ -392,12 +370,11 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     stage(a.e2 + b * a.e2_sb + h * a.e2_sh, a.e2_ss, 1);
     if constexpr (NST == 3) stage(po, a.e2_ss, 2);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the wave's own rows
-    const __bf16* at = smem + wave * NST * kBTileA;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      ef1[j] = in_row(j) ? *reinterpret_cast<const bf16x8*>(at + k_off[j]) : zero8;
-      ef2[j] = in_row(j) ? *reinterpret_cast<const bf16x8*>(at + kBTileA + k_off[j]) : zero8;
-      if constexpr (NST == 3) ef3[j] = in_row(j) ? *reinterpret_cast<const bf16x8*>(at + 2 * kBTileA + k_off[j]) : zero8;
+      ef1[j] = in_row(j) ? read_row(row_frag(stage0, j, 0)) : zero8;
+      ef2[j] = in_row(j) ? read_row(row_frag(stage0, j, T::Bytes)) : zero8;
+      if constexpr (NST == 3) ef3[j] = in_row(j) ? read_row(row_frag(stage0, j, 2 * T::Bytes)) : zero8;
     }
     __syncthreads();  // every wave holds its fragments: the staging area is the ring now
   }
@@ -405,9 +382,9 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
   if (!ain) {  // the chunks past the head dim of this wave's row groups (the loop's first barrier shows them to the others)
 #pragma unroll
     for (int i = 0; i < 2 * ((kBT / RPI) / NW); ++i) {
-      __bf16* at = smem + (i & 1) * kBStage + (wave + NW * (i >> 1)) * kBGK + lane * 8;
+      char* at = smem_raw_b + (i & 1) * kSlot + (wave + NW * (i >> 1)) * 1024 + lane * 16;
       *reinterpret_cast<uint4*>(at) = make_uint4(0u, 0u, 0u, 0u);
-      if constexpr (HAS2) *reinterpret_cast<uint4*>(at + kBTileA) = make_uint4(0u, 0u, 0u, 0u);
+      *reinterpret_cast<uint4*>(at + T::Bytes) = make_uint4(0u, 0u, 0u, 0u);
     }
   }
 
@@ -447,7 +424,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       drow[row] = row < a.Se ? ndelta_e : 0.f;
     }
   }
-  for (int t = 0; t < nt; ++t) {
+  auto tile = [&](int t, auto slot) __attribute__((always_inline)) {  // slot: t & 1, an int or an integral_constant
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of tile t has landed
     __syncthreads();                      // ... and everyone's; the other slot (tile t-1) is free
     int kt = t;
@@ -457,18 +434,18 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
       mixed = ec & 1;
       if (t + 1 < nt) {
         ec = entry(t + 1);
-        dma((t + 1) & 1, ec >> 1);
+        dma(slot ^ 1, ec >> 1);
       }
     } else {
-      if (t + 1 < nt) dma((t + 1) & 1, t + 1);
+      if (t + 1 < nt) dma(slot ^ 1, t + 1);
     }
-    if (idle) continue;
-    const __bf16* base = smem + (t & 1) * kBStage;
+    if (idle) return;
+    const unsigned base = smem_addr + (unsigned)(slot * kSlot);
 
     // Start values of the two MFMA chains: -delta for dP^T, so that the chain ends on dP - delta; and, when the
     // logits come out of the MFMAs in log2 units (PRE), -lse for S^T, so that exp2 applies to the chain's result
     // as it is.  Per-lane constants when the q rows are the entity rows, the tile's values from LDS otherwise.
-    [[maybe_unused]] const float* aux = reinterpret_cast<const float*>(base + kBAux);
+    [[maybe_unused]] auto aux4 = [&](int i) __attribute__((always_inline)) { return *(lds_f32x4_ptr)(base + (unsigned)(kAux + 4 * i)); };
     f32x16 S, dP;
     if constexpr (MODE == 0) {
 #pragma unroll
@@ -476,11 +453,11 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     } else {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const f32x4 dv = *reinterpret_cast<const f32x4*>(aux + 32 + 8 * g + 4 * hh);
+        const f32x4 dv = aux4(32 + 8 * g + 4 * hh);
 #pragma unroll
         for (int e = 0; e < 4; ++e) dP[4 * g + e] = dv[e];
         if constexpr (PRE) {
-          const f32x4 lv = *reinterpret_cast<const f32x4*>(aux + 8 * g + 4 * hh);
+          const f32x4 lv = aux4(8 * g + 4 * hh);
 #pragma unroll
           for (int e = 0; e < 4; ++e) S[4 * g + e] = lv[e];
         } else {
@@ -493,11 +470,9 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     // of the accumulation.  With LA > 0 a window of LA fragments runs ahead of the MFMAs (pinned by scheduling
     // barriers: left to itself the compiler waits for every read right before its MFMA).
     auto frag = [&](int n) __attribute__((always_inline)) {
-      if (n < NJ) return *reinterpret_cast<const bf16x8*>(base + k_off[n]);
-      if (n < 2 * NJ) return *reinterpret_cast<const bf16x8*>(base + kBTileA + k_off[n - NJ]);
-      const int jv = n - 2 * NJ;
-      const __bf16* src = base + v_off[jv % ND] + (jv / ND) * L::VH;
-      return read_vt_b(src, src + L::V8);
+      if (n < NJ) return read_row(row_frag(base, n, 0));
+      if (n < 2 * NJ) return read_row(row_frag(base, n - NJ, T::Bytes));
+      return vt_frag(base, n - 2 * NJ, 0);
     };
     [[maybe_unused]] bf16x8 win[LA > 0 ? LA : 1];
     if constexpr (LA > 0) {
@@ -524,10 +499,8 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     } else {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(j), ef1[j], S, 0, 0, 0);
-      if constexpr (HAS2) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) dP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(NJ + j), ef2[j], dP, 0, 0, 0);
-      }
+      for (int j = 0; j < NJ; ++j) dP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag(NJ + j), ef2[j], dP, 0, 0, 0);
     }
     // W = P or dS, eight logits (one B operand) at a time
     if constexpr (MODE == 0) {
@@ -551,7 +524,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
               const int col = kt * kBT + 8 * (2 * hb + g) + 4 * hh;
-              const f32x4 bv = *reinterpret_cast<const f32x4*>(aux + 8 * (2 * hb + g) + 4 * hh);
+              const f32x4 bv = aux4(8 * (2 * hb + g) + 4 * hh);
 #pragma unroll
               for (int e = 0; e < 4; ++e)
                 nl[4 * g + e] = col + e < Ss ? __builtin_fmaf(bv[e], kLog2e, nlse_e) : -INFINITY;  // whatever the padding holds
@@ -560,7 +533,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         } else {
 #pragma unroll
           for (int g = 0; g < 2; ++g) {
-            const f32x4 lv = *reinterpret_cast<const f32x4*>(aux + 8 * (2 * hb + g) + 4 * hh);
+            const f32x4 lv = aux4(8 * (2 * hb + g) + 4 * hh);
 #pragma unroll
             for (int e = 0; e < 4; ++e) nl[4 * g + e] = BIAS ? lv[e] + bias_e : lv[e];
           }
@@ -573,7 +546,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
         const float p0 = __builtin_amdgcn_exp2f(PRE ? S[8 * hb + e] : __builtin_fmaf(S[8 * hb + e], c, nl[e]));
         const float p1 = __builtin_amdgcn_exp2f(PRE ? S[8 * hb + e + 1] : __builtin_fmaf(S[8 * hb + e + 1], c, nl[e + 1]));
         // dS without its factor `scale`: applied once, to the accumulators
-        wpk[e >> 1] = HAS2 ? pack2(p0 * dP[8 * hb + e], p1 * dP[8 * hb + e + 1]) : pack2(p0, p1);
+        wpk[e >> 1] = pack2(p0 * dP[8 * hb + e], p1 * dP[8 * hb + e + 1]);
         if constexpr (BOTH) ppk[e >> 1] = pack2(p0, p1);
       }
       W[hb] = __builtin_bit_cast(bf16x8, u32x4{wpk[0], wpk[1], wpk[2], wpk[3]});
@@ -581,9 +554,7 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     }
     if constexpr (LA3 > 0) {  // merged pass: a window over the transposing reads of both accumulations
       auto frag3 = [&](int n) __attribute__((always_inline)) {
-        const int jv = n >> 1;
-        const __bf16* src = base + v_off[jv % ND] + (jv / ND) * L::VH + ((n & 1) ? kBTileB : 0);
-        return read_vt_b(src, src + L::V8);
+        return vt_frag(base, n >> 1, n & 1);
       };
       bf16x8 w3[LA3];
 #pragma unroll
@@ -599,24 +570,31 @@ __device__ __forceinline__ void attn_bwd_body(const BwdArgs& a) {
     } else
 #pragma unroll
     for (int jv = 0; jv < 2 * ND; ++jv) {
-      const __bf16* src = base + v_off[jv % ND] + (jv / ND) * L::VH;
       if constexpr (LA > 0) {
         acc[jv % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(win[(2 * NJ + jv) % LA], W[jv / ND], acc[jv % ND], 0, 0, 0);
         if (jv + LA < 2 * ND) win[(2 * NJ + jv) % LA] = frag(2 * NJ + jv + LA);
         __builtin_amdgcn_sched_barrier(0);
         continue;
       }
-      const bf16x8 f = read_vt_b(src, src + L::V8);
+      const bf16x8 f = vt_frag(base, jv, 0);
       acc[jv % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, W[jv / ND], acc[jv % ND], 0, 0, 0);
       if constexpr (BOTH) {
-        const bf16x8 f2 = read_vt_b(src + kBTileB, src + kBTileB + L::V8);
+        const bf16x8 f2 = vt_frag(base, jv, 1);
         acc2[jv % ND] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f2, Wp[jv / ND], acc2[jv % ND], 0, 0, 0);
       }
     }
+  };
+  if constexpr (CONST) {
+    for (int t = 0; t < nt; t += 2) {
+      tile(t, std::integral_constant<int, 0>{});
+      if (t + 1 >= nt) break;
+      tile(t + 1, std::integral_constant<int, 1>{});
+    }
+  } else {
+    for (int t = 0; t < nt; ++t) tile(t, t & 1);
   }
 
-  const float osc = HAS2 ? a.scale : 1.0f;  // dq = scale * dS k, dk = scale * dS^T q
-  static_assert(NW * kStageRows <= 2 * kBStage * 2, "the output staging tiles must fit the ring's LDS");
+  const float osc = a.scale;  // dq = scale * dS k, dk = scale * dS^T q
   // the lane number once more: the loop has no register for it (spills at head dim 128)
   const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   __syncthreads();  // every wave has finished reading the ring, and no load into it is in flight: it now stages the outputs
@@ -727,9 +705,9 @@ inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t 
 
 template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
 int launch_bwd_nw(hipStream_t st, BwdArgs a, int B) {
-  // the ring, or in front of it the waves' staged rows
-  constexpr int ring = 2 * bwd_slot_elems<MODE, HD, BIAS>() * 2, staged = NW * bwd_staged<MODE, HD>() * BwdLayout<HD>::TileA * 2;
-  constexpr int lds_bytes = ring > staged ? ring : staged;
+  // the ring, or in front of it the waves' staged rows and behind it their staged outputs
+  constexpr int ring = 2 * bwd_slot_bytes<MODE, HD, BIAS>(), staged = NW * bwd_staged<MODE, HD>() * BwdTile<HD>::Bytes, stored = NW * kStageRows;
+  constexpr int lds_bytes = ring > staged ? (ring > stored ? ring : stored) : (staged > stored ? staged : stored);
   a.net = (a.Se + NW * 32 - 1) / (NW * 32);
   const int64_t total = (int64_t)B * a.H * a.net * a.nsplit;
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
@@ -851,22 +829,20 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   a.tiles = tiles; a.tiles_sb = key_tiles_ints(Skv, 32);
   auto set = [](int64_t& sb, int64_t& ss, int64_t& sh, const mdattn_strides* s) { sb = s->batch; ss = s->seq; sh = s->head; };
   // dq: entity q / dout, stream k (scores), v (dP), k (accumulate)
-  a.e1 = (const __bf16*)q; a.e2 = (const __bf16*)dout; a.s1 = (const __bf16*)k; a.s2 = (const __bf16*)v; a.s3 = (const __bf16*)k;
+  a.e1 = (const __bf16*)q; a.e2 = (const __bf16*)dout; a.s1 = (const __bf16*)k; a.s2 = (const __bf16*)v;
   a.out = (__bf16*)dq; a.Se = Sq; a.Ss = Skv;
   set(a.e1_sb, a.e1_ss, a.e1_sh, q_strides); set(a.e2_sb, a.e2_ss, a.e2_sh, o_strides);
-  set(a.s1_sb, a.s1_ss, a.s1_sh, k_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, v_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, k_strides);
+  set(a.s1_sb, a.s1_ss, a.s1_sh, k_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, v_strides);
   set(a.o_sb, a.o_ss, a.o_sh, q_strides);
   a.waves = pq.waves; a.nsplit = pq.nsplit; a.tps = pq.tps; a.part = workspace + 2 * rows; a.part2 = nullptr;
   int rc = launch_bwd_any<0>(st, a, B);
   if (rc != MDATTN_OK) return rc;
   if (pq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B)) != MDATTN_OK) return rc;
   // dk and dv in one pass: entity k / v, stream q (scores, and accumulate for dk), dout (dP, and accumulate for dv)
-  a.e1 = (const __bf16*)k; a.e2 = (const __bf16*)v; a.s1 = (const __bf16*)q; a.s2 = (const __bf16*)dout; a.s3 = (const __bf16*)q;
-  a.s4 = (const __bf16*)dout;
+  a.e1 = (const __bf16*)k; a.e2 = (const __bf16*)v; a.s1 = (const __bf16*)q; a.s2 = (const __bf16*)dout;
   a.out = (__bf16*)dk; a.out2 = (__bf16*)dv; a.Se = Skv; a.Ss = Sq;
   set(a.e1_sb, a.e1_ss, a.e1_sh, k_strides); set(a.e2_sb, a.e2_ss, a.e2_sh, v_strides);
-  set(a.s1_sb, a.s1_ss, a.s1_sh, q_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, o_strides); set(a.s3_sb, a.s3_ss, a.s3_sh, q_strides);
-  set(a.s4_sb, a.s4_ss, a.s4_sh, o_strides);
+  set(a.s1_sb, a.s1_ss, a.s1_sh, q_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, o_strides);
   set(a.o_sb, a.o_ss, a.o_sh, k_strides); set(a.o2_sb, a.o2_ss, a.o2_sh, v_strides);
   a.waves = pkv.waves; a.nsplit = pkv.nsplit; a.tps = pkv.tps; a.part2 = a.part + pkv.floats;
   rc = launch_bwd_any<3>(st, a, B);
