@@ -327,14 +327,27 @@ std::optional<Table> as_table(const OptTensor& a, const OptTensor& b, int64_t s,
   t.cos = *a;
   return t;
 }
+// Replaces a tensor, or two of the same form (b may be undefined), by copies: dense ones in one launch, others as clones.
+void own(Tensor& a, Tensor& b) {
+  at::NoGradGuard guard;
+  const auto dense = [](const Tensor& t) { return t.is_cuda() && t.is_contiguous() && aligned(t) && !t.is_conj() && !t.is_neg(); };
+  if (dense(a) && a.nbytes() > 0 && a.nbytes() % 16 == 0 && (!b.defined() || (dense(b) && b.nbytes() == a.nbytes() && b.get_device() == a.get_device()))) {
+    Tensor x = at::empty(a.sizes(), a.options()), y = b.defined() ? at::empty(b.sizes(), b.options()) : Tensor();
+    if (mdattn_host_copy(stream(), ptr(a), mut(x), ptr(b), mut(y), (int64_t)a.nbytes()) == MDATTN_OK) {
+      a = x;
+      b = y;
+      return;
+    }
+  }
+  a = a.clone();
+  if (b.defined()) b = b.clone();
+}
 // The table as a node keeps it.  One that is read in place belongs to the caller, who may have made it in inference mode (autograd
-// refuses to save such a tensor) or may rewrite it before the backward: a dense copy of it, one launch (two for two planes),
-// where it was split into planes of its own before.  Half planes [S, D/2] were always saved as they are.
+// refuses to save such a tensor) or may rewrite it before the backward: a dense copy of it, one launch.  Half planes [S, D/2] were
+// always saved as they are.
 void own_table(Table& t) {
   if (!t.cos.defined() || t.kind == MDATTN_TABLE_PLANES) return;
-  at::NoGradGuard guard;
-  t.cos = t.cos.clone();
-  if (t.sin.defined()) t.sin = t.sin.clone();
+  own(t.cos, t.sin);
 }
 const float* table_ptr(const Tensor& t) { return t.defined() ? static_cast<const float*>(t.data_ptr()) : nullptr; }
 bool weight_ok(const Tensor& w, int64_t n, const Tensor& ref) { return bf16_on(w, ref) && w.is_contiguous() && w.numel() == n; }
@@ -591,7 +604,9 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     if (out.empty()) throw Refused{};
     // a weight with a factor is saved as a copy, as its product with the factor was: the caller's may be an inference tensor, or
     // be updated before the backward
-    ctx->save_for_backward({q, k, p.w_mul == 1.0 ? wq : wq.clone(), wk, cos, sin});
+    Tensor kept_wq = wq, none;
+    if (p.w_mul != 1.0) own(kept_wq, none);
+    ctx->save_for_backward({q, k, kept_wq, wk, cos, sin});
     ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode, (int64_t)q.scalar_type()});
     ctx->saved_data["f"] = c10::List<double>({p.eps, p.w_mul});
     ctx->set_materialize_grads(false);  // an output that the loss does not reach: no gradient for its input and weight

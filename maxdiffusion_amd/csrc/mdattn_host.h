@@ -19,6 +19,10 @@ int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D);
 int64_t mdattn_host_key_tiles_ints(int B, int Skv);
 int mdattn_host_key_tiles(void* stream, const void* keep, float* bias, int* tiles, int B, int Skv, int64_t bias_stride);
 
+/* Dense copies of one buffer, or of two (src1 and dst1 not null) of the same size, in one launch.  16-byte aligned, bytes a multiple
+ * of 16. */
+int mdattn_host_copy(void* stream, const void* src0, void* dst0, const void* src1, void* dst1, int64_t bytes);
+
 /* mdattn_quant_e4m3 of an attention call's q (premul q_premul, power-of-two scale), k (power-of-two scale) and v in two
  * launches.  ws: mdattn_host_quant3_floats floats, 16-byte aligned, of which [2 t] and [2 t + 1] become scale and absmax of
  * tensor t. */

@@ -360,3 +360,18 @@ def test_other_threads_run_during_a_call(dev):
     sys.setswitchinterval(interval)
     t.join()
   assert seen
+
+
+@pytest.mark.parametrize("n,two", [(4, False), (4 * 255, True), (4 * 256, False), (4 * 257, True), (128 * 4608, True)])
+def test_copies_of_one_and_two_buffers(dev, lib, n, two):
+  """mdattn_host_copy at the edges of its workgroups: what a training prologue keeps of a rotary table."""
+  import ctypes
+
+  a, b = torch.randn(n, device=dev), torch.randn(n, device=dev)
+  x, y = torch.zeros(n + 4, device=dev), torch.zeros(n + 4, device=dev)
+  P = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else None)
+  rc = lib.mdattn_host_copy(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), P(a), P(x), P(b if two else None),
+                            P(y if two else None), ctypes.c_int64(4 * n))
+  assert rc == 0
+  assert torch.equal(x[:n], a) and not x[n:].any()
+  assert torch.equal(y[:n], b if two else torch.zeros_like(b)) and not y[n:].any()
