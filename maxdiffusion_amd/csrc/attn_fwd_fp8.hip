@@ -271,20 +271,6 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
     };
     int zero = 0;
     asm volatile("" : "+s"(zero));  // an address the compiler cannot match with the hot path's: no reuse of its logits
-    // A row's reference point starts at the maximum of its first tile, formed in front of the softmax that the branch below would
-    // do twice.  With it, no request past the last tile, the tail's -inf only where there is a tail and whole-row stores: the whole
-    // entry 12 heads x 500 tokens 17.6 -> 15.8 us, 5 x 1,134 23.1 -> 21.8, 40 x 6,120 426 -> 417, 40 x 32,760 the same.
-    if (!BIAS && t == 0) {
-      float mx = row_max(Ks + zero);
-      if constexpr (PRE) {
-        if constexpr (CODE) mx = (mx - kCodeOne) * 0.125f;
-        ref += mx - kPOff;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) negref[i] = CODE ? kCodeOne - 8.0f * ref : -ref;
-      } else {
-        ref = fmaxf(ref, mx * c - kPOff);
-      }
-    }
     // ---- P = exp2(c*S - ref), f32 row sum, e4m3 pack in B-operand order.  The hot path takes no row
     // maximum: P is formed against the current reference point, and only a lane's sum over the tile (32 of the
     // row's 64 probabilities) beyond e4m3's largest value, so possibly one probability beyond it, sends the wave
@@ -344,7 +330,7 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
     // (a byte 0x7F decodes to NaN and poisons the sum; bytes above it are caught by their top bit)
     // PRE: a row's reference is set by the first tile in which it meets a finite logit: tile 0, unless a key bias
     // excludes all of that tile's keys (`fresh` then stays set and the row tries again on the next tile)
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(ls <= (CODE ? 3.0e38f : kPTrig)) || (hib & 0x80808080u) != 0u || (PRE && BIAS && fresh)) != 0, 0)) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(ls <= (CODE ? 3.0e38f : kPTrig)) || (hib & 0x80808080u) != 0u || (PRE && BIAS && fresh)) != 0 || (PRE && !BIAS && t == 0), 0)) {
       asm volatile("" : "+s"(zero));
       float mx = row_max(Ks + zero);
       float alpha;
@@ -357,8 +343,8 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
           alpha = fresh ? 0.f : __builtin_amdgcn_exp2f(-dm);
           fresh = fresh && !first;
         } else {
-          dm = fmaxf(mx - kPOff, 0.f);
-          alpha = __builtin_amdgcn_exp2f(-dm);
+          dm = t == 0 ? mx - kPOff : fmaxf(mx - kPOff, 0.f);
+          alpha = t == 0 ? 0.f : __builtin_amdgcn_exp2f(-dm);
         }
         ref += dm;
 #pragma unroll
@@ -429,7 +415,9 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
   tile(nt - 1, slot, std::true_type{});
 
   // ---- epilogue: the wave's 32 rows through the ring's LDS, so that a store instruction writes whole rows (as the lanes hold them it
-  // would write 16 bytes of each of 32 rows)
+  // would write 16 bytes of each of 32 rows).  With it, no request past the last tile and the tail's -inf only where there is a
+  // tail: the whole entry 40 heads x 32,760 tokens 8,945 -> 8,870 us, 20 x 6,762 277 -> 270, 12 x 500 17.1 -> 16.0.  (The first tile's
+  // maximum in front of its softmax, as the bf16 kernel takes it, costs the long call 0.9 % and gives the short ones nothing.)
   const float lt = CODE ? l : xhalf_sum(l);  // MODE 2: the MFMA already summed both halves of the row's keys
   const float inv = lt > 0.f ? a.v_scale[0] / lt : 0.f;  // rows whose keys are all excluded return 0 (and lse = -inf)
   constexpr int kRowB = HD * 2 + 16, kLPR = HD / 8, kRPS = 64 / kLPR;  // bytes of a staged row, lanes per row and rows per store
