@@ -10,7 +10,7 @@
 //                 once per tile; P feeds the dv accumulators and dS the dk ones: seven matrix products per call
 //                 where five are necessary (S and dP are formed in both passes).
 // Stream rows are walked in tiles of 32 through a 2-slot LDS ring filled by direct global->LDS loads.
-// Per tile, with the forward kernel's layouts and fragment reads:
+// Per tile, with the forward kernel's fragment orders:
 //   S^T  = stream1 . entity1^T      (A = tile rows by ds_read_b128, B = entity fragments)   lane = entity row
 //   dP^T = stream2 . entity2^T
 //   W    = exp2(c*S - lse*log2e) [* (dP - delta)]     f32, packed to bf16 in B-operand order (the factor `scale` of
