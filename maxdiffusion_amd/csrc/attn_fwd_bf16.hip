@@ -662,8 +662,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // that hold excluded keys.  4,096 keys and queries x 10 heads, nothing dropped / a key in every tile, from the bias: 106 / 106 us at head
   // dim 128, 72 / 71 at 64, 93 / 93 at 80; behind the chain: 100 / 110, 70 / 80, 89 / 99.
   constexpr bool kBiasFirst = BIAS == kKeyMask && ND < 4;
-  // kt: the tile; first: of this workgroup; mixed (kKeyMask): it holds excluded keys; slot: int or integral_constant
-  auto tile = [&](int kt, bool first, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {
+  // kt: the tile; first: of this workgroup, bool or integral_constant; mixed (kKeyMask): it holds excluded keys; slot: int or integral_constant
+  auto tile = [&](int kt, auto first, bool mixed, auto slot, auto masked) __attribute__((always_inline)) {
     const __bf16* base = smem + slot * STAGE;
     constexpr int kBlk = 32 * 64;  // a 32-key block of a head-dim-64 tile: 32 rows of 64 elements, in K and in V
     auto frag = [&](int n) __attribute__((always_inline)) {
@@ -902,35 +902,40 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       rf = rows(ef >> 1);
     }
   }
-  auto step = [&](int t, auto slot, int fill) __attribute__((always_inline)) {
+  // (with two slots the tile after t < nt - 1 exists: no question)
+  auto step = [&](int t, auto first, auto slot, int fill) __attribute__((always_inline)) {
     // vmcnt: this wave's share of tile t has landed (the SLOTS - 2 tiles requested after it may still be in flight)
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((SLOTS - 2) * (2 * GPW + (BIAS ? 1 : 0))));
     __syncthreads();                                  // ... and everyone's; slot `fill` (tile t-1) is free
     if constexpr (BIAS == kKeyMask) {
-      if (t + SLOTS - 1 < nt) dma(fill, ef >> 1, rf);
-      tile(ec >> 1, t == 0, ec & 1, slot, std::false_type{});
+      if (SLOTS == 2 || t + SLOTS - 1 < nt) dma(fill, ef >> 1, rf);
+      tile(ec >> 1, first, ec & 1, slot, std::false_type{});
       ec = SLOTS == 3 ? en : ef;
       en = ef;
       ef = entry(t + SLOTS);
       rf = rows(ef >> 1);
     } else {
-      if (t + SLOTS - 1 < nt) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
-      tile(t, t == 0, false, slot, std::false_type{});
+      if (SLOTS == 2 || t + SLOTS - 1 < nt) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
+      tile(t, first, false, slot, std::false_type{});
     }
   };
   if constexpr (HD == 64) {
     // Two copies of the loop body, one per ring slot: the slot is a compile-time constant in each, every fragment
     // address a lane constant plus an immediate offset, and the address arithmetic per tile is gone from a kernel that
-    // is bound by vector issue (1 % at 32 heads x 13,376 tokens; at head dim 128 the copies cost registers and lose).
-    for (int t = 0; t < nt - 1; t += 2) {
-      step(t, std::integral_constant<int, 0>{}, 1);
+    // is bound by vector issue (1 % at 32 heads x 13,376 tokens; at head dim 128 the copies cost registers and lose).  The first
+    // tile is a copy of its own: asked for in every tile it cost a SIMD with one wave 2 % (1 head x 11,007 keys and queries 138.7 us,
+    // 135.9 now, 5 x 5,368 69.8 and 68.7).  At head dim 128 that copy gave nothing at full tiles and lost 1 to 5 % with a tail of the
+    // last round at two workgroups per CU.
+    if (nt > 1) step(0, std::true_type{}, std::integral_constant<int, 0>{}, 1);
+    for (int t = 1; t < nt - 1; t += 2) {
+      step(t, std::false_type{}, std::integral_constant<int, 1>{}, 0);
       if (t + 1 >= nt - 1) break;
-      step(t + 1, std::integral_constant<int, 1>{}, 0);
+      step(t + 1, std::false_type{}, std::integral_constant<int, 0>{}, 1);
     }
   } else {
     int slot = 0, fill = SLOTS - 1;
     for (int t = 0; t < nt - 1; ++t) {
-      step(t, slot, fill);
+      step(t, t == 0, slot, fill);
       slot = slot == SLOTS - 1 ? 0 : slot + 1;
       fill = fill == SLOTS - 1 ? 0 : fill + 1;
     }

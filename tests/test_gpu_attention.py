@@ -445,3 +445,16 @@ def test_few_query_tiles_against_many_keys(dev, folded, H, sq, skv):
     o_run, l_run = ops.new_merge_state(1, sq, H, 128, dev)
     ops.flash_attention_merge(to_dev_bf16(q, dev), to_dev_bf16(keys, dev), to_dev_bf16(v, dev), o_run, l_run, scale=scale)
     _check(hsd(to_np(o_run)[:, rows]), to_np(l_run)[0][:, rows], ro, rl, "as a ring step")
+
+
+@pytest.mark.parametrize("folded", [False, True])
+@pytest.mark.parametrize("skv", [64, 65, 128, 129, 192, 250, 256, 257, 321, 384])
+def test_head_dim_64_one_to_six_key_tiles(dev, folded, skv):
+  """The first tile and the last have their own copies of the loop's body, the ones between take turns in two: every count at which one
+  of them is left out or is the same tile as another; sharp logits, so that reference points move behind the first tile."""
+  q, k, v = O.normal_bf16((1, 70, 3, 64), 0), O.normal_bf16((1, skv, 3, 64), 1), O.normal_bf16((1, skv, 3, 64), 2)
+  q = O.bf16_round(q * np.float32(5.0 * (ops.folded_q_mul(64) if folded else 1.0)))
+  scale = ops.FOLDED_SCALE if folded else 64**-0.5
+  out, lse = _run_np(q, k, v, dev, scale=scale)
+  ro, rl = O.attention(hsd(q), hsd(k), hsd(v), scale)
+  _check(hsd(out), lse[0], ro, rl, f"folded={folded} Skv={skv}")
