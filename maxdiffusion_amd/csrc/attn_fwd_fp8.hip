@@ -256,21 +256,6 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
         }
       }
     };
-    // The largest logit of each row's keys in the tile, the logits recomputed rather than kept: the hot path holds them only while
-    // it forms P.
-    auto row_max = [&](const char* Kb) __attribute__((always_inline)) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int blk = 0; blk < 2; ++blk) {
-        f32x16 S;
-        qk(S, blk, Kb);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, S[i]);
-      }
-      return xhalf_max(mx);
-    };
-    int zero = 0;
-    asm volatile("" : "+s"(zero));  // an address the compiler cannot match with the hot path's: no reuse of its logits
     // ---- P = exp2(c*S - ref), f32 row sum, e4m3 pack in B-operand order.  The hot path takes no row
     // maximum: P is formed against the current reference point, and only a lane's sum over the tile (32 of the
     // row's 64 probabilities) beyond e4m3's largest value, so possibly one probability beyond it, sends the wave
@@ -330,9 +315,20 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
     // (a byte 0x7F decodes to NaN and poisons the sum; bytes above it are caught by their top bit)
     // PRE: a row's reference is set by the first tile in which it meets a finite logit: tile 0, unless a key bias
     // excludes all of that tile's keys (`fresh` then stays set and the row tries again on the next tile)
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(ls <= (CODE ? 3.0e38f : kPTrig)) || (hib & 0x80808080u) != 0u || (PRE && BIAS && fresh)) != 0 || (PRE && !BIAS && t == 0), 0)) {
-      asm volatile("" : "+s"(zero));
-      float mx = row_max(Ks + zero);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(ls <= (CODE ? 3.0e38f : kPTrig)) || (hib & 0x80808080u) != 0u || (PRE && BIAS && fresh)) != 0 ||
+                         (PRE && !BIAS && t == 0), 0)) {
+      // The logits are recomputed rather than kept: the hot path holds them only while it forms P.
+      int zero = 0;
+      asm volatile("" : "+s"(zero));  // an address the compiler cannot match with the hot path's: no reuse of its logits
+      float mx = -INFINITY;
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        f32x16 S;
+        qk(S, blk, Ks + zero);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, S[i]);
+      }
+      mx = xhalf_max(mx);
       float alpha;
       if constexpr (PRE) {  // the logits are relative to the old reference (MODE 2: in code units, 56 at the reference)
         if constexpr (CODE) mx = (mx - kCodeOne) * 0.125f;
@@ -402,13 +398,29 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
   dma(0, 0);
   if (nt > 1) dma(1, 1);
   int slot = 0, fill = 2;
-  for (int t = 0; t < nt - 1; ++t) {
+  // Head dim 64 without a bias: the one step that requests nothing is a copy of its own, and the epilogue takes the lane's number
+  // from the loop.  Elsewhere the copy costs registers (spills), and so do the rows' places, which the compiler would form in front of
+  // the loop: there the epilogue asks for the lane once more.  Asked for in every step and with the places in registers, few rows
+  // against long sequences lost 2 %: 20 heads of 64 x 64 x 17,310 128.7 us, 125.4 now (130 with the lane asked for again), 40 of 128 x
+  // 88 x 18,145 174.8 and 173.5, under a mask 8 of 128 x 1,000 x 4,000 66.9 and 65.0.
+  constexpr bool LEAN = HD == 64 && !BIAS;
+  auto arrived = [&]() __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * GPW + (BIAS ? 1 : 0)));  // vmcnt: this wave's share of tile t has landed
     __syncthreads();                                  // ... and everyone's; slot `fill` (tile t-1) is free
-    if (t + 2 < nt) dma(fill, t + 2);
+  };
+  auto work = [&](int t) __attribute__((always_inline)) {
     tile(t, slot, std::false_type{});
     slot = slot == kSlots8 - 1 ? 0 : slot + 1;
     fill = fill == kSlots8 - 1 ? 0 : fill + 1;
+  };
+  for (int t = 0; t < (LEAN ? nt - 2 : nt - 1); ++t) {
+    arrived();
+    if (LEAN || t + 2 < nt) dma(fill, t + 2);
+    work(t);
+  }
+  if (LEAN && nt > 1) {
+    arrived();
+    work(nt - 2);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
@@ -418,6 +430,8 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
   // would write 16 bytes of each of 32 rows).  With it, no request past the last tile and the tail's -inf only where there is a
   // tail: the whole entry 40 heads x 32,760 tokens 8,945 -> 8,870 us, 20 x 6,762 277 -> 270, 12 x 500 17.1 -> 16.0.  (The first tile's
   // maximum in front of its softmax, as the bf16 kernel takes it, costs the long call 0.9 % and gives the short ones nothing.)
+  const int ln = LEAN ? lane : (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const int r32 = LEAN ? l32 : ln & 31, half = LEAN ? hh : ln >> 5;
   const float lt = CODE ? l : xhalf_sum(l);  // MODE 2: the MFMA already summed both halves of the row's keys
   const float inv = lt > 0.f ? a.v_scale[0] / lt : 0.f;  // rows whose keys are all excluded return 0 (and lse = -inf)
   constexpr int kRowB = HD * 2 + 16, kLPR = HD / 8, kRPS = 64 / kLPR;  // bytes of a staged row, lanes per row and rows per store
@@ -431,19 +445,19 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
       uint2 u;
       u.x = pack2(O[sl][4 * g] * inv, O[sl][4 * g + 1] * inv);
       u.y = pack2(O[sl][4 * g + 2] * inv, O[sl][4 * g + 3] * inv);
-      *reinterpret_cast<uint2*>(stage + l32 * kRowB + (sl * 32 + 8 * g + 4 * hh) * 2) = u;
+      *reinterpret_cast<uint2*>(stage + r32 * kRowB + (sl * 32 + 8 * g + 4 * half) * 2) = u;
     }
-  if (a.lse && hh == 0 && q0 + l32 < a.Sq)
-    a.lse[((int64_t)b * a.H + h) * a.Sq + q0 + l32] = (ref + __log2f(lt) - (CODE ? kCodeBiasLog2 : 0.f)) * kLn2;
+  if (a.lse && half == 0 && q0 + r32 < a.Sq)
+    a.lse[((int64_t)b * a.H + h) * a.Sq + q0 + r32] = (ref + __log2f(lt) - (CODE ? kCodeBiasLog2 : 0.f)) * kLn2;
   // LDS accesses of one wave execute in order: the reads see the writes above
-  const int rr = lane / kLPR, cc = lane % kLPR;
+  const int rr = ln / kLPR, cc = ln % kLPR;
   __bf16* p = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(q0 + rr) * a.o_ss + cc * 8;
-  const int64_t step = (int64_t)kRPS * a.o_ss;
+  const int64_t pitch = (int64_t)kRPS * a.o_ss;
   uint4 v[32 / kRPS];
 #pragma unroll
   for (int j = 0; j < 32 / kRPS; ++j) v[j] = *reinterpret_cast<const uint4*>(stage + (j * kRPS + rr) * kRowB + cc * 16);
 #pragma unroll
-  for (int j = 0; j < 32 / kRPS; ++j, p += step)
+  for (int j = 0; j < 32 / kRPS; ++j, p += pitch)
     if (q0 + j * kRPS + rr < a.Sq) st_nt(reinterpret_cast<uint4*>(p), v[j]);
 }
 
