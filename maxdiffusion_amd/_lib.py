@@ -63,6 +63,7 @@ SIGNATURES = {
 HOST_SIGNATURES = {
     "mdattn_bwd_split_workspace_floats": ([_I, _I, _I, _I, _I], _L),
     "mdattn_host_fwd_workspace_floats": ([_I, _I, _I, _I, _I], _L),
+    "mdattn_host_fwd_schedule": ([_I, _I, _I, _I, _I, _F], _I),
     "mdattn_host_norm_rope_fullrow": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _S], _I),
     "mdattn_host_norm_rope_qkv": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _S], _I),
     "mdattn_host_norm_rope_perhead": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _F, _S, _S], _I),

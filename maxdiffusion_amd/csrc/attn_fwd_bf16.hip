@@ -963,6 +963,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   store_rows_through_lds<ND, PADDED>(a, O, xhalf_sum(l), mc, b, h, q0, lane, smem_raw + wave * 32 * (ND * 64 + 16));
 }
 
+// scale * log2(e) == 1 (to f32 round-off): the caller folded the factor into q, and the kernels that leave the multiply per logit out run
+inline bool folded(float c) { return c > 1.0f - 1e-6f && c < 1.0f + 1e-6f; }
+
 template <int NW, int BIAS, int HD = 128, int DC = 0>
 static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   constexpr int BM = NW * 32;
@@ -980,9 +983,8 @@ static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
-  // scale * log2(e) == 1 (to f32 round-off): the caller folded the factor into q; the logits need no multiply.
   // With a key bias the logits are touched after the MFMAs anyway, so that variant keeps its FMA.
-  const bool pre = !BIAS && a.c > 1.0f - 1e-6f && a.c < 1.0f + 1e-6f;
+  const bool pre = !BIAS && folded(a.c);
   if (pre) MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, !BIAS, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   else MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, false, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   return launch_status();
@@ -1028,8 +1030,7 @@ static int launch_fwd(hipStream_t st, AttnArgs a, int B) {
   if (total > (int64_t)0x7FFFFFF0) return MDATTN_E_UNSUPPORTED;
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
-  // scale * log2(e) == 1 (to f32 round-off): the caller folded the factor into q; the logits need no multiply
-  const bool pre = a.c > 1.0f - 1e-6f && a.c < 1.0f + 1e-6f;
+  const bool pre = folded(a.c);
   auto kern = pre ? attn_fwd_bf16_kernel<NW, true> : attn_fwd_bf16_kernel<NW, false>;
   static LdsOptIn opted[2];
   if (lds_opt_in(opted[pre], reinterpret_cast<const void*>(kern), lds_bytes) != MDATTN_OK) return MDATTN_E_LAUNCH;
@@ -1069,25 +1070,29 @@ static int fill_args(AttnArgs& a, const void* q, const void* k, const void* v, v
   return MDATTN_OK;
 }
 
-// The schedule of a call at head dim 128 (1: pipelined, eight waves; 2: pipelined, four; 3: flat) by the lowest time in us; nt: 32-key
-// tiles.  Fitted to 1 .. 40 heads x 126 .. 40,000 queries x 126 .. 8,192 keys, within 10 % from 1,024 keys on:
+// The schedule of a call at head dim 128 whose keys are not cut (1: pipelined, eight waves; 2: pipelined, four; 3: flat) by the lowest
+// time in us; nt: 32-key tiles.  Fitted to 1 .. 40 heads x 126 .. 40,000 queries x 126 .. 8,192 keys, within 10 % from 1,024 keys on:
 //   pipelined, eight waves: one workgroup of 256 queries per CU, 0.55 us per tile while half of the CUs are busy, 0.82 (the power
 //     limit) when all are, rounds of 256;
 //   pipelined, four waves: 128 queries, one workgroup per CU, 0.41 to 0.47: the fastest where there is one for each CU at most;
-//   flat: 128 queries, three workgroups per CU, 0.55 / 0.92 / 1.34 with one, two, three of them; its start is the shortest.
-// Measured (pipelined 8 / pipelined 4 / flat): 20 heads x 1,024 queries x 4,096 keys 80 / 61 / 76, 4 x 8,192 x 4,096 80 / 67 / 80,
-// 40 x 2,048 x 4,096 188 / 193 / 164, 12 x 8,192 x 4,096 190 / 202 / 178, 20 x 16,384 x 4,096 553 / 662 / 567, 40 x 512 x 512 20.5 / 15.6 / 13.8.
+//   flat: 128 queries, three workgroups per CU, 0.55 / 0.93 / 1.34 with one, two, three of them, 0.65 / 0.72 (with the multiply per
+//     logit) when the first CU gets its second; its start is the shortest.
+// Measured through mdattn_fwd_bf16 and the ring step (pipelined 8 / pipelined 4 / flat; through mdattn_host_fwd_bf16 fwd_split below comes
+// first): 20 heads x 1,024 queries x 4,096 keys 80 / 61 / 76, 4 x 8,192 x 4,096 80 / 67 / 80, 40 x 2,048 x 4,096 188 / 193 / 164, 12 x 8,192 x 4,096
+// 190 / 202 / 178, 20 x 16,384 x 4,096 553 / 662 / 567, 40 x 512 x 512 20.5 / 15.6 / 13.8; 12 x 3,193 x 3,195, with the multiply 70 / 107 / 79, without
+// 68 / 103 / 70.  Over 340 shapes of 64 .. 2,048 workgroups and 32 .. 400 tiles the choice is 0.3 % behind the fastest on average.
 struct FwdSchedule {
   int variant;
   double us;
 };
-static FwdSchedule fwd_schedule(int64_t BH, int Sq, int Skv) {
+static FwdSchedule fwd_schedule(int64_t BH, int Sq, int Skv, bool pre) {
   const double nt = (Skv + 31) / 32;
   const int64_t w8 = BH * ((Sq + 255) / 256), w4 = BH * ((Sq + 127) / 128);
   const int64_t rest8 = w8 % 256, rest4 = w4 % 768;
   const double last8 = rest8 <= 128 ? 0.55 : 0.55 + 0.27 * (double)(rest8 - 128) / 128;
   const double us8 = 3.0 + (double)(w8 / 256) * (0.82 * nt + 7.5) + (rest8 ? last8 * nt + 7.5 : 0.0);
-  double last = rest4 == 0 ? 0.0 : rest4 <= 256 ? 0.55 : rest4 <= 512 ? 0.62 + 0.3 * (double)(rest4 - 256) / 256 : 1.22 + 0.1 * (double)(rest4 - 512) / 256;
+  const double two = (double)(rest4 - 256) / 256;
+  double last = rest4 == 0 ? 0.0 : rest4 <= 256 ? 0.55 : rest4 <= 512 ? (pre ? 0.65 + 0.28 * two : 0.72 + 0.26 * two) : 1.22 + 0.1 * (double)(rest4 - 512) / 256;
   if (w4 > 768 && rest4 > 0 && rest4 <= 512) last = rest4 <= 256 ? 0.48 : last < 0.8 ? 0.8 : last;  // the rounds before have not ended together
   FwdSchedule best{3, 4.0 + ((double)(w4 / 768) * 1.34 + last) * nt};
   if (us8 < best.us) best = {1, us8};
@@ -1097,11 +1102,15 @@ static FwdSchedule fwd_schedule(int64_t BH, int Sq, int Skv) {
   }
   return best;
 }
+extern "C" int mdattn_host_fwd_schedule(int B, int H, int Sq, int Skv, int D, float scale) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !native_head_dim(D)) return MDATTN_E_BADARG;
+  return D == kD ? fwd_schedule((int64_t)B * H, Sq, Skv, folded(scale * kLog2e)).variant : 3;
+}
 
 static int dispatch_fwd(hipStream_t st, const AttnArgs& a, int B, int Sq, int Skv, int D) {
   if (D == 64) return launch_flat<4, kNoBias, 64>(st, a, B);  // head dim 64: the flat schedule only
   // mdattn_set_fwd_schedule overrides the choice, for tests
-  const int forced = forced_fwd_schedule(), variant = forced ? forced : fwd_schedule((int64_t)B * a.H, Sq, Skv).variant;
+  const int forced = forced_fwd_schedule(), variant = forced ? forced : fwd_schedule((int64_t)B * a.H, Sq, Skv, folded(a.c)).variant;
   switch (variant) {
     case 1: return launch_fwd<8>(st, a, B);
     case 2: return launch_fwd<4>(st, a, B);
@@ -1137,8 +1146,13 @@ static FwdSplit fwd_split(int64_t BH, int Sq, int Skv, int D) {
     return tile_us * tps * (load > 1.0 ? load : 1.0);
   };
   double best_cost = 0.9 * walk(tiles, nt);
-  if (D == kD) {  // (the costs here leave out a workgroup's start, and are a tenth too high for 100 workgroups and more)
-    const FwdSchedule s = fwd_schedule(BH, Sq, Skv);
+  // Head dim 128: the whole call by its schedule's time, which the costs here meet when the workgroup's start, left out here, is taken
+  // off, and the flat kernel's lowered, the pipelined one's raised by a tenth.  The scale is not known here: the rates without the
+  // multiply.  Of 110 random calls that are cut, 1 .. 40 heads x 64 .. 8,192 queries x 1,000 .. 30,000 keys, two were more than 3 % slower
+  // than whole (24 x 1,298 x 12,731 253 us, 238 whole; 4 x 5,609 x 5,609 88 and 84), the others up to 7 times faster; 20 x 1,024 x 4,096 in two
+  // pieces 58 us, 60 whole, with the multiply 63 and 62.5.
+  if (D == kD) {
+    const FwdSchedule s = fwd_schedule(BH, Sq, Skv, true);
     const double whole = (s.variant == 2 ? 1.12 : 0.9) * (s.us - 4.0);
     best_cost = whole < best_cost ? whole : best_cost;
   }

@@ -42,6 +42,10 @@ int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void*
                          const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride, const int* tiles,
                          float* workspace, int64_t workspace_floats);
 
+/* The schedule (of mdattn_set_fwd_schedule) of a forward without a bias whose keys are not cut, as mdattn_fwd_bf16 and
+ * mdattn_fwd_bf16_merge choose it. */
+int mdattn_host_fwd_schedule(int B, int H, int Sq, int Skv, int D, float scale);
+
 /* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias with or without tiles) at the head dims of mdattn_host_fwd_bf16. */
 int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, void* dq,
                          void* dk, void* dv, float* workspace, int64_t workspace_floats, int B, int H, int Sq, int Skv, int D,
