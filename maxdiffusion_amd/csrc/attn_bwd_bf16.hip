@@ -663,10 +663,7 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
 // The stream is cut where its own rows leave a pass without workgroups: 12 heads x 32,760 queries x 512 keys: the dk / dv pass takes
 // 1312 us in one piece (24 workgroups) and 201 us in ten, + 13 us of bwd_reduce_kernel.
 constexpr int kMinSplitTiles = 8, kMaxSplit = 32;
-struct BwdPlan {
-  int waves, nsplit, tps;
-  int64_t floats;  // of one tensor's partials
-};
+using BwdPlan = mdattn_host_bwd_pass;
 inline double bwd_pass_us(int D, int tensors, int waves, int64_t wgs, int tps) {
   if (D <= 64) {  // workgroups of four waves, three per CU
     const double tile[3] = {tensors == 2 ? 0.74 : 0.54, tensors == 2 ? 1.15 : 0.8, tensors == 2 ? 1.45 : 1.1};  // with one, two, three of them
@@ -674,7 +671,7 @@ inline double bwd_pass_us(int D, int tensors, int waves, int64_t wgs, int tps) {
     return (double)(wgs / 768) * (tps * tile[2] + 4.0) + (rest ? tps * tile[(rest - 1) / 256] + 4.0 : 0.0);
   }
   const int slots = waves == 8 ? 256 : 512;
-  const int64_t rounds = wgs / slots, rest = wgs % slots;
+  const int64_t rounds = waves == 8 ? wgs / 256 : wgs / 512, rest = wgs - rounds * slots;
   const double tile = tensors == 2 ? (waves == 8 ? 1.65 : 1.75) : (waves == 8 ? 1.2 : 1.25);
   const double alone = waves == 8 ? tile : tensors == 2 ? 1.3 : 0.8;       // with the CU to itself
   const double full = tensors == 2 ? 0.0 : waves == 8 ? 10.0 : 5.5;        // of a start, when every CU reads its rows at once
@@ -687,20 +684,41 @@ inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t 
   const int nt = (Ss + kBT - 1) / kBT;
   const int64_t floats = BH * Se * D;
   const double partial = 1.5 * tensors * (double)floats * 4 / 5e6;  // (writing them is half hidden)
-  BwdPlan best{D > 64 ? 8 : 4, 1, nt, 0};
+  const int most = D > 64 ? 8 : 4;
+  BwdPlan best{most, 1, nt, 0};
   double best_cost = 1e300;
-  for (int waves = best.waves; waves >= 4; waves -= 4) {
+  for (int waves = most; waves >= 4; waves -= 4) {
     const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)), nt);
     if (cost < best_cost) { best_cost = cost; best.waves = waves; }
   }
-  for (int waves = D > 64 ? 8 : 4; waves >= 4; waves -= 4)
+  for (int waves = most; waves >= 4; waves -= 4) {
+    const int64_t entities = BH * ((Se + waves * 32 - 1) / (waves * 32));
+    // no cut is faster than its tiles on a full chip, the partials of two pieces and their launch
+    const double full_chip = D <= 64 ? (tensors == 2 ? 1.45 : 1.1) / 768 : waves == 8 ? (tensors == 2 ? 1.65 : 1.2) / 256 : (tensors == 2 ? 1.75 : 1.25) / 512;
+    if ((double)entities * nt * full_chip + 2 * partial + 6.0 >= best_cost * 0.95) continue;
     for (int n = 2; n <= kMaxSplit && nt / n >= kMinSplitTiles; ++n) {
       const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
       if (ns * floats * tensors > room) break;
-      const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)) * ns, tps) + partial * ns + 6.0;
+      const double cost = bwd_pass_us(D, tensors, waves, entities * ns, tps) + partial * ns + 6.0;
       if (cost < best_cost * 0.95) { best_cost = cost; best = {waves, ns, tps, ns * floats}; }
     }
+  }
   return best;
+}
+// The plan of a call without limits, and where a pass's partials do not fit, the best one for that pass that does.  Which cuts are
+// looked at decides where two are within 5 %: with the limit in the first search a call with the workspace of this very plan was launched
+// with another in one of forty shapes.
+inline mdattn_host_bwd_plan bwd_plans(int64_t BH, int Sq, int Skv, int D, int64_t room) {
+  mdattn_host_bwd_plan p{bwd_plan(BH, Sq, Skv, D, 1, INT64_MAX), bwd_plan(BH, Skv, Sq, D, 2, INT64_MAX)};
+  if (p.dq.floats > room) p.dq = bwd_plan(BH, Sq, Skv, D, 1, room);
+  if (2 * p.dkv.floats > room) p.dkv = bwd_plan(BH, Skv, Sq, D, 2, room);
+  return p;
+}
+// whether a pass of this plan covers its Ss stream rows, without an empty piece, and says the space it takes
+inline bool bwd_plan_ok(const BwdPlan& p, int64_t BH, int Se, int Ss, int D) {
+  const int64_t nt = ((int64_t)Ss + kBT - 1) / kBT;
+  return (p.waves == 4 || (p.waves == 8 && D > 64)) && p.pieces >= 1 && p.tiles >= 1 && (int64_t)p.pieces * p.tiles >= nt &&
+         (int64_t)(p.pieces - 1) * p.tiles < nt && p.floats == (p.pieces > 1 ? p.pieces * BH * Se * D : 0);
 }
 
 template <int MODE, int HD, bool BIAS, bool PRE, int DC, int NW>
@@ -779,12 +797,23 @@ extern "C" int64_t mdattn_bwd_workspace_floats(int B, int H, int Sq) {
   return 2 * (int64_t)B * H * (((int64_t)Sq + 31) / 32 * 32);
 }
 
+// the two passes run one after the other and their partials share the space
+static int64_t plan_floats(int B, int H, int Sq, const mdattn_host_bwd_plan& p) {
+  return mdattn_bwd_workspace_floats(B, H, Sq) + (p.dq.floats > 2 * p.dkv.floats ? p.dq.floats : 2 * p.dkv.floats);
+}
+
 extern "C" int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !native_head_dim(D)) return 0;
   const int64_t BH = (int64_t)B * H;
-  // the two passes run one after the other and their partials share the space
-  const int64_t dq = bwd_plan(BH, Sq, Skv, D, 1, INT64_MAX).floats, dkv = 2 * bwd_plan(BH, Skv, Sq, D, 2, INT64_MAX).floats;
-  return mdattn_bwd_workspace_floats(B, H, Sq) + (dq > dkv ? dq : dkv);
+  return plan_floats(B, H, Sq, bwd_plans(BH, Sq, Skv, D, INT64_MAX));
+}
+
+extern "C" int64_t mdattn_host_bwd_plan_floats(int B, int H, int Sq, int Skv, int D, int64_t workspace_floats, mdattn_host_bwd_plan* plan) {
+  const int64_t base = mdattn_bwd_workspace_floats(B, H, Sq);
+  if (base == 0 || Skv <= 0 || !native_head_dim(D) || (workspace_floats >= 0 && workspace_floats < base)) return 0;
+  const mdattn_host_bwd_plan p = bwd_plans((int64_t)B * H, Sq, Skv, D, workspace_floats < 0 ? INT64_MAX : workspace_floats - base);
+  if (plan) *plan = p;
+  return plan_floats(B, H, Sq, p);
 }
 
 // Shared body of mdattn_bwd_bf16 and mdattn_bwd_bf16_static: validation and the two passes.
@@ -793,7 +822,8 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
                    int B, int H, int Sq, int Skv, int D,
                    const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                    const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                   const float* key_bias, int64_t bias_stride, bool any_head_dim = false, const int* tiles = nullptr) {
+                   const float* key_bias, int64_t bias_stride, bool any_head_dim = false, const int* tiles = nullptr,
+                   const mdattn_host_bwd_plan* plan = nullptr) {
   if (!q || !k || !v || !out || !dout || !lse || !dq || !dk || !dv || !workspace) return MDATTN_E_BADARG;
   if (key_bias) {
     if (bias_stride < ((int64_t)Skv + 31) / 32 * 32 || bias_stride % 32 != 0) return MDATTN_E_BADARG;
@@ -822,7 +852,9 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
 
   // a stream is cut as far as the caller's workspace holds the partials (it always holds lse2 and delta)
   const int64_t BH = (int64_t)B * H;
-  const BwdPlan pq = bwd_plan(BH, Sq, Skv, D, 1, workspace_floats - 2 * rows), pkv = bwd_plan(BH, Skv, Sq, D, 2, workspace_floats - 2 * rows);
+  if (plan && (!bwd_plan_ok(plan->dq, BH, Sq, Skv, D) || !bwd_plan_ok(plan->dkv, BH, Skv, Sq, D) || workspace_floats < plan_floats(B, H, Sq, *plan)))
+    return MDATTN_E_BADARG;
+  const mdattn_host_bwd_plan p = plan ? *plan : bwd_plans(BH, Sq, Skv, D, workspace_floats - 2 * rows);
   BwdArgs a;
   a.lse2 = lse2; a.delta = delta; a.fwd = (const __bf16*)out; a.lse = lse; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;
@@ -834,19 +866,19 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   set(a.e1_sb, a.e1_ss, a.e1_sh, q_strides); set(a.e2_sb, a.e2_ss, a.e2_sh, o_strides);
   set(a.s1_sb, a.s1_ss, a.s1_sh, k_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, v_strides);
   set(a.o_sb, a.o_ss, a.o_sh, q_strides);
-  a.waves = pq.waves; a.nsplit = pq.nsplit; a.tps = pq.tps; a.part = workspace + 2 * rows; a.part2 = nullptr;
+  a.waves = p.dq.waves; a.nsplit = p.dq.pieces; a.tps = p.dq.tiles; a.part = workspace + 2 * rows; a.part2 = nullptr;
   int rc = launch_bwd_any<0>(st, a, B);
   if (rc != MDATTN_OK) return rc;
-  if (pq.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B)) != MDATTN_OK) return rc;
+  if (a.nsplit > 1 && (rc = launch_bwd_reduce(st, a, B)) != MDATTN_OK) return rc;
   // dk and dv in one pass: entity k / v, stream q (scores, and accumulate for dk), dout (dP, and accumulate for dv)
   a.e1 = (const __bf16*)k; a.e2 = (const __bf16*)v; a.s1 = (const __bf16*)q; a.s2 = (const __bf16*)dout;
   a.out = (__bf16*)dk; a.out2 = (__bf16*)dv; a.Se = Skv; a.Ss = Sq;
   set(a.e1_sb, a.e1_ss, a.e1_sh, k_strides); set(a.e2_sb, a.e2_ss, a.e2_sh, v_strides);
   set(a.s1_sb, a.s1_ss, a.s1_sh, q_strides); set(a.s2_sb, a.s2_ss, a.s2_sh, o_strides);
   set(a.o_sb, a.o_ss, a.o_sh, k_strides); set(a.o2_sb, a.o2_ss, a.o2_sh, v_strides);
-  a.waves = pkv.waves; a.nsplit = pkv.nsplit; a.tps = pkv.tps; a.part2 = a.part + pkv.floats;
+  a.waves = p.dkv.waves; a.nsplit = p.dkv.pieces; a.tps = p.dkv.tiles; a.part2 = a.part + p.dkv.floats;
   rc = launch_bwd_any<3>(st, a, B);
-  if (rc == MDATTN_OK && pkv.nsplit > 1) rc = launch_bwd_reduce(st, a, B);
+  if (rc == MDATTN_OK && a.nsplit > 1) rc = launch_bwd_reduce(st, a, B);
   return rc;
 }
 
@@ -876,9 +908,9 @@ extern "C" int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, 
                                     int B, int H, int Sq, int Skv, int D,
                                     const mdattn_strides* q_strides, const mdattn_strides* k_strides,
                                     const mdattn_strides* v_strides, const mdattn_strides* o_strides, float scale,
-                                    const float* key_bias, int64_t bias_stride, const int* tiles) {
+                                    const float* key_bias, int64_t bias_stride, const int* tiles, const mdattn_host_bwd_plan* plan) {
   return bwd_run((hipStream_t)stream, q, k, v, out, dout, lse, dq, dk, dv, workspace, workspace_floats, B, H, Sq, Skv, D,
-                 q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride, true, key_bias ? tiles : nullptr);
+                 q_strides, k_strides, v_strides, o_strides, scale, key_bias, bias_stride, true, key_bias ? tiles : nullptr, plan);
 }
 
 // ---------------------------------------------------------------------------------------------------

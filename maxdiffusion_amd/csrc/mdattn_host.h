@@ -11,7 +11,7 @@ extern "C" {
 
 /* Workspace of mdattn_bwd_bf16 / mdattn_bwd_bf16_bias with which a pass that has too few rows of its own to fill the chip
  * (cross-attention: dk / dv of a few hundred keys) is split over the other sequence: mdattn_bwd_workspace_floats plus the
- * f32 partial gradients.  With less, the call runs unsplit. */
+ * f32 partial gradients.  With less, it is split as far as the partials fit. */
 int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D);
 
 /* A [B, Skv] keep-mask (bytes) -> the additive bias of mdattn_key_mask_bias (-inf for excluded keys; bias_stride a multiple of
@@ -46,11 +46,26 @@ int mdattn_host_fwd_bf16(void* stream, const void* q, const void* k, const void*
  * mdattn_fwd_bf16_merge choose it. */
 int mdattn_host_fwd_schedule(int B, int H, int Sq, int Skv, int D, float scale);
 
-/* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias with or without tiles) at the head dims of mdattn_host_fwd_bf16. */
+/* How a backward call launches its passes, dq and dk with dv: waves per workgroup, pieces of the other sequence and 32-row tiles in each,
+ * floats of one tensor's partial gradients (0: one piece). */
+typedef struct {
+  int waves, pieces, tiles;
+  int64_t floats;
+} mdattn_host_bwd_pass;
+typedef struct {
+  mdattn_host_bwd_pass dq, dkv;
+} mdattn_host_bwd_plan;
+/* The plan (or null) of a call with a workspace of so many floats, at least mdattn_bwd_workspace_floats; negative: as many as it asks for.
+ * Returns how many it uses, 0 for sizes that are refused. */
+int64_t mdattn_host_bwd_plan_floats(int B, int H, int Sq, int Skv, int D, int64_t workspace_floats, mdattn_host_bwd_plan* plan);
+
+/* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias with or without tiles) at the head dims of mdattn_host_fwd_bf16.  plan: of these
+ * sizes; null: made from the workspace. */
 int mdattn_host_bwd_bf16(void* stream, const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, void* dq,
                          void* dk, void* dv, float* workspace, int64_t workspace_floats, int B, int H, int Sq, int Skv, int D,
                          const mdattn_strides* q_strides, const mdattn_strides* k_strides, const mdattn_strides* v_strides,
-                         const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride, const int* tiles);
+                         const mdattn_strides* o_strides, float scale, const float* key_bias, int64_t bias_stride, const int* tiles,
+                         const mdattn_host_bwd_plan* plan);
 
 /* The prologue and its backward with the rotary table in the layout the model made it in:
  *   PLANES    cos, sin f32 [S, D/2] (the layout of mdattn.h's entry points)
