@@ -62,7 +62,7 @@ SIGNATURES = {
 # what csrc/mdattn_host.h declares: entry points for this package's own host side
 HOST_SIGNATURES = {
     "mdattn_bwd_split_workspace_floats": ([_I, _I, _I, _I, _I], _L),
-    "mdattn_host_bwd_plan_floats": ([_I, _I, _I, _I, _I, _L, _P], _L),
+    "mdattn_host_bwd_plan_floats": ([_I, _I, _I, _I, _I, _I, _L, _P], _L),
     "mdattn_host_fwd_workspace_floats": ([_I, _I, _I, _I, _I], _L),
     "mdattn_host_fwd_schedule": ([_I, _I, _I, _I, _I, _F], _I),
     "mdattn_host_norm_rope_fullrow": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _L, _L, _S], _I),

@@ -664,23 +664,28 @@ __global__ __launch_bounds__(256) void bwd_reduce_kernel(BwdReduceArgs a) {
 // 1312 us in one piece (24 workgroups) and 201 us in ten, + 13 us of bwd_reduce_kernel.
 constexpr int kMinSplitTiles = 8, kMaxSplit = 32;
 using BwdPlan = mdattn_host_bwd_pass;
-inline double bwd_pass_us(int D, int tensors, int waves, int64_t wgs, int tps) {
+// A key bias or mask costs the dq pass 0.3 us per tile, whose sixteen bias values per lane stand between the products (measured 0.25 to 0.35 more
+// with one, two and three workgroups on a CU, at head dims 40 to 128); the dk / dv pass has one per lane and call.  Without that 2 x 4 heads
+// x 3,572 x 3,572 under a mask ran its dq pass whole, 125 us, 93 in three pieces, and 16 heads of 40 x 1,688 x 1,688 45 us, 33 in three.
+inline double bwd_bias_us(int tensors, bool bias) { return bias && tensors == 1 ? 0.3 : 0.0; }
+inline double bwd_pass_us(int D, int tensors, bool bias, int waves, int64_t wgs, int tps) {
+  const double more = bwd_bias_us(tensors, bias);
   if (D <= 64) {  // workgroups of four waves, three per CU
-    const double tile[3] = {tensors == 2 ? 0.74 : 0.54, tensors == 2 ? 1.15 : 0.8, tensors == 2 ? 1.45 : 1.1};  // with one, two, three of them
+    const double tile[3] = {more + (tensors == 2 ? 0.74 : 0.54), more + (tensors == 2 ? 1.15 : 0.8), more + (tensors == 2 ? 1.45 : 1.1)};  // with one, two, three of them
     const int64_t rest = wgs % 768;
     return (double)(wgs / 768) * (tps * tile[2] + 4.0) + (rest ? tps * tile[(rest - 1) / 256] + 4.0 : 0.0);
   }
   const int slots = waves == 8 ? 256 : 512;
   const int64_t rounds = waves == 8 ? wgs / 256 : wgs / 512, rest = wgs - rounds * slots;
-  const double tile = tensors == 2 ? (waves == 8 ? 1.65 : 1.75) : (waves == 8 ? 1.2 : 1.25);
-  const double alone = waves == 8 ? tile : tensors == 2 ? 1.3 : 0.8;       // with the CU to itself
+  const double tile = more + (tensors == 2 ? (waves == 8 ? 1.65 : 1.75) : (waves == 8 ? 1.2 : 1.25));
+  const double alone = waves == 8 ? tile : more + (tensors == 2 ? 1.3 : 0.8);       // with the CU to itself
   const double full = tensors == 2 ? 0.0 : waves == 8 ? 10.0 : 5.5;        // of a start, when every CU reads its rows at once
   double us = (double)rounds * (tps * tile + 4.0 + full);
   if (rest) us += tps * (rest <= 256 ? alone : tile) + 4.0 + full * (double)rest / slots;
   return us;
 }
 // entity rows Se, stream rows Ss; tensors: gradients the pass produces (2 in the dk / dv pass); room: floats for partials
-inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t room) {
+inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, bool bias, int64_t room) {
   const int nt = (Ss + kBT - 1) / kBT;
   const int64_t floats = BH * Se * D;
   const double partial = 1.5 * tensors * (double)floats * 4 / 5e6;  // (writing them is half hidden)
@@ -688,18 +693,19 @@ inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t 
   BwdPlan best{most, 1, nt, 0};
   double best_cost = 1e300;
   for (int waves = most; waves >= 4; waves -= 4) {
-    const double cost = bwd_pass_us(D, tensors, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)), nt);
+    const double cost = bwd_pass_us(D, tensors, bias, waves, BH * ((Se + waves * 32 - 1) / (waves * 32)), nt);
     if (cost < best_cost) { best_cost = cost; best.waves = waves; }
   }
   for (int waves = most; waves >= 4; waves -= 4) {
     const int64_t entities = BH * ((Se + waves * 32 - 1) / (waves * 32));
     // no cut is faster than its tiles on a full chip, the partials of two pieces and their launch
-    const double full_chip = D <= 64 ? (tensors == 2 ? 1.45 : 1.1) / 768 : waves == 8 ? (tensors == 2 ? 1.65 : 1.2) / 256 : (tensors == 2 ? 1.75 : 1.25) / 512;
-    if ((double)entities * nt * full_chip + 2 * partial + 6.0 >= best_cost * 0.95) continue;
+    const int slots = D <= 64 ? 768 : waves == 8 ? 256 : 512;
+    const double full_tile = D <= 64 ? (tensors == 2 ? 1.45 : 1.1) : tensors == 2 ? (waves == 8 ? 1.65 : 1.75) : (waves == 8 ? 1.2 : 1.25);
+    if ((double)entities * nt * (full_tile + bwd_bias_us(tensors, bias)) / slots + 2 * partial + 6.0 >= best_cost * 0.95) continue;
     for (int n = 2; n <= kMaxSplit && nt / n >= kMinSplitTiles; ++n) {
       const int tps = (nt + n - 1) / n, ns = (nt + tps - 1) / tps;
       if (ns * floats * tensors > room) break;
-      const double cost = bwd_pass_us(D, tensors, waves, entities * ns, tps) + partial * ns + 6.0;
+      const double cost = bwd_pass_us(D, tensors, bias, waves, entities * ns, tps) + partial * ns + 6.0;
       if (cost < best_cost * 0.95) { best_cost = cost; best = {waves, ns, tps, ns * floats}; }
     }
   }
@@ -708,10 +714,10 @@ inline BwdPlan bwd_plan(int64_t BH, int Se, int Ss, int D, int tensors, int64_t 
 // The plan of a call without limits, and where a pass's partials do not fit, the best one for that pass that does.  Which cuts are
 // looked at decides where two are within 5 %: with the limit in the first search a call with the workspace of this very plan was launched
 // with another in one of forty shapes.
-inline mdattn_host_bwd_plan bwd_plans(int64_t BH, int Sq, int Skv, int D, int64_t room) {
-  mdattn_host_bwd_plan p{bwd_plan(BH, Sq, Skv, D, 1, INT64_MAX), bwd_plan(BH, Skv, Sq, D, 2, INT64_MAX)};
-  if (p.dq.floats > room) p.dq = bwd_plan(BH, Sq, Skv, D, 1, room);
-  if (2 * p.dkv.floats > room) p.dkv = bwd_plan(BH, Skv, Sq, D, 2, room);
+inline mdattn_host_bwd_plan bwd_plans(int64_t BH, int Sq, int Skv, int D, bool bias, int64_t room) {
+  mdattn_host_bwd_plan p{bwd_plan(BH, Sq, Skv, D, 1, bias, INT64_MAX), bwd_plan(BH, Skv, Sq, D, 2, bias, INT64_MAX)};
+  if (p.dq.floats > room) p.dq = bwd_plan(BH, Sq, Skv, D, 1, bias, room);
+  if (2 * p.dkv.floats > room) p.dkv = bwd_plan(BH, Skv, Sq, D, 2, bias, room);
   return p;
 }
 // whether a pass of this plan covers its Ss stream rows, without an empty piece, and says the space it takes
@@ -805,13 +811,14 @@ static int64_t plan_floats(int B, int H, int Sq, const mdattn_host_bwd_plan& p) 
 extern "C" int64_t mdattn_bwd_split_workspace_floats(int B, int H, int Sq, int Skv, int D) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || !native_head_dim(D)) return 0;
   const int64_t BH = (int64_t)B * H;
-  return plan_floats(B, H, Sq, bwd_plans(BH, Sq, Skv, D, INT64_MAX));
+  const int64_t plain = plan_floats(B, H, Sq, bwd_plans(BH, Sq, Skv, D, false, INT64_MAX)), biased = plan_floats(B, H, Sq, bwd_plans(BH, Sq, Skv, D, true, INT64_MAX));
+  return plain > biased ? plain : biased;
 }
 
-extern "C" int64_t mdattn_host_bwd_plan_floats(int B, int H, int Sq, int Skv, int D, int64_t workspace_floats, mdattn_host_bwd_plan* plan) {
+extern "C" int64_t mdattn_host_bwd_plan_floats(int B, int H, int Sq, int Skv, int D, int key_bias, int64_t workspace_floats, mdattn_host_bwd_plan* plan) {
   const int64_t base = mdattn_bwd_workspace_floats(B, H, Sq);
   if (base == 0 || Skv <= 0 || !native_head_dim(D) || (workspace_floats >= 0 && workspace_floats < base)) return 0;
-  const mdattn_host_bwd_plan p = bwd_plans((int64_t)B * H, Sq, Skv, D, workspace_floats < 0 ? INT64_MAX : workspace_floats - base);
+  const mdattn_host_bwd_plan p = bwd_plans((int64_t)B * H, Sq, Skv, D, key_bias != 0, workspace_floats < 0 ? INT64_MAX : workspace_floats - base);
   if (plan) *plan = p;
   return plan_floats(B, H, Sq, p);
 }
@@ -854,7 +861,7 @@ static int bwd_run(hipStream_t st, const void* q, const void* k, const void* v, 
   const int64_t BH = (int64_t)B * H;
   if (plan && (!bwd_plan_ok(plan->dq, BH, Sq, Skv, D) || !bwd_plan_ok(plan->dkv, BH, Skv, Sq, D) || workspace_floats < plan_floats(B, H, Sq, *plan)))
     return MDATTN_E_BADARG;
-  const mdattn_host_bwd_plan p = plan ? *plan : bwd_plans(BH, Sq, Skv, D, workspace_floats - 2 * rows);
+  const mdattn_host_bwd_plan p = plan ? *plan : bwd_plans(BH, Sq, Skv, D, key_bias != nullptr, workspace_floats - 2 * rows);
   BwdArgs a;
   a.lse2 = lse2; a.delta = delta; a.fwd = (const __bf16*)out; a.lse = lse; a.H = H; a.Sp = Sp; a.D = D; a.c = scale * kLog2e; a.scale = scale;
   a.bias = key_bias; a.bias_sb = bias_stride;

@@ -200,7 +200,7 @@ struct FlashFn : torch::autograd::Function<FlashFn> {
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     const int B = (int)vq.b, H = (int)vq.h, Sq = (int)vq.s, Skv = (int)vk.s, D = (int)vq.d;
     mdattn_host_bwd_plan plan;
-    const int64_t nws = mdattn_host_bwd_plan_floats(B, H, Sq, Skv, D, -1, &plan);
+    const int64_t nws = mdattn_host_bwd_plan_floats(B, H, Sq, Skv, D, m.bias != nullptr, -1, &plan);
     Tensor ws = at::empty({nws}, lse.options());
     const mdattn_strides so{out.stride(0), out.stride(1), vq.d};
     const int rc = mdattn_host_bwd_bf16(stream(), ptr(q), ptr(k), ptr(v), ptr(out), ptr(dout), f32(lse), mut(dq), mut(dk), mut(dv), f32(ws), nws, B, H, Sq,

@@ -55,9 +55,9 @@ typedef struct {
 typedef struct {
   mdattn_host_bwd_pass dq, dkv;
 } mdattn_host_bwd_plan;
-/* The plan (or null) of a call with a workspace of so many floats, at least mdattn_bwd_workspace_floats; negative: as many as it asks for.
+/* The plan (or null) of a call, with a key bias or mask or without, and with a workspace of so many floats, at least mdattn_bwd_workspace_floats; negative: as many as it asks for.
  * Returns how many it uses, 0 for sizes that are refused. */
-int64_t mdattn_host_bwd_plan_floats(int B, int H, int Sq, int Skv, int D, int64_t workspace_floats, mdattn_host_bwd_plan* plan);
+int64_t mdattn_host_bwd_plan_floats(int B, int H, int Sq, int Skv, int D, int key_bias, int64_t workspace_floats, mdattn_host_bwd_plan* plan);
 
 /* mdattn_bwd_bf16 / mdattn_bwd_bf16_bias (key_bias with or without tiles) at the head dims of mdattn_host_fwd_bf16.  plan: of these
  * sizes; null: made from the workspace. */
