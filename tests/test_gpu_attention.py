@@ -424,10 +424,12 @@ def test_seeded_sweep_of_shapes_layouts_and_paths(dev, variant):
 
 
 @pytest.mark.parametrize("folded", [False, True])
-@pytest.mark.parametrize("H,sq,skv", [(2, 130, 2100), (3, 128, 1291), (1, 1, 4097), (12, 2690, 1420)])
-def test_few_query_tiles_against_many_keys(dev, folded, H, sq, skv):
-  """A workgroup per CU at most: the pipelined schedule of four waves, also as a ring step, and where a row's first 32 keys have
-  logits of -inf (a key with an infinite channel takes no part, like any key that is left out)."""
+@pytest.mark.parametrize("H,sq,skv,plain,with_factor", [(2, 130, 2100, 2, 2), (3, 128, 1291, 2, 2), (1, 1, 4097, 2, 2), (12, 2680, 1800, 2, 2), (12, 2690, 1420, 1, 3)])
+def test_few_query_tiles_against_many_keys(dev, lib, folded, H, sq, skv, plain, with_factor):
+  """A workgroup per CU at most: the pipelined schedule of four waves, on a few CUs and with 252 workgroups; with 264 one of the others.
+  Also as a ring step, and where a row's first 32 keys have logits of -inf (a key with an infinite channel takes no part, like any key
+  that is left out)."""
+  assert lib.mdattn_host_fwd_schedule(1, H, sq, skv, 128, ops.FOLDED_SCALE if folded else 128**-0.5) == (with_factor if folded else plain)
   q, k, v = O.normal_bf16((1, sq, H, 128), 0), O.normal_bf16((1, skv, H, 128), 1), O.normal_bf16((1, skv, H, 128), 2)
   q[..., 0] = -np.abs(q[..., 0]) - np.float32(0.5)
   scale = ops.FOLDED_SCALE if folded else 128**-0.5

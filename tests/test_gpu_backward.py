@@ -346,3 +346,39 @@ def test_backward_workgroups_of_four_and_eight_waves(dev, D, H, sq, skv, masked)
   ref = O.attention_bwd(hsd(q), hsd(k[:, keep[0]]), hsd(v[:, keep[0]]), hsd(do), D**-0.5)
   for g, r, name in ((got[0], ref[0], "dq"), (got[1][:, keep[0]], ref[1], "dk"), (got[2][:, keep[0]], ref[2], "dv")):
     _check(hsd(g), r, f"{name} H={H} Sq={sq} Skv={skv} D={D} masked={masked}")
+
+
+@pytest.mark.parametrize("D", [128, 96, 80])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("H,sq,skv,cut", [(12, 2777, 1475, False), (16, 4075, 4090, False), (6, 1990, 5990, True)])
+def test_dq_pass_of_eight_waves(dev, lib, D, masked, H, sq, skv, cut):
+  """Its two copies of the loop take turns at the ring's slots: an odd and an even number of tiles, cut and whole, over every tile and
+  over a mask's list, with a ragged last tile and a last workgroup with empty waves.  Each head against f32 on the GPU."""
+  from maxdiffusion_amd import attention_op as A
+  from test_plans import _plan
+
+  (waves, pieces, _, _), _, _ = _plan(lib, 1, H, sq, skv, D, int(masked))
+  assert waves == 8 and (pieces > 1) == cut
+  gen = torch.Generator(device=dev).manual_seed(sq)
+  mk = lambda s: torch.randn((1, s, H * D), generator=gen, device=dev).to(torch.bfloat16)
+  q, k, v, do = mk(sq), mk(skv), mk(skv), mk(sq)
+  keep = torch.ones((1, skv), dtype=torch.bool, device=dev)
+  if masked:
+    keep[:, 64:128] = keep[:, 1000:1100] = False  # whole tiles, which the list leaves out, and parts
+    keep[:, 70::7] = False
+  leaves = [x.requires_grad_(True) for x in (q, k, v)]
+  op = A.AttentionOp(attention_kernel="hip_flash", scale=D**-0.5, heads=H, dim_head=D, dtype=torch.bfloat16)
+  out = op.apply_attention(*leaves, attention_mask=keep if masked else None)
+  got = [g.view(-1, H, D) for g in torch.autograd.grad(out, leaves, do)]
+  assert not got[1][~keep[0]].any() and not got[2][~keep[0]].any()
+  heads = lambda x: x.detach().float().view(-1, H, D).transpose(0, 1).contiguous()
+  hq, hk, hv, hd = heads(q), heads(k)[:, keep[0]].contiguous(), heads(v)[:, keep[0]].contiguous(), heads(do)
+  want = [[], [], []]
+  for h in range(H):
+    p = torch.softmax((hq[h] @ hk[h].t()) * D**-0.5, -1)
+    dp = hd[h] @ hv[h].t()
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * D**-0.5
+    for to, x in zip(want, (ds @ hk[h], ds.t() @ hq[h], p.t() @ hd[h])):
+      to.append(x)
+  for name, g, w in zip(("dq", "dk", "dv"), (got[0], got[1][keep[0]], got[2][keep[0]]), want):
+    _check(to_np(g), to_np(torch.stack(w, 1)), f"{name} H={H} Sq={sq} Skv={skv} D={D} masked={masked}")
