@@ -328,28 +328,19 @@ std::optional<Table> as_table(const OptTensor& a, const OptTensor& b, int64_t s,
   t.cos = *a;
   return t;
 }
-// Replaces a tensor, or two of the same form (b may be undefined), by copies: dense ones in one launch, others as clones.
-void own(Tensor& a, Tensor& b) {
-  at::NoGradGuard guard;
-  const auto dense = [](const Tensor& t) { return t.is_cuda() && t.is_contiguous() && aligned(t) && !t.is_conj() && !t.is_neg(); };
-  if (dense(a) && a.nbytes() > 0 && a.nbytes() % 16 == 0 && (!b.defined() || (dense(b) && b.nbytes() == a.nbytes() && b.get_device() == a.get_device()))) {
-    Tensor x = at::empty(a.sizes(), a.options()), y = b.defined() ? at::empty(b.sizes(), b.options()) : Tensor();
-    if (mdattn_host_copy(stream(), ptr(a), mut(x), ptr(b), mut(y), (int64_t)a.nbytes()) == MDATTN_OK) {
-      a = x;
-      b = y;
-      return;
-    }
-  }
-  a = a.clone();
-  if (b.defined()) b = b.clone();
+// Replaces a tensor that in_place has accepted, or two of one size (b may be undefined), by copies, in one launch.  False, and nothing
+// replaced, for a size that is no multiple of 16 bytes: no kernel takes such rows either.
+bool own(Tensor& a, Tensor& b) {
+  const Tensor x = at::empty(a.sizes(), a.options()), y = b.defined() ? at::empty(b.sizes(), b.options()) : Tensor();
+  if (mdattn_host_copy(stream(), ptr(a), mut(x), ptr(b), mut(y), (int64_t)a.nbytes()) != MDATTN_OK) return false;
+  a = x;
+  b = y;
+  return true;
 }
 // The table as a node keeps it.  One that is read in place belongs to the caller, who may have made it in inference mode (autograd
 // refuses to save such a tensor) or may rewrite it before the backward: a dense copy of it, one launch.  Half planes [S, D/2] were
 // always saved as they are.
-void own_table(Table& t) {
-  if (!t.cos.defined() || t.kind == MDATTN_TABLE_PLANES) return;
-  own(t.cos, t.sin);
-}
+bool own_table(Table& t) { return !t.cos.defined() || t.kind == MDATTN_TABLE_PLANES || own(t.cos, t.sin); }
 const float* table_ptr(const Tensor& t) { return t.defined() ? static_cast<const float*>(t.data_ptr()) : nullptr; }
 bool weight_ok(const Tensor& w, int64_t n, const Tensor& ref) { return bf16_on(w, ref) && w.is_contiguous() && w.numel() == n; }
 
@@ -441,7 +432,7 @@ std::optional<variable_list> norm_rope(const Tensor& q, const OptTensor& k_, con
   const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
   if (wants_grad({&q, &k, &wq, &wk})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
-    own_table(*t);
+    if (!own_table(*t)) return std::nullopt;
     return unless_refused([&] { return FullrowFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(t->cos), opt(t->sin), p); });
   }
   variable_list out = fullrow_run(q, k, wq, wk, t->cos, t->sin, p);
@@ -510,7 +501,7 @@ std::optional<variable_list> norm_rope_perhead(const Tensor& q, const OptTensor&
   const Prologue p{q.size(2), t->kind, n_txt, eps, q_mul, bhsd};
   if (wants_grad({&q, &k, &wq, &wk, &wqt, &wkt})) {
     if (!q.is_non_overlapping_and_dense()) return std::nullopt;
-    own_table(*t);
+    if (!own_table(*t)) return std::nullopt;
     return unless_refused([&] { return PerheadFn::apply(q, opt(k), wq, k.defined() ? opt(wk) : std::nullopt, opt(wqt), opt(wkt), opt(t->cos), opt(t->sin), p); });
   }
   variable_list out = perhead_run(q, k, wq, wk, wqt, wkt, t->cos, t->sin, p);
@@ -575,7 +566,7 @@ std::optional<variable_list> norm_rope_qkv(const Tensor& x, const Tensor& bias, 
   if (!t) return std::nullopt;
   const Prologue p{heads, t->kind, 0, eps, q_mul, bhsd};
   if (wants_grad({&x, &bias, &wq, &wk})) {
-    own_table(*t);
+    if (!own_table(*t)) return std::nullopt;
     return unless_refused([&] { return QkvFn::apply(x, bias, wq, wk, opt(t->cos), opt(t->sin), p); });
   }
   variable_list out = qkv_run(x, bias, wq, wk, t->cos, t->sin, p);
@@ -606,7 +597,7 @@ struct RowsFn : torch::autograd::Function<RowsFn> {
     // a weight with a factor is saved as a copy, as its product with the factor was: the caller's may be an inference tensor, or
     // be updated before the backward
     Tensor kept_wq = wq, none;
-    if (p.w_mul != 1.0) own(kept_wq, none);
+    if (p.w_mul != 1.0 && !own(kept_wq, none)) throw Refused{};
     ctx->save_for_backward({q, k, kept_wq, wk, cos, sin});
     ctx->saved_data["i"] = c10::List<int64_t>({p.heads, p.mode, (int64_t)q.scalar_type()});
     ctx->saved_data["f"] = c10::List<double>({p.eps, p.w_mul});

@@ -69,8 +69,9 @@ __global__ __launch_bounds__(256) void finalize_kernel(const float4* __restrict_
   }
 }
 
-// Dense copies of one or two buffers (blockIdx.y), 16 bytes per lane: 2 x 2.4 MB 3 us, where the copies that the runtime launches
-// for a clone take 5 us each.
+// Dense copies of one or two buffers (blockIdx.y), 16 bytes per lane.  A launch's own time rules it at the sizes of rotary tables and
+// weights: 2 x 2.4 MB 5.4 us from memory and 2.8 from the caches, 2 x 8 KB 4.8 and 1.7, the runtime's copy of one of the two buffers 5.2
+// and 2.3, 4.8 and 1.4.  Two planes in one launch save the second, on the stream and on the host.
 __global__ __launch_bounds__(256) void copy_kernel(const uint4* src0, uint4* dst0, const uint4* src1, uint4* dst1, int64_t n16) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n16) (blockIdx.y ? dst1 : dst0)[i] = (blockIdx.y ? src1 : src0)[i];

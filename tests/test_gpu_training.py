@@ -411,6 +411,19 @@ def test_a_refused_training_call_raises_the_library_error(dev):
     assert e.value.code == -3
 
 
+@pytest.mark.parametrize("training", [False, True])
+def test_a_table_and_a_weight_too_small_to_be_copied(dev, training):
+  """Sizes that are no multiple of 16 bytes, which a training call's copies refuse: such a call ends as it does without them."""
+  mk = lambda n, dtype=torch.bfloat16: torch.randn((1, 3, n), device=dev).to(dtype).requires_grad_(training)
+  table = torch.polar(torch.ones((3, 1), device=dev), torch.rand((3, 1), device=dev))  # 24 bytes
+  w = torch.ones(6, device=dev)
+  for call in (lambda: A.hip_norm_rope(mk(4), mk(4), w[:4].bfloat16(), w[:4].bfloat16(), table, 2),
+               lambda: A.hip_norm_rope_ltx2(mk(6, torch.float32), mk(6, torch.float32), w, w, 1, rotary_emb=None, q_mul=0.5)):
+    with pytest.raises(_lib.MdattnError) as e:
+      call()
+    assert e.value.code == _lib.E_UNSUPPORTED
+
+
 def test_ltx2_gradient_of_the_query_alone(dev):
   """A loss that reaches one of q and k leaves the other and its weight without a gradient, and operands that need none get none."""
   q, k, wq, wk, H, g = _ltx2(dev)
