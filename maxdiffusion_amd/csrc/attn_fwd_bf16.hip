@@ -924,8 +924,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     // address a lane constant plus an immediate offset, and the address arithmetic per tile is gone from a kernel that
     // is bound by vector issue (1 % at 32 heads x 13,376 tokens; at head dim 128 the copies cost registers and lose).  The first
     // tile is a copy of its own: asked for in every tile it cost a SIMD with one wave 2 % (1 head x 11,007 keys and queries 138.7 us,
-    // 135.9 now, 5 x 5,368 69.8 and 68.7).  At head dim 128 that copy gave nothing at full tiles and lost 1 to 5 % with a tail of the
-    // last round at two workgroups per CU.
+    // 135.9 now, 5 x 5,368 69.8 and 68.7).
     if (nt > 1) step(0, std::true_type{}, std::integral_constant<int, 0>{}, 1);
     for (int t = 1; t < nt - 1; t += 2) {
       step(t, std::false_type{}, std::integral_constant<int, 1>{}, 0);
@@ -933,9 +932,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       step(t + 1, std::false_type{}, std::integral_constant<int, 0>{}, 1);
     }
   } else {
-    int slot = 0, fill = SLOTS - 1;
-    for (int t = 0; t < nt - 1; ++t) {
-      step(t, t == 0, slot, fill);
+    // Head dim 128: the first tile's copy pays beside an additive bias (2 heads x 1,000 queries x 6,000 keys 133.6 us without it, 127.8 now, 12 x
+    // 2,000 x 2,000 48.1 and 46.4, 40 x 2,000 x 2,000 95.2 and 91.9); the others lost 1 to 5 % where some CUs have two workgroups.
+    int slot = 0, fill = SLOTS - 1, t0 = 0;
+    if constexpr (BIAS == kKeyBias) {
+      if (nt > 1) step(t0++, std::true_type{}, slot++, fill);
+      fill = 0;
+    }
+    for (int t = t0; t < nt - 1; ++t) {
+      if constexpr (BIAS == kKeyBias) step(t, std::false_type{}, slot, fill);
+      else step(t, t == 0, slot, fill);
       slot = slot == SLOTS - 1 ? 0 : slot + 1;
       fill = fill == SLOTS - 1 ? 0 : fill + 1;
     }

@@ -191,3 +191,21 @@ def test_key_tile_lists(dev, lib, B, skv, density):
       assert (got[at + 1 + len(entries):at + 1 + nt] == -1).all()
       at += 1 + nt
   assert at == n
+
+
+@pytest.mark.parametrize("skv", [32, 33, 64, 65, 96, 97, 128, 129, 190])
+def test_additive_bias_one_to_six_key_tiles(dev, skv):
+  """Head dim 128: the first tile and the last are copies of the loop's body of their own; finite biases and an excluded key in
+  every tile.  out and lse against float64."""
+  H, sq = 3, 70
+  q, k, v = O.normal_bf16((1, sq, H, 128), 0), O.normal_bf16((1, skv, H, 128), 1), O.normal_bf16((1, skv, H, 128), 2)
+  bias = np.full((1, (skv + 31) // 32 * 32), -np.inf, np.float32)
+  bias[0, :skv] = 3.0 * np.random.default_rng(skv).standard_normal(skv)
+  bias[0, 5:skv:32] = -np.inf
+  out, lse = ops.flash_attention(to_dev_bf16(q, dev), to_dev_bf16(k, dev), to_dev_bf16(v, dev), return_lse=True, key_bias=torch.from_numpy(bias).to(dev))
+  logits = hsd(q).astype(np.float64) @ hsd(k).astype(np.float64).transpose(0, 2, 1) * 128**-0.5 + bias[0, :skv]
+  m = logits.max(-1, keepdims=True)
+  p = np.exp(logits - m)
+  total = p.sum(-1, keepdims=True)
+  assert rel_l2(hsd(to_np(out)), (p / total) @ hsd(v)) <= 6e-3  # bf16 roundings of the probabilities and of the output
+  assert np.abs(to_np(lse)[0] - (m + np.log(total))[..., 0]).max() <= 1e-3
