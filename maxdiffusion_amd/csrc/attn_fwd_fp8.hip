@@ -397,6 +397,11 @@ __device__ __forceinline__ void fp8_body(const Fp8Args& a, const float c, char* 
   // iteration t only the 2*GPW loads of tile t+1 may still be in flight once tile t is needed.
   dma(0, 0);
   if (nt > 1) dma(1, 1);
+  // Q has arrived: otherwise the compiler, which does not count the tiles' loads, waits for Q's where a tile's products begin, in every
+  // tile, and with a count that waits for the next tiles too.  (At head dim 128 without a bias and with a power-of-two scale it forms a
+  // first tile of its own, and this wait would only cost a short call 0.3 us.)  24 heads x 217 queries x 6,781 kept of 13,219 keys 224 ->
+  // 167 us, 160 x 581 x 3,313 of 8,914 385 -> 303, 4 of 64 x 160 x 15,547 of 17,740 236 -> 165; with other scales 40 x 88 x 18,145 293 -> 205.
+  if constexpr (BIAS || !PRE || HD == 64) __builtin_amdgcn_s_waitcnt(0x0F70);
   int slot = 0, fill = 2;
   // Head dim 64 without a bias: the one step that requests nothing is a copy of its own, and the epilogue takes the lane's number
   // from the loop.  Elsewhere the copy costs registers (spills), and so do the rows' places, which the compiler would form in front of
