@@ -902,7 +902,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       rf = rows(ef >> 1);
     }
   }
-  // (with two slots the tile after t < nt - 1 exists: no question)
+  // (with two slots the tile after t < nt - 1 exists: no question, but beside an additive bias the loop is 2 % faster with it)
   auto step = [&](int t, auto first, auto slot, int fill) __attribute__((always_inline)) {
     // vmcnt: this wave's share of tile t has landed (the SLOTS - 2 tiles requested after it may still be in flight)
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((SLOTS - 2) * (2 * GPW + (BIAS ? 1 : 0))));
@@ -915,32 +915,38 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       ef = entry(t + SLOTS);
       rf = rows(ef >> 1);
     } else {
-      if (SLOTS == 2 || t + SLOTS - 1 < nt) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
+      if ((SLOTS == 2 && !BIAS) || t + SLOTS - 1 < nt) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
       tile(t, first, false, slot, std::false_type{});
     }
   };
+  // The first tile as a copy of its own, or asked for in every tile.  The question costs a SIMD with one wave 2 to 4 %: at head dim 64 1 head x 11,007
+  // keys and queries 138.7 us, 135.9 with the copy, 5 x 5,368 69.8 and 68.7; beside an additive bias at 128 2 heads x 1,000 queries x 6,000 keys 133.6
+  // and 127.8, 40 x 2,000 x 2,000 95.2 and 91.9.  The copy costs the other two forms registers or the pace of a CU's workgroups: an
+  // additive bias at 64 2 % (5 x 5,392 x 7,188 104.9 and 106.9), the rest at 128 1 to 5 % where some CUs have two workgroups.
+  constexpr bool APART = HD == 64 ? BIAS != kKeyBias : BIAS == kKeyBias;
   if constexpr (HD == 64) {
     // Two copies of the loop body, one per ring slot: the slot is a compile-time constant in each, every fragment
     // address a lane constant plus an immediate offset, and the address arithmetic per tile is gone from a kernel that
-    // is bound by vector issue (1 % at 32 heads x 13,376 tokens; at head dim 128 the copies cost registers and lose).  The first
-    // tile is a copy of its own: asked for in every tile it cost a SIMD with one wave 2 % (1 head x 11,007 keys and queries 138.7 us,
-    // 135.9 now, 5 x 5,368 69.8 and 68.7).
-    if (nt > 1) step(0, std::true_type{}, std::integral_constant<int, 0>{}, 1);
-    for (int t = 1; t < nt - 1; t += 2) {
-      step(t, std::false_type{}, std::integral_constant<int, 1>{}, 0);
+    // is bound by vector issue (1 % at 32 heads x 13,376 tokens; at head dim 128 the copies cost registers and lose).
+    constexpr std::integral_constant<int, APART ? 1 : 0> one{};
+    constexpr std::integral_constant<int, APART ? 0 : 1> other{};
+    if constexpr (APART) {
+      if (nt > 1) step(0, std::true_type{}, other, one);
+    }
+    for (int t = APART; t < nt - 1; t += 2) {
+      if constexpr (APART) step(t, std::false_type{}, one, other);
+      else step(t, t == 0, one, other);
       if (t + 1 >= nt - 1) break;
-      step(t + 1, std::false_type{}, std::integral_constant<int, 0>{}, 1);
+      step(t + 1, std::false_type{}, other, one);
     }
   } else {
-    // Head dim 128: the first tile's copy pays beside an additive bias (2 heads x 1,000 queries x 6,000 keys 133.6 us without it, 127.8 now, 12 x
-    // 2,000 x 2,000 48.1 and 46.4, 40 x 2,000 x 2,000 95.2 and 91.9); the others lost 1 to 5 % where some CUs have two workgroups.
     int slot = 0, fill = SLOTS - 1, t0 = 0;
-    if constexpr (BIAS == kKeyBias) {
+    if constexpr (APART) {
       if (nt > 1) step(t0++, std::true_type{}, slot++, fill);
       fill = 0;
     }
     for (int t = t0; t < nt - 1; ++t) {
-      if constexpr (BIAS == kKeyBias) step(t, std::false_type{}, slot, fill);
+      if constexpr (APART) step(t, std::false_type{}, slot, fill);
       else step(t, t == 0, slot, fill);
       slot = slot == SLOTS - 1 ? 0 : slot + 1;
       fill = fill == SLOTS - 1 ? 0 : fill + 1;
