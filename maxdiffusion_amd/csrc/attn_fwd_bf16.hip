@@ -507,6 +507,7 @@ constexpr int kSlotsS = 3;
 // (nothing dropped: 109, 105, 100), of 64 81, 90, 72 (81, 73, 72); 512 queries x 75,600 keys x 40 heads of 128 1,575, 1,929, 1,693 (1,575,
 // 1,647, 1,505), of 64 1,072, 1,332, 1,021 (1,063, 1,051, 1,009): there a SIMD has one wave, and what stands between two tiles is the time.
 enum { kNoBias, kKeyBias, kKeyMask };
+enum { kNone, kYes, kAsk };  // whether a step of the loop requests a tile
 template <int NW, int BIAS, int HD, bool PRE, int DC = 0>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 3, HD == 64 ? 4 : 3))) void attn_fwd_bf16_flat_kernel(AttnArgs a) {
   constexpr bool PADDED = DC != 0;
@@ -592,7 +593,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     // every wave fetches the same values to the same place (a load more per wave and tile, counted in the loop's
     // s_waitcnt): lane l and lane l + 32 the bias of key l of the tile
     if constexpr (BIAS) {  // (a 64-key tile may reach past the padded bias row, whose length is a multiple of 32)
-      int col = kt * TS + (TS == 64 ? lane : l32);
+      int col = (BIAS == kKeyMask || kt < nt ? kt : nt - 1) * TS + (TS == 64 ? lane : l32);  // (an additive bias: the loads run past the end)
       col = col < bias_cols ? col : bias_cols - 1;
       lds_dma4(bias_row, (unsigned)col * 4u, Ks + TILES * 2u);
     }
@@ -890,7 +891,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       dma(1, en >> 1, rows(en >> 1));
     }
   } else if constexpr (SLOTS == 3) {
-    if (nt > 1) dma(1, 1, rows(1));
+    if (BIAS || nt > 1) dma(1, 1, rows(1));  // (an additive bias: as in the loop)
   }
   // kKeyMask: the tile to be requested next and its rows, known before the barrier: their arithmetic behind it would hold up the
   // request
@@ -902,8 +903,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       rf = rows(ef >> 1);
     }
   }
-  // (with two slots the tile after t < nt - 1 exists: no question, but beside an additive bias the loop is 2 % faster with it)
-  auto step = [&](int t, auto first, auto slot, int fill) __attribute__((always_inline)) {
+  auto step = [&](int t, auto first, auto slot, int fill, auto request) __attribute__((always_inline)) {
     // vmcnt: this wave's share of tile t has landed (the SLOTS - 2 tiles requested after it may still be in flight)
     __builtin_amdgcn_s_waitcnt(0x0F70 | ((SLOTS - 2) * (2 * GPW + (BIAS ? 1 : 0))));
     __syncthreads();                                  // ... and everyone's; slot `fill` (tile t-1) is free
@@ -915,7 +915,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
       ef = entry(t + SLOTS);
       rf = rows(ef >> 1);
     } else {
-      if ((SLOTS == 2 && !BIAS) || t + SLOTS - 1 < nt) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
+      if (request == kYes || (request == kAsk && t + SLOTS - 1 < nt)) dma(fill, t + SLOTS - 1, rows(t + SLOTS - 1));
       tile(t, first, false, slot, std::false_type{});
     }
   };
@@ -924,6 +924,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
   // and 127.8, 40 x 2,000 x 2,000 95.2 and 91.9.  The copy costs the other two forms registers or the pace of a CU's workgroups: an
   // additive bias at 64 2 % (5 x 5,392 x 7,188 104.9 and 106.9), the rest at 128 1 to 5 % where some CUs have two workgroups.
   constexpr bool APART = HD == 64 ? BIAS != kKeyBias : BIAS == kKeyBias;
+  // The request of the tile SLOTS - 1 ahead.  With two slots it always exists.  With three the last step has none: a copy of its own without the
+  // question (TAIL), the question in every step, or beside an additive bias a request past the end, whichever is the fastest form.  In the kernel
+  // with the multiply per logit the question cost 4 % where some CUs have two workgroups (5 heads x 3,372 x 3,372 53.0 us, 49.4 with the
+  // copy, 12 x 690 x 6,477 50.6 and 47.4, a ring step of 40 x 1,000 34.8 and 33.7; 40 x 40,000 x 256 258 and 256.5); without the multiply the copy costs short
+  // calls 1 to 2 % (40 x 40,000 x 256 249 and 254).  Beside a bias 40 x 819 x 9,709 238 us with the question, 231 without; 20 of 64 x 1,719 x 12,344
+  // 227 and 208.
+  constexpr bool TAIL = HD == 128 && BIAS == kNoBias && !PRE;
+  constexpr std::integral_constant<int, HD == 64 || TAIL || BIAS == kKeyBias ? kYes : kAsk> ahead{};
   if constexpr (HD == 64) {
     // Two copies of the loop body, one per ring slot: the slot is a compile-time constant in each, every fragment
     // address a lane constant plus an immediate offset, and the address arithmetic per tile is gone from a kernel that
@@ -931,25 +939,28 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
     constexpr std::integral_constant<int, APART ? 1 : 0> one{};
     constexpr std::integral_constant<int, APART ? 0 : 1> other{};
     if constexpr (APART) {
-      if (nt > 1) step(0, std::true_type{}, other, one);
+      if (nt > 1) step(0, std::true_type{}, other, one, ahead);
     }
     for (int t = APART; t < nt - 1; t += 2) {
-      if constexpr (APART) step(t, std::false_type{}, one, other);
-      else step(t, t == 0, one, other);
+      if constexpr (APART) step(t, std::false_type{}, one, other, ahead);
+      else step(t, t == 0, one, other, ahead);
       if (t + 1 >= nt - 1) break;
-      step(t + 1, std::false_type{}, other, one);
+      step(t + 1, std::false_type{}, other, one, ahead);
     }
   } else {
-    int slot = 0, fill = SLOTS - 1, t0 = 0;
+    int slot = 0, fill = SLOTS - 1, t = 0;
     if constexpr (APART) {
-      if (nt > 1) step(t0++, std::true_type{}, slot++, fill);
+      if (nt > 1) step(t++, std::true_type{}, slot++, fill, ahead);
       fill = 0;
     }
-    for (int t = t0; t < nt - 1; ++t) {
-      if constexpr (APART) step(t, std::false_type{}, slot, fill);
-      else step(t, t == 0, slot, fill);
+    for (; t < nt - (TAIL ? 2 : 1); ++t) {
+      if constexpr (APART) step(t, std::false_type{}, slot, fill, ahead);
+      else step(t, t == 0, slot, fill, ahead);
       slot = slot == SLOTS - 1 ? 0 : slot + 1;
       fill = fill == SLOTS - 1 ? 0 : fill + 1;
+    }
+    if constexpr (TAIL) {
+      if (t < nt - 1) step(t, t == 0, slot, fill, std::integral_constant<int, kNone>{});
     }
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);
