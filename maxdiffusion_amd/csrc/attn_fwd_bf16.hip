@@ -1,7 +1,7 @@
 // Non-causal flash-attention forward for gfx950 (MI355X), bf16 MFMA, head_dim 128.
 //
 // Work decomposition
-//   workgroup  = NW waves, each wave owns 32 query rows  (BM = NW*32 rows); two waves per SIMD
+//   workgroup  = NW waves, each wave owns 32 query rows  (BM = NW*32 rows); two waves per SIMD with eight waves, one with four
 //   K/V tiles  = 64 keys x 128, in a 4-deep LDS ring filled by direct global->LDS loads (no staging
 //                registers, no LDS store instructions).  Ring slot t%4 holds K(t) together with V(t-1):
 //                both are consumed in the same "period" (two 32-key iterations).  One barrier per
