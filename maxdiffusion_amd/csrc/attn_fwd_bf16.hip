@@ -197,6 +197,9 @@ __device__ __forceinline__ void store_rows_through_lds(const AttnArgs& a, const 
   }
 }
 
+// Read in place of the rows in front of V's first and behind its last.
+__device__ const u32x4 kZeros = {0u, 0u, 0u, 0u};
+
 template <int NW, bool PRE>
 __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -232,9 +235,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
   }
 
   // ---- direct global -> LDS loads of one ring slot: K(kt) and V(kt-1).  Wave w fills the row groups
-  // w, w+NW, ...  Rows outside the sequence re-read the nearest valid row: they only ever meet masked
-  // logits / zero probabilities, but must be finite.  Tiles that lie fully inside the sequence use a
-  // uniform base plus a lane offset that never changes.
+  // w, w+NW, ...  Rows of K past the end re-read the last row: they only ever meet masked logits.  Rows of V outside
+  // the sequence are zeros, not a row of V: their probabilities are zero, and zero times an infinite value
+  // would be NaN.  Tiles that lie fully inside the sequence use a uniform base plus a lane offset that never changes.
   const int grow = lane >> 4;                                  // row of the group this lane fills
   const int kcol = ((lane & 15) ^ grow) * 8;                   // K: logical chunk stored at this lane's position
   const int vcol = ((lane & 15) ^ (grow << 2)) * 8;            // V: same, segments permuted instead of chunks
@@ -258,11 +261,11 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_bf16_kernel(AttnArgs a) {
         const int g = wave + NW * i;
         int kk = kt * kBN + 4 * g + grow;
         kk = kk < a.Skv ? kk : a.Skv - 1;
-        int kvv = (kt - 1) * kBN + 4 * g + grow;
-        kvv = kvv < a.Skv ? kvv : a.Skv - 1;
-        kvv = kvv > 0 ? kvv : 0;
+        const int kvv = (kt - 1) * kBN + 4 * g + grow;
+        const __bf16* vrow = vp + (int64_t)kvv * a.v_ss + vcol;
+        if ((unsigned)kvv >= (unsigned)a.Skv) vrow = reinterpret_cast<const __bf16*>(&kZeros);
         lds_dma16(kp + (int64_t)kk * a.k_ss + kcol, Ks + (unsigned)(g * kGK) * 2u);
-        lds_dma16(vp + (int64_t)kvv * a.v_ss + vcol, Vs + (unsigned)(g * kGV) * 2u);
+        lds_dma16(vrow, Vs + (unsigned)(g * kGV) * 2u);
       }
     }
   };

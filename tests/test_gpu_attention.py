@@ -460,3 +460,27 @@ def test_head_dim_64_one_to_six_key_tiles(dev, folded, skv):
   out, lse = _run_np(q, k, v, dev, scale=scale)
   ro, rl = O.attention(hsd(q), hsd(k), hsd(v), scale)
   _check(hsd(out), lse[0], ro, rl, f"folded={folded} Skv={skv}")
+
+
+@pytest.mark.parametrize("folded", [False, True])
+@pytest.mark.parametrize("var", [1, 2, 3])
+@pytest.mark.parametrize("skv", [64, 96, 160, 1056, 1088])
+def test_infinite_values_in_the_first_and_the_last_row(dev, variant, var, skv, folded):
+  """Every key has weight, so a column in which one value is infinite is infinite in every row: the blocks in front of the first key
+  and behind the last multiply no value by zero.  The other columns are what they are without it."""
+  variant(var)
+  H, sq = 2, 70
+  q, k, v = O.normal_bf16((1, sq, H, 128), 0), O.normal_bf16((1, skv, H, 128), 1), O.normal_bf16((1, skv, H, 128), 2)
+  scale = ops.FOLDED_SCALE if folded else 128**-0.5
+  if folded:
+    q = O.bf16_round(q * np.float32(ops.folded_q_mul(128)))
+  plain, _ = _run_np(q, k, v, dev, scale=scale)
+  v[:, 0, :, 3], v[:, -1, :, 5] = np.inf, -np.inf
+  for got in (_run_np(q, k, v, dev, scale=scale)[0], None):
+    if got is None:  # as a ring step
+      o_run, l_run = ops.new_merge_state(1, sq, H, 128, dev)
+      ops.flash_attention_merge(to_dev_bf16(q, dev), to_dev_bf16(k, dev), to_dev_bf16(v, dev), o_run, l_run, scale=scale)
+      got = to_np(o_run)
+    assert (got[..., 3] == np.inf).all() and (got[..., 5] == -np.inf).all()
+    rest = [d for d in range(128) if d not in (3, 5)]
+    assert np.abs(got[..., rest] - plain[..., rest]).max() <= 2.0**-7 * np.abs(plain).max()  # the rounding of `plain` to bf16
