@@ -183,17 +183,26 @@ __device__ __forceinline__ void store_rows_through_lds(const AttnArgs& a, const 
   if (PADDED && cc * 8 >= a.D) return;
   __bf16* p = a.out + b * a.o_sb + h * a.o_sh + (int64_t)(row0 + rr) * a.o_ss + cc * 8;
   const int64_t step = (int64_t)RPI * a.o_ss;
-  // streaming stores: the output is written once and read by nobody here (1.5 % on the 512-key cross-attention)
+  // streaming stores: the output is written once and read by nobody here (1.5 % on the 512-key cross-attention); see cached_out
+  auto put = [&](__bf16* at, const uint4& u) __attribute__((always_inline)) {
+    if (PADDED && a.cached_out) {
+      asm volatile("" ::: "memory");  // the compiler would make one ordinary store of the two
+      *reinterpret_cast<uint4*>(at) = u;
+      asm volatile("" ::: "memory");
+    } else {
+      st_nt(reinterpret_cast<uint4*>(at), u);
+    }
+  };
   if (row0 + 32 <= a.Sq) {  // every read before the first store: one wait, no condition per row
     uint4 v[32 / RPI];
 #pragma unroll
     for (int j = 0; j < 32 / RPI; ++j) v[j] = *reinterpret_cast<const uint4*>(stage + (j * RPI + rr) * ROWB + cc * 16);
 #pragma unroll
-    for (int j = 0; j < 32 / RPI; ++j, p += step) st_nt(reinterpret_cast<uint4*>(p), v[j]);
+    for (int j = 0; j < 32 / RPI; ++j, p += step) put(p, v[j]);
   } else {
 #pragma unroll
     for (int j = 0; j < 32 / RPI; ++j, p += step)
-      if (row0 + j * RPI + rr < a.Sq) st_nt(reinterpret_cast<uint4*>(p), *reinterpret_cast<const uint4*>(stage + (j * RPI + rr) * ROWB + cc * 16));
+      if (row0 + j * RPI + rr < a.Sq) put(p, *reinterpret_cast<const uint4*>(stage + (j * RPI + rr) * ROWB + cc * 16));
   }
 }
 
@@ -992,6 +1001,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(HD == 6
 // scale * log2(e) == 1 (to f32 round-off): the caller folded the factor into q, and the kernels that leave the multiply per logit out run
 inline bool folded(float c) { return c > 1.0f - 1e-6f && c < 1.0f + 1e-6f; }
 
+// Whether the output of a head dim other than 64 and 128 is written by ordinary stores.  Rows of 80, 96, 144, 160 or 176 bytes share cache
+// lines with the neighbouring heads', whose workgroups run at other times: streaming stores send each part to memory by itself.  Ordinary
+// ones let the caches put the line together while the output fits them (streaming / ordinary, 4 x 20 heads, 77 keys: 5,000 queries at 80
+// 41 / 33 us, 9,500 74 / 60, 12,000 92 / 98; at 48 12,000 67 / 52, 20,000 110 / 116), at 72 and 88, whose parts are half sectors, at any size
+// (72: 8,000 73 / 52, 30,000 295 / 242).  Small outputs (2,000 at 80 15.7 / 16.3) and whole 64-byte pieces (96: 8,000 50.5 / 52) stay streaming.
+inline bool cached_out(int64_t rows, int D) {
+  const int64_t mib = rows * D * 2 >> 20;
+  return D % 32 != 0 && mib >= 32 && ((D > 64 && D % 16 != 0) || mib < 128);
+}
+
 template <int NW, int BIAS, int HD = 128, int DC = 0>
 static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   constexpr int BM = NW * 32;
@@ -1010,6 +1029,7 @@ static int launch_flat(hipStream_t st, AttnArgs a, int B) {
   a.total = (int)total;
   a.chunk = (a.total + 7) / 8;
   // With a key bias the logits are touched after the MFMAs anyway, so that variant keeps its FMA.
+  a.cached_out = DC != 0 && cached_out((int64_t)B * a.H * a.Sq, a.D);
   const bool pre = !BIAS && folded(a.c);
   if (pre) MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, !BIAS, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);
   else MDATTN_LAUNCH((attn_fwd_bf16_flat_kernel<NW, BIAS, HD, false, DC>), dim3(a.chunk * 8), dim3(NW * 64), lds_bytes, st, a);

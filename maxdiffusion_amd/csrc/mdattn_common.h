@@ -181,6 +181,7 @@ struct AttnArgs {
   // set, each leaves its un-normalised f32 output [split][B*H][Sq][D] and (reference point, sum of P) per row for
   // fwd_combine_kernel
   int nsplit, tps, BH;
+  int cached_out;  // flat kernel at head dims other than 64 and 128: the output by ordinary stores
   float* part;
   float2* ml;
 };

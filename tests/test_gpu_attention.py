@@ -484,3 +484,24 @@ def test_infinite_values_in_the_first_and_the_last_row(dev, variant, var, skv, f
     assert (got[..., 3] == np.inf).all() and (got[..., 5] == -np.inf).all()
     rest = [d for d in range(128) if d not in (3, 5)]
     assert np.abs(got[..., rest] - plain[..., rest]).max() <= 2.0**-7 * np.abs(plain).max()  # the rounding of `plain` to bf16
+
+
+@pytest.mark.parametrize("D", [40, 48, 72, 80])
+@pytest.mark.parametrize("masked", [False, True])
+def test_output_stores_of_narrow_rows_do_not_change_values(dev, D, masked):
+  """Rows of head dims that are no multiple of 32 are stored in two ways, by head dim and size of the output: 4 batch elements in one
+  call (above the 128 MiB where that changes at 40, 48 and 80) and each alone (below) give the same bits, the last query tile cut."""
+  B, H, sq, skv = 4, 20, {40: 22_001, 48: 18_001}.get(D, 11_001), 77
+  gen = torch.Generator(device=dev).manual_seed(D)
+  q, k, v = (torch.randn((B, s, H * D), generator=gen, device=dev).to(torch.bfloat16) for s in (sq, skv, skv))
+  keep = torch.rand((B, skv), generator=gen, device=dev) < 0.7 if masked else None
+  out = ops.flash_attention(q, k, v, scale=D**-0.5, heads=H, keep=keep)
+  ref = [ops.flash_attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], scale=D**-0.5, heads=H, keep=None if keep is None else keep[b:b + 1]) for b in range(B)]
+  assert torch.equal(out, torch.cat(ref))
+  rows = torch.tensor([0, 31, 32, 127, 128, sq - 2, sq - 1], device=dev)
+  split = lambda x: x.float().view(B, -1, H, D).transpose(1, 2)
+  logits = split(q[:, rows]) @ split(k).transpose(2, 3).contiguous() * D**-0.5
+  if masked:
+    logits = logits.masked_fill(~keep[:, None, None], -float("inf"))
+  exact = (logits.softmax(-1) @ split(v)).transpose(1, 2).reshape(B, -1, H * D)
+  assert (out[:, rows].float() - exact).abs().max() <= 2.0**-6 * exact.abs().max()  # P and the output in bf16: 2^-8 each, and the products' own
